@@ -165,6 +165,7 @@ int mlel_hip_conv2d(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const m
     MLEL_TRY(check_conv("conv2d", out, in, weights, bias, attr));
     int rc = try_conv2d_i8_direct(ctx, (hipStream_t)stream, out, in, weights, bias, attr, nullptr);
     if (rc == 0) rc = try_conv2d_i8_mfma(ctx, (hipStream_t)stream, out, in, weights, bias, attr, nullptr);
+    if (rc == 0) rc = try_conv2d_float(ctx, (hipStream_t)stream, out, in, weights, bias, attr, nullptr, nullptr);
     if (rc != 0) return rc < 0 ? rc : 0;
     return conv2d_generic_launch((hipStream_t)stream, out, in, weights, bias, attr);
 }
@@ -192,6 +193,7 @@ int mlel_hip_matmul(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const m
                  "matmul: integer/float mismatch between operands and output");
     int rc = try_matmul_i8_mfma(ctx, (hipStream_t)stream, out, a, b, attr, nullptr);
     if (rc == 0) rc = try_matmul_f16_mfma(ctx, (hipStream_t)stream, out, a, b, attr);
+    if (rc == 0) rc = try_matmul_float(ctx, (hipStream_t)stream, out, a, b, attr);
     if (rc != 0) return rc < 0 ? rc : 0;
     return matmul_generic_launch((hipStream_t)stream, out, a, b, attr);
 }

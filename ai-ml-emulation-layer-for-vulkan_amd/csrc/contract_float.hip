@@ -1,0 +1,608 @@
+// Floating-point contractions on the matrix cores: CONV2D (NHWC x OHWI, fp32 accumulator) over fp16, bf16 and fp32
+// tensors, and MATMUL over the same types with an fp32 result, for whatever extents and alignment gemm_f16.hip does not
+// take (reference arithmetic: conv2d.comp:40-116, matmul.comp:30-73; the order of the fp32 additions differs from the
+// shaders' sequential loops, the operands and the accumulator keep their types).
+//
+// One kernel body.  out[m][n] = sum_k X[m][k] * W[n][k]; k runs over 16-byte pieces (eight 16-bit or four 32-bit
+// elements), and a piece of X lies inside one tap of the convolution.  A block keeps stages of BKB bytes of K for its
+// BM rows and BN columns in shared memory, as pieces in XOR-swizzled slots (piece p of row r in slot
+// p ^ ((r >> SH) & mask), so that the sixteen lanes an LDS cycle serves meet sixteen different 16-byte banks), and every
+// type reads the same 128-bit operands: one v_mfma_f32_32x32x16 per piece pair for 16-bit types, four
+// v_mfma_f32_32x32x2_f32 for fp32 (the K order inside a piece pair is permuted alike on both sides).
+//   DIRECT: every piece is 16-byte aligned: buffer loads straight into shared memory, S stages deep, one barrier per
+//           stage.  A lane carries the (tap, channel) position of its piece along K, so that padding, strides, dilation
+//           and channel counts that are no multiple of a stage cost a few vector instructions and no second pass.
+//   else:   pieces are assembled in registers (unaligned rows, a K-major W, channel counts such as 3) and stored into
+//           two stage buffers; the next stage's loads are in flight while one is multiplied.
+// Small problems: with one tile of 64 x 64 per compute unit nothing but the stage depth hides the trip to memory, so the
+// tile shrinks to 32 x 32 and the four wavefronts of a block share a stage's K instead of its rows (WK = 4), summed
+// through shared memory at the end -- no exchange between blocks.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+#include "dispatch.hpp"
+
+namespace mlel {
+namespace {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kOob = 0x80000000u;
+
+struct BF16 {};  // tag: bf16 storage
+
+template <typename T> struct Elem;  // size, decode, encode of a storage type
+template <> struct Elem<_Float16> {
+    static constexpr int size = 2;
+    static __device__ __forceinline__ float get(uint32_t bits) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits); }
+    static __device__ __forceinline__ uint32_t put(float v, bool) {
+        return __half_as_ushort(f2h(v));
+    }
+};
+template <> struct Elem<BF16> {
+    static constexpr int size = 2;
+    static __device__ __forceinline__ float get(uint32_t bits) { return decode_bf16((uint16_t)bits); }
+    static __device__ __forceinline__ uint32_t put(float v, bool nearest) {
+        return nearest ? encode_bf16_rne(v) : encode_bf16_trunc(v);
+    }
+};
+template <> struct Elem<float> {
+    static constexpr int size = 4;
+    static __device__ __forceinline__ float get(uint32_t bits) { return __uint_as_float(bits); }
+    static __device__ __forceinline__ uint32_t put(float v, bool) { return __float_as_uint(v); }
+};
+
+struct FArgs {
+    const char *x, *w;
+    const char *bias, *res;  // of the output's type; res: of the output's shape and layout, or null
+    char *out;
+    int32_t M, N, K;                    // K in elements
+    int32_t tiles_m, tiles_n, total_tiles, chunk;
+    DivMagic div_per_batch, div_tiles_n, div_ohw, div_ow;
+    // X: row m is output position (image, oy, ox) of a convolution (a product: one "image" of M positions, one tap)
+    int32_t IC, KW, KH, H, W, sy, sx, pt, pl, dy, dx, OHW, OW;
+    uint32_t x_img, x_row, x_pix, x_bytes;  // byte strides and extent of one batch
+    // W: row-wise [N][K] with a pitch of ldw, or (w_kmajor) [K][N] with a pitch of ldw
+    uint32_t ldw, w_bytes;
+    int64_t x_batch, w_batch, o_batch;
+    uint32_t ldo, o_bytes;
+    int32_t bias_len;
+    int32_t wide_out;  // rows of the result in whole aligned 16-byte pieces
+    int32_t has_clamp, clamp_nan_ignore;
+    float clamp_lo, clamp_hi;
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ v4i rsrc_words(const void *p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
+}
+__device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const v4i v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+    return make_uint4((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w);
+}
+template <int SIZE>
+__device__ __forceinline__ uint32_t load_elem(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    if constexpr (SIZE == 2) return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0);
+    else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
+}
+// one wavefront-wide 16-byte-per-lane load straight into shared memory at lds_addr + 16 * lane; a lane whose offset lies
+// beyond the resource's extent leaves zeros.  The loop counts these loads itself (s_waitcnt vmcnt(N)).
+__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res)
+                 : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+template <typename T>
+__device__ __forceinline__ v16f multiply(uint4 w, uint4 x, v16f acc) {
+    if constexpr (std::is_same<T, _Float16>::value) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), acc, 0, 0, 0);
+    } else if constexpr (std::is_same<T, BF16>::value) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, w), __builtin_bit_cast(v8b, x), acc, 0, 0, 0);
+    } else {
+        const v4f a = __builtin_bit_cast(v4f, w), b = __builtin_bit_cast(v4f, x);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], acc, 0, 0, 0);
+        return acc;
+    }
+}
+
+// how a register-staged operand is fetched
+enum { F_PIECES = 0,   // aligned 16-byte pieces
+       F_ELEMS = 1,    // element by element along K
+       F_KMAJOR = 2 }; // W only: element by element down a column of [K][N] (consecutive lanes: consecutive columns)
+
+// T: operand type, TO: result type; BM x BN tile; WM x WN x WK wavefronts over rows, columns and the K of a stage
+template <typename T, typename TO, int BM, int BN, int WM, int WN, int WK, int BKB, int S, bool DIRECT, int XF, int WF>
+__global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const FArgs g) {
+    constexpr int NT = 64 * WM * WN * WK, E = 16 / Elem<T>::size, SZ = Elem<T>::size, SO = Elem<TO>::size;
+    constexpr int PPR = BKB / 16, SH = BKB == 64 ? 2 : (BKB == 128 ? 1 : 0);
+    constexpr int KK = BKB / 32, KKW = KK / WK;  // piece pairs per stage, and per wavefront
+    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+    constexpr int XI = BM * PPR / NT, WI = BN * PPR / NT, STAGE = (BM + BN) * BKB;
+    static_assert((BM * PPR) % NT == 0 && (BN * PPR) % NT == 0 && KK % WK == 0 && TM >= 1 && TN >= 1, "tile shape");
+    static_assert((NT / PPR) % 16 == 0, "the rows of one thread share their swizzle");
+    extern __shared__ __align__(16) char smem[];
+
+    const int lin = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % 8u) * g.chunk + (int)(blockIdx.x / 8u));
+    if (lin >= g.total_tiles) return;
+    const int batch = div_magic(lin, g.div_per_batch);
+    const int t_in = lin - batch * (g.tiles_m * g.tiles_n);
+    const int tile_m = div_magic(t_in, g.div_tiles_n), tile_n = t_in - tile_m * g.tiles_n;
+    const int m_base = tile_m * BM, n_base = tile_n * BN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_k = wave % WK, wave_n = (wave / WK) % WN, wave_m = wave / (WK * WN);
+
+    // ---- this thread's pieces: rows r0 + i * NT / PPR of X and of W, the same piece p of each (the swizzle repeats)
+    const int r0 = tid / PPR, p0 = (tid % PPR) ^ ((r0 >> SH) & (PPR - 1));
+    int32_t xb[XI], iy0[XI], ix0[XI];
+#pragma unroll
+    for (int i = 0; i < XI; i++) {
+        const int m = m_base + r0 + i * (NT / PPR);
+        const int img = div_magic(m, g.div_ohw), pos = m - img * g.OHW;
+        const int oy = div_magic(pos, g.div_ow), ox = pos - oy * g.OW;
+        iy0[i] = m < g.M ? oy * g.sy - g.pt : -0x40000000;
+        ix0[i] = ox * g.sx - g.pl;
+        xb[i] = (int32_t)((uint32_t)img * g.x_img + (uint32_t)(oy * g.sy - g.pt) * g.x_row + (uint32_t)ix0[i] * g.x_pix);
+    }
+    // position along K of this thread's piece in the stage that is fetched next: element kpos = tap * IC + ic
+    int kpos = p0 * E, ic = kpos, ky = 0, kx = 0;
+    auto wrap = [&](int &c, int &y, int &x) {
+        while (c >= g.IC && y < g.KH) {
+            c -= g.IC;
+            if (++x == g.KW) x = 0, y++;
+        }
+    };
+    wrap(ic, ky, kx);
+    auto tap_off = [&](int i, int c, int y, int x) {  // offset of channel c of a tap of row i, or beyond the extent
+        const int iy = iy0[i] + y * g.dy, ix = ix0[i] + x * g.dx;
+        const bool in = (uint32_t)iy < (uint32_t)g.H && (uint32_t)ix < (uint32_t)g.W && y < g.KH;
+        return in ? (uint32_t)xb[i] + (uint32_t)(y * g.dy) * g.x_row + (uint32_t)(x * g.dx) * g.x_pix + (uint32_t)(c * SZ) : kOob;
+    };
+    auto step_on = [&]() {
+        kpos += PPR * E;
+        ic += PPR * E;
+        wrap(ic, ky, kx);
+    };
+    const int n0 = n_base + r0;
+
+    v16f acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+
+    const int h = lane >> 5, lrow = lane & 31;
+    auto compute = [&](const char *st) {  // multiplies this wavefront's share of a stage
+#pragma unroll
+        for (int k = 0; k < KKW; k++) {
+            const int slot = (((wave_k * KKW + k) * 2 + h) ^ ((lrow >> SH) & (PPR - 1))) * 16;
+            uint4 xf[TM], wf[TN];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+                xf[i] = *reinterpret_cast<const uint4 *>(st + ((wave_m * TM + i) * 32 + lrow) * BKB + slot);
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                wf[j] = *reinterpret_cast<const uint4 *>(st + BM * BKB + ((wave_n * TN + j) * 32 + lrow) * BKB + slot);
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = multiply<T>(wf[j], xf[i], acc[i][j]);
+        }
+    };
+
+    const int nk = (g.K + PPR * E - 1) / (PPR * E);
+    const char *xp = g.x + (int64_t)batch * g.x_batch, *wp = g.w + (int64_t)batch * g.w_batch;
+    if constexpr (DIRECT) {
+        constexpr int NLA = XI + WI;
+        const v4i xres = rsrc_words(xp, g.x_bytes), wres = rsrc_words(wp, g.w_bytes);
+        const uint32_t lds0 =
+            (uint32_t) reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem) + (uint32_t)(wave * 1024);
+        auto request = [&](int buf) {  // the next stage into buffer `buf`; beyond K every lane fetches zeros
+            const uint32_t d = lds0 + (uint32_t)(buf * STAGE);
+#pragma unroll
+            for (int i = 0; i < XI; i++) load16_to_lds(xres, d + i * NT * 16, tap_off(i, ic, ky, kx));
+#pragma unroll
+            for (int i = 0; i < WI; i++) {
+                const int n = n0 + i * (NT / PPR);
+                load16_to_lds(wres, d + BM * BKB + i * NT * 16,
+                              n < g.N && kpos < g.K ? (uint32_t)n * g.ldw + (uint32_t)(kpos * SZ) : kOob);
+            }
+            step_on();
+        };
+#pragma unroll
+        for (int d = 0; d < S - 1; d++) request(d);
+        int cur = 0, nxt = S - 1;
+        for (int step = 0; step < nk; step++) {
+            // at most S - 2 stages outstanding: this thread's part of stage `step` has landed; the barrier extends that
+            // to the block, and says that every wavefront is done with the buffer the next request overwrites
+            wait_vmcnt<(S - 2) * NLA>();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            request(nxt);
+            compute(smem + cur * STAGE);
+            cur = cur + 1 == S ? 0 : cur + 1;
+            nxt = nxt + 1 == S ? 0 : nxt + 1;
+        }
+        wait_vmcnt<0>();  // requests beyond the last stage write (zeros) into the ring, which the epilogue reuses
+        __syncthreads();
+    } else {
+        const __amdgpu_buffer_rsrc_t xres = rsrc(xp, g.x_bytes), wres = rsrc(wp, g.w_bytes);
+        // W of a K-major operand: consecutive lanes hold consecutive columns, so that a column walk is coalesced
+        constexpr bool KM = WF == F_KMAJOR;
+        const int wn = KM ? tid % BN : r0, wpiece = KM ? tid / BN : 0;
+        constexpr int WSTEP = KM ? NT / BN : 0;  // pieces between two of this thread's pieces of one column
+        static_assert(!KM || NT % BN == 0 || BN % NT == 0, "columns per thread");
+        uint4 xr[XI], wr[WI];
+        auto pack = [](const uint32_t *v) {
+            if constexpr (SZ == 2)
+                return make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+            else
+                return make_uint4(v[0], v[1], v[2], v[3]);
+        };
+        int kstage = 0;  // first element of the stage that is fetched next
+        auto fetch = [&]() {
+#pragma unroll
+            for (int i = 0; i < XI; i++) {
+                if constexpr (XF == F_PIECES) {
+                    xr[i] = load16(xres, tap_off(i, ic, ky, kx));
+                } else {
+                    uint32_t v[E];
+                    int c = ic, y = ky, x = kx;
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        v[e] = load_elem<SZ>(xres, tap_off(i, c, y, x));
+                        c++;
+                        if (c == g.IC) {
+                            c = 0;
+                            if (++x == g.KW) x = 0, y++;
+                        }
+                    }
+                    xr[i] = pack(v);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < WI; i++) {
+                if constexpr (KM) {
+                    const int n = n_base + wn, k = kstage + (wpiece + i * WSTEP) * E;
+                    uint32_t v[E];
+#pragma unroll
+                    for (int e = 0; e < E; e++)
+                        v[e] = load_elem<SZ>(wres, n < g.N && k + e < g.K ? (uint32_t)(k + e) * g.ldw + (uint32_t)(n * SZ) : kOob);
+                    wr[i] = pack(v);
+                } else {
+                    const int n = n0 + i * (NT / PPR);
+                    const uint32_t off = (uint32_t)n * g.ldw + (uint32_t)(kpos * SZ);
+                    if constexpr (WF == F_PIECES) {
+                        wr[i] = load16(wres, n < g.N && kpos < g.K ? off : kOob);
+                    } else {
+                        uint32_t v[E];
+#pragma unroll
+                        for (int e = 0; e < E; e++) v[e] = load_elem<SZ>(wres, n < g.N && kpos + e < g.K ? off + e * SZ : kOob);
+                        wr[i] = pack(v);
+                    }
+                }
+            }
+            step_on();
+            kstage += PPR * E;
+        };
+        auto store = [&](char *st) {
+#pragma unroll
+            for (int i = 0; i < XI; i++) *reinterpret_cast<uint4 *>(st + (i * NT + tid) * 16) = xr[i];
+#pragma unroll
+            for (int i = 0; i < WI; i++) {
+                if constexpr (KM) {
+                    const int p = wpiece + i * WSTEP;
+                    *reinterpret_cast<uint4 *>(st + BM * BKB + wn * BKB + ((p ^ ((wn >> SH) & (PPR - 1))) * 16)) = wr[i];
+                } else {
+                    *reinterpret_cast<uint4 *>(st + BM * BKB + (i * NT + tid) * 16) = wr[i];
+                }
+            }
+        };
+        fetch();
+        store(smem);
+        if (nk > 1) fetch();
+        __syncthreads();
+        for (int step = 0; step < nk; step++) {
+            // (the barrier below closes the step that read the buffer stored to here)
+            if (step + 1 < nk) {
+                store(smem + ((step + 1) & 1) * STAGE);
+                if (step + 2 < nk) fetch();
+            }
+            compute(smem + (step & 1) * STAGE);
+            __syncthreads();
+        }
+    }
+
+    // ---- the K shares of a block's wavefronts, added in ascending order of K
+    if constexpr (WK > 1) {
+        float *red = reinterpret_cast<float *>(smem);
+        if (wave_k > 0) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        red[((((wave_k - 1) * WM * WN + wave / WK) * TM * TN + i * TN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+        }
+        __syncthreads();
+        if (wave_k == 0) {
+#pragma unroll
+            for (int s = 0; s < WK - 1; s++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++)
+                            acc[i][j][r] += red[(((s * WM * WN + wave / WK) * TM * TN + i * TN + j) * 16 + r) * 64 + lane];
+        }
+        __syncthreads();
+    }
+
+    // ---- bias and rounding, then through shared memory: a lane holds row m = lane % 32 of a sub-tile and, per register
+    // quad q, columns 8q + 4 * (lane / 32) ..; the stores below write whole runs of a row
+    constexpr int OP = BN * SO + 16;
+    const __amdgpu_buffer_rsrc_t bres = rsrc(g.bias, g.bias != nullptr ? (uint32_t)(g.bias_len * SO) : 0u);
+    if (WK == 1 || wave_k == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            float b[16];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int n = n_base + (wave_n * TN + j) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                b[r] = Elem<TO>::get(load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)(n * SO)));
+            }
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                char *row = smem + ((wave_m * TM + i) * 32 + lrow) * OP + ((wave_n * TN + j) * 32 + 4 * h) * SO;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    uint32_t v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        float s = acc[i][j][4 * q + e];
+                        if (g.bias != nullptr) s += b[4 * q + e];  // uniform (-0 + 0 would lose its sign)
+                        v[e] = Elem<TO>::put(s, false);
+                    }
+                    if constexpr (SO == 2)
+                        *reinterpret_cast<uint2 *>(row + 8 * q * SO) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+                    else
+                        *reinterpret_cast<uint4 *>(row + 8 * q * SO) = make_uint4(v[0], v[1], v[2], v[3]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t ores = rsrc(g.out + (int64_t)batch * g.o_batch, g.o_bytes);
+    const __amdgpu_buffer_rsrc_t rres = rsrc(g.res, g.res != nullptr ? g.o_bytes : 0u);
+    // ADD of the residual (one rounding, to nearest) and CLAMP, as the stand-alone operators compute them
+    auto finish = [&](uint32_t bits, uint32_t res_bits) {
+        if (g.res != nullptr) bits = Elem<TO>::put(Elem<TO>::get(bits) + Elem<TO>::get(res_bits), true);
+        if (g.has_clamp) {
+            float v = Elem<TO>::get(bits);
+            if (v != v && g.clamp_nan_ignore) v = g.clamp_lo;
+            if (v < g.clamp_lo) v = g.clamp_lo;
+            if (v > g.clamp_hi) v = g.clamp_hi;
+            bits = Elem<TO>::put(v, false);
+        }
+        return bits;
+    };
+    if (g.wide_out) {  // uniform
+        constexpr int OPPR = BN * SO / 16, EO = 16 / SO;
+        constexpr int NP = (BM * OPPR + NT - 1) / NT;
+        uint32_t off[NP];
+        uint4 res[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int p = i * NT + tid, m = m_base + p / OPPR, n = n_base + (p % OPPR) * EO;
+            off[i] = p < BM * OPPR && m < g.M && n < g.N ? (uint32_t)m * g.ldo + (uint32_t)(n * SO) : kOob;
+            res[i] = make_uint4(0, 0, 0, 0);
+        }
+        if (g.res != nullptr) {
+#pragma unroll
+            for (int i = 0; i < NP; i++) res[i] = load16(rres, off[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int p = i * NT + tid;
+            if (BM * OPPR % NT != 0 && p >= BM * OPPR) break;
+            uint4 v = *reinterpret_cast<const uint4 *>(smem + (p / OPPR) * OP + (p % OPPR) * 16);
+            if (g.res != nullptr || g.has_clamp) {
+                uint32_t *w = reinterpret_cast<uint32_t *>(&v);
+                const uint32_t *rw = reinterpret_cast<const uint32_t *>(&res[i]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if constexpr (SO == 2)
+                        w[e] = finish(w[e] & 0xffffu, rw[e] & 0xffffu) | (finish(w[e] >> 16, rw[e] >> 16) << 16);
+                    else
+                        w[e] = finish(w[e], rw[e]);
+                }
+            }
+            const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            __builtin_amdgcn_raw_buffer_store_b128(d, ores, (int)off[i], 0, kOutAux);
+        }
+    } else {
+        for (int p = tid; p < BM * BN; p += NT) {
+            const int r = p / BN, c = p % BN, m = m_base + r, n = n_base + c;
+            if (m >= g.M || n >= g.N) continue;
+            const uint32_t off = (uint32_t)m * g.ldo + (uint32_t)(n * SO);
+            uint32_t v;
+            if constexpr (SO == 2) v = *reinterpret_cast<const uint16_t *>(smem + r * OP + c * SO);
+            else v = *reinterpret_cast<const uint32_t *>(smem + r * OP + c * SO);
+            v = finish(v, g.res != nullptr ? load_elem<SO>(rres, off) : 0u);
+            if constexpr (SO == 2) __builtin_amdgcn_raw_buffer_store_b16((short)v, ores, (int)off, 0, kOutAux);
+            else __builtin_amdgcn_raw_buffer_store_b32((int)v, ores, (int)off, 0, kOutAux);
+        }
+    }
+}
+
+template <typename T, typename TO, int BM, int BN, int WM, int WN, int WK, int BKB, int S, bool DIRECT, int XF, int WF>
+int launch_tile(FArgs &g, int64_t batches, hipStream_t s) {
+    constexpr int SO = Elem<TO>::size;
+    constexpr size_t operands = (size_t)S * (BM + BN) * BKB, result = (size_t)BM * (BN * SO + 16);
+    constexpr size_t shares = (size_t)(WK - 1) * BM * BN * 4;
+    constexpr size_t sm = std::max(operands, std::max(result, shares));
+    static_assert(sm <= 160 * 1024, "shared memory of a compute unit");
+    g.tiles_m = (g.M + BM - 1) / BM;
+    g.tiles_n = (g.N + BN - 1) / BN;
+    const int64_t total = (int64_t)g.tiles_m * g.tiles_n * batches;
+    MLEL_REQUIRE(total < (int64_t(1) << 30), MLEL_ERR_LIMIT, "contraction: %lld tiles", (long long)total);
+    g.total_tiles = (int)total;
+    g.chunk = (int)((total + 7) / 8);
+    g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
+    g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
+    auto kernel = contract_float_kernel<T, TO, BM, BN, WM, WN, WK, BKB, S, DIRECT, XF, WF>;
+    static const bool raised = sm <= 48 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) == hipSuccess;
+    (void)raised;
+    kernel<<<dim3((unsigned)(g.chunk * 8)), dim3(64 * WM * WN * WK), sm, s>>>(g);
+    MLEL_TRY(check_launch("floating-point contraction"));
+    return 1;
+}
+
+// Tile choice.  128 x 128 from two tiles per compute unit on; 64 x 64 from half a tile per compute unit on; below that
+// 32 x 32 with the wavefronts sharing K.
+template <typename T, typename TO, bool DIRECT, int XF, int WF>
+int launch_shape(mlel_ctx *ctx, FArgs &g, int64_t batches, hipStream_t s) {
+    const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+    auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batches; };
+    constexpr int S2 = DIRECT ? 3 : 2;
+    if constexpr (DIRECT) {
+        if (tiles(128, 128) >= 2 * cus && g.N > 64) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 4, DIRECT, XF, WF>(g, batches, s);
+    }
+    if (tiles(64, 64) * 2 >= cus) return launch_tile<T, TO, 64, 64, 2, 2, 1, 128, S2, DIRECT, XF, WF>(g, batches, s);
+    return launch_tile<T, TO, 32, 32, 1, 1, 4, 256, S2, DIRECT, XF, WF>(g, batches, s);
+}
+
+// `pieces`: both operands in aligned 16-byte pieces along K
+template <typename T>
+int launch_conv(mlel_ctx *ctx, FArgs &g, bool pieces, hipStream_t s) {
+    return pieces ? launch_shape<T, T, true, F_PIECES, F_PIECES>(ctx, g, 1, s)
+                  : launch_shape<T, T, false, F_ELEMS, F_ELEMS>(ctx, g, 1, s);
+}
+template <typename T>
+int launch_product(mlel_ctx *ctx, FArgs &g, int64_t batches, bool x_pieces, bool w_pieces, bool w_kmajor, hipStream_t s) {
+    if (x_pieces && w_pieces) return launch_shape<T, float, true, F_PIECES, F_PIECES>(ctx, g, batches, s);
+    if (!w_kmajor) return launch_shape<T, float, false, F_ELEMS, F_ELEMS>(ctx, g, batches, s);
+    return x_pieces ? launch_shape<T, float, false, F_PIECES, F_KMAJOR>(ctx, g, batches, s)
+                    : launch_shape<T, float, false, F_ELEMS, F_KMAJOR>(ctx, g, batches, s);
+}
+
+bool aligned16(const void *p, std::initializer_list<int64_t> strides) {
+    if (((uintptr_t)p % 16) != 0) return false;
+    for (int64_t v : strides)
+        if (v % 16 != 0) return false;
+    return true;
+}
+constexpr int64_t kLim = (int64_t(1) << 31) - 4096;
+
+}  // namespace
+
+// CONV2D with an fp32 accumulator, optionally followed by the ADD of a residual of the output's shape and by a CLAMP
+// (each computed as the stand-alone operator would).  Returns 1 when launched, 0 to decline.
+int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
+                     const mlel_tensor *bias, const mlel_conv2d_attr *a, const mlel_tensor *residual,
+                     const mlel_clamp_attr *clamp) {
+    const int dt = in->dtype;
+    if ((dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32) || w->dtype != dt || out->dtype != dt ||
+        a->acc_type != MLEL_ACC_F32 || a->input_zp != 0 || a->weight_zp != 0)
+        return 0;
+    if (!is_packed(in) || !is_packed(w) || !is_packed(out) || !is_packed(bias)) return 0;
+    const int64_t sz = dt_size(dt), N = in->dims[0], H = in->dims[1], W = in->dims[2], IC = in->dims[3];
+    const int64_t OC = w->dims[0], KH = w->dims[1], KW = w->dims[2], OH = out->dims[1], OW = out->dims[2];
+    if (w->dims[3] != IC || out->dims[0] != N || out->dims[3] != OC) return 0;
+    if (N <= 0 || H <= 0 || W <= 0 || IC <= 0 || OC <= 0 || KH <= 0 || KW <= 0 || OH <= 0 || OW <= 0) return 0;
+    if (bias->dims[0] != 1 && bias->dims[0] < OC) return 0;
+    if (a->stride[0] <= 0 || a->stride[1] <= 0 || a->dilation[0] <= 0 || a->dilation[1] <= 0) return 0;
+    const int64_t K = KH * KW * IC, M = N * OH * OW, small = 1 << 20;
+    if (N * H * W * IC * sz >= kLim || OC * K * sz >= kLim || M * OC * sz >= kLim || K >= (1 << 24) || M >= (1 << 30)) return 0;
+    // coordinates and taps stay far inside 31 bits
+    if (H >= small || W >= small || OH >= small || OW >= small || KH >= 4096 || KW >= 4096 || a->stride[0] >= 1024 ||
+        a->stride[1] >= 1024 || a->dilation[0] >= 1024 || a->dilation[1] >= 1024)
+        return 0;
+    for (int i = 0; i < 4; i++)
+        if (a->pad[i] < -small || a->pad[i] > small) return 0;
+    if (residual != nullptr && (residual->dtype != dt || !is_packed(residual) || !same_shape(residual, out))) return 0;
+    FArgs g{};
+    g.x = static_cast<const char *>(in->ptr), g.w = static_cast<const char *>(w->ptr);
+    g.bias = static_cast<const char *>(bias->ptr), g.out = static_cast<char *>(out->ptr);
+    g.res = residual != nullptr ? static_cast<const char *>(residual->ptr) : nullptr;
+    g.M = (int)M, g.N = (int)OC, g.K = (int)K;
+    g.IC = (int)IC, g.KW = (int)KW, g.KH = (int)KH, g.H = (int)H, g.W = (int)W;
+    g.sy = a->stride[0], g.sx = a->stride[1], g.pt = a->pad[0], g.pl = a->pad[2], g.dy = a->dilation[0], g.dx = a->dilation[1];
+    g.OHW = (int)(OH * OW), g.OW = (int)OW;
+    g.div_ohw = make_div_magic((uint32_t)g.OHW), g.div_ow = make_div_magic((uint32_t)g.OW);
+    g.x_pix = (uint32_t)(IC * sz), g.x_row = (uint32_t)(W * IC * sz), g.x_img = (uint32_t)(H * W * IC * sz);
+    g.x_bytes = (uint32_t)(N * H * W * IC * sz), g.w_bytes = (uint32_t)(OC * K * sz), g.ldw = (uint32_t)(K * sz);
+    g.ldo = (uint32_t)(OC * sz), g.o_bytes = (uint32_t)(M * OC * sz);
+    g.bias_len = bias->dims[0] == 1 ? 1 : (int)OC;
+    const bool pieces = aligned16(in->ptr, {IC * sz}) && aligned16(w->ptr, {IC * sz});
+    g.wide_out = aligned16(out->ptr, {OC * sz}) && (residual == nullptr || aligned16(residual->ptr, {}));
+    if (clamp != nullptr) {
+        g.has_clamp = 1, g.clamp_nan_ignore = clamp->nan_mode == MLEL_NAN_IGNORE;
+        g.clamp_lo = (float)clamp->min_val, g.clamp_hi = (float)clamp->max_val;
+        if (dt == MLEL_F16) g.clamp_lo = (float)(_Float16)g.clamp_lo, g.clamp_hi = (float)(_Float16)g.clamp_hi;
+    }
+    if (dt == MLEL_F16) return launch_conv<_Float16>(ctx, g, pieces, s);
+    if (dt == MLEL_BF16) return launch_conv<BF16>(ctx, g, pieces, s);
+    return launch_conv<float>(ctx, g, pieces, s);
+}
+
+// MATMUL over fp16, bf16 or fp32 operands with an fp32 result.  Returns 1 when launched, 0 to decline.
+int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
+                     const mlel_matmul_attr *attr) {
+    const int dt = a->dtype;
+    if ((dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32) || b->dtype != dt || out->dtype != MLEL_F32 || attr->a_zp != 0 ||
+        attr->b_zp != 0)
+        return 0;
+    const int64_t sz = dt_size(dt), NB = out->dims[0], M = out->dims[1], N = out->dims[2], K = a->dims[2];
+    // (a contraction shorter than one matrix instruction is mostly padding there)
+    if (NB <= 0 || M <= 0 || N <= 0 || K < 16) return 0;
+    if (a->dims[0] < NB || b->dims[0] < NB || a->dims[1] < M || b->dims[1] < K || b->dims[2] < N) return 0;
+    if (a->strides[2] != sz || out->strides[2] != 4 || a->strides[1] < K * sz || out->strides[1] < N * 4) return 0;
+    const bool rows = K > 1 && b->strides[1] == sz && b->strides[2] >= b->dims[1] * sz;
+    if (!rows && (b->strides[2] != sz || b->strides[1] < N * sz)) return 0;
+    for (const mlel_tensor *t : {out, a, b})
+        for (int i = 0; i < 3; i++)
+            if (t->strides[i] < 0 || t->strides[i] % dt_size(t->dtype) != 0) return 0;
+    const int64_t ldw = rows ? b->strides[2] : b->strides[1];
+    if (M * a->strides[1] >= kLim || (rows ? N : K) * ldw >= kLim || M * out->strides[1] >= kLim || K >= (1 << 24) ||
+        M >= (1 << 30) || N >= (1 << 30))
+        return 0;
+    FArgs g{};
+    g.x = static_cast<const char *>(a->ptr), g.w = static_cast<const char *>(b->ptr), g.out = static_cast<char *>(out->ptr);
+    g.M = (int)M, g.N = (int)N, g.K = (int)K;
+    g.IC = (int)K, g.KW = g.KH = 1, g.H = 1, g.W = (int)M, g.sy = g.sx = g.dy = g.dx = 1;
+    g.OHW = g.OW = (int)M;
+    g.div_ohw = make_div_magic((uint32_t)g.OHW), g.div_ow = make_div_magic((uint32_t)g.OW);
+    g.x_pix = (uint32_t)a->strides[1];
+    g.x_bytes = (uint32_t)((M - 1) * a->strides[1] + K * sz);
+    g.ldw = (uint32_t)ldw;
+    g.w_bytes = (uint32_t)(((rows ? N : K) - 1) * ldw + (rows ? K : N) * sz);
+    g.ldo = (uint32_t)out->strides[1], g.o_bytes = (uint32_t)((M - 1) * out->strides[1] + N * 4);
+    g.x_batch = a->strides[0], g.w_batch = b->strides[0], g.o_batch = out->strides[0];
+    const bool xp = aligned16(a->ptr, {a->strides[0], a->strides[1], K * sz});
+    const bool wp = rows && aligned16(b->ptr, {b->strides[0], ldw, K * sz});
+    g.wide_out = aligned16(out->ptr, {out->strides[0], out->strides[1], N * 4});
+    if (dt == MLEL_F16) return launch_product<_Float16>(ctx, g, NB, xp, wp, !rows, s);
+    if (dt == MLEL_BF16) return launch_product<BF16>(ctx, g, NB, xp, wp, !rows, s);
+    return launch_product<float>(ctx, g, NB, xp, wp, !rows, s);
+}
+
+}  // namespace mlel

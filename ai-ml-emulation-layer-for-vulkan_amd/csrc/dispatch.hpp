@@ -129,6 +129,14 @@ bool chain_is_gelu_tanh(const mlel_chain *chain);
 int try_matmul_f16_group(mlel_ctx *ctx, hipStream_t s, int n, const mlel_tensor *const *outs, const mlel_tensor *a,
                          const mlel_tensor *const *bs, const mlel_tensor *const *biases, const mlel_matmul_attr *attr);
 
+// ---- CONV2D and MATMUL over fp16, bf16 and fp32 tensors (contract_float.hip) ----
+// `residual` (of the output's type and shape) and `clamp` may be null: ADD and CLAMP behind the convolution
+int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
+                     const mlel_tensor *bias, const mlel_conv2d_attr *a, const mlel_tensor *residual,
+                     const mlel_clamp_attr *clamp);
+int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
+                     const mlel_matmul_attr *attr);
+
 // ---- 1x1 CONV2D + RESCALE (+CLAMP) and 3x3 DEPTHWISE_CONV2D + RESCALE (+CLAMP) in one launch (conv_dw_i8.hip) ----
 // 1 when taken (with `launch` false: when the extents, types and strides are covered; pointers are not looked at)
 int try_conv2d_dwconv_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in,
