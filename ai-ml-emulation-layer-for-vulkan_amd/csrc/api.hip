@@ -480,6 +480,8 @@ int mlel_hip_transpose_conv2d(mlel_ctx *ctx, void *stream, const mlel_tensor *ou
     MLEL_REQUIRE(attr->stride[0] > 0 && attr->stride[1] > 0, MLEL_ERR_INVALID, "transpose_conv2d: stride must be positive");
     MLEL_REQUIRE(attr->acc_type >= MLEL_ACC_I32 && attr->acc_type <= MLEL_ACC_I64, MLEL_ERR_INVALID,
                  "Unsupported acc type %u", attr->acc_type);
+    const int rc = try_tconv2d_i8(ctx, (hipStream_t)stream, out, in, weights, bias, attr, nullptr);
+    if (rc != 0) return rc < 0 ? rc : 0;
     return tconv2d_launch((hipStream_t)stream, out, in, weights, bias, attr);
 }
 

@@ -113,6 +113,14 @@ int try_conv2d_i8_direct(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, c
 int try_matmul_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a,
                        const mlel_tensor *b, const mlel_matmul_attr *attr, const FusedEpilogue *epi);
 
+// ---- int8 contractions over ragged rows and TRANSPOSE_CONV2D (contract_i8.hip) ----
+int try_conv2d_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
+                         const mlel_tensor *bias, const mlel_conv2d_attr *a, const FusedEpilogue *epi);
+int try_tconv2d_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
+                   const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi);
+int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
+                         const mlel_matmul_attr *attr, const FusedEpilogue *epi);
+
 // ---- fp16 MFMA MATMUL with fp32 result (gemm_f16.hip) ----
 // `residual`: an fp16 tensor of the output's shape added to the fused form's fp16 result (a second, fp16 ADD)
 int try_matmul_f16_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a,

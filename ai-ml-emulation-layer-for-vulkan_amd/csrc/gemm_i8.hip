@@ -16,7 +16,9 @@ struct SplitScratch {
     bool from_ctx = true;  // look the workspace up in the context when a split is wanted
 };
 
-int launch_gemm(mlel_ctx *ctx, hipStream_t s, GemmArgs &g, const SplitScratch &scratch) {
+// `ragged`: tried first when no fetch mode of aligned pieces applies (contract_i8.hip); returns 1 when it launched
+template <typename Ragged>
+int launch_gemm(mlel_ctx *ctx, hipStream_t s, GemmArgs &g, const SplitScratch &scratch, const Ragged &ragged) {
     // operand fetch modes
     int xmode = X_GENERIC, wmode = W_GENERIC;
     const bool small = g.x_bytes != 0 && g.w_bytes != 0;  // both operand extents fit 31-bit buffer offsets
@@ -36,6 +38,8 @@ int launch_gemm(mlel_ctx *ctx, hipStream_t s, GemmArgs &g, const SplitScratch &s
                       (xmode == X_PLAIN && (wmode == W_KMAJOR || wmode == W_KMAJOR4)) ||
                       (xmode == X_PLAIN4 && wmode == W_ROWS4);
     if (!fast) {
+        const int rc = ragged();
+        if (rc != 0) return rc < 0 ? rc : 0;
         xmode = X_GENERIC;
         wmode = W_GENERIC;
     }
@@ -278,7 +282,7 @@ int try_conv2d_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
         sc.counters = static_scratch->counters;
         sc.partial_bytes = static_scratch->partial_bytes;
     }
-    MLEL_TRY(launch_gemm(ctx, s, g, sc));
+    MLEL_TRY(launch_gemm(ctx, s, g, sc, [&] { return try_conv2d_i8_ragged(ctx, s, out, in, w, bias, a, epi); }));
     if (static_scratch != nullptr && static_scratch->used_split != nullptr) *static_scratch->used_split = g.splits > 1;
     return 1;
 }
@@ -346,7 +350,7 @@ int try_matmul_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
             return 1;
         }
     }
-    MLEL_TRY(launch_gemm(ctx, s, g, SplitScratch{}));
+    MLEL_TRY(launch_gemm(ctx, s, g, SplitScratch{}, [&] { return try_matmul_i8_ragged(ctx, s, out, A, B, attr, epi); }));
     return 1;
 }
 
