@@ -265,6 +265,10 @@ FUSED_SIGNATURES = {
     "elementwise_chain": [_T, C.POINTER(Chain)],
     "matmul_bias_cast_chain": [_T, _T, _T, _T, C.POINTER(MatmulAttr), C.POINTER(Chain)],
     "attention_f16": [_T, _T, _T, _T, C.POINTER(Chain)],
+    "conv2d_add_clamp": [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, C.POINTER(ClampAttr)],
+    "transpose_conv2d_rescale_clamp": [_T, _T, _T, _T, C.POINTER(Tconv2dAttr), C.POINTER(Epilogue)],
+    "concat_conv2d_rescale_clamp": [_T, _T, _T, _T, _T, C.POINTER(Conv2dAttr), C.POINTER(Epilogue)],
+    "resize_rescale": [_T, _T, C.POINTER(ResizeAttr), C.POINTER(Epilogue), C.c_int32],
     "rescale_add_rescale": [_T, _T, C.POINTER(Epilogue), _T, C.POINTER(Epilogue), C.POINTER(Epilogue)],
 }
 
@@ -308,6 +312,10 @@ RUNTIME_SIGNATURES = {
                                                    C.POINTER(Conv2dAttr)]),
     "mlel_hip_conv2d_conv2d_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, _T,
                                                    C.POINTER(Conv2dAttr)]),
+    "mlel_hip_conv2d_add_clamp_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T]),
+    "mlel_hip_transpose_conv2d_rescale_clamp_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Tconv2dAttr)]),
+    "mlel_hip_concat_conv2d_in_kernel": (C.c_int, [_T, _T, _T, _T, _T, C.POINTER(Conv2dAttr)]),
+    "mlel_hip_resize_rescale_in_kernel": (C.c_int, [_T, _T, C.POINTER(ResizeAttr), C.c_int32]),
     "mlel_hip_conv2d_avgpool_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), C.c_int32,
                                                     C.POINTER(Pool2dAttr)]),
 }

@@ -433,6 +433,8 @@ int mlel_hip_argmax(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const m
     MLEL_TRY(check_supported(in, "argmax in"));
     MLEL_REQUIRE((int)axis < in->rank && out->rank == in->rank - 1 && out->dtype == MLEL_I32, MLEL_ERR_INVALID,
                  "argmax: the output is int32 with the axis removed");
+    const int rc = try_argmax_rows((hipStream_t)stream, out, in, axis, nan_mode);
+    if (rc != 0) return rc < 0 ? rc : 0;
     return argmax_launch((hipStream_t)stream, out, in, axis, nan_mode);
 }
 
@@ -548,6 +550,8 @@ int mlel_hip_resize(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const m
     MLEL_REQUIRE(attr->scale[0] > 0 && attr->scale[2] > 0, MLEL_ERR_INVALID, "resize: scale numerators must be positive");
     MLEL_REQUIRE(attr->mode == MLEL_RESIZE_NEAREST || attr->mode == MLEL_RESIZE_BILINEAR, MLEL_ERR_INVALID,
                  "resize: mode %u", attr->mode);
+    const int rc = try_resize_i8((hipStream_t)stream, out, in, attr, nullptr);
+    if (rc != 0) return rc < 0 ? rc : 0;
     return resize_launch((hipStream_t)stream, out, in, attr);
 }
 
@@ -1168,6 +1172,96 @@ int mlel_hip_conv2d_avgpool_in_kernel(const mlel_tensor *out, const mlel_tensor 
     if (!conv_result_like(&mid, in, weights, attr, conv_dtype, nullptr)) return 0;
     const FusedEpilogue unused{};  // the requantisation constants do not decide whether the kernel takes the case
     return try_conv2d_avgpool_cols(nullptr, out, &mid, in, weights, bias, attr, &unused, pool, true) == 1 ? 1 : 0;
+}
+
+// ---- fused forms without a fallback: MLEL_ERR_UNSUPPORTED where the *_in_kernel query answers 0 ----
+
+int mlel_hip_conv2d_add_clamp_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *weights,
+                                        const mlel_tensor *bias, const mlel_conv2d_attr *attr, const mlel_tensor *residual) {
+    if (out == nullptr || in == nullptr || weights == nullptr || bias == nullptr || attr == nullptr) return 0;
+    if (out->rank != 4 || in->rank != 4 || weights->rank != 4 || bias->rank != 1 || bias->dtype != out->dtype) return 0;
+    return try_conv2d_float(nullptr, nullptr, out, in, weights, bias, attr, residual, nullptr, true) == 1 ? 1 : 0;
+}
+
+int mlel_hip_conv2d_add_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                              const mlel_tensor *weights, const mlel_tensor *bias, const mlel_conv2d_attr *attr,
+                              const mlel_tensor *residual, const mlel_clamp_attr *clamp) {
+    MLEL_TRY(require_ctx(ctx, "conv2d_add_clamp"));
+    MLEL_TRY(check_conv("conv2d_add_clamp", out, in, weights, bias, attr));
+    if (residual != nullptr) MLEL_TRY(check_tensor(residual, "conv2d_add_clamp residual"));
+    const int rc = try_conv2d_float(ctx, (hipStream_t)stream, out, in, weights, bias, attr, residual, clamp);
+    if (rc != 0) return rc < 0 ? rc : 0;
+    return set_error(MLEL_ERR_UNSUPPORTED, "conv2d_add_clamp: not a case of the one-launch kernel");
+}
+
+int mlel_hip_transpose_conv2d_rescale_clamp_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *weights,
+                                                      const mlel_tensor *bias, const mlel_tconv2d_attr *attr) {
+    if (out == nullptr || in == nullptr || weights == nullptr || bias == nullptr || attr == nullptr) return 0;
+    if (out->rank != 4 || in->rank != 4 || weights->rank != 4 || bias->rank != 1) return 0;
+    const FusedEpilogue unused{};
+    return try_tconv2d_i8(nullptr, nullptr, out, in, weights, bias, attr, &unused, true) == 1 ? 1 : 0;
+}
+
+int mlel_hip_transpose_conv2d_rescale_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                                            const mlel_tensor *weights, const mlel_tensor *bias,
+                                            const mlel_tconv2d_attr *attr, const mlel_epilogue *epi) {
+    MLEL_TRY(require_ctx(ctx, "transpose_conv2d_rescale_clamp"));
+    MLEL_REQUIRE(attr != nullptr, MLEL_ERR_INVALID, "transpose_conv2d_rescale_clamp: null attribute");
+    for (const mlel_tensor *t : {out, in, weights, bias}) MLEL_TRY(check_supported(t, "transpose_conv2d_rescale_clamp"));
+    MLEL_REQUIRE(out->rank == 4 && in->rank == 4 && weights->rank == 4 && bias->rank == 1, MLEL_ERR_INVALID,
+                 "transpose_conv2d_rescale_clamp: ranks must be 4,4,4,1");
+    FusedEpilogue fe;
+    MLEL_TRY(make_epilogue(epi, MLEL_I32, out, out->dims[3], &fe));
+    const int rc = try_tconv2d_i8(ctx, (hipStream_t)stream, out, in, weights, bias, attr, &fe);
+    if (rc != 0) return rc < 0 ? rc : 0;
+    return set_error(MLEL_ERR_UNSUPPORTED, "transpose_conv2d_rescale_clamp: not a case of the one-launch kernel");
+}
+
+int mlel_hip_concat_conv2d_in_kernel(const mlel_tensor *out, const mlel_tensor *in1, const mlel_tensor *in2,
+                                     const mlel_tensor *weights, const mlel_tensor *bias, const mlel_conv2d_attr *attr) {
+    if (out == nullptr || in1 == nullptr || in2 == nullptr || weights == nullptr || bias == nullptr || attr == nullptr) return 0;
+    if (out->rank != 4 || in1->rank != 4 || in2->rank != 4 || weights->rank != 4 || bias->rank != 1) return 0;
+    const FusedEpilogue unused{};
+    return try_conv2d_i8_ragged(nullptr, nullptr, out, in1, weights, bias, attr, &unused, in2, true) == 1 ? 1 : 0;
+}
+
+int mlel_hip_concat_conv2d_rescale_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in1,
+                                         const mlel_tensor *in2, const mlel_tensor *weights, const mlel_tensor *bias,
+                                         const mlel_conv2d_attr *attr, const mlel_epilogue *epi) {
+    MLEL_TRY(require_ctx(ctx, "concat_conv2d_rescale_clamp"));
+    MLEL_REQUIRE(out != nullptr && attr != nullptr, MLEL_ERR_INVALID, "concat_conv2d_rescale_clamp: null argument");
+    MLEL_TRY(check_tensor(out, "concat_conv2d_rescale_clamp out"));
+    MLEL_TRY(check_supported(in2, "concat_conv2d_rescale_clamp in2"));
+    MLEL_REQUIRE(in2->rank == 4, MLEL_ERR_INVALID, "concat_conv2d_rescale_clamp: rank of the second input");
+    mlel_tensor acc_view = packed_like(out, MLEL_I32, out->ptr);
+    MLEL_TRY(check_conv("concat_conv2d_rescale_clamp", &acc_view, in1, weights, bias, attr));
+    FusedEpilogue fe;
+    MLEL_TRY(make_epilogue(epi, MLEL_I32, out, out->dims[3], &fe));
+    const int rc = try_conv2d_i8_ragged(ctx, (hipStream_t)stream, out, in1, weights, bias, attr, &fe, in2);
+    if (rc != 0) return rc < 0 ? rc : 0;
+    return set_error(MLEL_ERR_UNSUPPORTED, "concat_conv2d_rescale_clamp: not a case of the one-launch kernel");
+}
+
+int mlel_hip_resize_rescale_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *attr, int32_t argmax) {
+    if (out == nullptr || in == nullptr || attr == nullptr || in->rank != 4 || out->rank != (argmax ? 3 : 4)) return 0;
+    return (argmax ? try_resize_argmax_i8(nullptr, out, in, attr, nullptr, true) : try_resize_i8(nullptr, out, in, attr, nullptr, true)) == 1 ? 1 : 0;
+}
+
+int mlel_hip_resize_rescale(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                            const mlel_resize_attr *attr, const mlel_epilogue *epi, int32_t argmax) {
+    MLEL_TRY(require_ctx(ctx, "resize_rescale"));
+    MLEL_REQUIRE(attr != nullptr, MLEL_ERR_INVALID, "resize_rescale: null attribute");
+    MLEL_TRY(check_supported(out, "resize_rescale out"));
+    MLEL_TRY(check_supported(in, "resize_rescale in"));
+    MLEL_REQUIRE(in->rank == 4 && out->rank == (argmax ? 3 : 4), MLEL_ERR_INVALID, "resize_rescale: ranks");
+    mlel_tensor image = *in;  // the type the RESCALE has: the labels of an ARGMAX are int32 whatever it was
+    image.dtype = MLEL_I8;
+    FusedEpilogue fe;
+    MLEL_TRY(make_epilogue(epi, MLEL_I32, argmax ? &image : out, 1, &fe));
+    const int rc = argmax ? try_resize_argmax_i8((hipStream_t)stream, out, in, attr, &fe)
+                          : try_resize_i8((hipStream_t)stream, out, in, attr, &fe);
+    if (rc != 0) return rc < 0 ? rc : 0;
+    return set_error(MLEL_ERR_UNSUPPORTED, "resize_rescale: not a case of the one-launch kernel");
 }
 
 int mlel_hip_rescale_add_rescale(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in1,

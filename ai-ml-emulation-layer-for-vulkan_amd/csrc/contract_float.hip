@@ -515,10 +515,11 @@ constexpr int64_t kLim = (int64_t(1) << 31) - 4096;
 }  // namespace
 
 // CONV2D with an fp32 accumulator, optionally followed by the ADD of a residual of the output's shape and by a CLAMP
-// (each computed as the stand-alone operator would).  Returns 1 when launched, 0 to decline.
+// (each computed as the stand-alone operator would).  Returns 1 when launched (`probe`: when types and extents are covered;
+// pointers are not looked at), 0 to decline.
 int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
                      const mlel_tensor *bias, const mlel_conv2d_attr *a, const mlel_tensor *residual,
-                     const mlel_clamp_attr *clamp) {
+                     const mlel_clamp_attr *clamp, bool probe) {
     const int dt = in->dtype;
     if ((dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32) || w->dtype != dt || out->dtype != dt ||
         a->acc_type != MLEL_ACC_F32 || a->input_zp != 0 || a->weight_zp != 0)
@@ -539,6 +540,7 @@ int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     for (int i = 0; i < 4; i++)
         if (a->pad[i] < -small || a->pad[i] > small) return 0;
     if (residual != nullptr && (residual->dtype != dt || !is_packed(residual) || !same_shape(residual, out))) return 0;
+    if (probe) return 1;
     FArgs g{};
     g.x = static_cast<const char *>(in->ptr), g.w = static_cast<const char *>(w->ptr);
     g.bias = static_cast<const char *>(bias->ptr), g.out = static_cast<char *>(out->ptr);

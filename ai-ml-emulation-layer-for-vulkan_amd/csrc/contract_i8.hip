@@ -27,7 +27,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 struct IArgs {
-    const int8_t *x, *w;
+    const int8_t *x, *x2, *w;           // x2: the second operand of a CONCAT along the channels, or null
     char *out;
     const int32_t *bias;  // or null
     int32_t bias_len;
@@ -36,11 +36,11 @@ struct IArgs {
     DivMagic div_phase, div_per_batch, div_tiles_n, div_ohw, div_ow;
     // row m of a phase: image, y', x'; its taps (jy, jx), jy < taps_y, read input row y' * sy + base_y + jy * dy.
     // CONV2D has one phase (phase_y = phase_x = 1); TRANSPOSE_CONV2D has sy x sx, of unit stride and dy = dx = -1
-    int32_t IC, KH, KW, H, W, OHW, OW;  // OHW, OW: positions of a phase per image and per row
+    int32_t IC, IC1, KH, KW, H, W, OHW, OW;  // OHW, OW: positions of a phase per image and per row; IC1: channels of x
     int32_t sy, sx, pt, pl, dy, dx, phase_y, phase_x;
     int32_t out_h, out_w;               // extents of the output image
     int64_t x_batch, w_batch, o_batch;
-    uint32_t x_img, x_row, x_pix, x_bytes, ldw, w_bytes;
+    uint32_t x_pix, x_bytes, x2_bytes, ldw, w_bytes;  // x_pix: bytes from one position of x to the next
     int32_t zx, zw;
     const char *mult;
     const int8_t *shift;
@@ -89,8 +89,9 @@ __device__ __forceinline__ int32_t sum_bytes(uint4 v, int32_t acc) {
 }
 
 // SO: bytes of a result (1: requantised int8 / uint8, 4: the int32 accumulator, or the requantised int32);
-// XC: bytes per chunk; KM: W is [K][N] (a product), else rows of K
-template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM>
+// XC: bytes per chunk; KM: W is [K][N] (a product), else rows of K; DUAL: X is two tensors side by side along the channels
+// (CONCAT read in place: a tap's chunks are those of the first tensor, then those of the second)
+template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM, bool DUAL>
 __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IArgs g) {
     constexpr int NT = 64 * WM * WN * WK;
     constexpr int PPR = BKB / 16, SH = BKB == 64 ? 2 : (BKB == 128 ? 1 : 0);
@@ -132,13 +133,14 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     }
     const int taps = taps_y * taps_x;
     constexpr int CP = 16 / XC;                // chunks per piece
-    const int cpt = (g.IC + XC - 1) / XC;      // chunks per tap
+    const int cpt1 = DUAL ? (g.IC1 + XC - 1) / XC : (g.IC + XC - 1) / XC;
+    const int cpt = DUAL ? cpt1 + (g.IC - g.IC1 + XC - 1) / XC : cpt1;  // chunks per tap
     const int n_chunks = taps * cpt;
     const int nk = (n_chunks + PPR * CP - 1) / (PPR * CP);
 
     const int r0 = tid / PPR, p0 = (tid % PPR) ^ ((r0 >> SH) & (PPR - 1));
     const int8_t *xp = g.x + (int64_t)batch * g.x_batch, *wp = g.w + (int64_t)batch * g.w_batch;
-    int32_t xb[XI], iy0[XI], ix0[XI];
+    int32_t xb[XI], iy0[XI], ix0[XI];  // xb: index of the position the first tap meets
 #pragma unroll
     for (int i = 0; i < XI; i++) {
         const int m = m_base + r0 + i * (NT / PPR);
@@ -146,7 +148,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
         const int y = div_magic(pos, g.div_ow), x = pos - y * g.OW;
         iy0[i] = m < g.M ? y * g.sy + by : -0x40000000;
         ix0[i] = x * g.sx + bx;
-        xb[i] = (int32_t)((uint32_t)img * g.x_img + (uint32_t)(y * g.sy + by) * g.x_row + (uint32_t)ix0[i] * g.x_pix);
+        xb[i] = (img * g.H + y * g.sy + by) * g.W + ix0[i];
     }
     if (tid < BM + BN) sums[tid] = 0;
     if (BM + BN > NT && tid + NT < BM + BN) sums[tid + NT] = 0;
@@ -176,7 +178,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     };
     wrap(cq, jy, jx);
     const uint32_t zx4 = (uint32_t)(uint8_t)g.zx * 0x01010101u;
-    const bool tail = g.IC % XC != 0;          // a tap's last chunk holds bytes of its neighbour
+    // a tap's last chunk holds bytes of its neighbour
+    const bool tail = DUAL ? (g.IC1 % XC != 0 || (g.IC - g.IC1) % XC != 0) : g.IC % XC != 0;
     const bool mask_x = tail && g.zw != 0;     // they count only where the weights' zero point does
 
     v16i acc[TM][TN];
@@ -190,6 +193,14 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     // ---- fetch: X pieces and W pieces of the next stage into one of two register sets
     const int wq = tid % (BN / 4), wpc = tid / (BN / 4);  // K-major: column group and piece of this thread
     int kbase = 0;                                        // K-major: first k of the stage
+    // chunk c of a tap: bytes of it that are channels, and its place among the weights of the tap
+    auto remaining = [&](int c) { return DUAL ? (c < cpt1 ? g.IC1 - c * XC : g.IC - g.IC1 - (c - cpt1) * XC) : g.IC - c * XC; };
+    auto channel = [&](int c) { return DUAL && c >= cpt1 ? g.IC1 + (c - cpt1) * XC : c * XC; };
+    auto load_x = [&](int pix, int c) {
+        if (DUAL && c >= cpt1)
+            return load_chunk<XC>(g.x2, (uint32_t)pix * (uint32_t)(g.IC - g.IC1) + (uint32_t)((c - cpt1) * XC), g.x2_bytes);
+        return load_chunk<XC>(xp, (uint32_t)pix * g.x_pix + (uint32_t)(c * XC), g.x_bytes);
+    };
     auto fetch = [&](uint4(&xr)[XI], uint4(&wr)[WI]) {
         const bool live = jy < taps_y && taps_x > 0;
 #pragma unroll
@@ -199,10 +210,10 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
                 const uint32_t fill = live ? zx4 : 0u;  // (nothing beyond K, where the sums of rows end too)
                 uint4 v = make_uint4(fill, fill, fill, fill);
                 if (live && (uint32_t)iy < (uint32_t)g.H && (uint32_t)ix < (uint32_t)g.W) {
-                    v = load_chunk<16>(xp, (uint32_t)xb[i] + (uint32_t)(jy * g.dy) * g.x_row + (uint32_t)(jx * g.dx) * g.x_pix + (uint32_t)(cq * 16), g.x_bytes);
+                    v = load_x(xb[i] + jy * g.dy * g.W + jx * g.dx, cq);
                 }
                 if (mask_x) {  // uniform
-                    const int rem = g.IC - cq * 16;
+                    const int rem = remaining(cq);
                     v = make_uint4(keep_bytes(v.x, rem), keep_bytes(v.y, rem - 4), keep_bytes(v.z, rem - 8), keep_bytes(v.w, rem - 12));
                 }
                 xr[i] = v;
@@ -214,8 +225,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
                     const int iy = iy0[i] + y * g.dy, ix = ix0[i] + x * g.dx;
                     v[e] = y < taps_y ? zx4 : 0u;
                     if (y < taps_y && (uint32_t)iy < (uint32_t)g.H && (uint32_t)ix < (uint32_t)g.W)
-                        v[e] = load_chunk<4>(xp, (uint32_t)xb[i] + (uint32_t)(y * g.dy) * g.x_row + (uint32_t)(x * g.dx) * g.x_pix + (uint32_t)(c * 4), g.x_bytes).x;
-                    if (mask_x) v[e] = keep_bytes(v[e], g.IC - c * 4);
+                        v[e] = load_x(xb[i] + y * g.dy * g.W + x * g.dx, c).x;
+                    if (mask_x) v[e] = keep_bytes(v[e], remaining(c));
                     if (++c == cpt) {
                         c = 0;
                         if (++x == taps_x) x = 0, y++;
@@ -249,9 +260,9 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
                 if constexpr (XC == 16) {
                     uint4 v = make_uint4(0, 0, 0, 0);
                     if (in && live)
-                        v = load_chunk<16>(wp, row + (uint32_t)(((ky0 + jy * g.phase_y) * g.KW + kx0 + jx * g.phase_x) * g.IC + cq * 16), g.w_bytes);
+                        v = load_chunk<16>(wp, row + (uint32_t)(((ky0 + jy * g.phase_y) * g.KW + kx0 + jx * g.phase_x) * g.IC + channel(cq)), g.w_bytes);
                     if (tail) {  // uniform
-                        const int rem = g.IC - cq * 16;
+                        const int rem = remaining(cq);
                         v = make_uint4(keep_bytes(v.x, rem), keep_bytes(v.y, rem - 4), keep_bytes(v.z, rem - 8), keep_bytes(v.w, rem - 12));
                     }
                     wr[i] = v;
@@ -262,8 +273,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
                     for (int e = 0; e < 4; e++) {
                         v[e] = 0;
                         if (in && y < taps_y)
-                            v[e] = load_chunk<4>(wp, row + (uint32_t)(((ky0 + y * g.phase_y) * g.KW + kx0 + x * g.phase_x) * g.IC + c * 4), g.w_bytes).x;
-                        if (tail) v[e] = keep_bytes(v[e], g.IC - c * 4);
+                            v[e] = load_chunk<4>(wp, row + (uint32_t)(((ky0 + y * g.phase_y) * g.KW + kx0 + x * g.phase_x) * g.IC + channel(c)), g.w_bytes).x;
+                        if (tail) v[e] = keep_bytes(v[e], remaining(c));
                         if (++c == cpt) {
                             c = 0;
                             if (++x == taps_x) x = 0, y++;
@@ -485,7 +496,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     }
 }
 
-template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM>
+template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM, bool DUAL>
 int launch_tile(IArgs &g, hipStream_t s) {
     constexpr size_t operands = (size_t)2 * (BM + BN) * BKB, result = (size_t)BM * (BN * SO + 16);
     constexpr size_t sm = operands + (BM + BN) * 4 + BN * 32;
@@ -500,7 +511,7 @@ int launch_tile(IArgs &g, hipStream_t s) {
     g.div_phase = make_div_magic((uint32_t)per_phase);
     g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
     g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
-    auto kernel = contract_i8_kernel<FUSED, SO, BM, BN, WM, WN, WK, BKB, XC, KM>;
+    auto kernel = contract_i8_kernel<FUSED, SO, BM, BN, WM, WN, WK, BKB, XC, KM, DUAL>;
     static const bool raised = sm <= 48 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) == hipSuccess;
     (void)raised;
@@ -511,19 +522,21 @@ int launch_tile(IArgs &g, hipStream_t s) {
 
 // Tile choice: 32 columns when N fits them, else 64; from half a tile per compute unit on four wavefronts share the rows,
 // below that they share K over a 32 x 32 tile.
-template <bool FUSED, int SO, int XC, bool KM>
+template <bool FUSED, int SO, int XC, bool KM, bool DUAL>
 int launch_shape(mlel_ctx *ctx, IArgs &g, hipStream_t s) {
     const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
     const int64_t phases = (int64_t)g.phase_y * g.phase_x * g.batches;
     auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * phases; };
-    if (g.N <= 32 && tiles(128, 32) * 2 >= cus) return launch_tile<FUSED, SO, 128, 32, 4, 1, 1, 128, XC, KM>(g, s);
-    if (g.N > 32 && tiles(64, 64) * 2 >= cus) return launch_tile<FUSED, SO, 64, 64, 2, 2, 1, 128, XC, KM>(g, s);
-    return launch_tile<FUSED, SO, 32, 32, 1, 1, 4, 256, XC, KM>(g, s);
+    if (g.N <= 32 && tiles(128, 32) * 2 >= cus) return launch_tile<FUSED, SO, 128, 32, 4, 1, 1, 128, XC, KM, DUAL>(g, s);
+    if (g.N > 32 && tiles(64, 64) * 2 >= cus) return launch_tile<FUSED, SO, 64, 64, 2, 2, 1, 128, XC, KM, DUAL>(g, s);
+    return launch_tile<FUSED, SO, 32, 32, 1, 1, 4, 256, XC, KM, DUAL>(g, s);
 }
 
 template <int XC, bool KM>
 int launch_out(mlel_ctx *ctx, IArgs &g, bool fused, hipStream_t s) {
-    return fused ? launch_shape<true, 1, XC, KM>(ctx, g, s) : launch_shape<false, 4, XC, KM>(ctx, g, s);
+    if constexpr (!KM)
+        if (g.x2 != nullptr) return launch_shape<true, 1, XC, false, true>(ctx, g, s);
+    return fused ? launch_shape<true, 1, XC, KM, false>(ctx, g, s) : launch_shape<false, 4, XC, KM, false>(ctx, g, s);
 }
 
 constexpr int64_t kLim = (int64_t(1) << 31) - 4096;
@@ -538,30 +551,36 @@ bool fill_epilogue(IArgs &g, const mlel_tensor *out, const FusedEpilogue *epi) {
     return true;
 }
 
-// CONV2D (out_pad null) or TRANSPOSE_CONV2D described by the same record
-int try_conv(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
-             const mlel_tensor *bias, const FusedEpilogue *epi, uint32_t acc_type, int32_t zx, int32_t zw,
-             const int32_t *pad, const int32_t *stride, const int32_t *dilation, bool transposed) {
+// CONV2D (over `in`, or over `in` and `in2` side by side along the channels) or TRANSPOSE_CONV2D; `probe`: judge types and
+// extents only
+int try_conv(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *in2,
+             const mlel_tensor *w, const mlel_tensor *bias, const FusedEpilogue *epi, uint32_t acc_type, int32_t zx, int32_t zw,
+             const int32_t *pad, const int32_t *stride, const int32_t *dilation, bool transposed, bool probe) {
     if (in->dtype != MLEL_I8 || w->dtype != MLEL_I8 || bias->dtype != MLEL_I32 || acc_type != MLEL_ACC_I32) return 0;
     IArgs g{};
-    if (!fill_epilogue(g, out, epi)) return 0;
+    if (probe ? dt_size(out->dtype) != 1 : !fill_epilogue(g, out, epi)) return 0;
     if (zx < -128 || zx > 127 || zw < -128 || zw > 127) return 0;
     if (!is_packed(in) || !is_packed(w) || !is_packed(out) || !is_packed(bias)) return 0;
-    const int64_t N = in->dims[0], H = in->dims[1], W = in->dims[2], IC = in->dims[3];
+    const int64_t N = in->dims[0], H = in->dims[1], W = in->dims[2], IC1 = in->dims[3], IC = IC1 + (in2 ? in2->dims[3] : 0);
+    if (in2 != nullptr && (in2->dtype != MLEL_I8 || !is_packed(in2) || in2->dims[0] != N || in2->dims[1] != H || in2->dims[2] != W ||
+                           epi == nullptr || in2->dims[3] <= 0 || N * H * W * in2->dims[3] < 16))
+        return 0;
     const int64_t OC = w->dims[0], KH = w->dims[1], KW = w->dims[2], OH = out->dims[1], OW = out->dims[2], small = 1 << 20;
     if (w->dims[3] != IC || out->dims[0] != N || out->dims[3] != OC) return 0;
-    if (N <= 0 || H <= 0 || W <= 0 || IC <= 0 || OC <= 0 || KH <= 0 || KW <= 0 || OH <= 0 || OW <= 0) return 0;
+    if (N <= 0 || H <= 0 || W <= 0 || IC1 <= 0 || OC <= 0 || KH <= 0 || KW <= 0 || OH <= 0 || OW <= 0) return 0;
     if (bias->dims[0] != 1 && bias->dims[0] < OC) return 0;
-    if (N * H * W * IC >= kLim || OC * KH * KW * IC >= kLim || N * H * W * IC < 16 || OC * KH * KW * IC < 16) return 0;
+    if (N * H * W * IC >= kLim || OC * KH * KW * IC >= kLim || N * H * W * IC1 < 16 || OC * KH * KW * IC < 16) return 0;
     if (N * OH * OW >= (int64_t(1) << 30) || H >= small || W >= small || OH >= small || OW >= small || KH >= 4096 || KW >= 4096) return 0;
     for (int i = 0; i < 2; i++)
         if (stride[i] <= 0 || stride[i] >= 1024 || dilation[i] <= 0 || dilation[i] >= 1024) return 0;
     for (int i = 0; i < 4; i++)
         if (pad[i] < -small || pad[i] > small) return 0;
+    if (probe) return 1;
     g.x = static_cast<const int8_t *>(in->ptr), g.w = static_cast<const int8_t *>(w->ptr);
+    if (in2 != nullptr) g.x2 = static_cast<const int8_t *>(in2->ptr), g.x2_bytes = (uint32_t)(N * H * W * in2->dims[3]);
     g.out = static_cast<char *>(out->ptr), g.bias = static_cast<const int32_t *>(bias->ptr), g.bias_len = (int)bias->dims[0];
     g.N = (int)OC, g.batches = 1;
-    g.IC = (int)IC, g.KH = (int)KH, g.KW = (int)KW, g.H = (int)H, g.W = (int)W;
+    g.IC = (int)IC, g.IC1 = (int)IC1, g.KH = (int)KH, g.KW = (int)KW, g.H = (int)H, g.W = (int)W;
     g.pt = pad[0], g.pl = pad[2];
     g.out_h = (int)OH, g.out_w = (int)OW;
     int64_t ph = OH, pw = OW;
@@ -573,25 +592,29 @@ int try_conv(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_te
     }
     g.M = (int)(N * ph * pw), g.OHW = (int)(ph * pw), g.OW = (int)pw;
     g.div_ohw = make_div_magic((uint32_t)g.OHW), g.div_ow = make_div_magic((uint32_t)g.OW);
-    g.x_pix = (uint32_t)IC, g.x_row = (uint32_t)(W * IC), g.x_img = (uint32_t)(H * W * IC);
-    g.x_bytes = (uint32_t)(N * H * W * IC), g.ldw = (uint32_t)(KH * KW * IC), g.w_bytes = (uint32_t)(OC * KH * KW * IC);
+    g.x_pix = (uint32_t)IC1;
+    g.x_bytes = (uint32_t)(N * H * W * IC1), g.ldw = (uint32_t)(KH * KW * IC), g.w_bytes = (uint32_t)(OC * KH * KW * IC);
     g.zx = zx, g.zw = zw;
     // chunks of 16 bytes where they waste less than a quarter of the loads' width, dwords for fewer channels
-    const bool wide = ((IC + 15) / 16) * 16 * 4 <= ((IC + 3) / 4) * 4 * 5;
+    const auto fetched = [&](int64_t c) { return (IC1 + c - 1) / c * c + (IC - IC1 + c - 1) / c * c; };
+    const bool wide = fetched(16) * 4 <= fetched(4) * 5;
     return wide ? launch_out<16, false>(ctx, g, epi != nullptr, s) : launch_out<4, false>(ctx, g, epi != nullptr, s);
 }
 
 }  // namespace
 
 int try_conv2d_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
-                         const mlel_tensor *bias, const mlel_conv2d_attr *a, const FusedEpilogue *epi) {
-    return try_conv(ctx, s, out, in, w, bias, epi, a->acc_type, a->input_zp, a->weight_zp, a->pad, a->stride, a->dilation, false);
+                         const mlel_tensor *bias, const mlel_conv2d_attr *a, const FusedEpilogue *epi, const mlel_tensor *in2,
+                         bool probe) {
+    return try_conv(ctx, s, out, in, in2, w, bias, epi, a->acc_type, a->input_zp, a->weight_zp, a->pad, a->stride, a->dilation,
+                    false, probe);
 }
 
 int try_tconv2d_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
-                   const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi) {
+                   const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi, bool probe) {
     const int32_t unit[2] = {1, 1};
-    return try_conv(ctx, s, out, in, w, bias, epi, a->acc_type, a->input_zp, a->weight_zp, a->out_pad, a->stride, unit, true);
+    return try_conv(ctx, s, out, in, nullptr, w, bias, epi, a->acc_type, a->input_zp, a->weight_zp, a->out_pad, a->stride, unit,
+                    true, probe);
 }
 
 int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
@@ -612,7 +635,7 @@ int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, c
     if (xb >= kLim || wb >= kLim || xb < 16 || wb < 16 || M * N * 4 >= kLim || NB >= (1 << 20)) return 0;
     g.x = static_cast<const int8_t *>(a->ptr), g.w = static_cast<const int8_t *>(b->ptr), g.out = static_cast<char *>(out->ptr);
     g.M = (int)M, g.N = (int)N, g.batches = (int)NB;
-    g.IC = (int)K, g.KH = g.KW = 1, g.H = 1, g.W = (int)M, g.OHW = g.OW = (int)M;
+    g.IC = g.IC1 = (int)K, g.KH = g.KW = 1, g.H = 1, g.W = (int)M, g.OHW = g.OW = (int)M;
     g.sy = g.sx = g.dy = g.dx = g.phase_y = g.phase_x = 1, g.out_h = 1, g.out_w = (int)M;
     g.div_ohw = make_div_magic((uint32_t)M), g.div_ow = make_div_magic((uint32_t)M);
     g.x_batch = a->strides[0], g.w_batch = b->strides[0], g.o_batch = out->strides[0];

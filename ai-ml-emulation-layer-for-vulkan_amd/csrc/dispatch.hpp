@@ -114,10 +114,13 @@ int try_matmul_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
                        const mlel_tensor *b, const mlel_matmul_attr *attr, const FusedEpilogue *epi);
 
 // ---- int8 contractions over ragged rows and TRANSPOSE_CONV2D (contract_i8.hip) ----
+// `in2`: the second operand of a CONCAT along the channels, read in place (fused form only); `probe`: judge types and
+// extents only (the epilogue's constants do not decide)
 int try_conv2d_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
-                         const mlel_tensor *bias, const mlel_conv2d_attr *a, const FusedEpilogue *epi);
+                         const mlel_tensor *bias, const mlel_conv2d_attr *a, const FusedEpilogue *epi,
+                         const mlel_tensor *in2 = nullptr, bool probe = false);
 int try_tconv2d_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
-                   const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi);
+                   const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi, bool probe = false);
 int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
                          const mlel_matmul_attr *attr, const FusedEpilogue *epi);
 
@@ -141,7 +144,7 @@ int try_matmul_f16_group(mlel_ctx *ctx, hipStream_t s, int n, const mlel_tensor 
 // `residual` (of the output's type and shape) and `clamp` may be null: ADD and CLAMP behind the convolution
 int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
                      const mlel_tensor *bias, const mlel_conv2d_attr *a, const mlel_tensor *residual,
-                     const mlel_clamp_attr *clamp);
+                     const mlel_clamp_attr *clamp, bool probe = false);
 int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
                      const mlel_matmul_attr *attr);
 
@@ -157,6 +160,14 @@ bool attention_f16_supported(const mlel_tensor *out, const mlel_tensor *q, const
                              const mlel_chain *chain);
 int try_attention_f16(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt,
                       const mlel_tensor *v, const mlel_chain *chain);
+
+// ---- RESIZE of int8 images, alone (`epi` null), with its RESCALE, and with the ARGMAX behind that; ARGMAX over rows
+// (ops_resize.hip) ----
+int try_resize_i8(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *a,
+                  const FusedEpilogue *epi, bool probe = false);
+int try_resize_argmax_i8(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *a,
+                         const FusedEpilogue *epi, bool probe = false);
+int try_argmax_rows(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, uint32_t axis, uint32_t nan_mode);
 
 // ---- floating-point elementwise / reduce specialisations (ops_float.hip) ----
 int try_binary_float_fast(mlel_ctx *ctx, hipStream_t s, int op, const mlel_tensor *out, const mlel_tensor *in1,

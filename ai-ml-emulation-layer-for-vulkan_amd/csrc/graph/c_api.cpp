@@ -292,6 +292,10 @@ std::string opLabel(const OpNode &op) {
     case OpKind::FusedConv2D: return std::string("CONV2D+RESCALE") + (op.hasClamp ? "+CLAMP" : "");
     case OpKind::FusedDepthwiseConv2D: return std::string("DEPTHWISE_CONV2D+RESCALE") + (op.hasClamp ? "+CLAMP" : "");
     case OpKind::FusedMatmul: return std::string("MATMUL+RESCALE") + (op.hasClamp ? "+CLAMP" : "");
+    case OpKind::FusedConv2DFloat: return std::string("CONV2D") + (op.flag ? "+ADD" : "") + (op.hasClamp ? "+CLAMP" : "");
+    case OpKind::FusedTransposeConv2D: return std::string("TRANSPOSE_CONV2D+RESCALE") + (op.hasClamp ? "+CLAMP" : "");
+    case OpKind::FusedConcatConv2D: return std::string("CONCAT+CONV2D+RESCALE") + (op.hasClamp ? "+CLAMP" : "");
+    case OpKind::FusedResize: return std::string("RESIZE+RESCALE") + (op.flag ? "+ARGMAX" : "");
     case OpKind::FusedRescaleAddRescale: return "RESCALE+RESCALE+ADD+RESCALE";
     case OpKind::FusedConv2DResidual:
         return std::string("CONV2D+RESCALE") + (op.hasClamp ? "+CLAMP" : "") + "+RESCALE+RESCALE+ADD+RESCALE";

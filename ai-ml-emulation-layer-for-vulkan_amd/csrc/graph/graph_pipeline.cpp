@@ -590,7 +590,7 @@ bool isSmallInt(int32_t dt) { return dt == MLEL_I8 || dt == MLEL_I16 || dt == ML
 }  // namespace
 
 void GraphPipeline::fuse() {
-    // Pattern 1: CONV2D | DEPTHWISE_CONV2D | MATMUL (int8 x int8 -> int32)  ->  RESCALE  [-> CLAMP]
+    // Pattern 1: CONV2D | DEPTHWISE_CONV2D | TRANSPOSE_CONV2D | MATMUL (int8 x int8 -> int32)  ->  RESCALE  [-> CLAMP]
     // Legal when the int32 accumulator tensor (and, for the CLAMP, the RESCALE result) is a private intermediate
     // with exactly one consumer.  The fused kernels compute exactly RESCALE(CLAMP) of the int32 accumulator, so the
     // result is bit-identical to the three operators run one after another.
@@ -598,13 +598,13 @@ void GraphPipeline::fuse() {
         OpNode &op = *opPtr;
         if (op.fusedAway) continue;
         const bool isConv = op.kind == OpKind::Conv2D, isDw = op.kind == OpKind::DepthwiseConv2D,
-                   isMm = op.kind == OpKind::Matmul;
-        if (!isConv && !isDw && !isMm) continue;
+                   isMm = op.kind == OpKind::Matmul, isTc = op.kind == OpKind::TransposeConv2D;
+        if (!isConv && !isDw && !isMm && !isTc) continue;
         const auto &acc = op.outputs[0];
         if (acc->getFormat() != MLEL_I32 || op.inputs[0]->getFormat() != MLEL_I8 ||
             op.inputs[1]->getFormat() != MLEL_I8 || !isPrivateIntermediate(*acc))
             continue;
-        if (!isMm && op.conv.acc_type != MLEL_ACC_I32) continue;
+        if (!isMm && (isTc ? op.tconv.acc_type : op.conv.acc_type) != MLEL_ACC_I32) continue;
         const auto users = consumersOf(ops, acc.get());
         if (users.size() != 1 || users[0]->kind != OpKind::Rescale || users[0]->inputs[0].get() != acc.get()) continue;
         OpNode &rs = *users[0];
@@ -612,6 +612,10 @@ void GraphPipeline::fuse() {
         if (!isSmallInt(rsOut->getFormat()) || !sameShape(*acc, *rsOut) || !rsOut->isPacked() || !scaleTensorsOk(rs) ||
             rs.rescale.input_unsigned)
             continue;
+        if (isTc) {  // one launch or none: the fused entry point has no route of its own for other operands
+            const mlel_tensor o = rsOut->view(), x = op.inputs[0]->view(), w = op.inputs[1]->view(), b = op.inputs[2]->view();
+            if (rs.rescale.input_zp != 0 || mlel_hip_transpose_conv2d_rescale_clamp_in_kernel(&o, &x, &w, &b, &op.tconv) == 0) continue;
+        }
         // optional CLAMP
         OpNode *clamp = nullptr;
         if (isPrivateIntermediate(*rsOut) && !rs.rescale.output_unsigned) {
@@ -621,7 +625,8 @@ void GraphPipeline::fuse() {
                 rsUsers[0]->outputs[0]->isPacked() && rsUsers[0]->clamp.min_val <= rsUsers[0]->clamp.max_val)
                 clamp = rsUsers[0];
         }
-        op.kind = isConv ? OpKind::FusedConv2D : (isDw ? OpKind::FusedDepthwiseConv2D : OpKind::FusedMatmul);
+        op.kind = isConv ? OpKind::FusedConv2D
+                         : (isDw ? OpKind::FusedDepthwiseConv2D : (isTc ? OpKind::FusedTransposeConv2D : OpKind::FusedMatmul));
         op.epilogue = RescaleSpec{rs.inputs[1], rs.inputs[2], rs.rescale};
         rs.fusedAway = true;
         TensorPtr finalOut = rsOut;
@@ -633,6 +638,113 @@ void GraphPipeline::fuse() {
         }
         op.outputs[0] = finalOut;
         finalOut->setProducer(&op);
+    }
+
+    // Pattern 1b (skip connection): a fused CONV2D whose image is the private result of a CONCAT of two tensors along the
+    // channels reads the two where they lie (mlel_hip_concat_conv2d_in_kernel decides); the CONCAT, one launch per operand,
+    // disappears.
+    for (const auto &opPtr : ops) {
+        OpNode &conv = *opPtr;
+        if (conv.fusedAway || conv.kind != OpKind::FusedConv2D || conv.epilogue.attr.input_zp != 0) continue;
+        const TensorPtr joined = conv.inputs[0];
+        if (!isPrivateIntermediate(*joined) || consumersOf(ops, joined.get()).size() != 1) continue;
+        std::vector<OpNode *> writers;
+        for (const auto &other : ops)
+            if (!other->fusedAway && other->outputs[0].get() == joined.get()) writers.push_back(other.get());
+        if (writers.size() != 2 || writers[0]->kind != OpKind::Concat || writers[1]->kind != OpKind::Concat) continue;
+        if (writers[0]->offset != 0) std::swap(writers[0], writers[1]);
+        const TensorPtr x1 = writers[0]->inputs[0], x2 = writers[1]->inputs[0];
+        if (joined->getRank() != 4 || x1->getRank() != 4 || x2->getRank() != 4 || writers[0]->axis != 3 || writers[1]->axis != 3 ||
+            writers[0]->offset != 0 || writers[1]->offset != static_cast<uint32_t>(x1->getDimensions()[3]) ||
+            x1->getDimensions()[3] + x2->getDimensions()[3] != joined->getDimensions()[3])
+            continue;
+        const mlel_tensor o = conv.outputs[0]->view(), a = x1->view(), b = x2->view(), w = conv.inputs[1]->view(),
+                          bias = conv.inputs[2]->view();
+        if (mlel_hip_concat_conv2d_in_kernel(&o, &a, &b, &w, &bias, &conv.conv) == 0) continue;
+        conv.kind = OpKind::FusedConcatConv2D;
+        conv.inputs = {x1, conv.inputs[1], conv.inputs[2], x2};
+        writers[0]->fusedAway = writers[1]->fusedAway = true;
+    }
+
+    // Pattern 1c: RESIZE (int8 -> int32) -> per-tensor RESCALE to int8 [-> ARGMAX over the channels], on what the one-launch
+    // kernels take (mlel_hip_resize_rescale_in_kernel decides): the int32 image never reaches memory, nor, in front of an
+    // ARGMAX, the int8 one.
+    for (const auto &opPtr : ops) {
+        OpNode &resize = *opPtr;
+        if (resize.fusedAway || resize.kind != OpKind::Resize) continue;
+        const TensorPtr wide = resize.outputs[0];
+        if (wide->getFormat() != MLEL_I32 || !isPrivateIntermediate(*wide)) continue;
+        auto users = consumersOf(ops, wide.get());
+        if (users.size() != 1 || users[0]->kind != OpKind::Rescale || users[0]->inputs[0].get() != wide.get()) continue;
+        OpNode &rs = *users[0];
+        if (rs.outputs[0]->getFormat() != MLEL_I8 || !sameShape(*wide, *rs.outputs[0]) || !scaleTensorsOk(rs) ||
+            rs.rescale.per_channel || rs.rescale.input_unsigned || rs.rescale.output_unsigned)
+            continue;
+        const mlel_tensor x = resize.inputs[0]->view(), y = rs.outputs[0]->view();
+        OpNode *argmax = nullptr;
+        if (isPrivateIntermediate(*rs.outputs[0])) {
+            users = consumersOf(ops, rs.outputs[0].get());
+            if (users.size() == 1 && users[0]->kind == OpKind::Argmax && users[0]->axis == 3) {
+                const mlel_tensor labels = users[0]->outputs[0]->view();
+                if (mlel_hip_resize_rescale_in_kernel(&labels, &x, &resize.resize, 1)) argmax = users[0];
+            }
+        }
+        if (argmax == nullptr && mlel_hip_resize_rescale_in_kernel(&y, &x, &resize.resize, 0) == 0) continue;
+        resize.kind = OpKind::FusedResize;
+        resize.epilogue = RescaleSpec{rs.inputs[1], rs.inputs[2], rs.rescale};
+        resize.flag = argmax != nullptr;
+        resize.outputs[0] = argmax ? argmax->outputs[0] : rs.outputs[0];
+        resize.outputs[0]->setProducer(&resize);
+        rs.fusedAway = true;
+        if (argmax) argmax->fusedAway = true;
+    }
+
+    // Pattern 1d (floating-point convolution): CONV2D [-> ADD of a tensor of the same shape that exists before the
+    // convolution runs] [-> CLAMP], on what the one-launch kernel takes (mlel_hip_conv2d_add_clamp_in_kernel decides).
+    // Every step is rounded as the stand-alone operator rounds it.
+    for (size_t at = 0; at < ops.size(); at++) {
+        OpNode &conv = *ops[at];
+        if (conv.fusedAway || conv.kind != OpKind::Conv2D) continue;
+        TensorPtr result = conv.outputs[0];
+        const int32_t dt = result->getFormat();
+        if (dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32) continue;
+        const mlel_tensor o = result->view(), x = conv.inputs[0]->view(), w = conv.inputs[1]->view(), b = conv.inputs[2]->view();
+        OpNode *add = nullptr, *clamp = nullptr;
+        TensorPtr residual;
+        const auto onlyUser = [&](const TensorPtr &t) -> OpNode * {
+            if (!isPrivateIntermediate(*t)) return nullptr;
+            const auto users = consumersOf(ops, t.get());
+            return users.size() == 1 ? users[0] : nullptr;
+        };
+        OpNode *next = onlyUser(result);
+        if (next != nullptr && next->kind == OpKind::Binary && next->selector == MLEL_BIN_ADD &&
+            next->inputs[0].get() != next->inputs[1].get()) {
+            const TensorPtr other = next->inputs[next->inputs[0].get() == result.get() ? 1 : 0];
+            bool early = other->getProducer() == nullptr && (other->getKind() != TensorKind::Session || other->isGraphInput);
+            for (size_t k = 0; k < at && !early; k++) early = ops[k].get() == other->getProducer();
+            const mlel_tensor r = other->view();
+            if (early && sameShape(*other, *result) && sameShape(*next->outputs[0], *result) && next->outputs[0]->getFormat() == dt &&
+                next->outputs[0]->isPacked() && mlel_hip_conv2d_add_clamp_in_kernel(&o, &x, &w, &b, &conv.conv, &r)) {
+                add = next;
+                residual = other;
+                result = add->outputs[0];
+                next = onlyUser(result);
+            }
+        }
+        if (next != nullptr && next->kind == OpKind::Clamp && next->outputs[0]->getFormat() == dt &&
+            sameShape(*next->outputs[0], *result) && next->outputs[0]->isPacked() && next->clamp.min_val <= next->clamp.max_val &&
+            mlel_hip_conv2d_add_clamp_in_kernel(&o, &x, &w, &b, &conv.conv, nullptr)) {
+            clamp = next;
+            result = clamp->outputs[0];
+        }
+        if (add == nullptr && clamp == nullptr) continue;
+        conv.kind = OpKind::FusedConv2DFloat;
+        conv.flag = add != nullptr;
+        conv.hasClamp = clamp != nullptr;
+        if (add) conv.inputs.push_back(residual), add->fusedAway = true;
+        if (clamp) conv.clamp = clamp->clamp, clamp->fusedAway = true;
+        conv.outputs[0] = result;
+        result->setProducer(&conv);
     }
 
     // Pattern 2 (residual add): RESCALE(a -> i32), RESCALE(b -> i32), ADD(i32), RESCALE(-> i8/i16/i32)
@@ -1676,6 +1788,14 @@ bool batchOperands(const OpNode &op, std::vector<size_t> &ins) {
     case OpKind::Table:
         ins = {0};
         return true;
+    case OpKind::FusedTransposeConv2D:
+        ins = {0};
+        return true;
+    case OpKind::FusedConv2DFloat:
+        ins = {0};
+        if (op.flag) ins.push_back(3);
+        return true;
+    case OpKind::FusedConcatConv2D:
     case OpKind::FusedConv2DResidual:
         ins = {0, 3};
         return true;
@@ -2001,6 +2121,13 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
     case OpKind::Reverse: rc = mlel_hip_reverse(ctx, stream, &out, &in[0], op.axis); break;
     case OpKind::Tile: rc = mlel_hip_tile(ctx, stream, &out, &in[0]); break;
     case OpKind::Select: rc = mlel_hip_select(ctx, stream, &out, &in[0], &in[1], &in[2]); break;
+    case OpKind::FusedConv2DFloat:
+        rc = mlel_hip_conv2d_add_clamp(ctx, stream, &out, &in[0], &in[1], &in[2], &op.conv, op.flag ? &in[3] : nullptr,
+                                       op.hasClamp ? &op.clamp : nullptr);
+        break;
+    case OpKind::FusedResize:
+    case OpKind::FusedTransposeConv2D:
+    case OpKind::FusedConcatConv2D:
     case OpKind::FusedConv2D:
     case OpKind::FusedDepthwiseConv2D:
     case OpKind::FusedMatmul: {
@@ -2008,6 +2135,12 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
         const mlel_epilogue e = makeEpilogue(op.epilogue, &mult, &shift, op.hasClamp, op.clamp);
         if (op.kind == OpKind::FusedConv2D)
             rc = mlel_hip_conv2d_rescale_clamp(ctx, stream, &out, &in[0], &in[1], &in[2], &op.conv, &e);
+        else if (op.kind == OpKind::FusedConcatConv2D)
+            rc = mlel_hip_concat_conv2d_rescale_clamp(ctx, stream, &out, &in[0], &in[3], &in[1], &in[2], &op.conv, &e);
+        else if (op.kind == OpKind::FusedTransposeConv2D)
+            rc = mlel_hip_transpose_conv2d_rescale_clamp(ctx, stream, &out, &in[0], &in[1], &in[2], &op.tconv, &e);
+        else if (op.kind == OpKind::FusedResize)
+            rc = mlel_hip_resize_rescale(ctx, stream, &out, &in[0], &op.resize, &e, op.flag ? 1 : 0);
         else if (op.kind == OpKind::FusedDepthwiseConv2D)
             rc = mlel_hip_dwconv_rescale_clamp(ctx, stream, &out, &in[0], &in[1], &in[2], &op.conv, &e);
         else

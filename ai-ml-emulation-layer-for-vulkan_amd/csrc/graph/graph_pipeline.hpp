@@ -99,6 +99,7 @@ enum class OpKind {
     // produced by the fusion pass only
     FusedConv2D, FusedDepthwiseConv2D, FusedMatmul, FusedRescaleAddRescale, FusedMatmulBiasCast, FusedElementwise,
     FusedConv2DResidual, FusedAttention, FusedConv2DDepthwise, FusedConv2DConv2D, FusedConv2DAvgPool,
+    FusedConv2DFloat, FusedTransposeConv2D, FusedConcatConv2D, FusedResize,
 };
 
 struct RescaleSpec {
@@ -159,6 +160,9 @@ class OpNode {
     // FusedConv2DAvgPool: a 1x1 convolution (+RESCALE, +CLAMP) and the AVG_POOL2D over all positions behind it; inputs =
     // {x, weights, bias}; conv / epilogue / hasClamp / clamp belong to the convolution, pool to the pooling, selector
     // is the type the convolution's result had
+    // FusedConv2DFloat: CONV2D over floating-point tensors with an ADD (inputs[3] is its other operand, `flag` set) and / or
+    // a CLAMP behind it; FusedTransposeConv2D: epilogue (+ clamp) as for FusedConv2D; FusedConcatConv2D: FusedConv2D over
+    // inputs[0] and inputs[3] side by side along the channels; FusedResize: RESIZE, RESCALE (epilogue) and, with `flag`, ARGMAX
     mlel_conv2d_attr convFirst{};
     mlel_clamp_attr clampFirst{};
     bool hasClampFirst = false;

@@ -1,0 +1,292 @@
+// RESIZE of int8 images, alone, with the RESCALE that follows it, and with the ARGMAX behind that (the head of a network that
+// labels pixels), and ARGMAX over the last axis (reference arithmetic: resize.comp:57-134, rescale.comp:27-72,
+// argmax.comp:26-66).
+//
+// Bound: memory for RESIZE alone (its int32 result is 16 times a fourfold smaller int8 input), the vector units for the
+// fused forms, which write one byte or one label in place of it.  The row coordinates belong to a block, the column is one
+// multiplication away; the generic kernel, which these replace for dense tensors, took six 64-bit divisions per element.
+#include "common.hpp"
+#include "dispatch.hpp"
+
+namespace mlel {
+namespace {
+
+constexpr int kBlock = 256;
+
+struct ResizeArgs {
+    const int8_t *in;
+    char *out;
+    int32_t H, W, C, OH, OW;
+    int32_t yn, yd, xn, xd, off_y, off_x;
+    int32_t bias_y, bias_x, bias_qy, bias_qx;  // multiples of yn, xn that make the coordinates non-negative, and quotients
+    DivMagic div_yn, div_xn, div_c;
+    int32_t bilinear, per_row, whole;          // elements of an output row; rows in aligned groups of four elements
+    const char *mult;                          // RESCALE, per tensor
+    const int8_t *shift;
+    int32_t mult16;
+    RescaleParams rp;
+};
+
+// the two neighbours of an output coordinate and the weight of the second
+struct Axis {
+    int32_t i0, i1, r;
+};
+__device__ __forceinline__ Axis axis_of(int32_t o, int32_t n, int32_t d, int32_t off, int32_t bias, int32_t bias_q,
+                                        const DivMagic &div, int32_t extent) {
+    const int32_t p = o * d + off;
+    const int32_t q = div_magic(p + bias, div) - bias_q;  // floor(p / n)
+    Axis a;
+    a.r = p - q * n;
+    a.i0 = q > 0 ? q : 0;
+    const uint32_t next = (uint32_t)(q + 1), last = (uint32_t)extent - 1u;
+    a.i1 = (int32_t)(next < last ? next : last);
+    return a;
+}
+
+__device__ __forceinline__ ChanScale scale_of(const ResizeArgs &g) {
+    const int32_t m = g.mult16 ? (int32_t) *reinterpret_cast<const int16_t *>(g.mult) : *reinterpret_cast<const int32_t *>(g.mult);
+    return make_chan_scale(m, g.shift[0], g.rp);
+}
+
+enum { R_I32, R_I8 };  // result: the int32 of RESIZE, or its RESCALE to int8
+
+// four consecutive elements of an output row per thread; FUSED: RESCALE (R_I8 without FUSED: RESIZE nearest, int8 result)
+template <int OUT, bool FUSED>
+__global__ void __launch_bounds__(kBlock) resize_i8_kernel(const ResizeArgs g) {
+    const int e0 = (int)(blockIdx.x * kBlock + threadIdx.x) * 4;
+    if (e0 >= g.per_row) return;
+    const int oy = blockIdx.y, img = blockIdx.z;
+    const Axis y = axis_of(oy, g.yn, g.yd, g.off_y, g.bias_y, g.bias_qy, g.div_yn, g.H);
+    const int8_t *base = g.in + (int64_t)img * g.H * g.W * g.C;
+    const int8_t *row0 = base + (int64_t)y.i0 * g.W * g.C, *row1 = base + (int64_t)y.i1 * g.W * g.C;
+    if (!g.bilinear) row0 = 2 * y.r >= g.yn ? row1 : row0;
+    ChanScale cs{};
+    if constexpr (FUSED) cs = scale_of(g);
+    int32_t v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int f = min(e0 + e, g.per_row - 1), ox = div_magic(f, g.div_c), c = f - ox * g.C;
+        const Axis x = axis_of(ox, g.xn, g.xd, g.off_x, g.bias_x, g.bias_qx, g.div_xn, g.W);
+        if (g.bilinear) {
+            const int32_t a = row0[x.i0 * g.C + c], b = row0[x.i1 * g.C + c], p = row1[x.i0 * g.C + c], q = row1[x.i1 * g.C + c];
+            v[e] = (a * (g.xn - x.r) + b * x.r) * (g.yn - y.r) + (p * (g.xn - x.r) + q * x.r) * y.r;
+        } else {
+            v[e] = row0[(2 * x.r >= g.xn ? x.i1 : x.i0) * g.C + c];
+        }
+        if constexpr (FUSED) v[e] = requant_chan(v[e], cs, g.rp);
+    }
+    const int64_t at = ((int64_t)img * g.OH + oy) * g.per_row + e0;
+    if constexpr (OUT == R_I32) {
+        int32_t *o = reinterpret_cast<int32_t *>(g.out) + at;
+        if (g.whole) {
+            store16_result(o, make_uint4((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e0 + e < g.per_row) o[e] = v[e];
+        }
+    } else {
+        char *o = g.out + at;
+        if (g.whole) {
+            *reinterpret_cast<uint32_t *>(o) = (uint32_t)(v[0] & 255) | (uint32_t)(v[1] & 255) << 8 | (uint32_t)(v[2] & 255) << 16 |
+                                               (uint32_t)v[3] << 24;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e0 + e < g.per_row) o[e] = (char)v[e];
+        }
+    }
+}
+
+// RESIZE (bilinear) -> RESCALE to int8 -> ARGMAX over the channels: one output position per thread.  RESCALE with a
+// multiplier that is not negative never turns a smaller value into a larger one, so a channel can only become the maximum
+// when its interpolated value exceeds every earlier one; only then is it rescaled (ties after rounding keep the first).
+__global__ void __launch_bounds__(kBlock) resize_argmax_kernel(const ResizeArgs g) {
+    const int ox = blockIdx.x * kBlock + threadIdx.x;
+    if (ox >= g.OW) return;
+    const int oy = blockIdx.y, img = blockIdx.z;
+    const Axis y = axis_of(oy, g.yn, g.yd, g.off_y, g.bias_y, g.bias_qy, g.div_yn, g.H);
+    const Axis x = axis_of(ox, g.xn, g.xd, g.off_x, g.bias_x, g.bias_qx, g.div_xn, g.W);
+    const int8_t *base = g.in + (int64_t)img * g.H * g.W * g.C;
+    const int8_t *p00 = base + ((int64_t)y.i0 * g.W + x.i0) * g.C, *p01 = base + ((int64_t)y.i0 * g.W + x.i1) * g.C;
+    const int8_t *p10 = base + ((int64_t)y.i1 * g.W + x.i0) * g.C, *p11 = base + ((int64_t)y.i1 * g.W + x.i1) * g.C;
+    const int32_t w00 = (g.yn - y.r) * (g.xn - x.r), w01 = (g.yn - y.r) * x.r, w10 = y.r * (g.xn - x.r), w11 = y.r * x.r;
+    const ChanScale cs = scale_of(g);
+    // (no sum of this RESIZE may leave int32 when it is scaled, or the order would not survive)
+    const int64_t bound = (int64_t)128 * g.yn * g.xn;
+    const bool monotone = cs.mult >= 0 && ((bound * cs.mult + cs.round_pos) >> cs.shift) < (int64_t(1) << 30);
+    int32_t best = 0, best_r = -128, best_a = INT32_MIN;
+    auto channel = [&](int c, int32_t a) {
+        if (monotone && a <= best_a && c > 0) return;
+        best_a = a;
+        const int32_t r = requant_chan(a, cs, g.rp);
+        if (r > best_r) best_r = r, best = c;
+    };
+    int c = 0;
+    for (; c + 4 <= g.C; c += 4) {
+        uint32_t d[4];
+        __builtin_memcpy(&d[0], p00 + c, 4);
+        __builtin_memcpy(&d[1], p01 + c, 4);
+        __builtin_memcpy(&d[2], p10 + c, 4);
+        __builtin_memcpy(&d[3], p11 + c, 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            channel(c + e, (int8_t)(d[0] >> (8 * e)) * w00 + (int8_t)(d[1] >> (8 * e)) * w01 + (int8_t)(d[2] >> (8 * e)) * w10 +
+                               (int8_t)(d[3] >> (8 * e)) * w11);
+    }
+    for (; c < g.C; c++) channel(c, p00[c] * w00 + p01[c] * w01 + p10[c] * w10 + p11[c] * w11);
+    reinterpret_cast<int32_t *>(g.out)[((int64_t)img * g.OH + oy) * g.OW + ox] = best;
+}
+
+// ARGMAX over the last axis of dense rows: G lanes per row (a power of two), each scanning every G-th chunk of V elements;
+// then the larger value, and of equal values the smaller index, wins
+struct ArgmaxArgs {
+    const char *in;
+    int32_t *out;
+    int64_t rows;
+    int32_t cols, ignore_nan;
+};
+template <typename T>
+__device__ __forceinline__ float as_key(T v);
+template <> __device__ __forceinline__ float as_key<int8_t>(int8_t v) { return (float)v; }
+template <> __device__ __forceinline__ float as_key<_Float16>(_Float16 v) { return (float)v; }
+template <> __device__ __forceinline__ float as_key<float>(float v) { return v; }
+
+template <typename T, int G>
+__global__ void __launch_bounds__(kBlock) argmax_rows_kernel(const ArgmaxArgs g) {
+    constexpr int V = 4;
+    const int lane = threadIdx.x % G;
+    const int64_t row = (int64_t)blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    const bool live = row < g.rows;
+    const T *p = reinterpret_cast<const T *>(g.in) + (live ? row : 0) * g.cols;
+    const float lowest = sizeof(T) == 1 ? -128.f : (sizeof(T) == 2 ? -65504.f : -3.402823466e+38f);
+    float best = lowest;
+    int at = 0;
+    auto take = [&](T raw, int c) {
+        float v = as_key(raw);
+        if (v != v) {  // the first NaN is the maximum, or is passed over
+            if (g.ignore_nan) return;
+            if (best != best) return;
+            best = NAN, at = c;
+            return;
+        }
+        if (v > best) best = v, at = c;
+    };
+    for (int c = lane * V; c < g.cols; c += G * V) {
+        if (c + V <= g.cols) {
+            T v[V];
+            __builtin_memcpy(v, p + c, sizeof(v));
+#pragma unroll
+            for (int e = 0; e < V; e++) take(v[e], c + e);
+        } else {
+            for (int e = c; e < g.cols; e++) take(p[e], e);
+        }
+    }
+#pragma unroll
+    for (int m = 1; m < G; m <<= 1) {
+        const float ov = __shfl_xor(best, m);
+        const int oa = __shfl_xor(at, m);
+        const bool on = ov != ov, mine = best != best;
+        // a lane that met nothing above the lowest value holds index 0, the answer for such a row
+        const bool wins = on != mine ? on : (on ? oa < at : (ov > best || (ov == best && oa < at)));
+        if (wins) best = ov, at = oa;
+    }
+    if (live && lane == 0) g.out[row] = at;
+}
+
+template <typename T>
+void launch_argmax(const ArgmaxArgs &g, hipStream_t s) {
+    // four lanes for every 64 columns, at least one load per lane
+    const int chunks = (g.cols + 3) / 4;
+    auto go = [&](auto n) {
+        constexpr int G = decltype(n)::value;
+        argmax_rows_kernel<T, G><<<dim3((unsigned)((g.rows + kBlock / G - 1) / (kBlock / G))), dim3(kBlock), 0, s>>>(g);
+    };
+    if (chunks <= 2) go(std::integral_constant<int, 1>{});
+    else if (chunks <= 32) go(std::integral_constant<int, 4>{});
+    else if (chunks <= 128) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 64>{});
+}
+
+// what the kernels' 32-bit coordinates assume; fills everything but the RESCALE
+bool describe(ResizeArgs &g, const mlel_tensor *out_image, const mlel_tensor *in, const mlel_resize_attr *a) {
+    if (in->dtype != MLEL_I8 || !is_packed(in)) return false;
+    const int64_t N = in->dims[0], H = in->dims[1], W = in->dims[2], C = in->dims[3];
+    const int64_t OH = out_image->dims[1], OW = out_image->dims[2];
+    if (out_image->dims[0] != N || N <= 0 || H <= 0 || W <= 0 || C <= 0 || OH <= 0 || OW <= 0 || N > 65535 || OH > 65535) return false;
+    if (H > 32767 || W > 32767 || OW * C >= (1 << 28) || N * H * W * C >= (int64_t(1) << 40)) return false;
+    const int32_t *s = a->scale;
+    for (int i = 0; i < 4; i++)
+        if (s[i] <= 0 || s[i] > 2048) return false;
+    for (int i = 0; i < 2; i++)
+        if (a->offset[i] < -(1 << 20) || a->offset[i] > (1 << 20)) return false;
+    // the shader's coordinates are int16: they stay so for every position
+    if (((OH - 1) * s[1] + a->offset[0]) / s[0] > 32000 || ((OW - 1) * s[3] + a->offset[1]) / s[2] > 32000) return false;
+    if (OH * s[1] >= (1 << 28) || OW * s[3] >= (1 << 28)) return false;
+    g.in = static_cast<const int8_t *>(in->ptr);
+    g.H = (int)H, g.W = (int)W, g.C = (int)C, g.OH = (int)OH, g.OW = (int)OW, g.per_row = (int)(OW * C);
+    g.yn = s[0], g.yd = s[1], g.xn = s[2], g.xd = s[3], g.off_y = a->offset[0], g.off_x = a->offset[1];
+    g.bias_qy = a->offset[0] < 0 ? -a->offset[0] / s[0] + 1 : 0, g.bias_y = g.bias_qy * s[0];
+    g.bias_qx = a->offset[1] < 0 ? -a->offset[1] / s[2] + 1 : 0, g.bias_x = g.bias_qx * s[2];
+    g.div_yn = make_div_magic((uint32_t)g.yn), g.div_xn = make_div_magic((uint32_t)g.xn), g.div_c = make_div_magic((uint32_t)g.C);
+    g.bilinear = a->mode == MLEL_RESIZE_BILINEAR;
+    return true;
+}
+
+bool fill_scale(ResizeArgs &g, const FusedEpilogue *epi) {
+    if (epi->p.per_channel) return false;
+    g.mult = static_cast<const char *>(epi->mult->ptr);
+    g.shift = static_cast<const int8_t *>(epi->shift->ptr);
+    g.mult16 = epi->scale32 ? 0 : 1;
+    g.rp = epi->p;
+    return true;
+}
+
+}  // namespace
+
+int try_resize_i8(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *a,
+                  const FusedEpilogue *epi, bool probe) {
+    ResizeArgs g{};
+    if (!is_packed(out) || out->dims[3] != in->dims[3] || !describe(g, out, in, a)) return 0;
+    if (out->dtype != MLEL_I32 && out->dtype != MLEL_I8) return 0;
+    if (probe) return out->dtype == MLEL_I8;
+    g.whole = g.per_row % 4 == 0 && ((uintptr_t)out->ptr % (out->dtype == MLEL_I32 ? 16 : 4)) == 0;
+    // (an int8 result without a RESCALE would be the truncated sum)
+    if (epi == nullptr && out->dtype == MLEL_I8 && g.bilinear) return 0;
+    if (epi != nullptr && (out->dtype != MLEL_I8 || !fill_scale(g, epi))) return 0;
+    g.out = static_cast<char *>(out->ptr);
+    const dim3 grid((unsigned)((g.per_row + 4 * kBlock - 1) / (4 * kBlock)), (unsigned)g.OH, (unsigned)in->dims[0]);
+    if (epi != nullptr) resize_i8_kernel<R_I8, true><<<grid, dim3(kBlock), 0, s>>>(g);
+    else if (out->dtype == MLEL_I32) resize_i8_kernel<R_I32, false><<<grid, dim3(kBlock), 0, s>>>(g);
+    else resize_i8_kernel<R_I8, false><<<grid, dim3(kBlock), 0, s>>>(g);
+    MLEL_TRY(check_launch("resize int8"));
+    return 1;
+}
+
+int try_resize_argmax_i8(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *a,
+                         const FusedEpilogue *epi, bool probe) {
+    ResizeArgs g{};
+    if (out->dtype != MLEL_I32 || !is_packed(out) || a->mode != MLEL_RESIZE_BILINEAR || !describe(g, out, in, a)) return 0;
+    if (probe) return 1;
+    if (((uintptr_t)out->ptr % 4) != 0 || !fill_scale(g, epi) || g.rp.out_lo < -128 || g.rp.out_hi > 127) return 0;
+    g.out = static_cast<char *>(out->ptr);
+    resize_argmax_kernel<<<dim3((unsigned)((g.OW + kBlock - 1) / kBlock), (unsigned)g.OH, (unsigned)in->dims[0]), dim3(kBlock), 0, s>>>(g);
+    MLEL_TRY(check_launch("resize + rescale + argmax int8"));
+    return 1;
+}
+
+int try_argmax_rows(hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, uint32_t axis, uint32_t nan_mode) {
+    if ((int)axis != in->rank - 1 || !is_packed(in) || !is_packed(out) || out->dtype != MLEL_I32) return 0;
+    if (in->dtype != MLEL_I8 && in->dtype != MLEL_F16 && in->dtype != MLEL_F32) return 0;
+    const int64_t cols = in->dims[in->rank - 1], rows = numel(out);
+    if (cols <= 0 || cols >= (1 << 30) || rows <= 0 || rows * cols != numel(in) || rows >= (int64_t(1) << 31)) return 0;
+    const ArgmaxArgs g{static_cast<const char *>(in->ptr), static_cast<int32_t *>(out->ptr), rows, (int32_t)cols,
+                       nan_mode == MLEL_NAN_IGNORE ? 1 : 0};
+    if (in->dtype == MLEL_I8) launch_argmax<int8_t>(g, s);
+    else if (in->dtype == MLEL_F16) launch_argmax<_Float16>(g, s);
+    else launch_argmax<float>(g, s);
+    MLEL_TRY(check_launch("argmax rows"));
+    return 1;
+}
+
+}  // namespace mlel

@@ -586,6 +586,38 @@ int mlel_hip_conv2d_rescale_clamp_avgpool(mlel_ctx *ctx, void *stream, const mle
 int mlel_hip_conv2d_avgpool_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *weights,
                                       const mlel_tensor *bias, const mlel_conv2d_attr *attr, int32_t conv_dtype,
                                       const mlel_pool2d_attr *pool);
+/* out = CLAMP?( ADD?( CONV2D(in, w, bias), residual ) ) over fp16, bf16 or fp32 tensors of one type with an fp32
+ * accumulator, one launch: every step rounded as the stand-alone operator rounds it.  `residual` (of out's type and
+ * shape) and `clamp` may be NULL.  Composition of conv2d.comp:40-116, elementwise_binary.comp:146-173 and
+ * clamp.comp:24-53.  Zero zero points, dense operands; anything else is MLEL_ERR_UNSUPPORTED (nothing is allocated and
+ * nothing falls back).  The _in_kernel query judges by types, extents and strides without touching the device. */
+int mlel_hip_conv2d_add_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                              const mlel_tensor *weights, const mlel_tensor *bias, const mlel_conv2d_attr *attr,
+                              const mlel_tensor *residual, const mlel_clamp_attr *clamp);
+int mlel_hip_conv2d_add_clamp_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *weights,
+                                        const mlel_tensor *bias, const mlel_conv2d_attr *attr, const mlel_tensor *residual);
+/* out(8-bit) = CLAMP?(RESCALE(TRANSPOSE_CONV2D(in, w, bias))), int8 operands, one launch; byte for byte the operators one
+ * after another (transpose_conv2d.comp:31-70, rescale.comp:27-72, clamp.comp:24-53).  No fallback; _in_kernel as above. */
+int mlel_hip_transpose_conv2d_rescale_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                                            const mlel_tensor *weights, const mlel_tensor *bias,
+                                            const mlel_tconv2d_attr *attr, const mlel_epilogue *epi);
+int mlel_hip_transpose_conv2d_rescale_clamp_in_kernel(const mlel_tensor *out, const mlel_tensor *in,
+                                                      const mlel_tensor *weights, const mlel_tensor *bias,
+                                                      const mlel_tconv2d_attr *attr);
+/* out(8-bit) = CLAMP?(RESCALE(CONV2D( CONCAT(in1, in2) along the channels, w, bias ))), int8 operands: the convolution reads
+ * both tensors in place (concat.comp, then as mlel_hip_conv2d_rescale_clamp).  No fallback; _in_kernel as above. */
+int mlel_hip_concat_conv2d_rescale_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in1,
+                                         const mlel_tensor *in2, const mlel_tensor *weights, const mlel_tensor *bias,
+                                         const mlel_conv2d_attr *attr, const mlel_epilogue *epi);
+int mlel_hip_concat_conv2d_in_kernel(const mlel_tensor *out, const mlel_tensor *in1, const mlel_tensor *in2,
+                                     const mlel_tensor *weights, const mlel_tensor *bias, const mlel_conv2d_attr *attr);
+/* RESIZE (int8 -> int32) -> per-tensor RESCALE to int8 in one launch, and with `argmax` != 0 the ARGMAX over the channels
+ * behind it too (`out` is then the int32 [N, OH, OW] of labels; bilinear only): resize.comp:57-134, rescale.comp:27-72,
+ * argmax.comp:26-66.  No fallback; _in_kernel as above. */
+int mlel_hip_resize_rescale(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
+                            const mlel_resize_attr *attr, const mlel_epilogue *epi, int32_t argmax);
+int mlel_hip_resize_rescale_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_resize_attr *attr,
+                                      int32_t argmax);
 /* 1 when mlel_hip_conv2d_dwconv_rescale_clamp takes these operands, judged by types, extents, strides and attributes
  * only (data pointers are not looked at; no device is touched), else 0. */
 int mlel_hip_conv2d_dwconv_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w1,
