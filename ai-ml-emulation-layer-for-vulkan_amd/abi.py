@@ -265,6 +265,7 @@ FUSED_SIGNATURES = {
     "elementwise_chain": [_T, C.POINTER(Chain)],
     "matmul_bias_cast_chain": [_T, _T, _T, _T, C.POINTER(MatmulAttr), C.POINTER(Chain)],
     "attention_f16": [_T, _T, _T, _T, C.POINTER(Chain)],
+    "attention_rows_f16": [_T, _T, _T, _T, C.POINTER(Chain)],
     "conv2d_add_clamp": [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, C.POINTER(ClampAttr)],
     "transpose_conv2d_rescale_clamp": [_T, _T, _T, _T, C.POINTER(Tconv2dAttr), C.POINTER(Epilogue)],
     "concat_conv2d_rescale_clamp": [_T, _T, _T, _T, _T, C.POINTER(Conv2dAttr), C.POINTER(Epilogue)],
@@ -308,6 +309,7 @@ RUNTIME_SIGNATURES = {
     "mlel_hip_copy_kernel_variant": (C.c_int, [_V, _V, _V, _V, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_int]),
     "mlel_hip_matmul_chain_in_kernel": (C.c_int, [C.POINTER(Chain)]),
     "mlel_hip_attention_f16_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Chain)]),
+    "mlel_hip_attention_rows_f16_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Chain)]),
     "mlel_hip_conv2d_dwconv_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, _T,
                                                    C.POINTER(Conv2dAttr)]),
     "mlel_hip_conv2d_conv2d_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, _T,

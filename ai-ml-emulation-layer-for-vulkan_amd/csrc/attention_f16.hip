@@ -37,9 +37,11 @@ constexpr int kRows = 64;       // query rows per block
 constexpr int kHead = 64;       // head size: K of the first product, N of the second
 constexpr int kChunk = 64;      // keys per chunk of K^T / V
 constexpr int kChunkPitch = 2 * kChunk + 32;  // bytes per K row of a chunk: 4 rows x 32 B land on distinct banks
+constexpr int kKeyPitch = 2 * kHead + 16;     // bytes per key of a chunk of K by rows: 36 banks apart, so that the
+                                              // sixteen lanes of a 128-bit access meet distinct banks
 constexpr int kMaxKeys = 512;   // 16 pieces of 16 bytes per thread
+constexpr int kMaxKeysRagged = 1024;  // two registers' worth of that
 constexpr int kPassKeys = 256;  // keys of a row that sit in shared memory at a time
-constexpr int kPasses = kMaxKeys / kPassKeys;
 constexpr int kPassChunks = kPassKeys / kChunk;
 constexpr int kPassPieces = kPassKeys / 32;  // 16-byte pieces per thread and pass
 
@@ -47,7 +49,8 @@ struct AttnArgs {
     const char *q, *kt, *v;
     char *out;
     const uint16_t *scale;  // the chain's single-element fp16 input (SCALED), else unused
-    int32_t M, S, batches, strips;
+    int32_t M, S, batches, strips;  // S: the number of keys, rounded up to whole chunks in the ragged form
+    int32_t keys;                   // the number of keys
     int64_t q_batch, kt_batch, v_batch, o_batch;  // bytes
     uint32_t ldq, ldkt, ldv, ldo;                 // bytes per row
     uint32_t q_bytes, kt_bytes, v_bytes, o_bytes; // per-batch extents (all below 2^31)
@@ -75,8 +78,27 @@ __device__ __forceinline__ v8h as_v8h(const uint4 &u) {
     return c.h;
 }
 
-template <bool SCALED>
+// The softmax's row values beyond the last key take `fill` (two fp16 values): the words of a 16-byte piece whose first
+// key is `left` keys before the end of the row.
+__device__ __forceinline__ uint4 past_end(uint4 x, int left, uint32_t fill) {
+    uint32_t *w = &x.x;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t keep = left >= 2 * i + 2 ? 0xffffffffu : (left == 2 * i + 1 ? 0x0000ffffu : 0u);
+        w[i] = (w[i] & keep) | (fill & ~keep);
+    }
+    return x;
+}
+
+// KROWS: the ragged form.  K arrives by rows [S][64] (a projection writes it so without transposing, and rows of any S
+// stay 16-byte aligned; the matrix operand is then a plain 128-bit read of shared memory), and neither M nor S need be a
+// multiple of anything: rows of K and V beyond S are fetched as zeros, scores beyond S are the smallest fp16 value for
+// the maximum and their exponentials zero (adding zero to the fold and to the product changes no bit), query rows beyond
+// M are computed from zeros and not stored.  Six heads of 197 queries and keys: 10.3 us, where the transposition of K, two
+// products and nine elementwise and reduction passes took 455 us (the two reductions of unaligned rows 184 us each).
+template <bool SCALED, bool KROWS, int MAXKEYS>
 __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g) {
+    constexpr int kPasses = MAXKEYS / kPassKeys;
     extern __shared__ __align__(16) char smem[];
     const int SP = min(g.S, kPassKeys) * 2 + 16;  // pitch of a score row (bytes): consecutive rows start four banks apart
     char *st = smem;               // [64][SP]: one pass of S, later of EXP(..), later of P
@@ -88,7 +110,7 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
                  "s"(g.kt), "s"(g.v), "s"(g.out), "s"(g.scale), "s"(g.M), "s"(g.S), "s"(g.batches), "s"(g.strips),
                  "s"(g.q_batch), "s"(g.kt_batch), "s"(g.v_batch), "s"(g.o_batch), "s"(g.ldq), "s"(g.ldkt), "s"(g.ldv),
                  "s"(g.ldo), "s"(g.q_bytes), "s"(g.kt_bytes), "s"(g.v_bytes), "s"(g.o_bytes), "s"(g.view), "s"(g.v_nb2),
-                 "s"(g.v_m2), "s"(g.v_n2), "s"(g.vs_nb1), "s"(g.vs_nb2), "s"(g.vs_m1), "s"(g.vs_m2), "s"(g.vs_n1));
+                 "s"(g.v_m2), "s"(g.v_n2), "s"(g.vs_nb1), "s"(g.vs_nb2), "s"(g.vs_m1), "s"(g.vs_m2), "s"(g.vs_n1), "s"(g.keys));
     const int lin = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % 8u) * g.chunk + (int)(blockIdx.x / 8u));
     if (lin >= g.total) return;
     const int batch = div_magic(lin, g.div_strips);
@@ -121,6 +143,11 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
     };
     // a chunk is 64 rows of 128 bytes: two 16-byte pieces per thread
     const int c_row = tid >> 2, c_piece = (tid & 3) * 2;
+    auto keys_store = [&](const uint4 (&r)[2]) {
+        constexpr int pitch = KROWS ? kKeyPitch : kChunkPitch;
+        *reinterpret_cast<uint4 *>(cb + c_row * pitch + c_piece * 16) = r[0];
+        *reinterpret_cast<uint4 *>(cb + c_row * pitch + c_piece * 16 + 16) = r[1];
+    };
     auto chunk_store = [&](const uint4 (&r)[2]) {
         *reinterpret_cast<uint4 *>(cb + c_row * kChunkPitch + c_piece * 16) = r[0];
         *reinterpret_cast<uint4 *>(cb + c_row * kChunkPitch + c_piece * 16 + 16) = r[1];
@@ -128,7 +155,8 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
     const int nchunks = g.S / kChunk;
     uint4 cr[2];
     auto fetch_kt = [&](int c) {  // rows = k (the head dimension), columns = the chunk's keys
-        const uint32_t off = (uint32_t)c_row * g.ldkt + (uint32_t)(c * kChunk + c_piece * 8) * 2;
+        const uint32_t off = KROWS ? (uint32_t)(c * kChunk + c_row) * g.ldkt + (uint32_t)c_piece * 16
+                                   : (uint32_t)c_row * g.ldkt + (uint32_t)(c * kChunk + c_piece * 8) * 2;
         cr[0] = load16(kres, c < nchunks ? off : kOob);
         cr[1] = load16(kres, c < nchunks ? off + 16 : kOob);
     };
@@ -148,7 +176,8 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
     // full rate (measured: quarter + 4 uu, the threads 16 bytes apart, takes 1.6 times as long).  A pass has an even
     // number of pieces per thread, so this is a bijection onto the row's pieces.
     auto piece_off = [&](int, int uu) { return (2 * quarter + (uu & 1) + 8 * (uu >> 1)) * 16; };
-    uint4 val[kMaxKeys / 32];
+    auto keys_left = [&](int h, int uu) { return g.keys - h * kPassKeys - piece_off(h, uu) / 2; };
+    uint4 val[MAXKEYS / 32];
     uint32_t scale_w = 0;
     if (SCALED) {
         const uint32_t bits = *g.scale;
@@ -170,14 +199,17 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
             const int c_end = min(nchunks, (h + 1) * kPassChunks);
             for (int c = h * kPassChunks; c < c_end; c++) {
                 __syncthreads();  // every wavefront has read the previous chunk (and the previous pass its scores)
-                chunk_store(cr);
+                keys_store(cr);
                 __syncthreads();
                 fetch_kt(c + 1);
                 v16f acc;
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[r] = 0.f;
 #pragma unroll
-                for (int kk = 0; kk < 4; kk++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(b_frag(kk), qf[kk], acc, 0, 0, 0);
+                for (int kk = 0; kk < 4; kk++) {
+                    const v8h kf = KROWS ? *reinterpret_cast<const v8h *>(cb + (wn * 32 + a_row) * kKeyPitch + kk * 32 + a_kg * 16) : b_frag(kk);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kk], acc, 0, 0, 0);
+                }
                 // lane holds row lane % 32 of the tile and, per register quad q, columns 8 q + 4 (lane / 32) .. + 3
                 char *srow = st + (wm * 32 + (lane & 31)) * SP + ((c - h * kPassChunks) * kChunk + wn * 32 + 4 * (lane >> 5)) * 2;
 #pragma unroll
@@ -204,6 +236,7 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
                         x = static_apply<F_MUL>(x, make_uint4(scale_w, scale_w, scale_w, scale_w));
                         asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
                     }
+                    if (KROWS) x = past_end(x, keys_left(h, uu), 0xfbfffbffu);  // -65504
                     val[u] = x;
                     // REDUCE_MAX: exact; a NaN or an infinity anywhere in the row makes the maximum a NaN (as the row program)
                     special |= (((x.x & 0x7fff7fffu) + 0x03ff03ffu) | ((x.y & 0x7fff7fffu) + 0x03ff03ffu) |
@@ -226,13 +259,13 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
     const uint32_t mbits = (uint32_t)__half_as_ushort(f2h(special != 0 ? __builtin_nanf("") : mx));
     const uint4 mrow = make_uint4(mbits | (mbits << 16), mbits | (mbits << 16), mbits | (mbits << 16), mbits | (mbits << 16));
 #pragma unroll
-    for (int u = 0; u < kMaxKeys / 32; u++) {
+    for (int u = 0; u < MAXKEYS / 32; u++) {
         if (u < ppt) {
             uint4 d = static_apply<F_SUB>(val[u], mrow);
             asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z), "+v"(d.w));
             uint4 e = static_apply<F_EXP>(d, d);
             asm volatile("" : "+v"(e.x), "+v"(e.y), "+v"(e.z), "+v"(e.w));
-            val[u] = e;
+            val[u] = KROWS ? past_end(e, keys_left(u / kPassPieces, u % kPassPieces), 0u) : e;
         }
     }
     // REDUCE_SUM: left to right in fp16, one lane per row, a pass of the rows at a time; the first chunk of V is on its
@@ -365,6 +398,7 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
             const uint32_t n1 = fast_n ? __umulhi((uint32_t)n, magic_n) : (dn == 1 ? (uint32_t)n : (uint32_t)n / dn);
             off = m1 * g.vs_m1 + ((uint32_t)m - m1 * dm) * g.vs_m2 + n1 * g.vs_n1 + ((uint32_t)n - n1 * dn) * 2;
         }
+        if (KROWS && m >= g.M) off = kOob;
         v4i v;
         v.x = (int)piece.x, v.y = (int)piece.y, v.z = (int)piece.z, v.w = (int)piece.w;
         __builtin_amdgcn_raw_buffer_store_b128(v, ores, (int)off, 0, kOutAux);
@@ -406,22 +440,25 @@ int softmax_form(const mlel_chain *c) {
 }
 
 // 1 when the three operators are a case for the kernel; `with_pointers`: also check the base addresses
+// `krows`: the ragged form, `kt` is K [NB, S, 64]
 int describe(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt, const mlel_tensor *v,
-             const mlel_chain *chain, bool with_pointers, AttnArgs *filled) {
+             const mlel_chain *chain, bool krows, bool with_pointers, AttnArgs *filled) {
     const int form = softmax_form(chain);
     if (form < 0) return 0;
     if (q->dtype != MLEL_F16 || kt->dtype != MLEL_F16 || v->dtype != MLEL_F16 || out->dtype != MLEL_F16) return 0;
     if (q->rank != 3 || kt->rank != 3 || v->rank != 3 || (out->rank != 3 && out->rank != 6)) return 0;
-    const int64_t NB = q->dims[0], M = q->dims[1], S = kt->dims[2];
-    if (q->dims[2] != kHead || kt->dims[0] != NB || kt->dims[1] != kHead || v->dims[0] != NB || v->dims[1] != S ||
+    const int64_t NB = q->dims[0], M = q->dims[1], S = kt->dims[krows ? 1 : 2];
+    if (q->dims[2] != kHead || kt->dims[0] != NB || kt->dims[krows ? 2 : 1] != kHead || v->dims[0] != NB || v->dims[1] != S ||
         v->dims[2] != kHead)
         return 0;
-    if (NB <= 0 || M <= 0 || M % kRows != 0 || S < kChunk || S > kMaxKeys || S % kChunk != 0) return 0;
+    if (NB <= 0 || M <= 0) return 0;
+    if (krows ? S < 1 || S > kMaxKeysRagged : M % kRows != 0 || S < kChunk || S > kMaxKeys || S % kChunk != 0) return 0;
+    const int64_t strips = (M + kRows - 1) / kRows;
     if (!dense_rows(q) || !dense_rows(kt) || !dense_rows(v)) return 0;
     if (!aligned16(q, with_pointers) || !aligned16(kt, with_pointers) || !aligned16(v, with_pointers)) return 0;
     const int64_t lim = (int64_t(1) << 31) - 64;
-    const int64_t qb = M * q->strides[1], kb = kHead * kt->strides[1], vb = S * v->strides[1];
-    if (qb >= lim || kb >= lim || vb >= lim || NB * (M / kRows) >= (int64_t(1) << 30)) return 0;
+    const int64_t qb = M * q->strides[1], kb = (krows ? S : kHead) * kt->strides[1], vb = S * v->strides[1];
+    if (qb >= lim || kb >= lim || vb >= lim || M >= (1 << 24) || NB * strips >= (int64_t(1) << 30)) return 0;
     AttnArgs g{};
     if (out->rank == 3) {
         if (out->dims[0] != NB || out->dims[1] != M || out->dims[2] != kHead || out->strides[2] != 2) return 0;
@@ -458,9 +495,10 @@ int describe(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt
     g.scale = form == 1 ? static_cast<const uint16_t *>(chain->inputs[1]->ptr) : nullptr;
     if (with_pointers && form == 1 && (g.scale == nullptr || ((uintptr_t)g.scale % 2) != 0)) return 0;
     g.M = (int32_t)M;
-    g.S = (int32_t)S;
+    g.S = (int32_t)((S + kChunk - 1) / kChunk * kChunk);
+    g.keys = (int32_t)S;
     g.batches = (int32_t)NB;
-    g.strips = (int32_t)(M / kRows);
+    g.strips = (int32_t)strips;
     g.div_strips = make_div_magic((uint32_t)g.strips);
     g.q_batch = q->strides[0];
     g.kt_batch = kt->strides[0];
@@ -471,42 +509,44 @@ int describe(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt
     g.q_bytes = (uint32_t)qb;
     g.kt_bytes = (uint32_t)kb;
     g.v_bytes = (uint32_t)vb;
-    g.total = (int32_t)(NB * (M / kRows));
+    g.total = (int32_t)(NB * strips);
     g.chunk = (g.total + 7) / 8;
     if (filled != nullptr) *filled = g;
     return form == 1 ? 2 : 1;
 }
 
-}  // namespace
-
-bool attention_f16_supported(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt, const mlel_tensor *v,
-                             const mlel_chain *chain) {
-    return describe(out, q, kt, v, chain, false, nullptr) != 0;
+template <bool SCALED, bool KROWS, int MAXKEYS>
+void launch(mlel_ctx *ctx, AttnArgs &g, hipStream_t s) {
+    const size_t sm = (size_t)kRows * (std::min(g.S, kPassKeys) * 2 + 16) + (size_t)kChunk * kChunkPitch;
+    g.fold_span = std::max(1, (ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256) / 8);
+    auto kernel = attention_f16_kernel<SCALED, KROWS, MAXKEYS>;
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   kRows * (kPassKeys * 2 + 16) + kChunk * kChunkPitch) == hipSuccess;
+    (void)raised;
+    kernel<<<dim3((unsigned)(g.chunk * 8)), dim3(kBlock), sm, s>>>(g);
 }
 
-int try_attention_f16(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt,
-                      const mlel_tensor *v, const mlel_chain *chain) {
+}  // namespace
+
+bool attention_f16_supported(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *k, const mlel_tensor *v,
+                             const mlel_chain *chain, bool krows) {
+    return describe(out, q, k, v, chain, krows, false, nullptr) != 0;
+}
+
+int try_attention_f16(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *k,
+                      const mlel_tensor *v, const mlel_chain *chain, bool krows) {
     AttnArgs g{};
-    const int form = describe(out, q, kt, v, chain, true, &g);
+    const int form = describe(out, q, k, v, chain, krows, true, &g);
     if (form == 0) return 0;
-    const size_t sm = (size_t)kRows * (std::min(g.S, kPassKeys) * 2 + 16) + (size_t)kChunk * kChunkPitch;
-    const dim3 grid((unsigned)(g.chunk * 8));
-    g.fold_span = std::max(1, (ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256) / 8);
-    if (form == 2) {
-        auto kernel = attention_f16_kernel<true>;
-        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       kRows * (kPassKeys * 2 + 16) + kChunk * kChunkPitch) == hipSuccess;
-        (void)raised;
-        kernel<<<grid, dim3(kBlock), sm, s>>>(g);
-    } else {
-        auto kernel = attention_f16_kernel<false>;
-        static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       kRows * (kPassKeys * 2 + 16) + kChunk * kChunkPitch) == hipSuccess;
-        (void)raised;
-        kernel<<<grid, dim3(kBlock), sm, s>>>(g);
-    }
+    // the ragged form's instance: as few registers for the row values as the keys need (one, two or four passes)
+    if (!krows)
+        form == 2 ? launch<true, false, kMaxKeys>(ctx, g, s) : launch<false, false, kMaxKeys>(ctx, g, s);
+    else if (g.S <= kPassKeys)
+        form == 2 ? launch<true, true, kPassKeys>(ctx, g, s) : launch<false, true, kPassKeys>(ctx, g, s);
+    else if (g.S <= kMaxKeys)
+        form == 2 ? launch<true, true, kMaxKeys>(ctx, g, s) : launch<false, true, kMaxKeys>(ctx, g, s);
+    else
+        form == 2 ? launch<true, true, kMaxKeysRagged>(ctx, g, s) : launch<false, true, kMaxKeysRagged>(ctx, g, s);
     MLEL_TRY(check_launch("attention fp16"));
     return 1;
 }

@@ -156,10 +156,11 @@ int try_conv2d_dwconv_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, c
                          const mlel_conv2d_attr *a2, const FusedEpilogue *e2, bool launch);
 
 // ---- scores, softmax and the product with V of fp16 attention heads in one launch (attention_f16.hip) ----
-bool attention_f16_supported(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt, const mlel_tensor *v,
-                             const mlel_chain *chain);
-int try_attention_f16(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt,
-                      const mlel_tensor *v, const mlel_chain *chain);
+// `krows`: `k` is K [NB, S, 64] and neither M nor S need be a multiple of anything; else K^T [NB, 64, S]
+bool attention_f16_supported(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *k, const mlel_tensor *v,
+                             const mlel_chain *chain, bool krows);
+int try_attention_f16(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *k,
+                      const mlel_tensor *v, const mlel_chain *chain, bool krows);
 
 // ---- RESIZE of int8 images, alone (`epi` null), with its RESCALE, and with the ARGMAX behind that; ARGMAX over rows
 // (ops_resize.hip) ----

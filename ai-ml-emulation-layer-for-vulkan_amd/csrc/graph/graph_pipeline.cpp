@@ -585,6 +585,10 @@ bool scaleTensorsOk(const OpNode &rescale) {
            m->getFormat() == (rescale.rescale.scale32 ? MLEL_I32 : MLEL_I16) && s->getFormat() == MLEL_I8;
 }
 
+// Below this many blocks of 64 query rows the three launches of an attention whose rows of scores are aligned, which
+// spread over more compute units, are as fast as the one.
+constexpr int64_t kFewAttentionBlocks = 20;
+
 bool isSmallInt(int32_t dt) { return dt == MLEL_I8 || dt == MLEL_I16 || dt == MLEL_I32; }
 
 }  // namespace
@@ -831,6 +835,120 @@ void GraphPipeline::fuse() {
         }
     }
 
+    // Pattern 4a (attention over any number of keys): MATMUL(q, K^T) -> CAST [-> MUL by one value] -> softmax over the last
+    // axis -> MATMUL with V -> CAST, every value between them private, where K^T is the private result of a TRANSPOSE (and a
+    // RESHAPE) read nowhere else.  The TRANSPOSE then leaves K by rows (its last two permutation entries exchanged; the
+    // projection in front of it takes even that into its stores, pattern 4e) and the seven to eleven operators become one
+    // launch that keeps the scores on the chip (mlel_hip_attention_rows_f16).  A number of keys that pattern 7 takes, or
+    // whose rows of scores are whole 16-byte pieces while the heads give only a few blocks, is left to it and to the three
+    // launches.
+    for (const auto &opPtr : ops) {
+        OpNode &qk = *opPtr;
+        if (qk.fusedAway || qk.kind != OpKind::Matmul || qk.outputs[0]->getFormat() != MLEL_F32 || qk.outputs[0]->getRank() != 3 ||
+            qk.matmul.a_zp != 0 || qk.matmul.b_zp != 0)
+            continue;
+        // the only reader of a private value
+        const auto reader = [&](const TensorPtr &t) -> OpNode * {
+            if (!isPrivateIntermediate(*t)) return nullptr;
+            const auto users = consumersOf(ops, t.get());
+            return users.size() == 1 ? users[0] : nullptr;
+        };
+        const auto isF16 = [](const OpNode *op) { return op != nullptr && op->outputs[0]->getFormat() == MLEL_F16 && op->inputs[0]->getRank() == 3; };
+        const auto isReduce = [&](const OpNode *op, int which) {
+            return isF16(op) && op->kind == OpKind::Reduce && op->selector == which && op->axis == 2 && op->nanMode == MLEL_NAN_PROPAGATE;
+        };
+        const auto isUnary = [&](const OpNode *op, int which) { return isF16(op) && op->kind == OpKind::Unary && op->selector == which; };
+        const TensorPtr q = qk.inputs[0], kt = qk.inputs[1];
+        if (q->getFormat() != MLEL_F16 || kt->getFormat() != MLEL_F16) continue;
+        OpNode *cast = reader(qk.outputs[0]);
+        if (!isF16(cast) || cast->kind != OpKind::Cast) continue;
+        std::vector<OpNode *> folded{&qk, cast};
+        TensorPtr x = cast->outputs[0], scale;
+        if (OpNode *mul = reader(x); isF16(mul) && mul->kind == OpKind::Mul && mul->shift == 0 && mul->inputs[0].get() == x.get()) {
+            scale = mul->inputs[1];
+            if (scale->getProducer() != nullptr || scale->getFormat() != MLEL_F16 || scale->getShapeSize() != 1) continue;
+            folded.push_back(mul);
+            x = mul->outputs[0];
+        }
+        const auto two = [&](const TensorPtr &t, OpNode *&a, OpNode *&b) {
+            if (!isPrivateIntermediate(*t)) return false;
+            const auto users = consumersOf(ops, t.get());
+            if (users.size() != 2) return false;
+            a = users[0], b = users[1];
+            return true;
+        };
+        OpNode *max = nullptr, *sub = nullptr, *sum = nullptr, *mul = nullptr;
+        if (!two(x, max, sub) || !isReduce(max, MLEL_RED_MAX) || !isF16(sub) || sub->kind != OpKind::Binary ||
+            sub->selector != MLEL_BIN_SUB || sub->inputs[0].get() != x.get() || sub->inputs[1].get() != max->outputs[0].get() ||
+            reader(max->outputs[0]) != sub)
+            continue;
+        OpNode *exp = reader(sub->outputs[0]);
+        if (!isUnary(exp, MLEL_UN_EXP) || !two(exp->outputs[0], sum, mul) || !isReduce(sum, MLEL_RED_SUM)) continue;
+        OpNode *recip = reader(sum->outputs[0]);
+        if (!isUnary(recip, MLEL_UN_RECIPROCAL) || reader(recip->outputs[0]) != mul || !isF16(mul) || mul->kind != OpKind::Mul ||
+            mul->shift != 0 || mul->inputs[0].get() != exp->outputs[0].get() || mul->inputs[1].get() != recip->outputs[0].get())
+            continue;
+        const TensorPtr prob = mul->outputs[0];
+        OpNode *pv = reader(prob);
+        if (pv == nullptr || pv->kind != OpKind::Matmul || pv->inputs[0].get() != prob.get() || pv->inputs[1].get() == prob.get() ||
+            pv->matmul.a_zp != 0 || pv->matmul.b_zp != 0 || pv->outputs[0]->getFormat() != MLEL_F32)
+            continue;
+        OpNode *last = reader(pv->outputs[0]);
+        if (!isF16(last) || last->kind != OpKind::Cast || !last->outputs[0]->isPacked()) continue;
+        folded.insert(folded.end(), {max, sub, exp, sum, recip, mul, last});
+        // where K^T comes from
+        OpNode *reshape = kt->getProducer();
+        if (reshape == nullptr || reshape->fusedAway || reshape->kind != OpKind::Reshape || reader(kt) != &qk) continue;
+        OpNode *transpose = reshape->inputs[0]->getProducer();
+        if (transpose == nullptr || transpose->fusedAway || transpose->kind != OpKind::Transpose ||
+            reader(reshape->inputs[0]) != reshape)
+            continue;
+        std::vector<int64_t> moved = reshape->inputs[0]->getDimensions(), rows = kt->getDimensions();
+        const size_t r = moved.size();
+        if (r < 2 || moved[r - 1] != rows[2] || moved[r - 2] != rows[1]) continue;
+        std::swap(moved[r - 1], moved[r - 2]);
+        std::swap(rows[1], rows[2]);
+        const int64_t heads = rows[0], keys = rows[1], queries = q->getDimensions()[1];
+        const bool others = keys % 64 == 0 && keys <= 512 && queries % 64 == 0;  // pattern 7
+        if (others || (keys % 8 == 0 && heads * ((queries + 63) / 64) < kFewAttentionBlocks)) continue;
+        // the softmax chain as the kernel reads it: value 0 the first product, value 1 the scale
+        mlel_chain query{};
+        mlel_tensor scaleView{};
+        const int o = scale ? 2 : 0;
+        std::vector<mlel_chain_step> steps;
+        if (scale) steps.push_back({MLEL_CHAIN_MUL, 0, 0, 1, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_REDUCE, MLEL_RED_MAX, o, 0, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_BINARY, MLEL_BIN_SUB, o, o + 1, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_UNARY, MLEL_UN_EXP, o + 2, 0, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_REDUCE, MLEL_RED_SUM, o + 3, 0, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_UNARY, MLEL_UN_RECIPROCAL, o + 4, 0, MLEL_F16});
+        steps.push_back({MLEL_CHAIN_MUL, 0, o + 3, o + 5, MLEL_F16});
+        query.n_inputs = scale ? 2 : 1;
+        query.n_steps = static_cast<int32_t>(steps.size());
+        if (scale) {
+            scaleView = scale->view();
+            query.inputs[1] = &scaleView;
+        }
+        for (size_t i = 0; i < steps.size(); i++) query.steps[i] = steps[i];
+        const TensorDescriptor keyRows(MLEL_F16, rows, {}, TensorKind::Session);
+        const mlel_tensor qv = q->view(), kv = keyRows.view(), vv = pv->inputs[1]->view(), ov = last->outputs[0]->view();
+        if (mlel_hip_attention_rows_f16_in_kernel(&ov, &qv, &kv, &vv, &query) == 0) continue;
+        std::swap(transpose->vec[r - 1], transpose->vec[r - 2]);
+        transpose->outputs[0] = makeTensor(MLEL_F16, moved);
+        transpose->outputs[0]->setProducer(transpose);
+        reshape->inputs[0] = transpose->outputs[0];
+        reshape->outputs[0] = makeTensor(MLEL_F16, rows);
+        reshape->outputs[0]->setProducer(reshape);
+        pv->kind = OpKind::FusedAttention;
+        pv->selector = 1;
+        pv->inputs = {q, reshape->outputs[0], pv->inputs[1]};
+        if (scale) pv->inputs.push_back(scale);
+        pv->chain = steps;
+        pv->outputs[0] = last->outputs[0];
+        pv->outputs[0]->setProducer(pv);
+        for (OpNode *op : folded) op->fusedAway = true;
+    }
+
     // Pattern 4 (fp16 projections): MATMUL (fp16 x fp16 -> fp32)  [-> ADD of an fp32 constant of one or N values]
     // -> CAST to fp16.  The fused kernel adds in fp32 and rounds once to fp16, exactly like the operators it replaces.
     for (const auto &opPtr : ops) {
@@ -882,10 +1000,12 @@ void GraphPipeline::fuse() {
     // RESHAPE that splits each of NB, M, N into at most two extents, itself read only by a TRANSPOSE that keeps the
     // innermost extent innermost or makes the inner row extent the innermost one (K transposed for the scores).
     // The product then writes the transposed tensor directly, through a strided view
-    // (mlel_hip_matmul_bias_cast with a six-dimensional output); the two data-movement operators disappear.
+    // (mlel_hip_matmul_bias_cast with a six-dimensional output); the two data-movement operators disappear.  The same for
+    // the head merge behind the attention of pattern 4a.
     for (const auto &opPtr : ops) {
         OpNode &mm = *opPtr;
-        if (mm.fusedAway || mm.kind != OpKind::FusedMatmulBiasCast || mm.flag) continue;
+        const bool attention = mm.kind == OpKind::FusedAttention;
+        if (mm.fusedAway || (mm.kind != OpKind::FusedMatmulBiasCast && !attention) || mm.flag) continue;
         const TensorPtr h = mm.outputs[0];
         if (!isPrivateIntermediate(*h) || h->getRank() != 3) continue;
         auto users = consumersOf(ops, h.get());
@@ -938,7 +1058,7 @@ void GraphPipeline::fuse() {
         }
         // eight contiguous elements along the innermost column extent or, for a transposing view, along the
         // innermost row extent
-        const size_t inner = vs[5] == 2 ? 5 : 3;
+        const size_t inner = vs[5] == 2 || attention ? 5 : 3;
         bool aligned = vs[inner] == 2 && vd[inner] % 8 == 0;
         for (size_t k = 0; k < 6; k++) aligned = aligned && (k == inner || vs[k] % 16 == 0);
         if (!aligned) continue;
@@ -2238,7 +2358,7 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
                 view.strides[k] = op.viewStrides[k];
             }
         }
-        rc = mlel_hip_attention_f16(ctx, stream, &view, &in[0], &in[1], &in[2], &c);
+        rc = (op.selector == 1 ? mlel_hip_attention_rows_f16 : mlel_hip_attention_f16)(ctx, stream, &view, &in[0], &in[1], &in[2], &c);
         break;
     }
     case OpKind::FusedConv2DDepthwise: {

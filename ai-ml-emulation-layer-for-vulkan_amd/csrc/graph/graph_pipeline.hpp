@@ -146,7 +146,8 @@ class OpNode {
     // when that view's extents are non-zero
     std::vector<std::pair<std::array<int64_t, 6>, std::array<int64_t, 6>>> extraProductViews;
     // FusedAttention: inputs = {q, kt, v, the softmax chain's inputs from 1 on}; `chain` is the softmax region between
-    // the two products (its value 0 is the first product); viewDims / viewStrides as for FusedMatmulBiasCast
+    // the two products (its value 0 is the first product); viewDims / viewStrides as for FusedMatmulBiasCast; selector 1:
+    // inputs[1] is K by rows instead of K^T
     RescaleSpec scaleA, scaleB;      // FusedRescaleAddRescale: the two input stages (epilogue = output stage)
     // FusedConv2DResidual: epilogue (+ clamp) belongs to the convolution; scaleA rescales its 8-bit result, scaleB the
     // residual (inputs[3]), scaleOut their sum; `flag` is set when the residual was the addition's first operand

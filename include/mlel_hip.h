@@ -536,6 +536,12 @@ int mlel_hip_attention_f16(mlel_ctx *ctx, void *stream, const mlel_tensor *out, 
  * (data pointers are not looked at; no device is touched), else 0. */
 int mlel_hip_attention_f16_in_kernel(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *kt,
                                      const mlel_tensor *v, const mlel_chain *softmax);
+/* The same with K by rows (k [NB, S, 64], as a projection writes it without transposing) for any M and 1 <= S <= 1024:
+ * rows of any number of keys stay aligned in this layout. */
+int mlel_hip_attention_rows_f16(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *q,
+                                const mlel_tensor *k, const mlel_tensor *v, const mlel_chain *softmax);
+int mlel_hip_attention_rows_f16_in_kernel(const mlel_tensor *out, const mlel_tensor *q, const mlel_tensor *k,
+                                          const mlel_tensor *v, const mlel_chain *softmax);
 
 /* out(int8) = CLAMP?(RESCALE(DEPTHWISE_CONV2D( CLAMP?(RESCALE(CONV2D(in, w1, b1))), w2, b2 ))): the expansion (1x1,
  * unit stride, no padding) and the 3x3 depthwise stage (stride 1 or 2) of an inverted-residual block in one launch.  A
