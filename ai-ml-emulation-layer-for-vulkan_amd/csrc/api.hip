@@ -297,7 +297,8 @@ int mlel_hip_avg_pool2d(mlel_ctx *ctx, void *stream, const mlel_tensor *out, con
                  "avg_pool2d: rank 4 tensors of one type");
     MLEL_REQUIRE(attr->acc_type >= 1 && attr->acc_type <= 4, MLEL_ERR_INVALID, "Unsupported AVG_POOL2D acc type %u",
                  attr->acc_type);
-    const int rc = try_avgpool_fast(ctx, (hipStream_t)stream, out, in, attr);
+    int rc = try_avgpool_fast(ctx, (hipStream_t)stream, out, in, attr);
+    if (rc == 0) rc = try_pool_float((hipStream_t)stream, true, out, in, attr);
     if (rc != 0) return rc < 0 ? rc : 0;
     return pool_generic_launch((hipStream_t)stream, true, out, in, attr);
 }
@@ -310,7 +311,8 @@ int mlel_hip_max_pool2d(mlel_ctx *ctx, void *stream, const mlel_tensor *out, con
     MLEL_TRY(check_supported(in, "max_pool2d in"));
     MLEL_REQUIRE(out->rank == 4 && in->rank == 4 && in->dtype == out->dtype, MLEL_ERR_INVALID,
                  "max_pool2d: rank 4 tensors of one type");
-    const int rc = try_maxpool_fast(ctx, (hipStream_t)stream, out, in, attr);
+    int rc = try_maxpool_fast(ctx, (hipStream_t)stream, out, in, attr);
+    if (rc == 0) rc = try_pool_float((hipStream_t)stream, false, out, in, attr);
     if (rc != 0) return rc < 0 ? rc : 0;
     return pool_generic_launch((hipStream_t)stream, false, out, in, attr);
 }

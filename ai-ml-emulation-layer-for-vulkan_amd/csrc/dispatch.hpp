@@ -196,6 +196,8 @@ int try_avgpool_fast(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
 // ops_vec.hip: packed integer tensors, 128 bits per thread
 int try_maxpool_fast(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in,
                      const mlel_pool2d_attr *a);
+// ops_pool.hip: fp16, bf16 and fp32 images
+int try_pool_float(hipStream_t s, bool avg, const mlel_tensor *out, const mlel_tensor *in, const mlel_pool2d_attr *a);
 int try_table_fast(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in,
                    const mlel_tensor *table);
 int try_transpose_fast(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in,

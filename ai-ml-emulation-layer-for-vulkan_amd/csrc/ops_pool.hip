@@ -1,0 +1,238 @@
+// MAX_POOL2D and AVG_POOL2D over NHWC fp16, bf16 and fp32 images, 16 bytes of channels per thread (reference results:
+// maxpool2d.comp:23-72, avgpool2d.comp:27-75; the order of the fp32 additions of a large window differs from the shader's
+// loop, the operands and the accumulator keep their types).  What they decline runs one thread per element
+// (ops_generic.hip).
+//
+// A window of a few taps: one thread per piece of one output position, its taps read in the shader's order; consecutive
+// lanes hold consecutive pieces, so a wavefront reads whole pixels.  Bound by the reads: 4 x 112 x 112 x 64 fp16 into
+// 56 x 56 (2 x 2): 6.4 MB in and 1.6 MB out.
+// A window of kSplitTaps taps and more (the global average in front of a classifier: few outputs, hundreds of taps): 32
+// threads share the window of one piece, taps dealt in turn with four loads in flight, and add up through shared memory;
+// eight pieces (128 bytes of a pixel) to a block, so a tap is one whole cache line.  One thread per output walked the
+// window's 196 taps one behind the other (4 x 14 x 14 x 256 fp16: 209 us, 4 blocks on the machine).
+#include "common.hpp"
+#include "dispatch.hpp"
+
+namespace mlel {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kPieces = 8, kParts = kBlock / kPieces;
+constexpr int kSplitTaps = 32;
+
+struct PoolFloatArgs {
+    const char *x;
+    char *out;
+    int32_t H, W, OH, OW, groups;  // groups: 16-byte pieces per pixel
+    int64_t x_sn, x_sy, x_sx, o_sn, o_sy, o_sx;
+    int32_t kh, kw, sy, sx, pad_t, pad_l, zi, ignore_nan;
+    int64_t items;  // N * OH * OW * groups
+    DivMagic div_groups, div_ow, div_oh;
+};
+
+template <int DT>
+struct Piece {
+    static constexpr int n = DT == MLEL_F32 ? 4 : 8;
+    static __device__ __forceinline__ void load(const char *p, float (&v)[n]) {
+        const uint4 u = *reinterpret_cast<const uint4 *>(p);
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            if constexpr (DT == MLEL_F32)
+                v[i] = __uint_as_float(w[i]);
+            else if constexpr (DT == MLEL_BF16)
+                v[i] = __uint_as_float(i & 1 ? w[i / 2] & 0xffff0000u : w[i / 2] << 16);
+            else
+                v[i] = __half2float(__ushort_as_half((unsigned short)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu)));
+        }
+    }
+    static __device__ __forceinline__ void store(char *p, const float (&v)[n]) {
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            if constexpr (DT == MLEL_F32) {
+                w[i] = __float_as_uint(v[i]);
+            } else {
+                uint16_t h;
+                raw_st_f(reinterpret_cast<char *>(&h), DT, v[i]);
+                w[i / 2] |= (uint32_t)h << (16 * (i & 1));
+            }
+        }
+        store16_result(p, make_uint4(w[0], w[1], w[2], w[3]));
+    }
+};
+
+struct Window {
+    int n, oy, ox, group, y0, y1, x0, x1;
+};
+__device__ __forceinline__ Window window_of(const PoolFloatArgs &a, int item) {
+    Window w;
+    int rest = div_magic(item, a.div_groups);
+    w.group = item - rest * a.groups;
+    int up = div_magic(rest, a.div_ow);
+    w.ox = rest - up * a.OW;
+    w.n = div_magic(up, a.div_oh);
+    w.oy = up - w.n * a.OH;
+    const int ty = w.oy * a.sy - a.pad_t, tx = w.ox * a.sx - a.pad_l;
+    w.y0 = max(0, ty), w.y1 = min(a.H, ty + a.kh);
+    w.x0 = max(0, tx), w.x1 = min(a.W, tx + a.kw);
+    return w;
+}
+
+template <int DT, bool AVG>
+__global__ void __launch_bounds__(kBlock) pool_float_kernel(const PoolFloatArgs a) {
+    constexpr int n = Piece<DT>::n;
+    const int64_t item = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (item >= a.items) return;
+    const Window w = window_of(a, (int)item);
+    const char *xb = a.x + w.n * a.x_sn + w.group * 16;
+    float acc[n];
+#pragma unroll
+    for (int i = 0; i < n; i++) acc[i] = AVG ? 0.f : (a.ignore_nan ? NAN : dt_lowest_f(DT));
+    int count = 0;
+    auto take = [&](const float (&v)[n]) {
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            if (AVG) {
+                acc[i] += v[i] - (float)a.zi;
+            } else if (a.ignore_nan) {
+                acc[i] = isnan(v[i]) ? acc[i] : (isnan(acc[i]) || acc[i] < v[i] ? v[i] : acc[i]);
+            } else {
+                acc[i] = isnan(acc[i]) ? acc[i] : (isnan(v[i]) || acc[i] < v[i] ? v[i] : acc[i]);
+            }
+        }
+        count++;
+    };
+    for (int y = w.y0; y < w.y1; y++) {
+        const char *row = xb + y * a.x_sy;
+        int x = w.x0;
+        for (; x + 2 <= w.x1; x += 2) {  // two loads in flight
+            float v0[n], v1[n];
+            Piece<DT>::load(row + x * a.x_sx, v0);
+            Piece<DT>::load(row + (x + 1) * a.x_sx, v1);
+            take(v0);
+            take(v1);
+        }
+        for (; x < w.x1; x++) {
+            float v[n];
+            Piece<DT>::load(row + x * a.x_sx, v);
+            take(v);
+        }
+    }
+    if (AVG) {
+#pragma unroll
+        for (int i = 0; i < n; i++) acc[i] /= (float)count;
+    }
+    Piece<DT>::store(a.out + w.n * a.o_sn + w.oy * a.o_sy + w.ox * a.o_sx + w.group * 16, acc);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(kBlock) avgpool_float_split_kernel(const PoolFloatArgs a) {
+    constexpr int n = Piece<DT>::n;
+    __shared__ float partial[kParts][kPieces][n];
+    const int slot = threadIdx.x % kPieces, part = threadIdx.x / kPieces;
+    const int64_t item = (int64_t)blockIdx.x * kPieces + slot;
+    const bool live = item < a.items;
+    const Window w = window_of(a, live ? (int)item : 0);
+    const int nx = w.x1 - w.x0, count = w.y1 > w.y0 && nx > 0 ? (w.y1 - w.y0) * nx : 0;
+    const char *xb = a.x + w.n * a.x_sn + w.group * 16;
+    float acc[n];
+#pragma unroll
+    for (int i = 0; i < n; i++) acc[i] = 0.f;
+    int y = w.y0, x = w.x0 + part;
+    for (int t = part; t < count; t += 4 * kParts) {
+        float v[4][n];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            while (x >= w.x1) x -= nx, y++;
+            const bool in = t + k * kParts < count;
+            Piece<DT>::load(xb + (in ? y : w.y0) * a.x_sy + (in ? x : w.x0) * a.x_sx, v[k]);
+            x += kParts;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (t + k * kParts < count) {
+#pragma unroll
+                for (int i = 0; i < n; i++) acc[i] += v[k][i] - (float)a.zi;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < n; i++) partial[part][slot][i] = acc[i];
+    __syncthreads();
+    // one thread per value
+    if (threadIdx.x < kPieces * n) {
+        const float *p = &partial[0][0][0] + threadIdx.x;
+        float sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < kParts; k++) sum += p[k * kPieces * n];
+        partial[0][0][threadIdx.x] = sum;
+    }
+    __syncthreads();
+    if (part != 0 || !live) return;
+#pragma unroll
+    for (int i = 0; i < n; i++) acc[i] = partial[0][slot][i] / (float)count;
+    Piece<DT>::store(a.out + w.n * a.o_sn + w.oy * a.o_sy + w.ox * a.o_sx + w.group * 16, acc);
+}
+
+template <int DT>
+void launch_pool(const PoolFloatArgs &g, bool avg, bool split, hipStream_t s) {
+    const int per_block = split ? kPieces : kBlock;
+    const dim3 grid((unsigned)((g.items + per_block - 1) / per_block));
+    if (split)
+        avgpool_float_split_kernel<DT><<<grid, dim3(kBlock), 0, s>>>(g);
+    else if (avg)
+        pool_float_kernel<DT, true><<<grid, dim3(kBlock), 0, s>>>(g);
+    else
+        pool_float_kernel<DT, false><<<grid, dim3(kBlock), 0, s>>>(g);
+}
+
+}  // namespace
+
+int try_pool_float(hipStream_t s, bool avg, const mlel_tensor *out, const mlel_tensor *in, const mlel_pool2d_attr *a) {
+    const int dt = in->dtype;
+    if (dt != out->dtype || (dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32)) return 0;
+    if (avg && a->acc_type != MLEL_ACC_F32) return 0;  // a fp16 accumulator rounds after every addition: in order only
+    const int64_t N = out->dims[0], OH = out->dims[1], OW = out->dims[2], C = out->dims[3], size = dt_size(dt);
+    if (in->dims[3] != C || in->dims[0] < N || C * size % 16 != 0 || in->strides[3] != size || out->strides[3] != size) return 0;
+    for (int i = 0; i < 3; i++)
+        if (in->strides[i] % 16 != 0 || out->strides[i] % 16 != 0 || in->strides[i] < 0 || out->strides[i] < 0) return 0;
+    if (((uintptr_t)in->ptr % 16) != 0 || ((uintptr_t)out->ptr % 16) != 0) return 0;
+    const int64_t lim = int64_t(1) << 15;  // coordinates whose products stay in 32 bits
+    if (a->kernel[0] < 1 || a->kernel[1] < 1 || a->stride[0] < 1 || a->stride[1] < 1 || a->pad[0] < 0 || a->pad[2] < 0) return 0;
+    if (a->kernel[0] >= lim || a->kernel[1] >= lim || a->stride[0] >= lim || a->stride[1] >= lim || a->pad[0] >= lim ||
+        a->pad[2] >= lim || in->dims[1] >= lim || in->dims[2] >= lim || OH >= lim || OW >= lim || C >= (1 << 24))
+        return 0;
+    const int64_t groups = C * size / 16, items = N * OH * OW * groups;
+    if (items >= (int64_t(1) << 30) || N >= (int64_t(1) << 30)) return 0;
+    if (items <= 0) return 1;
+    PoolFloatArgs g{};
+    g.x = static_cast<const char *>(in->ptr);
+    g.out = static_cast<char *>(out->ptr);
+    g.H = (int)in->dims[1];
+    g.W = (int)in->dims[2];
+    g.OH = (int)OH;
+    g.OW = (int)OW;
+    g.groups = (int)groups;
+    g.x_sn = in->strides[0], g.x_sy = in->strides[1], g.x_sx = in->strides[2];
+    g.o_sn = out->strides[0], g.o_sy = out->strides[1], g.o_sx = out->strides[2];
+    g.kh = a->kernel[0], g.kw = a->kernel[1];
+    g.sy = a->stride[0], g.sx = a->stride[1];
+    g.pad_t = a->pad[0], g.pad_l = a->pad[2];
+    g.zi = a->input_zp;
+    g.ignore_nan = !avg && a->nan_mode == MLEL_NAN_IGNORE;
+    g.items = items;
+    g.div_groups = make_div_magic((uint32_t)groups);
+    g.div_ow = make_div_magic((uint32_t)OW);
+    g.div_oh = make_div_magic((uint32_t)OH);
+    const bool split = avg && (int64_t)g.kh * g.kw >= kSplitTaps && items < 256 * 256;
+    if (dt == MLEL_F16)
+        launch_pool<MLEL_F16>(g, avg, split, s);
+    else if (dt == MLEL_BF16)
+        launch_pool<MLEL_BF16>(g, avg, split, s);
+    else
+        launch_pool<MLEL_F32>(g, avg, split, s);
+    MLEL_TRY(check_launch(avg ? "avg_pool2d float" : "max_pool2d float"));
+    return 1;
+}
+
+}  // namespace mlel
