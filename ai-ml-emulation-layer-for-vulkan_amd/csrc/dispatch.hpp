@@ -121,6 +121,10 @@ int try_conv2d_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, c
                          const mlel_tensor *in2 = nullptr, bool probe = false);
 int try_tconv2d_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *w,
                    const mlel_tensor *bias, const mlel_tconv2d_attr *a, const FusedEpilogue *epi, bool probe = false);
+// the same convolutions from a piece of the image in shared memory (conv_patch_i8.hip); called by the two above
+int try_conv_patch_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *in2,
+                      const mlel_tensor *w, const mlel_tensor *bias, const FusedEpilogue *epi, int32_t zx, int32_t zw,
+                      const int32_t *pad, const int32_t *stride, const int32_t *dilation, bool transposed);
 int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
                          const mlel_matmul_attr *attr, const FusedEpilogue *epi);
 
