@@ -133,6 +133,9 @@ struct ViewDiv {
 // K per step, `buffer_load ... lds` into a ring of four unpadded stages whose 16-byte pieces are XOR-swizzled (piece p
 // of row r in slot p ^ ((r >> 2) & 3)), 128-bit operand reads without bank conflicts and without the transposing
 // reads of the K-major tile, one barrier per step, reads of the next half step issued before the multiplies of this one.
+// The ring is four stages deep, eight for the 64 x 64 tile: it is taken where a compute unit gets one or two blocks, and the
+// stages in flight are then all that hides the trip to memory.
+constexpr int ring_stages(int bm, int bn) { return bm * bn <= 64 * 64 ? 8 : 4; }
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int BKH, bool BROWS = false>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const HGemmArgs g) {
     constexpr int NT = 64 * WAVES_M * WAVES_N;  // four or eight wavefronts
@@ -221,7 +224,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const 
     };
     if constexpr (BROWS) {
         // ---- direct-to-LDS main loop (K % 32 == 0: whole 64-byte steps)
-        constexpr int BK = 64, DL_S = 4, DL_STAGE = (BM + BN) * BK;
+        constexpr int BK = 64, DL_S = ring_stages(BM, BN), DL_STAGE = (BM + BN) * BK;
         constexpr int XI = BM * 4 / NT, WI = BN * 4 / NT;  // 16-byte pieces per thread and stage
         // (request counts above 15 need the upper bits of the vmcnt field, a path no instance has exercised)
         static_assert((BM * 4) % NT == 0 && (BN * 4) % NT == 0 && (DL_S - 1) * (XI + WI) < 16, "whole pieces per thread");
@@ -572,7 +575,7 @@ void launch_k(const HGemmArgs &args, bool cast_epilogue, dim3 grid, hipStream_t 
     g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
     g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
     g.div_group = make_div_magic((uint32_t)(g.tiles_n_group > 0 ? g.tiles_n_group : 1));
-    constexpr size_t operands = BROWS ? (size_t)4 * (BM + BN) * 64
+    constexpr size_t operands = BROWS ? (size_t)ring_stages(BM, BN) * (BM + BN) * 64
                                       : (size_t)2 * BM * (BKH * 2 + 16) + (size_t)2 * BKH * (2 * BN + 32);
     constexpr size_t result = std::max((size_t)BM * (BN * 2 + 16), (size_t)BN * (BM * 2 + 16));
     constexpr size_t sm = std::max(operands, result);
@@ -761,10 +764,21 @@ int launch_args(mlel_ctx *ctx, hipStream_t s, HGemmArgs &g, bool bias_cast) {
     // tile with or without one.
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256) * NB;
     if (g.b_rows) {
-        // row-wise B: the direct-to-LDS loop; the 256 x 256 tile under the same condition as below, else 128 x 128 of
+        // row-wise B: the direct-to-LDS loop; 64 x 64 tiles where there are few, the 256 x 256 tile under the same condition as below, else 128 x 128 of
         // eight wavefronts, whatever the extents (rows beyond M or N are fetched as zeros)
         const int64_t tn128 = (N + 127) / 128;
-        if (g.groups == 1 && g.K >= 256 && tiles256 * 4 >= 3 * (int64_t)cus && tiles256 <= 2 * (int64_t)cus) {
+        const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * g.groups * NB;
+        // Few tiles (one or two of 64 x 64 per compute unit): 64 x 64 over four wavefronts.  197 rows, 1536 -> 384: 8 blocks of
+        // 128 x 128 took 15.7 us, 24 of these 6; an encoder block of 8 x 197 rows, 768 columns: 107.7 -> 100.7 us with the
+        // line at two tiles per unit, 105.7 at four.
+        if (tiles64 <= 2 * (int64_t)cus) {
+            g.tiles_m = (int)((M + 63) / 64);
+            g.tiles_n_group = (int)((N + 63) / 64);
+            g.tiles_n = g.tiles_n_group * g.groups;
+            g.total_tiles = (int)tiles64;
+            g.chunk = (int)((tiles64 + 7) / 8);
+            launch_k<64, 64, 2, 2, 32, true>(g, bias_cast, dim3((unsigned)(g.chunk * 8)), s);
+        } else if (g.groups == 1 && g.K >= 256 && tiles256 * 4 >= 3 * (int64_t)cus && tiles256 <= 2 * (int64_t)cus) {
             g.tiles_m = (int)((M + 255) / 256);
             g.tiles_n_group = (int)((N + 255) / 256);
             g.tiles_n = g.tiles_n_group;

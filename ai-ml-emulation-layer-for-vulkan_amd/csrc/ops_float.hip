@@ -1100,9 +1100,10 @@ struct RowStaticArgs {
 constexpr int kRowStaticPieces = 4;      // pieces per thread and value when a row is spread as widely as it goes
 constexpr int kRowStaticMaxPieces = 12;  // the most a thread holds when rows are packed more densely into wavefronts
 
-template <class P, int NP>
+template <class P, int NP, bool DPP>
 struct RowStaticState {
     uint4 f[P::n_full][NP];
+    uint4 col[P::n_inputs][NP];        // DPP: the per-column inputs, fetched with the rows
     uint32_t r[P::n_row];              // a per-row value, the half in both halves of the word
     uint32_t one[P::n_inputs];         // single-element inputs, likewise
     const RowStaticArgs *g;
@@ -1114,8 +1115,8 @@ struct RowStaticState {
 
 __device__ __forceinline__ uint4 splat_word(uint32_t w) { return make_uint4(w, w, w, w); }
 
-template <class P, int NP, int V>
-__device__ __forceinline__ uint4 row_static_piece(const RowStaticState<P, NP> &c, int u) {
+template <class P, int NP, bool DPP, int V>
+__device__ __forceinline__ uint4 row_static_piece(const RowStaticState<P, NP, DPP> &c, int u) {
     if constexpr (P::cls[V] == SC_FULL) {
         return c.f[P::slot[V]][u];
     } else if constexpr (P::cls[V] == SC_ROW) {
@@ -1123,17 +1124,56 @@ __device__ __forceinline__ uint4 row_static_piece(const RowStaticState<P, NP> &c
     } else if constexpr (P::cls[V] == SC_ONE) {
         return splat_word(c.one[V]);
     } else {
+        if constexpr (DPP) return c.col[V][u];
         const int sg = c.part + u * c.tpr;
         return sg < c.segs ? *reinterpret_cast<const uint4 *>(c.g->in[V] + sg * 16) : make_uint4(0, 0, 0, 0);
     }
 }
 
-template <class P, int NP, int S>
-__device__ __forceinline__ void row_static_run(RowStaticState<P, NP> &c) {
+// The left-to-right fp16 sum of a row whose 16-byte piece s lies in lane s % 16 of the row's sixteen lanes, register s / 16.
+// Every lane adds every element: v_add_f16 with the element taken from lane n of the sixteen (DPP row_newbcast), one
+// instruction per element and nothing but registers.  Bound by the chain of dependent additions, 9 clocks each.  Through
+// shared memory, with the row's first thread alone adding, it was 20 -- the reads take 5, and a wavefront with only a few of
+// its lanes active issues an addition every 8 - 19 clocks instead of every 7 when its SIMD has nothing else to run (measured
+// with 1 - 256 blocks of one row chain per wavefront).
+template <int NP>
+__device__ __forceinline__ uint32_t fold_row16(const uint4 (&f)[NP], int part, int segs) {
+    uint32_t acc = 0;
+    for (int u = 0; u < NP; u++) {  // (not unrolled: 128 additions are 1 KiB of instructions)
+        if (u * 16 >= segs) break;  // uniform
+        uint4 x = f[0];
+#pragma unroll
+        for (int k = 1; k < NP; k++)
+            if (u == k) x = f[k];  // uniform
+        const bool in = part + u * 16 < segs;
+        uint32_t lo[4] = {in ? x.x : 0u, in ? x.y : 0u, in ? x.z : 0u, in ? x.w : 0u}, hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) hi[k] = lo[k] >> 16;
+        asm volatile("s_nop 1" : "+v"(lo[0]), "+v"(lo[1]), "+v"(lo[2]), "+v"(lo[3]), "+v"(hi[0]), "+v"(hi[1]), "+v"(hi[2]), "+v"(hi[3]));
+#define MLEL_FOLD2(n, k)                                                                                                        \
+    "v_add_f16_dpp %0, %" #k ", %0 row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
+#define MLEL_FOLD8(n)                                                                                                           \
+    MLEL_FOLD2(n, 1) MLEL_FOLD2(n, 5) MLEL_FOLD2(n, 2) MLEL_FOLD2(n, 6) MLEL_FOLD2(n, 3) MLEL_FOLD2(n, 7) MLEL_FOLD2(n, 4) MLEL_FOLD2(n, 8)
+        asm volatile(MLEL_FOLD8(0) MLEL_FOLD8(1) MLEL_FOLD8(2) MLEL_FOLD8(3) MLEL_FOLD8(4) MLEL_FOLD8(5) MLEL_FOLD8(6) MLEL_FOLD8(7)
+                     MLEL_FOLD8(8) MLEL_FOLD8(9) MLEL_FOLD8(10) MLEL_FOLD8(11) MLEL_FOLD8(12) MLEL_FOLD8(13) MLEL_FOLD8(14)
+                     MLEL_FOLD8(15)
+                     : "+v"(acc)
+                     : "v"(lo[0]), "v"(lo[1]), "v"(lo[2]), "v"(lo[3]), "v"(hi[0]), "v"(hi[1]), "v"(hi[2]), "v"(hi[3]));
+#undef MLEL_FOLD8
+#undef MLEL_FOLD2
+    }
+    return acc & 0xffffu;
+}
+
+template <class P, int NP, bool DPP, int S>
+__device__ __forceinline__ void row_static_run(RowStaticState<P, NP, DPP> &c) {
     if constexpr (S < P::n_steps) {
         constexpr int OP = P::steps[S].op, A = P::steps[S].a, B = P::steps[S].b, V = P::n_inputs + S;
         constexpr bool last = S + 1 == P::n_steps;
-        if constexpr (OP == F_RED_SUM) {
+        if constexpr (OP == F_RED_SUM && DPP) {
+            const uint32_t sum = fold_row16<NP>(c.f[P::slot[A]], c.part, c.segs);
+            c.r[P::slot[V]] = sum | (sum << 16);
+        } else if constexpr (OP == F_RED_SUM) {
             // the operand into the row's staging area, then the row's first thread folds it; the row's threads are
             // lanes of one wavefront, whose shared-memory operations complete in program order
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1219,13 +1259,13 @@ __device__ __forceinline__ void row_static_run(RowStaticState<P, NP> &c) {
             const uint32_t bits = (uint32_t)__half_as_ushort(f2h(special != 0 ? __builtin_nanf("") : mx));
             c.r[P::slot[V]] = bits | (bits << 16);
         } else if constexpr (P::cls[V] == SC_ROW) {
-            uint4 r = static_apply<OP>(row_static_piece<P, NP, A>(c, 0), row_static_piece<P, NP, B>(c, 0));
+            uint4 r = static_apply<OP>(row_static_piece<P, NP, DPP, A>(c, 0), row_static_piece<P, NP, DPP, B>(c, 0));
             asm volatile("" : "+v"(r.x));  // rounded here, as the stand-alone operator rounds: no contraction across steps
             c.r[P::slot[V]] = r.x;
         } else {
 #pragma unroll
             for (int u = 0; u < NP; u++) {
-                uint4 r = static_apply<OP>(row_static_piece<P, NP, A>(c, u), row_static_piece<P, NP, B>(c, u));
+                uint4 r = static_apply<OP>(row_static_piece<P, NP, DPP, A>(c, u), row_static_piece<P, NP, DPP, B>(c, u));
                 asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z), "+v"(r.w));
                 if constexpr (last) {
                     const int sg = c.part + u * c.tpr;
@@ -1236,13 +1276,13 @@ __device__ __forceinline__ void row_static_run(RowStaticState<P, NP> &c) {
                 }
             }
         }
-        row_static_run<P, NP, S + 1>(c);
+        row_static_run<P, NP, DPP, S + 1>(c);
     }
 }
 
 // the full inputs into registers (four pieces requested at once), the single elements into both halves of a word
-template <class P, int NP, int K>
-__device__ __forceinline__ void row_static_load(RowStaticState<P, NP> &c) {
+template <class P, int NP, bool DPP, int K>
+__device__ __forceinline__ void row_static_load(RowStaticState<P, NP, DPP> &c) {
     if constexpr (K < P::n_inputs) {
         if constexpr (P::cls[K] == SC_FULL) {
 #pragma unroll
@@ -1252,28 +1292,34 @@ __device__ __forceinline__ void row_static_load(RowStaticState<P, NP> &c) {
                                          ? *reinterpret_cast<const uint4 *>(c.g->in[K] + (c.row * c.g->cols + sg * 8) * 2)
                                          : make_uint4(0, 0, 0, 0);
             }
+        } else if constexpr (P::cls[K] == SC_COL && DPP) {
+#pragma unroll
+            for (int u = 0; u < NP; u++) {
+                const int sg = c.part + u * c.tpr;
+                c.col[K][u] = sg < c.segs ? *reinterpret_cast<const uint4 *>(c.g->in[K] + sg * 16) : make_uint4(0, 0, 0, 0);
+            }
         } else if constexpr (P::cls[K] == SC_ONE) {
             const uint32_t bits = *reinterpret_cast<const uint16_t *>(c.g->in[K]);
             c.one[K] = bits | (bits << 16);
         }
-        row_static_load<P, NP, K + 1>(c);
+        row_static_load<P, NP, DPP, K + 1>(c);
     }
 }
 
-template <class P, int NP>
+template <class P, int NP, bool DPP>
 __global__ void __launch_bounds__(kBlock) row_static_f16_kernel(const RowStaticArgs g) {
     extern __shared__ __align__(16) char lds[];
-    RowStaticState<P, NP> c;
+    RowStaticState<P, NP, DPP> c;
     c.g = &g;
-    c.tpr = 1 << g.tpr_log;
+    c.tpr = DPP ? 16 : 1 << g.tpr_log;
     c.part = (int)threadIdx.x & (c.tpr - 1);
     const int rr = (int)threadIdx.x >> g.tpr_log;
     c.row = (int64_t)blockIdx.x * (kBlock >> g.tpr_log) + rr;
     c.live = c.row < g.rows;
     c.segs = g.cols >> 3;
     c.stage = lds + rr * (g.cols * 2 + 16);
-    row_static_load<P, NP, 0>(c);
-    row_static_run<P, NP, 0>(c);
+    row_static_load<P, NP, DPP, 0>(c);
+    row_static_run<P, NP, DPP, 0>(c);
 }
 
 // the chain is P's program over inputs of P's shapes (`classes`: the RowClass of every input, `ops`: FOp / F_RED_*)
@@ -1291,13 +1337,13 @@ bool matches_row_static(const mlel_chain *c, const int8_t *classes, const int *o
     return true;
 }
 
-template <class P, int NP>
+template <class P, int NP, bool DPP>
 int launch_row_static_pieces(hipStream_t s, const RowStaticArgs &g, int64_t rows, int64_t cols) {
     const int64_t rows_per_block = kBlock >> g.tpr_log;
     const int64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
     MLEL_REQUIRE(blocks < (int64_t(1) << 31), MLEL_ERR_LIMIT, "row chain: too many rows");
-    const size_t smem = (size_t)rows_per_block * (size_t)(cols * 2 + 16);
-    row_static_f16_kernel<P, NP><<<dim3((unsigned)blocks), dim3(kBlock), smem, s>>>(g);
+    const size_t smem = DPP ? 0 : (size_t)rows_per_block * (size_t)(cols * 2 + 16);
+    row_static_f16_kernel<P, NP, DPP><<<dim3((unsigned)blocks), dim3(kBlock), smem, s>>>(g);
     return check_launch("row chain (compiled program)");
 }
 
@@ -1315,15 +1361,25 @@ int launch_row_static(hipStream_t s, const mlel_tensor *out, const mlel_chain *c
     // every 4: two wavefronts fold side by side on a SIMD at full speed each, a third slows all three.  Rows are
     // therefore packed more densely (fewer threads per row, more pieces per thread) until there are at most two
     // wavefronts per SIMD of the device (256 compute units of four) or a thread is full.
+    // Sixteen lanes to a row (fold_row16) when twelve pieces a lane hold it: LayerNorm over 197 x 768 15.0 -> 5.9 us, 4096 x 768
+    // 10.9 -> 6.6, 9000 x 768 18.7 -> 12.5; the same time as the rule below from some 65 536 rows on.
     const auto pieces = [&](int log) { return (segs + (int64_t(1) << log) - 1) >> log; };
     const auto wavefronts = [&](int log) { return (rows + (64 >> log) - 1) / (64 >> log); };
+    for (int k = 0; k < c->n_inputs; k++) g.in[k] = static_cast<const char *>(c->inputs[k]->ptr);
+    if (pieces(4) <= kRowStaticMaxPieces) {
+        g.tpr_log = 4;
+        const int64_t n = pieces(4);
+        if (n <= 4) return launch_row_static_pieces<P, 4, true>(s, g, rows, cols);
+        if (n <= 6) return launch_row_static_pieces<P, 6, true>(s, g, rows, cols);
+        if (n <= 8) return launch_row_static_pieces<P, 8, true>(s, g, rows, cols);
+        return launch_row_static_pieces<P, kRowStaticMaxPieces, true>(s, g, rows, cols);
+    }
     while (tpr_log > 0 && wavefronts(tpr_log) > 2048 && pieces(tpr_log - 1) <= kRowStaticMaxPieces) tpr_log--;
     g.tpr_log = tpr_log;
-    for (int k = 0; k < c->n_inputs; k++) g.in[k] = static_cast<const char *>(c->inputs[k]->ptr);
     const int64_t np = pieces(tpr_log);
-    if (np <= 4) return launch_row_static_pieces<P, 4>(s, g, rows, cols);
-    if (np <= 8) return launch_row_static_pieces<P, 8>(s, g, rows, cols);
-    return launch_row_static_pieces<P, kRowStaticMaxPieces>(s, g, rows, cols);
+    if (np <= 4) return launch_row_static_pieces<P, 4, false>(s, g, rows, cols);
+    if (np <= 8) return launch_row_static_pieces<P, 8, false>(s, g, rows, cols);
+    return launch_row_static_pieces<P, kRowStaticMaxPieces, false>(s, g, rows, cols);
 }
 
 }  // namespace
