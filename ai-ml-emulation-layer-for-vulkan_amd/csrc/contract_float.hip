@@ -10,10 +10,10 @@
 // type reads the same 128-bit operands: one v_mfma_f32_32x32x16 per piece pair for 16-bit types, four
 // v_mfma_f32_32x32x2_f32 for fp32 (the K order inside a piece pair is permuted alike on both sides).
 //   DIRECT: every piece is 16-byte aligned: buffer loads straight into shared memory, S stages deep, one barrier per
-//           stage.  A lane carries the (tap, channel) position of its piece along K, so that padding, strides, dilation
-//           and channel counts that are no multiple of a stage cost a few vector instructions and no second pass.
-//   else:   pieces are assembled in registers (unaligned rows, a K-major W, channel counts such as 3) and stored into
-//           two stage buffers; the next stage's loads are in flight while one is multiplied.
+//           stage.  A lane carries the position of its piece along K, from which tap and channel follow, so that padding,
+//           strides, dilation and channel counts that are no multiple of a stage cost a few vector instructions.
+//   else:   pieces from any address are loaded into registers, S stages ahead, and stored into two stage buffers; a K-major W
+//           keeps its rows in shared memory and is transposed by the reads (ds_read_b64_tr_b16; fp32 reads columns).
 // Small problems: with one tile of 64 x 64 per compute unit nothing but the stage depth hides the trip to memory, so the
 // tile shrinks to 32 x 32 and the four wavefronts of a block share a stage's K instead of its rows (WK = 4), summed
 // through shared memory at the end -- no exchange between blocks.
@@ -31,6 +31,9 @@ typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) v4s lds_v4s;
 
 constexpr uint32_t kOob = 0x80000000u;
 
@@ -63,7 +66,7 @@ struct FArgs {
     char *out;
     int32_t M, N, K;                    // K in elements
     int32_t tiles_m, tiles_n, total_tiles, chunk;
-    DivMagic div_per_batch, div_tiles_n, div_ohw, div_ow;
+    DivMagic div_per_batch, div_tiles_n, div_ohw, div_ow, div_ppr;
     // X: row m is output position (image, oy, ox) of a convolution (a product: one "image" of M positions, one tap)
     int32_t IC, KW, KH, H, W, sy, sx, pt, pl, dy, dx, OHW, OW;
     uint32_t x_img, x_row, x_pix, x_bytes;  // byte strides and extent of one batch
@@ -71,6 +74,7 @@ struct FArgs {
     uint32_t ldw, w_bytes;
     int64_t x_batch, w_batch, o_batch;
     uint32_t ldo, o_bytes;
+    uint32_t ic_magic, kw_magic;  // k / IC = mulhi(k, ic_magic), tap / KW = tap kw_magic >> 16 (DIRECT)
     int32_t bias_len;
     int32_t wide_out;  // rows of the result in whole aligned 16-byte pieces
     int32_t has_clamp, clamp_nan_ignore;
@@ -95,8 +99,9 @@ __device__ __forceinline__ uint32_t load_elem(__amdgpu_buffer_rsrc_t r, uint32_t
 }
 // one wavefront-wide 16-byte-per-lane load straight into shared memory at lds_addr + 16 * lane; a lane whose offset lies
 // beyond the resource's extent leaves zeros.  The loop counts these loads itself (s_waitcnt vmcnt(N)).
-__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res)
+__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res),
+                 "s"(scalar_offset)
                  : "memory");
 }
 template <int N>
@@ -104,6 +109,20 @@ __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
+// 16 x 16: the same over four pieces
+template <typename T>
+__device__ __forceinline__ v4f multiply(uint4 w, uint4 x, v4f acc) {
+    if constexpr (std::is_same<T, _Float16>::value) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), acc, 0, 0, 0);
+    } else if constexpr (std::is_same<T, BF16>::value) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, w), __builtin_bit_cast(v8b, x), acc, 0, 0, 0);
+    } else {
+        const v4f a = __builtin_bit_cast(v4f, w), b = __builtin_bit_cast(v4f, x);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+        return acc;
+    }
+}
 template <typename T>
 __device__ __forceinline__ v16f multiply(uint4 w, uint4 x, v16f acc) {
     if constexpr (std::is_same<T, _Float16>::value) {
@@ -120,17 +139,32 @@ __device__ __forceinline__ v16f multiply(uint4 w, uint4 x, v16f acc) {
 
 // how a register-staged operand is fetched
 enum { F_PIECES = 0,   // aligned 16-byte pieces
-       F_ELEMS = 1,    // element by element along K
-       F_KMAJOR = 2 }; // W only: element by element down a column of [K][N] (consecutive lanes: consecutive columns)
+       F_ROWS = 1,     // products: 16-byte pieces of rows from any address
+       F_RUNS = 2,     // convolutions: the taps of a kernel row are one run of KW IC elements, padded to whole pieces of K, that
+                       // lie anywhere; elements outside the image or beyond the run are zeros
+       F_ELEMS = 3,    // element by element along K (convolutions dilated along the row)
+       F_KMAJOR = 4 }; // W of a product only: pieces of the rows of [K][N], from any address, transposed on their way out of
+                       // shared memory
+
+constexpr int stage_bytes(int bm, int bn, int bkb, int size, bool km) {
+    return km ? bm * bkb + (bkb / size) * (bn * size + 32) : (bm + bn) * bkb;
+}
 
 // T: operand type, TO: result type; BM x BN tile; WM x WN x WK wavefronts over rows, columns and the K of a stage
 template <typename T, typename TO, int BM, int BN, int WM, int WN, int WK, int BKB, int S, bool DIRECT, int XF, int WF>
 __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const FArgs g) {
     constexpr int NT = 64 * WM * WN * WK, E = 16 / Elem<T>::size, SZ = Elem<T>::size, SO = Elem<TO>::size;
     constexpr int PPR = BKB / 16, SH = BKB == 64 ? 2 : (BKB == 128 ? 1 : 0);
-    constexpr int KK = BKB / 32, KKW = KK / WK;  // piece pairs per stage, and per wavefront
-    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
-    constexpr int XI = BM * PPR / NT, WI = BN * PPR / NT, STAGE = (BM + BN) * BKB;
+    constexpr int MT = BM / WM >= 32 ? 32 : 16, MP = 64 / MT, AR = MT * MT / 64;  // matrix tile; its pieces of K and result registers
+    constexpr int KK = BKB / (16 * MP), KKW = KK / WK;  // matrix steps per stage, and per wavefront
+    constexpr int TM = BM / WM / MT, TN = BN / WN / MT;
+    typedef typename std::conditional<MT == 32, v16f, v4f>::type acc_t;
+    constexpr int XI = BM * PPR / NT, WI = BN * PPR / NT;
+    constexpr bool KM = WF == F_KMAJOR;
+    // a K-major W keeps its rows: the pad puts the four rows a transposing read meets (16 bits), or the two the halves of a
+    // wavefront read (fp32), on distinct banks
+    constexpr int WPITCH = BN * SZ + 32, KROWS = BKB / SZ, WCH = BN * SZ / 16;
+    constexpr int STAGE = stage_bytes(BM, BN, BKB, SZ, KM);
     static_assert((BM * PPR) % NT == 0 && (BN * PPR) % NT == 0 && KK % WK == 0 && TM >= 1 && TN >= 1, "tile shape");
     static_assert((NT / PPR) % 16 == 0, "the rows of one thread share their swizzle");
     extern __shared__ __align__(16) char smem[];
@@ -157,14 +191,14 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
         xb[i] = (int32_t)((uint32_t)img * g.x_img + (uint32_t)(oy * g.sy - g.pt) * g.x_row + (uint32_t)ix0[i] * g.x_pix);
     }
     // position along K of this thread's piece in the stage that is fetched next: element kpos = tap * IC + ic
-    int kpos = p0 * E, ic = kpos, ky = 0, kx = 0;
+    int kpos = p0 * E, ic = kpos, ky = 0, kx = 0;  // (DIRECT keeps kpos alone)
     auto wrap = [&](int &c, int &y, int &x) {
         while (c >= g.IC && y < g.KH) {
             c -= g.IC;
             if (++x == g.KW) x = 0, y++;
         }
     };
-    wrap(ic, ky, kx);
+    if constexpr (!DIRECT) wrap(ic, ky, kx);
     auto tap_off = [&](int i, int c, int y, int x) {  // offset of channel c of a tap of row i, or beyond the extent
         const int iy = iy0[i] + y * g.dy, ix = ix0[i] + x * g.dx;
         const bool in = (uint32_t)iy < (uint32_t)g.H && (uint32_t)ix < (uint32_t)g.W && y < g.KH;
@@ -177,90 +211,227 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
     };
     const int n0 = n_base + r0;
 
-    v16f acc[TM][TN];
+    acc_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+            for (int r = 0; r < AR; r++) acc[i][j][r] = 0.f;
 
-    const int h = lane >> 5, lrow = lane & 31;
-    auto compute = [&](const char *st) {  // multiplies this wavefront's share of a stage
+    const int h = lane / MT, lrow = lane % MT;
+    // this wavefront's operands of a stage; `between` runs while they are on their way, then they are multiplied
+    auto compute = [&](const char *st, auto between) {
+        uint4 xf[KKW][TM], wf[KKW][TN];
 #pragma unroll
         for (int k = 0; k < KKW; k++) {
-            const int slot = (((wave_k * KKW + k) * 2 + h) ^ ((lrow >> SH) & (PPR - 1))) * 16;
-            uint4 xf[TM], wf[TN];
+            const int slot = (((wave_k * KKW + k) * MP + h) ^ ((lrow >> SH) & (PPR - 1))) * 16;
 #pragma unroll
             for (int i = 0; i < TM; i++)
-                xf[i] = *reinterpret_cast<const uint4 *>(st + ((wave_m * TM + i) * 32 + lrow) * BKB + slot);
+                xf[k][i] = *reinterpret_cast<const uint4 *>(st + ((wave_m * TM + i) * MT + lrow) * BKB + slot);
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                wf[j] = *reinterpret_cast<const uint4 *>(st + BM * BKB + ((wave_n * TN + j) * 32 + lrow) * BKB + slot);
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = multiply<T>(wf[j], xf[i], acc[i][j]);
+            for (int j = 0; j < TN; j++) {
+                if constexpr (!KM) {
+                    wf[k][j] = *reinterpret_cast<const uint4 *>(st + BM * BKB + ((wave_n * TN + j) * MT + lrow) * BKB + slot);
+                } else if constexpr (SZ == 2) {
+                    // 16-lane group q covers columns 16 (q & 1) .., k group q / 2; its lane s points at row s / 4, columns 4 (s % 4)
+                    const char *p = st + BM * BKB + ((wave_k * KKW + k) * 16 + 8 * (lane >> 5) + ((lane & 15) >> 2)) * WPITCH +
+                                    ((wave_n * TN + j) * 32 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)p);
+                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + 4 * WPITCH));
+                    const v8s both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                    wf[k][j] = __builtin_bit_cast(uint4, both);
+                } else {
+                    const char *p = st + BM * BKB + ((wave_k * KKW + k) * 8 + 4 * h) * WPITCH + ((wave_n * TN + j) * 32 + lrow) * 4;
+                    wf[k][j] = make_uint4(*reinterpret_cast<const uint32_t *>(p), *reinterpret_cast<const uint32_t *>(p + WPITCH),
+                                          *reinterpret_cast<const uint32_t *>(p + 2 * WPITCH), *reinterpret_cast<const uint32_t *>(p + 3 * WPITCH));
+                }
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
+        between();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < KKW; k++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = multiply<T>(wf[k][j], xf[k][i], acc[i][j]);
     };
+    auto nothing = [] {};
 
-    const int nk = (g.K + PPR * E - 1) / (PPR * E);
+    const int run = g.KW * g.IC, ppr = (run + E - 1) / E;  // F_RUNS: elements and pieces of a kernel row
+    const int nk = XF == F_RUNS ? (g.KH * ppr + PPR - 1) / PPR : (g.K + PPR * E - 1) / (PPR * E);
     const char *xp = g.x + (int64_t)batch * g.x_batch, *wp = g.w + (int64_t)batch * g.w_batch;
     if constexpr (DIRECT) {
         constexpr int NLA = XI + WI;
         const v4i xres = rsrc_words(xp, g.x_bytes), wres = rsrc_words(wp, g.w_bytes);
         const uint32_t lds0 =
             (uint32_t) reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem) + (uint32_t)(wave * 1024);
-        auto request = [&](int buf) {  // the next stage into buffer `buf`; beyond K every lane fetches zeros
-            const uint32_t d = lds0 + (uint32_t)(buf * STAGE);
+        // A wavefront that has its SIMD to itself issues an instruction every 7 clocks or so, and the loop is a few dozen of
+        // them beside eight matrix instructions: what a request costs is what the loop takes.  So the taps a row meets inside
+        // the image are a bit each, the place of a piece among them comes from two multiplications, and W's rows advance by
+        // the scalar offset alone (4 x 56 x 56 x 64, 3 x 3: 0.40 -> 0.21 us per tap, of 3.9 + 9 x that).
+        uint32_t my[XI], mx[XI], wo[WI];
 #pragma unroll
-            for (int i = 0; i < XI; i++) load16_to_lds(xres, d + i * NT * 16, tap_off(i, ic, ky, kx));
+        for (int i = 0; i < XI; i++) {
+            my[i] = mx[i] = 0;
+            for (int y = 0; y < g.KH; y++) my[i] |= (uint32_t)(iy0[i] + y * g.dy) < (uint32_t)g.H ? 1u << y : 0u;  // uniform trip count
+            for (int x = 0; x < g.KW; x++) mx[i] |= (uint32_t)(ix0[i] + x * g.dx) < (uint32_t)g.W ? 1u << x : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < WI; i++) {
+            const int n = n0 + i * (NT / PPR);
+            wo[i] = n < g.N ? (uint32_t)n * g.ldw + (uint32_t)(p0 * 16) : kOob;
+        }
+        const uint32_t y_step = (uint32_t)g.dy * g.x_row, x_step = (uint32_t)g.dx * g.x_pix;
+        int asked = 0;  // stages requested so far
+        auto request = [&](int buf) {  // the next stage into buffer `buf`; beyond K there is no tap, and W is zeros
+            const uint32_t d = lds0 + (uint32_t)(buf * STAGE);
+            const int tap = (int)__umulhi((uint32_t)kpos, g.ic_magic), c = kpos - (int)__umul24((uint32_t)tap, (uint32_t)g.IC);
+            const int y = (int)(__umul24((uint32_t)tap, g.kw_magic) >> 16), x = tap - (int)__umul24((uint32_t)y, (uint32_t)g.KW);
+            const uint32_t t = __umul24((uint32_t)y, y_step) + __umul24((uint32_t)x, x_step) + (uint32_t)(c * SZ);
+            const bool partial = (asked + 1) * PPR * E > g.K;  // uniform: the last stage ends beyond K
+#pragma unroll
+            for (int i = 0; i < XI; i++) {
+                const uint32_t in = (uint32_t)(__builtin_amdgcn_sbfe((int)my[i], y, 1) & __builtin_amdgcn_sbfe((int)mx[i], x, 1));
+                uint32_t off = (in & ((uint32_t)xb[i] + t)) | (~in & kOob);
+                load16_to_lds(xres, d + i * NT * 16, off, 0);
+            }
 #pragma unroll
             for (int i = 0; i < WI; i++) {
-                const int n = n0 + i * (NT / PPR);
-                load16_to_lds(wres, d + BM * BKB + i * NT * 16,
-                              n < g.N && kpos < g.K ? (uint32_t)n * g.ldw + (uint32_t)(kpos * SZ) : kOob);
+                uint32_t off = wo[i];
+                if (partial) {
+                    off = kpos < g.K ? off : kOob;
+                    asm volatile("" : "+v"(off));  // (a branch, not a select in every stage)
+                }
+                load16_to_lds(wres, d + BM * BKB + i * NT * 16, off, (uint32_t)(asked * BKB));
             }
-            step_on();
+            kpos += PPR * E;
+            asked++;
         };
 #pragma unroll
-        for (int d = 0; d < S - 1; d++) request(d);
-        int cur = 0, nxt = S - 1;
-        for (int step = 0; step < nk; step++) {
-            // at most S - 2 stages outstanding: this thread's part of stage `step` has landed; the barrier extends that
-            // to the block, and says that every wavefront is done with the buffer the next request overwrites
-            wait_vmcnt<(S - 2) * NLA>();
+        for (int d = 0; d < S - 1; d++)
+            if (d < nk) request(d);  // uniform
+        // this thread's part of a stage has landed when at most the later stages are outstanding; the barrier extends that to
+        // the block, and says that every wavefront is done with the buffer the next request overwrites
+        auto meet = [&]() {
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            request(nxt);
-            compute(smem + cur * STAGE);
-            cur = cur + 1 == S ? 0 : cur + 1;
-            nxt = nxt + 1 == S ? 0 : nxt + 1;
+        };
+        int step = 0;
+        while (step + S - 1 < nk) {  // unrolled over the ring: a stage's place is a constant
+#pragma unroll
+            for (int d = 0; d < S; d++) {
+                if (step + S - 1 < nk) {  // uniform
+                    wait_vmcnt<(S - 2) * NLA>();
+                    meet();
+                    compute(smem + d * STAGE, [&] { request((d + S - 1) % S); });
+                    step++;
+                }
+            }
         }
-        wait_vmcnt<0>();  // requests beyond the last stage write (zeros) into the ring, which the epilogue reuses
+        int cur = step % S;
+        // the last S - 1 stages: nothing is left to request
+        auto drain = [&](auto self, auto left) {
+            constexpr int R = decltype(left)::value;
+            if constexpr (R > 0) {
+                if (nk - step >= R) {  // uniform
+                    wait_vmcnt<(R - 1) * NLA>();
+                    meet();
+                    compute(smem + cur * STAGE, nothing);
+                    cur = cur + 1 == S ? 0 : cur + 1;
+                    step++;
+                }
+                self(self, std::integral_constant<int, R - 1>{});
+            }
+        };
+        drain(drain, std::integral_constant<int, S - 1>{});
         __syncthreads();
     } else {
         const __amdgpu_buffer_rsrc_t xres = rsrc(xp, g.x_bytes), wres = rsrc(wp, g.w_bytes);
-        // W of a K-major operand: consecutive lanes hold consecutive columns, so that a column walk is coalesced
-        constexpr bool KM = WF == F_KMAJOR;
-        const int wn = KM ? tid % BN : r0, wpiece = KM ? tid / BN : 0;
-        constexpr int WSTEP = KM ? NT / BN : 0;  // pieces between two of this thread's pieces of one column
-        static_assert(!KM || NT % BN == 0 || BN % NT == 0, "columns per thread");
-        uint4 xr[XI], wr[WI];
+        struct Set {
+            uint4 x[XI], w[WI];
+        };
         auto pack = [](const uint32_t *v) {
             if constexpr (SZ == 2)
                 return make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
             else
                 return make_uint4(v[0], v[1], v[2], v[3]);
         };
-        int kstage = 0;  // first element of the stage that is fetched next
-        auto fetch = [&]() {
+        // elements lo .. hi - 1 of a piece, the others zeros
+        auto keep = [&](uint4 v, int lo, int hi) {
+            uint32_t *w = &v.x;
 #pragma unroll
-            for (int i = 0; i < XI; i++) {
-                if constexpr (XF == F_PIECES) {
-                    xr[i] = load16(xres, tap_off(i, ic, ky, kx));
+            for (int k = 0; k < 4; k++) {
+                if constexpr (SZ == 4) {
+                    w[k] = k >= lo && k < hi ? w[k] : 0u;
                 } else {
+                    const uint32_t low = 2 * k >= lo && 2 * k < hi ? 0xffffu : 0u, high = 2 * k + 1 >= lo && 2 * k + 1 < hi ? 0xffff0000u : 0u;
+                    w[k] &= low | high;
+                }
+            }
+            return v;
+        };
+        // elements lo .. hi - 1 of the piece at byte `off`: one load where the whole piece lies inside the operand, else
+        // element by element
+        auto load_run = [&](const char *base, __amdgpu_buffer_rsrc_t res, uint32_t bytes, int64_t off, int lo, int hi) {
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (lo >= hi) return v;
+            if (off >= 0 && off + 16 <= (int64_t)bytes) {
+                __builtin_memcpy(&v, base + off, 16);
+            } else {
+                uint32_t e[E];
+#pragma unroll
+                for (int k = 0; k < E; k++) e[k] = load_elem<SZ>(res, k >= lo && k < hi ? (uint32_t)(off + k * SZ) : kOob);
+                return pack(e);
+            }
+            return lo > 0 || hi < E ? keep(v, lo, hi) : v;
+        };
+        // F_ROWS and F_KMAJOR walk K by a scalar offset; a row beyond the operand is its last row (its results are not stored).
+        // The stage that reaches beyond K, and whole operands of less than a piece, take load_run.
+        uint32_t xo[XI], wo[WI];
+        int back[WI];  // F_KMAJOR: elements by which the piece that would reach beyond a row lies further in front
+#pragma unroll
+        for (int i = 0; i < XI; i++) xo[i] = XF == F_ROWS ? (uint32_t)min(m_base + r0 + i * (NT / PPR), g.M - 1) * g.x_pix + (uint32_t)(p0 * 16) : 0u;
+#pragma unroll
+        for (int i = 0; i < WI; i++) {
+            const int id = i * NT + tid, n = n_base + (id % WCH) * E;
+            back[i] = KM ? min(max(n + E - g.N, 0), n) : 0;
+            wo[i] = KM ? (uint32_t)(id / WCH) * g.ldw + (uint32_t)((n - back[i]) * SZ)
+                       : (uint32_t)min(n0 + i * (NT / PPR), g.N - 1) * g.ldw + (uint32_t)(p0 * 16);
+        }
+        const bool edge = KM && n_base + BN > g.N;  // uniform
+        // a piece moved `by` elements to the front (zeros behind)
+        auto forward = [&](uint4 v, int by) {
+            const uint32_t d = (uint32_t)by * SZ / 4, sh = (uint32_t)by * SZ % 4 * 8;
+            uint32_t w[5] = {v.x, v.y, v.z, v.w, 0};
+            if (d & 1) w[0] = w[1], w[1] = w[2], w[2] = w[3], w[3] = 0;
+            if (d & 2) w[0] = w[2], w[1] = w[3], w[2] = w[3] = 0;
+            return make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], sh), __builtin_amdgcn_alignbit(w[2], w[1], sh),
+                              __builtin_amdgcn_alignbit(w[3], w[2], sh), __builtin_amdgcn_alignbit(w[4], w[3], sh));
+        };
+        const bool tiny = (XF == F_ROWS && g.x_bytes < 16) || g.w_bytes < 16 || (KM && g.N < E);
+        int stage_k = 0;            // first element (F_RUNS: first piece) of the stage that is fetched next
+        auto fetch = [&](Set &r) {
+            if constexpr (XF == F_RUNS) {
+                const int pi = stage_k + p0, y = div_magic(pi, g.div_ppr), q = pi - y * ppr, e0 = q * E;
+#pragma unroll
+                for (int i = 0; i < XI; i++) {
+                    const bool in = (uint32_t)(iy0[i] + y * g.dy) < (uint32_t)g.H && y < g.KH;
+                    const int lo = min(max(-ix0[i], 0), g.KW) * g.IC - e0, hi = min(g.W - ix0[i], g.KW) * g.IC - e0;
+                    r.x[i] = load_run(xp, xres, g.x_bytes, (int64_t)xb[i] + (int64_t)(y * g.dy) * g.x_row + e0 * SZ, lo, in ? hi : INT32_MIN);
+                }
+#pragma unroll
+                for (int i = 0; i < WI; i++) {
+                    const int n = n0 + i * (NT / PPR);
+                    r.w[i] = load_run(wp, wres, g.w_bytes, (int64_t)n * g.ldw + (int64_t)(y * run + e0) * SZ, 0,
+                                      n < g.N && y < g.KH ? run - e0 : 0);
+                }
+            } else if constexpr (XF == F_ELEMS) {
+#pragma unroll
+                for (int i = 0; i < XI; i++) {
                     uint32_t v[E];
                     int c = ic, y = ky, x = kx;
 #pragma unroll
@@ -272,59 +443,112 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
                             if (++x == g.KW) x = 0, y++;
                         }
                     }
-                    xr[i] = pack(v);
+                    r.x[i] = pack(v);
                 }
-            }
 #pragma unroll
-            for (int i = 0; i < WI; i++) {
-                if constexpr (KM) {
-                    const int n = n_base + wn, k = kstage + (wpiece + i * WSTEP) * E;
+                for (int i = 0; i < WI; i++) {
+                    const int n = n0 + i * (NT / PPR);
                     uint32_t v[E];
 #pragma unroll
                     for (int e = 0; e < E; e++)
-                        v[e] = load_elem<SZ>(wres, n < g.N && k + e < g.K ? (uint32_t)(k + e) * g.ldw + (uint32_t)(n * SZ) : kOob);
-                    wr[i] = pack(v);
-                } else {
-                    const int n = n0 + i * (NT / PPR);
-                    const uint32_t off = (uint32_t)n * g.ldw + (uint32_t)(kpos * SZ);
-                    if constexpr (WF == F_PIECES) {
-                        wr[i] = load16(wres, n < g.N && kpos < g.K ? off : kOob);
-                    } else {
-                        uint32_t v[E];
+                        v[e] = load_elem<SZ>(wres, n < g.N && kpos + e < g.K ? (uint32_t)n * g.ldw + (uint32_t)((kpos + e) * SZ) : kOob);
+                    r.w[i] = pack(v);
+                }
+            } else {  // the stage that reaches beyond K, and operands of less than a piece
 #pragma unroll
-                        for (int e = 0; e < E; e++) v[e] = load_elem<SZ>(wres, n < g.N && kpos + e < g.K ? off + e * SZ : kOob);
-                        wr[i] = pack(v);
+                for (int i = 0; i < XI; i++)
+                    r.x[i] = load_run(xp, xres, g.x_bytes, (int64_t)stage_k * SZ + xo[i], 0, g.K - stage_k - p0 * E);
+#pragma unroll
+                for (int i = 0; i < WI; i++) {
+                    if constexpr (KM) {
+                        const int id = i * NT + tid, k = stage_k + id / WCH, n = n_base + (id % WCH) * E;
+                        r.w[i] = load_run(wp, wres, g.w_bytes, (int64_t)k * g.ldw + (int64_t)(n - back[i]) * SZ, 0, k < g.K && n < g.N ? E : 0);
+                    } else {
+                        r.w[i] = load_run(wp, wres, g.w_bytes, (int64_t)stage_k * SZ + wo[i], 0, g.K - stage_k - p0 * E);
                     }
                 }
             }
-            step_on();
-            kstage += PPR * E;
+            if constexpr (XF == F_ELEMS) step_on();
+            stage_k += XF == F_RUNS ? PPR : PPR * E;
         };
-        auto store = [&](char *st) {
+        auto store = [&](char *st, const Set &r) {
 #pragma unroll
-            for (int i = 0; i < XI; i++) *reinterpret_cast<uint4 *>(st + (i * NT + tid) * 16) = xr[i];
+            for (int i = 0; i < XI; i++) *reinterpret_cast<uint4 *>(st + (i * NT + tid) * 16) = r.x[i];
 #pragma unroll
             for (int i = 0; i < WI; i++) {
-                if constexpr (KM) {
-                    const int p = wpiece + i * WSTEP;
-                    *reinterpret_cast<uint4 *>(st + BM * BKB + wn * BKB + ((p ^ ((wn >> SH) & (PPR - 1))) * 16)) = wr[i];
-                } else {
-                    *reinterpret_cast<uint4 *>(st + BM * BKB + (i * NT + tid) * 16) = wr[i];
-                }
+                const int id = i * NT + tid;
+                uint4 v = r.w[i];
+                if (edge) v = forward(v, back[i]);
+                *reinterpret_cast<uint4 *>(st + BM * BKB + (KM ? (id / WCH) * WPITCH + (id % WCH) * 16 : id * 16)) = v;
             }
         };
-        fetch();
-        store(smem);
-        if (nk > 1) fetch();
-        __syncthreads();
-        for (int step = 0; step < nk; step++) {
-            // (the barrier below closes the step that read the buffer stored to here)
-            if (step + 1 < nk) {
-                store(smem + ((step + 1) & 1) * STAGE);
-                if (step + 2 < nk) fetch();
+        // S register sets, two stage buffers: stage s passes through set s % S and buffer s % 2, and is asked for S stages
+        // before it is stored
+        static_assert(S % 2 == 0, "a set meets one buffer");
+        Set r[S];
+        if constexpr (XF == F_ROWS) {
+            // The whole stages without a condition around a load -- behind one the compiler no longer knows how many loads are
+            // on their way, and waits for all of them; requests beyond the last whole stage ask for it again.
+            const int nkw = tiny ? 0 : g.K / (PPR * E);
+            auto ask = [&](Set &v, int stage) {
+                stage = min(stage, nkw - 1);
+                const char *xa = xp + (int64_t)stage * BKB, *wa = wp + (int64_t)stage * (KM ? (int64_t)KROWS * g.ldw : BKB);
+#pragma unroll
+                for (int i = 0; i < XI; i++) __builtin_memcpy(&v.x[i], xa + xo[i], 16);
+#pragma unroll
+                for (int i = 0; i < WI; i++) __builtin_memcpy(&v.w[i], wa + wo[i], 16);
+            };
+            if (nkw > 0) {  // uniform
+#pragma unroll
+                for (int d = 0; d < S; d++) ask(r[d], d);
+                store(smem, r[0]);
+                ask(r[0], S);
+                __syncthreads();
+                int step = 0;
+                for (; step + S <= nkw; step += S) {
+#pragma unroll
+                    for (int d = 0; d < S; d++) {
+                        store(smem + ((d + 1) & 1) * STAGE, r[(d + 1) % S]);
+                        ask(r[(d + 1) % S], step + d + 1 + S);
+                        compute(smem + (d & 1) * STAGE, nothing);
+                        __syncthreads();
+                    }
+                }
+#pragma unroll
+                for (int d = 0; d + 1 < S; d++) {
+                    if (step + d < nkw) {  // uniform
+                        store(smem + ((d + 1) & 1) * STAGE, r[(d + 1) % S]);
+                        compute(smem + (d & 1) * STAGE, nothing);
+                        __syncthreads();
+                    }
+                }
             }
-            compute(smem + (step & 1) * STAGE);
+            stage_k = nkw * PPR * E;
+            while (stage_k < g.K) {  // (tiny operands: all of their stages)
+                fetch(r[0]);
+                store(smem, r[0]);
+                __syncthreads();
+                compute(smem, nothing);
+                __syncthreads();
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < S; d++)
+                if (d < nk) fetch(r[d]);
+            store(smem, r[0]);
+            if (S < nk) fetch(r[0]);
             __syncthreads();
+            for (int step = 0; step < nk; step += S) {
+#pragma unroll
+                for (int d = 0; d < S; d++) {
+                    if (step + d < nk) {  // uniform
+                        if (step + d + 1 < nk) store(smem + ((d + 1) & 1) * STAGE, r[(d + 1) % S]);
+                        if (step + d + 1 + S < nk) fetch(r[(d + 1) % S]);
+                        compute(smem + (d & 1) * STAGE, nothing);
+                        __syncthreads();
+                    }
+                }
+            }
         }
     }
 
@@ -337,8 +561,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
 #pragma unroll
                 for (int j = 0; j < TN; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        red[((((wave_k - 1) * WM * WN + wave / WK) * TM * TN + i * TN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+                    for (int r = 0; r < AR; r++)
+                        red[((((wave_k - 1) * WM * WN + wave / WK) * TM * TN + i * TN + j) * AR + r) * 64 + lane] = acc[i][j][r];
         }
         __syncthreads();
         if (wave_k == 0) {
@@ -349,30 +573,30 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
 #pragma unroll
                     for (int j = 0; j < TN; j++)
 #pragma unroll
-                        for (int r = 0; r < 16; r++)
-                            acc[i][j][r] += red[(((s * WM * WN + wave / WK) * TM * TN + i * TN + j) * 16 + r) * 64 + lane];
+                        for (int r = 0; r < AR; r++)
+                            acc[i][j][r] += red[(((s * WM * WN + wave / WK) * TM * TN + i * TN + j) * AR + r) * 64 + lane];
         }
         __syncthreads();
     }
 
-    // ---- bias and rounding, then through shared memory: a lane holds row m = lane % 32 of a sub-tile and, per register
-    // quad q, columns 8q + 4 * (lane / 32) ..; the stores below write whole runs of a row
+    // ---- bias and rounding, then through shared memory: a lane holds row m = lane % MT of a sub-tile and, per register
+    // quad q, columns 4 MP q + 4 * (lane / MT) ..; the stores below write whole runs of a row
     constexpr int OP = BN * SO + 16;
     const __amdgpu_buffer_rsrc_t bres = rsrc(g.bias, g.bias != nullptr ? (uint32_t)(g.bias_len * SO) : 0u);
     if (WK == 1 || wave_k == 0) {
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            float b[16];
+            float b[AR];
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int n = n_base + (wave_n * TN + j) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+            for (int r = 0; r < AR; r++) {
+                const int n = n_base + (wave_n * TN + j) * MT + 4 * MP * (r >> 2) + 4 * h + (r & 3);
                 b[r] = Elem<TO>::get(load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)(n * SO)));
             }
 #pragma unroll
             for (int i = 0; i < TM; i++) {
-                char *row = smem + ((wave_m * TM + i) * 32 + lrow) * OP + ((wave_n * TN + j) * 32 + 4 * h) * SO;
+                char *row = smem + ((wave_m * TM + i) * MT + lrow) * OP + ((wave_n * TN + j) * MT + 4 * h) * SO;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
+                for (int q = 0; q < AR / 4; q++) {
                     uint32_t v[4];
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
@@ -381,9 +605,9 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
                         v[e] = Elem<TO>::put(s, false);
                     }
                     if constexpr (SO == 2)
-                        *reinterpret_cast<uint2 *>(row + 8 * q * SO) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+                        *reinterpret_cast<uint2 *>(row + 4 * MP * q * SO) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
                     else
-                        *reinterpret_cast<uint4 *>(row + 8 * q * SO) = make_uint4(v[0], v[1], v[2], v[3]);
+                        *reinterpret_cast<uint4 *>(row + 4 * MP * q * SO) = make_uint4(v[0], v[1], v[2], v[3]);
                 }
             }
         }
@@ -455,7 +679,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
 template <typename T, typename TO, int BM, int BN, int WM, int WN, int WK, int BKB, int S, bool DIRECT, int XF, int WF>
 int launch_tile(FArgs &g, int64_t batches, hipStream_t s) {
     constexpr int SO = Elem<TO>::size;
-    constexpr size_t operands = (size_t)S * (BM + BN) * BKB, result = (size_t)BM * (BN * SO + 16);
+    constexpr size_t operands = (size_t)(DIRECT ? S : 2) * stage_bytes(BM, BN, BKB, Elem<T>::size, WF == F_KMAJOR), result = (size_t)BM * (BN * SO + 16);
     constexpr size_t shares = (size_t)(WK - 1) * BM * BN * 4;
     constexpr size_t sm = std::max(operands, std::max(result, shares));
     static_assert(sm <= 160 * 1024, "shared memory of a compute unit");
@@ -467,6 +691,7 @@ int launch_tile(FArgs &g, int64_t batches, hipStream_t s) {
     g.chunk = (int)((total + 7) / 8);
     g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
     g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
+    g.div_ppr = make_div_magic((uint32_t)((g.KW * (int64_t)g.IC * Elem<T>::size + 15) / 16));
     auto kernel = contract_float_kernel<T, TO, BM, BN, WM, WN, WK, BKB, S, DIRECT, XF, WF>;
     static const bool raised = sm <= 48 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) == hipSuccess;
@@ -477,31 +702,52 @@ int launch_tile(FArgs &g, int64_t batches, hipStream_t s) {
 }
 
 // Tile choice.  128 x 128 from two tiles per compute unit on; 64 x 64 from half a tile per compute unit on; below that
-// 32 x 32 with the wavefronts sharing K.
+// 32 x 32 with the wavefronts sharing K, and 16 x 16 where even those leave half of the machine idle: the time is then the
+// chain of one block's products, four times shorter (fp32 convolutions, 7 x 13 x 96: 11.2 -> 5 us; a network of them, one image
+// of 112 x 208: 99 -> 74 us).  The ring needs no more than three stages: eight, for the blocks that have a compute unit to
+// themselves, changed nothing.
 template <typename T, typename TO, bool DIRECT, int XF, int WF>
 int launch_shape(mlel_ctx *ctx, FArgs &g, int64_t batches, hipStream_t s) {
     const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
     auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batches; };
-    constexpr int S2 = DIRECT ? 3 : 2;
     if constexpr (DIRECT) {
         if (tiles(128, 128) >= 2 * cus && g.N > 64) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 4, DIRECT, XF, WF>(g, batches, s);
+        if (tiles(64, 64) * 2 >= cus) return launch_tile<T, TO, 64, 64, 2, 2, 2, 128, 3, DIRECT, XF, WF>(g, batches, s);
+        if (tiles(32, 32) * 2 <= cus) return launch_tile<T, TO, 16, 16, 1, 1, 4, 256, 3, DIRECT, XF, WF>(g, batches, s);
+        return launch_tile<T, TO, 32, 32, 1, 1, 4, 256, 3, DIRECT, XF, WF>(g, batches, s);
     }
-    if (tiles(64, 64) * 2 >= cus) return launch_tile<T, TO, 64, 64, 2, 2, 1, 128, S2, DIRECT, XF, WF>(g, batches, s);
-    return launch_tile<T, TO, 32, 32, 1, 1, 4, 256, S2, DIRECT, XF, WF>(g, batches, s);
+    if constexpr (!DIRECT) {
+        // 128 x 128 tiles from one per compute unit on, unless most of one would be padding; products take eight wavefronts on
+        // the smaller tiles where K is long: a wavefront that has a SIMD to itself issues an instruction every 7 clocks, two
+        // share the work of a stage (7 x 4000 x 900 fp32: 32.6 -> 25.3 us, 4 x 2274 x 3609 x 32 fp16: 25.2 -> 19.6 us)
+        if (WF == F_KMAJOR && g.M > 64 && g.N > 64 && tiles(128, 128) >= cus) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 2, DIRECT, XF, WF>(g, batches, s);
+        constexpr int W2 = XF == F_ROWS ? 2 : 1;
+        if (tiles(64, 64) * 2 >= cus) {
+            if (W2 == 2 && g.K * (int64_t)Elem<T>::size >= 1024) return launch_tile<T, TO, 64, 64, 2, 2, W2, 128, 2, DIRECT, XF, WF>(g, batches, s);
+            return launch_tile<T, TO, 64, 64, 2, 2, 1, 128, 2, DIRECT, XF, WF>(g, batches, s);
+        }
+        return launch_tile<T, TO, 32, 32, 1, 1, 4 * W2, 256, 2, DIRECT, XF, WF>(g, batches, s);
+    }
+    return 0;
 }
 
-// `pieces`: both operands in aligned 16-byte pieces along K
+// quotients of one multiplication: exact for k IC < 2^32 and up to 1024 taps
+void set_tap_magics(FArgs &g) {
+    g.ic_magic = (uint32_t)((uint64_t(1) << 32) / (uint32_t)g.IC + 1);
+    g.kw_magic = 65536u / (uint32_t)g.KW + 1;
+}
+
+// `direct`: both operands in aligned 16-byte pieces along K
 template <typename T>
-int launch_conv(mlel_ctx *ctx, FArgs &g, bool pieces, hipStream_t s) {
-    return pieces ? launch_shape<T, T, true, F_PIECES, F_PIECES>(ctx, g, 1, s)
-                  : launch_shape<T, T, false, F_ELEMS, F_ELEMS>(ctx, g, 1, s);
+int launch_conv(mlel_ctx *ctx, FArgs &g, bool direct, hipStream_t s) {
+    if (direct) return launch_shape<T, T, true, F_PIECES, F_PIECES>(ctx, g, 1, s);
+    return g.dx == 1 ? launch_shape<T, T, false, F_RUNS, F_RUNS>(ctx, g, 1, s) : launch_shape<T, T, false, F_ELEMS, F_ELEMS>(ctx, g, 1, s);
 }
 template <typename T>
 int launch_product(mlel_ctx *ctx, FArgs &g, int64_t batches, bool x_pieces, bool w_pieces, bool w_kmajor, hipStream_t s) {
     if (x_pieces && w_pieces) return launch_shape<T, float, true, F_PIECES, F_PIECES>(ctx, g, batches, s);
-    if (!w_kmajor) return launch_shape<T, float, false, F_ELEMS, F_ELEMS>(ctx, g, batches, s);
-    return x_pieces ? launch_shape<T, float, false, F_PIECES, F_KMAJOR>(ctx, g, batches, s)
-                    : launch_shape<T, float, false, F_ELEMS, F_KMAJOR>(ctx, g, batches, s);
+    if (!w_kmajor) return launch_shape<T, float, false, F_ROWS, F_ROWS>(ctx, g, batches, s);
+    return launch_shape<T, float, false, F_ROWS, F_KMAJOR>(ctx, g, batches, s);
 }
 
 bool aligned16(const void *p, std::initializer_list<int64_t> strides) {
@@ -555,15 +801,19 @@ int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     g.ldo = (uint32_t)(OC * sz), g.o_bytes = (uint32_t)(M * OC * sz);
     g.bias_len = bias->dims[0] == 1 ? 1 : (int)OC;
     const bool pieces = aligned16(in->ptr, {IC * sz}) && aligned16(w->ptr, {IC * sz});
+    // the DIRECT form's taps are bits of a word and its divisions single multiplications
+    const bool direct = pieces && KH <= 32 && KW <= 32 && (K + 1024) * IC < (int64_t(1) << 32) &&
+                        g.dy * (int64_t)g.x_row < (1 << 24) && g.dx * (int64_t)g.x_pix < (1 << 24);
+    set_tap_magics(g);
     g.wide_out = aligned16(out->ptr, {OC * sz}) && (residual == nullptr || aligned16(residual->ptr, {}));
     if (clamp != nullptr) {
         g.has_clamp = 1, g.clamp_nan_ignore = clamp->nan_mode == MLEL_NAN_IGNORE;
         g.clamp_lo = (float)clamp->min_val, g.clamp_hi = (float)clamp->max_val;
         if (dt == MLEL_F16) g.clamp_lo = (float)(_Float16)g.clamp_lo, g.clamp_hi = (float)(_Float16)g.clamp_hi;
     }
-    if (dt == MLEL_F16) return launch_conv<_Float16>(ctx, g, pieces, s);
-    if (dt == MLEL_BF16) return launch_conv<BF16>(ctx, g, pieces, s);
-    return launch_conv<float>(ctx, g, pieces, s);
+    if (dt == MLEL_F16) return launch_conv<_Float16>(ctx, g, direct, s);
+    if (dt == MLEL_BF16) return launch_conv<BF16>(ctx, g, direct, s);
+    return launch_conv<float>(ctx, g, direct, s);
 }
 
 // MATMUL over fp16, bf16 or fp32 operands with an fp32 result.  Returns 1 when launched, 0 to decline.
@@ -599,7 +849,9 @@ int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     g.w_bytes = (uint32_t)(((rows ? N : K) - 1) * ldw + (rows ? K : N) * sz);
     g.ldo = (uint32_t)out->strides[1], g.o_bytes = (uint32_t)((M - 1) * out->strides[1] + N * 4);
     g.x_batch = a->strides[0], g.w_batch = b->strides[0], g.o_batch = out->strides[0];
-    const bool xp = aligned16(a->ptr, {a->strides[0], a->strides[1], K * sz});
+    set_tap_magics(g);
+    // (the DIRECT form's division by K is one multiplication)
+    const bool xp = aligned16(a->ptr, {a->strides[0], a->strides[1], K * sz}) && (K + 1024) * K < (int64_t(1) << 32);
     const bool wp = rows && aligned16(b->ptr, {b->strides[0], ldw, K * sz});
     g.wide_out = aligned16(out->ptr, {out->strides[0], out->strides[1], N * 4});
     if (dt == MLEL_F16) return launch_product<_Float16>(ctx, g, NB, xp, wp, !rows, s);

@@ -93,3 +93,59 @@ def test_matmul_float_vs_oracle(run, oracle, case, dt, b_rows):
     out = to.download()
     run.done()
     np.testing.assert_allclose(out, exp, rtol=0, atol=2e-5)
+
+
+# ---- edges of the register-staged forms: stages that reach beyond K, pieces that reach beyond a row or the operand,
+# operands of less than a piece, tiles of every size
+EDGES = [
+    # batches, m, k, n
+    (1, 1, 16, 1), (2, 3, 17, 5), (1, 33, 64, 31), (1, 40, 65, 33), (3, 70, 127, 72), (1, 130, 130, 129), (2, 5, 515, 40), (1, 65, 1029, 66),
+    (1, 1500, 33, 1400), (40, 150, 48, 150), (20, 190, 550, 65),
+]
+
+
+@pytest.mark.parametrize("b_rows", [False, True], ids=["k_major", "row_wise"])
+@pytest.mark.parametrize("dt", [abi.F16, abi.BF16, abi.F32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", EDGES, ids=["x".join(map(str, c)) for c in EDGES])
+def test_matmul_edges(run, case, dt, b_rows):
+    nb, m, k, n = case
+    rng = np.random.default_rng(zlib.crc32(repr(case).encode()))
+    a, b = values(rng, (nb, m, k), dt), values(rng, (nb, k, n), dt)
+    want = np.matmul(floats(a).astype(np.float64), floats(b).astype(np.float64))
+    ta, tb, to = run.put(a), run.put(b), run.new(abi.F32, (nb, m, n))
+    view = tb.view
+    if b_rows:
+        es = abi.DTYPE_SIZE[dt]
+        stored = run.put(np.ascontiguousarray(np.transpose(b, (0, 2, 1))), dt)
+        view = abi.make_tensor(stored.ptr, dt, (nb, k, n), [n * k * es, es, k * es])
+    run.dev.op("matmul", to.ref, ta.ref, C.byref(view), C.byref(abi.MatmulAttr(0, 0)))
+    got = to.download()
+    run.done()
+    np.testing.assert_allclose(got, want, rtol=0, atol=3e-6 * np.sqrt(k) * max(1.0, np.abs(want).max()))
+
+
+CONV_EDGES = [
+    # n, h, w, ic, oc, kernel, stride, dilation, pad
+    (1, 7, 9, 3, 40, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (2, 9, 8, 3, 64, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3)),
+    (1, 5, 6, 5, 7, (2, 5), (1, 1), (2, 1), (1, 1, 4, 4)), (1, 6, 5, 6, 9, (3, 3), (1, 1), (1, 2), (1, 1, 2, 2)),
+    (1, 13, 11, 24, 20, (5, 3), (1, 2), (2, 2), (4, 4, 2, 2)), (3, 30, 31, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+    (1, 6, 6, 8, 12, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)), (2, 70, 66, 40, 128, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("dt", [abi.F16, abi.BF16, abi.F32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", CONV_EDGES, ids=["_".join(map(str, c[1:5] + c[5] + c[7])) for c in CONV_EDGES])
+def test_convolution_edges(run, case, dt):
+    n, h, w, ic, oc, (kh, kw), (sy, sx), (dy, dx), pad = case
+    rng = np.random.default_rng(zlib.crc32(repr(case).encode()))
+    x, wt, b = values(rng, (n, h, w, ic), dt), values(rng, (oc, kh, kw, ic), dt, 0.2), values(rng, (oc,), dt)
+    oh, ow = (h + pad[0] + pad[1] - (kh - 1) * dy - 1) // sy + 1, (w + pad[2] + pad[3] - (kw - 1) * dx - 1) // sx + 1
+    xp = np.pad(floats(x).astype(np.float64), ((0, 0), (pad[0], pad[1]), (pad[2], pad[3]), (0, 0)))
+    want = np.zeros((n, oh, ow, oc)) + floats(b)
+    for ky in range(kh):
+        for kx in range(kw):
+            part = xp[:, ky * dy:ky * dy + (oh - 1) * sy + 1:sy, kx * dx:kx * dx + (ow - 1) * sx + 1:sx]
+            want += part @ floats(wt)[:, ky, kx].astype(np.float64).T
+    attr = abi.conv2d_attr(pad, (sy, sx), (dy, dx), acc_type=abi.ACC_F32)
+    got = floats(run.conv2d(x, wt, b, (n, oh, ow, oc), dt, attr))
+    np.testing.assert_allclose(got, want, rtol=1.01 * STEP[dt], atol=1e-5 * max(1.0, np.abs(want).max()))
