@@ -1,7 +1,7 @@
-// int8 contractions whose rows are not made of aligned 16-byte pieces, on the matrix cores: CONV2D with any channel count,
-// TRANSPOSE_CONV2D, and MATMUL with ragged K or N -- what gemm_i8.hip's fetch modes and conv_direct.hip do not take
-// (reference arithmetic: conv2d.comp:40-116, transpose_conv2d.comp:31-70, matmul.comp:30-73; RESCALE and CLAMP of the
-// fused forms: rescale.comp:27-72, clamp.comp:24-53).  int32 sums wrap, so the order of the additions is immaterial.
+// int8 convolutions whose rows are not made of aligned 16-byte pieces, on the matrix cores: CONV2D with any channel count and
+// TRANSPOSE_CONV2D -- what gemm_i8.hip's fetch modes and conv_direct.hip do not take (reference arithmetic: conv2d.comp:40-116,
+// transpose_conv2d.comp:31-70; RESCALE and CLAMP of the fused forms: rescale.comp:27-72, clamp.comp:24-53).  int32 sums wrap,
+// so the order of the additions is immaterial.
 //
 // out[m][n] = sum_k X[m][k] * W[n][k].  K is padded per tap: a tap's IC bytes are fetched in chunks of XC bytes (16, or 4
 // for few channels) wherever they lie -- the chip loads dwords from any byte address, and a loop over single bytes, which
@@ -31,15 +31,14 @@ struct IArgs {
     char *out;
     const int32_t *bias;  // or null
     int32_t bias_len;
-    int32_t M, N, batches;
+    int32_t M, N;
     int32_t tiles_m, tiles_n, total_tiles, chunk, tiles_phase;
-    DivMagic div_phase, div_per_batch, div_tiles_n, div_ohw, div_ow;
+    DivMagic div_phase, div_tiles_n, div_ohw, div_ow;
     // row m of a phase: image, y', x'; its taps (jy, jx), jy < taps_y, read input row y' * sy + base_y + jy * dy.
     // CONV2D has one phase (phase_y = phase_x = 1); TRANSPOSE_CONV2D has sy x sx, of unit stride and dy = dx = -1
     int32_t IC, IC1, KH, KW, H, W, OHW, OW;  // OHW, OW: positions of a phase per image and per row; IC1: channels of x
     int32_t sy, sx, pt, pl, dy, dx, phase_y, phase_x;
     int32_t out_h, out_w;               // extents of the output image
-    int64_t x_batch, w_batch, o_batch;
     uint32_t x_pix, x_bytes, x2_bytes, ldw, w_bytes;  // x_pix: bytes from one position of x to the next
     int32_t zx, zw;
     const char *mult;
@@ -89,19 +88,17 @@ __device__ __forceinline__ int32_t sum_bytes(uint4 v, int32_t acc) {
 }
 
 // SO: bytes of a result (1: requantised int8 / uint8, 4: the int32 accumulator, or the requantised int32);
-// XC: bytes per chunk; KM: W is [K][N] (a product), else rows of K; DUAL: X is two tensors side by side along the channels
+// XC: bytes per chunk; DUAL: X is two tensors side by side along the channels
 // (CONCAT read in place: a tap's chunks are those of the first tensor, then those of the second)
-template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM, bool DUAL>
+template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool DUAL>
 __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IArgs g) {
     constexpr int NT = 64 * WM * WN * WK;
     constexpr int PPR = BKB / 16, SH = BKB == 64 ? 2 : (BKB == 128 ? 1 : 0);
     constexpr int KK = BKB / 32, KKW = KK / WK;
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr int XI = BM * PPR / NT, STAGE = (BM + BN) * BKB;
-    constexpr int QW = BN / 4 * PPR;                        // K-major: items of four columns by one piece
-    constexpr int WI = KM ? 4 : (BN * PPR + NT - 1) / NT;  // pieces of W per thread
+    constexpr int WI = (BN * PPR + NT - 1) / NT;  // pieces of W per thread
     static_assert((BM * PPR) % NT == 0 && KK % WK == 0 && TM >= 1 && TN >= 1 && (NT / PPR) % 16 == 0, "tile shape");
-    static_assert(!KM || (QW <= NT && XC == 16), "K-major items");
     extern __shared__ __align__(16) char smem[];
     int32_t *sums = reinterpret_cast<int32_t *>(smem + 2 * STAGE);  // [BM] of X, [BN] of W
     struct Scale {
@@ -113,9 +110,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     const int lin_all = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % 8u) * g.chunk + (int)(blockIdx.x / 8u));
     if (lin_all >= g.total_tiles) return;
     const int phase = div_magic(lin_all, g.div_phase), lin = lin_all - phase * g.tiles_phase;
-    const int batch = div_magic(lin, g.div_per_batch);
-    const int t_in = lin - batch * (g.tiles_m * g.tiles_n);
-    const int tile_m = div_magic(t_in, g.div_tiles_n), tile_n = t_in - tile_m * g.tiles_n;
+    const int tile_m = div_magic(lin, g.div_tiles_n), tile_n = lin - tile_m * g.tiles_n;
     const int m_base = tile_m * BM, n_base = tile_n * BN;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_k = wave % WK, wave_n = (wave / WK) % WN, wave_m = wave / (WK * WN);
@@ -139,7 +134,6 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     const int nk = (n_chunks + PPR * CP - 1) / (PPR * CP);
 
     const int r0 = tid / PPR, p0 = (tid % PPR) ^ ((r0 >> SH) & (PPR - 1));
-    const int8_t *xp = g.x + (int64_t)batch * g.x_batch, *wp = g.w + (int64_t)batch * g.w_batch;
     int32_t xb[XI], iy0[XI], ix0[XI];  // xb: index of the position the first tap meets
 #pragma unroll
     for (int i = 0; i < XI; i++) {
@@ -191,15 +185,13 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
 
     // ---- fetch: X pieces and W pieces of the next stage into one of two register sets
-    const int wq = tid % (BN / 4), wpc = tid / (BN / 4);  // K-major: column group and piece of this thread
-    int kbase = 0;                                        // K-major: first k of the stage
     // chunk c of a tap: bytes of it that are channels, and its place among the weights of the tap
     auto remaining = [&](int c) { return DUAL ? (c < cpt1 ? g.IC1 - c * XC : g.IC - g.IC1 - (c - cpt1) * XC) : g.IC - c * XC; };
     auto channel = [&](int c) { return DUAL && c >= cpt1 ? g.IC1 + (c - cpt1) * XC : c * XC; };
     auto load_x = [&](int pix, int c) {
         if (DUAL && c >= cpt1)
             return load_chunk<XC>(g.x2, (uint32_t)pix * (uint32_t)(g.IC - g.IC1) + (uint32_t)((c - cpt1) * XC), g.x2_bytes);
-        return load_chunk<XC>(xp, (uint32_t)pix * g.x_pix + (uint32_t)(c * XC), g.x_bytes);
+        return load_chunk<XC>(g.x, (uint32_t)pix * g.x_pix + (uint32_t)(c * XC), g.x_bytes);
     };
     auto fetch = [&](uint4(&xr)[XI], uint4(&wr)[WI]) {
         const bool live = jy < taps_y && taps_x > 0;
@@ -235,53 +227,35 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
                 xr[i] = make_uint4(v[0], v[1], v[2], v[3]);
             }
         }
-        if constexpr (KM) {
-            // four columns n .. n + 3 by sixteen k: dwords along a row of [K][N], transposed in registers
-            const int n = n_base + wq * 4, k = kbase + wpc * 16;
-            uint32_t d[16];
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                d[e] = 0;
-                if (tid < QW && n < g.N && k + e < g.IC)
-                    d[e] = load_chunk<4>(wp, (uint32_t)(k + e) * g.ldw + (uint32_t)n, g.w_bytes).x;
-            }
-            uint32_t t[4][4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) transpose_4x4(d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3], t[q]);
-#pragma unroll
-            for (int c = 0; c < 4; c++) wr[c] = make_uint4(t[0][c], t[1][c], t[2][c], t[3][c]);
-            kbase += PPR * 16;
-        } else {
-#pragma unroll
-            for (int i = 0; i < WI; i++) {
-                const int r = r0 + i * (NT / PPR), n = n_base + r;
-                const bool in = n < g.N && ((BN * PPR) % NT == 0 || r < BN);
-                const uint32_t row = (uint32_t)n * g.ldw;
-                if constexpr (XC == 16) {
-                    uint4 v = make_uint4(0, 0, 0, 0);
-                    if (in && live)
-                        v = load_chunk<16>(wp, row + (uint32_t)(((ky0 + jy * g.phase_y) * g.KW + kx0 + jx * g.phase_x) * g.IC + channel(cq)), g.w_bytes);
-                    if (tail) {  // uniform
-                        const int rem = remaining(cq);
-                        v = make_uint4(keep_bytes(v.x, rem), keep_bytes(v.y, rem - 4), keep_bytes(v.z, rem - 8), keep_bytes(v.w, rem - 12));
-                    }
-                    wr[i] = v;
-                } else {
-                    uint32_t v[4];
-                    int c = cq, y = jy, x = jx;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        v[e] = 0;
-                        if (in && y < taps_y)
-                            v[e] = load_chunk<4>(wp, row + (uint32_t)(((ky0 + y * g.phase_y) * g.KW + kx0 + x * g.phase_x) * g.IC + channel(c)), g.w_bytes).x;
-                        if (tail) v[e] = keep_bytes(v[e], remaining(c));
-                        if (++c == cpt) {
-                            c = 0;
-                            if (++x == taps_x) x = 0, y++;
-                        }
-                    }
-                    wr[i] = make_uint4(v[0], v[1], v[2], v[3]);
+        for (int i = 0; i < WI; i++) {
+            const int r = r0 + i * (NT / PPR), n = n_base + r;
+            const bool in = n < g.N && ((BN * PPR) % NT == 0 || r < BN);
+            const uint32_t row = (uint32_t)n * g.ldw;
+            if constexpr (XC == 16) {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (in && live)
+                    v = load_chunk<16>(g.w, row + (uint32_t)(((ky0 + jy * g.phase_y) * g.KW + kx0 + jx * g.phase_x) * g.IC + channel(cq)), g.w_bytes);
+                if (tail) {  // uniform
+                    const int rem = remaining(cq);
+                    v = make_uint4(keep_bytes(v.x, rem), keep_bytes(v.y, rem - 4), keep_bytes(v.z, rem - 8), keep_bytes(v.w, rem - 12));
                 }
+                wr[i] = v;
+            } else {
+                uint32_t v[4];
+                int c = cq, y = jy, x = jx;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[e] = 0;
+                    if (in && y < taps_y)
+                        v[e] = load_chunk<4>(g.w, row + (uint32_t)(((ky0 + y * g.phase_y) * g.KW + kx0 + x * g.phase_x) * g.IC + channel(c)), g.w_bytes).x;
+                    if (tail) v[e] = keep_bytes(v[e], remaining(c));
+                    if (++c == cpt) {
+                        c = 0;
+                        if (++x == taps_x) x = 0, y++;
+                    }
+                }
+                wr[i] = make_uint4(v[0], v[1], v[2], v[3]);
             }
         }
         cq += PPR * CP;
@@ -300,13 +274,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
         }
 #pragma unroll
         for (int i = 0; i < WI; i++) {
-            if constexpr (KM) {
-                const int r = wq * 4 + i;
-                if (tid < QW)
-                    *reinterpret_cast<uint4 *>(st + BM * BKB + r * BKB + ((wpc ^ ((r >> SH) & (PPR - 1))) * 16)) = wr[i];
-            } else if ((BN * PPR) % NT == 0 || i * NT + tid < BN * PPR) {
+            if ((BN * PPR) % NT == 0 || i * NT + tid < BN * PPR)
                 *reinterpret_cast<uint4 *>(st + BM * BKB + (i * NT + tid) * 16) = wr[i];
-            }
             if (g.zx != 0) wsum[i] = sum_bytes(wr[i], wsum[i]);  // uniform
         }
     };
@@ -359,11 +328,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     if (g.zx != 0) {
 #pragma unroll
         for (int i = 0; i < WI; i++) {
-            if constexpr (KM) {
-                if (tid < QW) atomicAdd(&sums[BM + wq * 4 + i], wsum[i]);
-            } else if ((BN * PPR) % NT == 0 || i * NT + tid < BN * PPR) {
-                atomicAdd(&sums[BM + r0 + i * (NT / PPR)], wsum[i]);
-            }
+            if ((BN * PPR) % NT == 0 || i * NT + tid < BN * PPR) atomicAdd(&sums[BM + r0 + i * (NT / PPR)], wsum[i]);
         }
     }
     if constexpr (WK > 1) {
@@ -396,7 +361,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
 
     // ---- zero points, bias, RESCALE; the tile goes through shared memory and leaves in runs of a row
     constexpr int OP = BN * SO + 16;
-    char *ob = g.out + (int64_t)batch * g.o_batch;
+    char *ob = g.out;
     // a tile that holds whole rows of a dense result is one run of memory: it is laid down without gaps and leaves in
     // 16-byte pieces whatever N is (m_base is a multiple of 32)
     const bool dense = g.phase_y * g.phase_x == 1 && g.tiles_n == 1 && (g.N * SO) % 16 != 0 && ((uintptr_t)ob % 16) == 0;
@@ -496,22 +461,21 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     }
 }
 
-template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool KM, bool DUAL>
+template <bool FUSED, int SO, int BM, int BN, int WM, int WN, int WK, int BKB, int XC, bool DUAL>
 int launch_tile(IArgs &g, hipStream_t s) {
     constexpr size_t operands = (size_t)2 * (BM + BN) * BKB, result = (size_t)BM * (BN * SO + 16);
     constexpr size_t sm = operands + (BM + BN) * 4 + BN * 32;
     static_assert(result <= operands && sm <= 64 * 1024 && operands % 16 == 0 && (BM + BN) % 4 == 0, "shared memory");
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    const int64_t per_phase = (int64_t)g.tiles_m * g.tiles_n * g.batches, total = per_phase * g.phase_y * g.phase_x;
+    const int64_t per_phase = (int64_t)g.tiles_m * g.tiles_n, total = per_phase * g.phase_y * g.phase_x;
     MLEL_REQUIRE(total < (int64_t(1) << 30), MLEL_ERR_LIMIT, "contraction: %lld tiles", (long long)total);
     g.tiles_phase = (int)per_phase;
     g.total_tiles = (int)total;
     g.chunk = (int)((total + 7) / 8);
     g.div_phase = make_div_magic((uint32_t)per_phase);
-    g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
     g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
-    auto kernel = contract_i8_kernel<FUSED, SO, BM, BN, WM, WN, WK, BKB, XC, KM, DUAL>;
+    auto kernel = contract_i8_kernel<FUSED, SO, BM, BN, WM, WN, WK, BKB, XC, DUAL>;
     static const bool raised = sm <= 48 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) == hipSuccess;
     (void)raised;
@@ -522,21 +486,20 @@ int launch_tile(IArgs &g, hipStream_t s) {
 
 // Tile choice: 32 columns when N fits them, else 64; from half a tile per compute unit on four wavefronts share the rows,
 // below that they share K over a 32 x 32 tile.
-template <bool FUSED, int SO, int XC, bool KM, bool DUAL>
+template <bool FUSED, int SO, int XC, bool DUAL>
 int launch_shape(mlel_ctx *ctx, IArgs &g, hipStream_t s) {
     const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
-    const int64_t phases = (int64_t)g.phase_y * g.phase_x * g.batches;
+    const int64_t phases = (int64_t)g.phase_y * g.phase_x;
     auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * phases; };
-    if (g.N <= 32 && tiles(128, 32) * 2 >= cus) return launch_tile<FUSED, SO, 128, 32, 4, 1, 1, 128, XC, KM, DUAL>(g, s);
-    if (g.N > 32 && tiles(64, 64) * 2 >= cus) return launch_tile<FUSED, SO, 64, 64, 2, 2, 1, 128, XC, KM, DUAL>(g, s);
-    return launch_tile<FUSED, SO, 32, 32, 1, 1, 4, 256, XC, KM, DUAL>(g, s);
+    if (g.N <= 32 && tiles(128, 32) * 2 >= cus) return launch_tile<FUSED, SO, 128, 32, 4, 1, 1, 128, XC, DUAL>(g, s);
+    if (g.N > 32 && tiles(64, 64) * 2 >= cus) return launch_tile<FUSED, SO, 64, 64, 2, 2, 1, 128, XC, DUAL>(g, s);
+    return launch_tile<FUSED, SO, 32, 32, 1, 1, 4, 256, XC, DUAL>(g, s);
 }
 
-template <int XC, bool KM>
+template <int XC>
 int launch_out(mlel_ctx *ctx, IArgs &g, bool fused, hipStream_t s) {
-    if constexpr (!KM)
-        if (g.x2 != nullptr) return launch_shape<true, 1, XC, false, true>(ctx, g, s);
-    return fused ? launch_shape<true, 1, XC, KM, false>(ctx, g, s) : launch_shape<false, 4, XC, KM, false>(ctx, g, s);
+    if (g.x2 != nullptr) return launch_shape<true, 1, XC, true>(ctx, g, s);
+    return fused ? launch_shape<true, 1, XC, false>(ctx, g, s) : launch_shape<false, 4, XC, false>(ctx, g, s);
 }
 
 constexpr int64_t kLim = (int64_t(1) << 31) - 4096;
@@ -581,7 +544,7 @@ int try_conv(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_te
     g.x = static_cast<const int8_t *>(in->ptr), g.w = static_cast<const int8_t *>(w->ptr);
     if (in2 != nullptr) g.x2 = static_cast<const int8_t *>(in2->ptr), g.x2_bytes = (uint32_t)(N * H * W * in2->dims[3]);
     g.out = static_cast<char *>(out->ptr), g.bias = static_cast<const int32_t *>(bias->ptr), g.bias_len = (int)bias->dims[0];
-    g.N = (int)OC, g.batches = 1;
+    g.N = (int)OC;
     g.IC = (int)IC, g.IC1 = (int)IC1, g.KH = (int)KH, g.KW = (int)KW, g.H = (int)H, g.W = (int)W;
     g.pt = pad[0], g.pl = pad[2];
     g.out_h = (int)OH, g.out_w = (int)OW;
@@ -600,7 +563,7 @@ int try_conv(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_te
     // chunks of 16 bytes where they waste less than a quarter of the loads' width, dwords for fewer channels
     const auto fetched = [&](int64_t c) { return (IC1 + c - 1) / c * c + (IC - IC1 + c - 1) / c * c; };
     const bool wide = fetched(16) * 4 <= fetched(4) * 5;
-    return wide ? launch_out<16, false>(ctx, g, epi != nullptr, s) : launch_out<4, false>(ctx, g, epi != nullptr, s);
+    return wide ? launch_out<16>(ctx, g, epi != nullptr, s) : launch_out<4>(ctx, g, epi != nullptr, s);
 }
 
 }  // namespace
@@ -617,33 +580,6 @@ int try_tconv2d_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const m
     const int32_t unit[2] = {1, 1};
     return try_conv(ctx, s, out, in, nullptr, w, bias, epi, a->acc_type, a->input_zp, a->weight_zp, a->out_pad, a->stride, unit,
                     true, probe);
-}
-
-int try_matmul_i8_ragged(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
-                         const mlel_matmul_attr *attr, const FusedEpilogue *epi) {
-    if (a->dtype != MLEL_I8 || b->dtype != MLEL_I8) return 0;
-    IArgs g{};
-    if (!fill_epilogue(g, out, epi)) return 0;
-    if (attr->a_zp < -128 || attr->a_zp > 127 || attr->b_zp < -128 || attr->b_zp > 127) return 0;
-    const int64_t NB = out->dims[0], M = out->dims[1], N = out->dims[2], K = a->dims[2];
-    if (NB <= 0 || M <= 0 || N <= 0 || K <= 0 || !is_packed(out)) return 0;
-    if (a->dims[0] < NB || b->dims[0] < NB || a->dims[1] < M || b->dims[1] != K || b->dims[2] < N) return 0;
-    const bool rows = K > 1 && N > 1 && b->strides[1] == 1 && b->strides[2] >= K;
-    if (a->strides[2] != 1 || a->strides[1] < K || (!rows && (b->strides[2] != 1 || b->strides[1] < N))) return 0;
-    for (const mlel_tensor *t : {a, b})
-        if (t->strides[0] < 0) return 0;
-    const int64_t ldw = rows ? b->strides[2] : b->strides[1];
-    const int64_t xb = (M - 1) * a->strides[1] + K, wb = ((rows ? N : K) - 1) * ldw + (rows ? K : N);
-    if (xb >= kLim || wb >= kLim || xb < 16 || wb < 16 || M * N * 4 >= kLim || NB >= (1 << 20)) return 0;
-    g.x = static_cast<const int8_t *>(a->ptr), g.w = static_cast<const int8_t *>(b->ptr), g.out = static_cast<char *>(out->ptr);
-    g.M = (int)M, g.N = (int)N, g.batches = (int)NB;
-    g.IC = g.IC1 = (int)K, g.KH = g.KW = 1, g.H = 1, g.W = (int)M, g.OHW = g.OW = (int)M;
-    g.sy = g.sx = g.dy = g.dx = g.phase_y = g.phase_x = 1, g.out_h = 1, g.out_w = (int)M;
-    g.div_ohw = make_div_magic((uint32_t)M), g.div_ow = make_div_magic((uint32_t)M);
-    g.x_batch = a->strides[0], g.w_batch = b->strides[0], g.o_batch = out->strides[0];
-    g.x_pix = (uint32_t)a->strides[1], g.x_bytes = (uint32_t)xb, g.ldw = (uint32_t)ldw, g.w_bytes = (uint32_t)wb;
-    g.zx = attr->a_zp, g.zw = attr->b_zp;
-    return rows ? launch_out<16, false>(ctx, g, epi != nullptr, s) : launch_out<16, true>(ctx, g, epi != nullptr, s);
 }
 
 }  // namespace mlel
