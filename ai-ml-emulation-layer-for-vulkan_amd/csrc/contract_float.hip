@@ -220,6 +220,32 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             for (int r = 0; r < AR; r++) acc[i][j][r] = 0.f;
 
     const int h = lane / MT, lrow = lane % MT;
+
+    // ---- what the epilogue needs, asked for in front of the operands (behind the loop its trip to memory stands alone): the
+    // bias of this lane's columns and the pieces of the residual.  NQ: register quads this wavefront finishes, of NB columns' worth
+    constexpr int NQ = WK == 1 ? AR / 4 * TM * TN : (AR / 4 > WK ? AR / 4 / WK : 1), NB = WK == 1 ? AR / 4 * TN : NQ;
+    static_assert(WK == 1 || TM * TN == 1, "one sub-tile where K is shared");
+    auto quad_col = [&](int u) {  // first column of quad u, within the tile
+        return WK == 1 ? (wave_n * TN + u / (AR / 4) % TN) * MT + 4 * MP * (u % (AR / 4)) + 4 * h
+                       : wave_n * TN * MT + 4 * MP * (wave_k * NQ + u) + 4 * h;
+    };
+    constexpr int OP = BN * SO + 16, OPPR = BN * SO / 16, EO = 16 / SO, NP = (BM * OPPR + NT - 1) / NT;
+    const __amdgpu_buffer_rsrc_t bres = rsrc(g.bias, g.bias != nullptr ? (uint32_t)(g.bias_len * SO) : 0u);
+    const __amdgpu_buffer_rsrc_t ores = rsrc(g.out + (int64_t)batch * g.o_batch, g.o_bytes);
+    const __amdgpu_buffer_rsrc_t rres = rsrc(g.res, g.res != nullptr ? g.o_bytes : 0u);
+    uint32_t bias_bits[NB][4], off[NP];
+    uint4 res[NP];
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            bias_bits[u][e] = load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)((n_base + quad_col(u) + e) * SO));
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int p = i * NT + tid, m = m_base + p / OPPR, n = n_base + (p % OPPR) * EO;
+        off[i] = p < BM * OPPR && m < g.M && n < g.N ? (uint32_t)m * g.ldo + (uint32_t)(n * SO) : kOob;
+        res[i] = load16(rres, g.wide_out ? off[i] : kOob);
+    }
     // this wavefront's operands of a stage; `between` runs while they are on their way, then they are multiplied
     auto compute = [&](const char *st, auto between) {
         uint4 xf[KKW][TM], wf[KKW][TN];
@@ -552,69 +578,51 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
         }
     }
 
-    // ---- the K shares of a block's wavefronts, added in ascending order of K
+    // ---- the K shares of a block's wavefronts, added in ascending order of K: they leave their quads in shared memory, and each
+    // of the first few takes an equal part of them, in every wavefront what it then rounds and stores
+    v4f own[NQ];
     if constexpr (WK > 1) {
-        float *red = reinterpret_cast<float *>(smem);
-        if (wave_k > 0) {
+        v4f *red = reinterpret_cast<v4f *>(smem) + wave / WK * (AR * 16) + lane;
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+        for (int q = 0; q < AR / 4; q++)
+            red[(wave_k * WM * WN * (AR / 4) + q) * 64] = v4f{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]};
+        __syncthreads();
+        if (wave_k < AR / 4) {
 #pragma unroll
-                for (int j = 0; j < TN; j++)
+            for (int u = 0; u < NQ; u++) {
+                own[u] = red[(wave_k * NQ + u) * 64];
 #pragma unroll
-                    for (int r = 0; r < AR; r++)
-                        red[((((wave_k - 1) * WM * WN + wave / WK) * TM * TN + i * TN + j) * AR + r) * 64 + lane] = acc[i][j][r];
+                for (int s = 1; s < WK; s++) own[u] += red[(s * WM * WN * (AR / 4) + wave_k * NQ + u) * 64];
+            }
         }
         __syncthreads();
-        if (wave_k == 0) {
+    } else {
 #pragma unroll
-            for (int s = 0; s < WK - 1; s++)
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-#pragma unroll
-                        for (int r = 0; r < AR; r++)
-                            acc[i][j][r] += red[(((s * WM * WN + wave / WK) * TM * TN + i * TN + j) * AR + r) * 64 + lane];
+        for (int u = 0; u < NQ; u++) {
+            const acc_t &t = acc[u / (AR / 4 * TN)][u / (AR / 4) % TN];
+            own[u] = v4f{t[u % (AR / 4) * 4], t[u % (AR / 4) * 4 + 1], t[u % (AR / 4) * 4 + 2], t[u % (AR / 4) * 4 + 3]};
         }
-        __syncthreads();
     }
 
     // ---- bias and rounding, then through shared memory: a lane holds row m = lane % MT of a sub-tile and, per register
     // quad q, columns 4 MP q + 4 * (lane / MT) ..; the stores below write whole runs of a row
-    constexpr int OP = BN * SO + 16;
-    const __amdgpu_buffer_rsrc_t bres = rsrc(g.bias, g.bias != nullptr ? (uint32_t)(g.bias_len * SO) : 0u);
-    if (WK == 1 || wave_k == 0) {
+    if (WK == 1 || wave_k < AR / 4) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            float b[AR];
+        for (int u = 0; u < NQ; u++) {
+            const int i = u / (AR / 4 * TN);
+            char *row = smem + ((wave_m * TM + i) * MT + lrow) * OP + quad_col(u) * SO;
+            uint32_t v[4];
 #pragma unroll
-            for (int r = 0; r < AR; r++) {
-                const int n = n_base + (wave_n * TN + j) * MT + 4 * MP * (r >> 2) + 4 * h + (r & 3);
-                b[r] = Elem<TO>::get(load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)(n * SO)));
+            for (int e = 0; e < 4; e++) {
+                float s = own[u][e];
+                if (g.bias != nullptr) s += Elem<TO>::get(bias_bits[u % NB][e]);  // uniform (-0 + 0 would lose its sign)
+                v[e] = Elem<TO>::put(s, false);
             }
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                char *row = smem + ((wave_m * TM + i) * MT + lrow) * OP + ((wave_n * TN + j) * MT + 4 * h) * SO;
-#pragma unroll
-                for (int q = 0; q < AR / 4; q++) {
-                    uint32_t v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        float s = acc[i][j][4 * q + e];
-                        if (g.bias != nullptr) s += b[4 * q + e];  // uniform (-0 + 0 would lose its sign)
-                        v[e] = Elem<TO>::put(s, false);
-                    }
-                    if constexpr (SO == 2)
-                        *reinterpret_cast<uint2 *>(row + 4 * MP * q * SO) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
-                    else
-                        *reinterpret_cast<uint4 *>(row + 4 * MP * q * SO) = make_uint4(v[0], v[1], v[2], v[3]);
-                }
-            }
+            if constexpr (SO == 2) *reinterpret_cast<uint2 *>(row) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+            else *reinterpret_cast<uint4 *>(row) = make_uint4(v[0], v[1], v[2], v[3]);
         }
     }
     __syncthreads();
-    const __amdgpu_buffer_rsrc_t ores = rsrc(g.out + (int64_t)batch * g.o_batch, g.o_bytes);
-    const __amdgpu_buffer_rsrc_t rres = rsrc(g.res, g.res != nullptr ? g.o_bytes : 0u);
     // ADD of the residual (one rounding, to nearest) and CLAMP, as the stand-alone operators compute them
     auto finish = [&](uint32_t bits, uint32_t res_bits) {
         if (g.res != nullptr) bits = Elem<TO>::put(Elem<TO>::get(bits) + Elem<TO>::get(res_bits), true);
@@ -627,51 +635,46 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
         }
         return bits;
     };
-    if (g.wide_out) {  // uniform
-        constexpr int OPPR = BN * SO / 16, EO = 16 / SO;
-        constexpr int NP = (BM * OPPR + NT - 1) / NT;
-        uint32_t off[NP];
-        uint4 res[NP];
+    auto finish16 = [&](uint4 v, uint4 r) {
+        uint32_t *w = reinterpret_cast<uint32_t *>(&v);
+        const uint32_t *rw = reinterpret_cast<const uint32_t *>(&r);
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int p = i * NT + tid, m = m_base + p / OPPR, n = n_base + (p % OPPR) * EO;
-            off[i] = p < BM * OPPR && m < g.M && n < g.N ? (uint32_t)m * g.ldo + (uint32_t)(n * SO) : kOob;
-            res[i] = make_uint4(0, 0, 0, 0);
+        for (int e = 0; e < 4; e++) {
+            if constexpr (SO == 2) w[e] = finish(w[e] & 0xffffu, rw[e] & 0xffffu) | (finish(w[e] >> 16, rw[e] >> 16) << 16);
+            else w[e] = finish(w[e], rw[e]);
         }
-        if (g.res != nullptr) {
+        return v;
+    };
 #pragma unroll
-            for (int i = 0; i < NP; i++) res[i] = load16(rres, off[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int p = i * NT + tid;
-            if (BM * OPPR % NT != 0 && p >= BM * OPPR) break;
-            uint4 v = *reinterpret_cast<const uint4 *>(smem + (p / OPPR) * OP + (p % OPPR) * 16);
-            if (g.res != nullptr || g.has_clamp) {
-                uint32_t *w = reinterpret_cast<uint32_t *>(&v);
-                const uint32_t *rw = reinterpret_cast<const uint32_t *>(&res[i]);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    if constexpr (SO == 2)
-                        w[e] = finish(w[e] & 0xffffu, rw[e] & 0xffffu) | (finish(w[e] >> 16, rw[e] >> 16) << 16);
-                    else
-                        w[e] = finish(w[e], rw[e]);
-                }
-            }
+    for (int i = 0; i < NP; i++) {
+        const int p = i * NT + tid;
+        if (BM * OPPR % NT != 0 && p >= BM * OPPR) break;
+        const char *src = smem + (p / OPPR) * OP + (p % OPPR) * 16;
+        uint4 v = *reinterpret_cast<const uint4 *>(src);
+        if (g.wide_out) {  // uniform
+            if (g.res != nullptr || g.has_clamp) v = finish16(v, res[i]);
             const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
             __builtin_amdgcn_raw_buffer_store_b128(d, ores, (int)off[i], 0, kOutAux);
+            continue;
         }
-    } else {
-        for (int p = tid; p < BM * BN; p += NT) {
-            const int r = p / BN, c = p % BN, m = m_base + r, n = n_base + c;
-            if (m >= g.M || n >= g.N) continue;
-            const uint32_t off = (uint32_t)m * g.ldo + (uint32_t)(n * SO);
-            uint32_t v;
-            if constexpr (SO == 2) v = *reinterpret_cast<const uint16_t *>(smem + r * OP + c * SO);
-            else v = *reinterpret_cast<const uint32_t *>(smem + r * OP + c * SO);
-            v = finish(v, g.res != nullptr ? load_elem<SO>(rres, off) : 0u);
-            if constexpr (SO == 2) __builtin_amdgcn_raw_buffer_store_b16((short)v, ores, (int)off, 0, kOutAux);
-            else __builtin_amdgcn_raw_buffer_store_b32((int)v, ores, (int)off, 0, kOutAux);
+        // rows that are no whole pieces: 16 bytes at any element's address, through the L2, which joins the lines that rows
+        // share; the end of a row element by element
+        if (off[i] == kOob) continue;
+        const int n = n_base + (p % OPPR) * EO;
+        if (n + EO <= g.N) {
+            if (g.res != nullptr) __builtin_memcpy(&res[i], g.res + off[i], 16);
+            if (g.res != nullptr || g.has_clamp) v = finish16(v, res[i]);
+            __builtin_memcpy(g.out + (int64_t)batch * g.o_batch + off[i], &v, 16);
+            continue;
+        }
+        for (int e = 0; e < g.N - n; e++) {
+            uint32_t x;
+            if constexpr (SO == 2) x = reinterpret_cast<const uint16_t *>(src)[e];
+            else x = reinterpret_cast<const uint32_t *>(src)[e];
+            const uint32_t at = off[i] + (uint32_t)(e * SO);
+            x = finish(x, g.res != nullptr ? load_elem<SO>(rres, at) : 0u);
+            if constexpr (SO == 2) __builtin_amdgcn_raw_buffer_store_b16((short)x, ores, (int)at, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b32((int)x, ores, (int)at, 0, 0);
         }
     }
 }
@@ -680,7 +683,7 @@ template <typename T, typename TO, int BM, int BN, int WM, int WN, int WK, int B
 int launch_tile(FArgs &g, int64_t batches, hipStream_t s) {
     constexpr int SO = Elem<TO>::size;
     constexpr size_t operands = (size_t)(DIRECT ? S : 2) * stage_bytes(BM, BN, BKB, Elem<T>::size, WF == F_KMAJOR), result = (size_t)BM * (BN * SO + 16);
-    constexpr size_t shares = (size_t)(WK - 1) * BM * BN * 4;
+    constexpr size_t shares = WK > 1 ? (size_t)WK * BM * BN * 4 : 0;
     constexpr size_t sm = std::max(operands, std::max(result, shares));
     static_assert(sm <= 160 * 1024, "shared memory of a compute unit");
     g.tiles_m = (g.M + BM - 1) / BM;

@@ -149,3 +149,20 @@ def test_convolution_edges(run, case, dt):
     attr = abi.conv2d_attr(pad, (sy, sx), (dy, dx), acc_type=abi.ACC_F32)
     got = floats(run.conv2d(x, wt, b, (n, oh, ow, oc), dt, attr))
     np.testing.assert_allclose(got, want, rtol=1.01 * STEP[dt], atol=1e-5 * max(1.0, np.abs(want).max()))
+
+
+@pytest.mark.parametrize("dt", [abi.F16, abi.F32], ids=["f16", "f32"])
+@pytest.mark.parametrize("oc", [1, 7, 20, 33, 96])
+def test_residual_of_ragged_rows(run, oc, dt):
+    """ADD and CLAMP behind a convolution whose output rows are no whole 16-byte pieces: what the operators give one by one."""
+    rng = np.random.default_rng(oc)
+    x, wt, b = values(rng, (1, 9, 11, 24), dt), values(rng, (oc, 3, 3, 24), dt, 0.2), values(rng, (oc,), dt)
+    res = values(rng, (1, 9, 11, oc), dt)
+    attr = abi.conv2d_attr((1, 1, 1, 1), acc_type=abi.ACC_F32)
+    alone = run.conv2d(x, wt, b, res.shape, dt, attr)
+    want = np.clip((alone + res).astype(res.dtype), -0.5, 1.25).astype(res.dtype)
+    tx, tw, tb, tr, to = run.put(x), run.put(wt), run.put(b), run.put(res), run.new(dt, res.shape)
+    run.dev.op("conv2d_add_clamp", to.ref, tx.ref, tw.ref, tb.ref, C.byref(attr), tr.ref, C.byref(abi.ClampAttr(-0.5, 1.25, 0)))
+    got = to.download()
+    run.done()
+    np.testing.assert_array_equal(got, want)
