@@ -266,6 +266,7 @@ FUSED_SIGNATURES = {
     "matmul_bias_cast_chain": [_T, _T, _T, _T, C.POINTER(MatmulAttr), C.POINTER(Chain)],
     "attention_f16": [_T, _T, _T, _T, C.POINTER(Chain)],
     "attention_rows_f16": [_T, _T, _T, _T, C.POINTER(Chain)],
+    "matmul_add": [_T, _T, _T, C.POINTER(MatmulAttr), _T],
     "conv2d_add_clamp": [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, C.POINTER(ClampAttr)],
     "transpose_conv2d_rescale_clamp": [_T, _T, _T, _T, C.POINTER(Tconv2dAttr), C.POINTER(Epilogue)],
     "concat_conv2d_rescale_clamp": [_T, _T, _T, _T, _T, C.POINTER(Conv2dAttr), C.POINTER(Epilogue)],
@@ -314,6 +315,7 @@ RUNTIME_SIGNATURES = {
                                                    C.POINTER(Conv2dAttr)]),
     "mlel_hip_conv2d_conv2d_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T, _T,
                                                    C.POINTER(Conv2dAttr)]),
+    "mlel_hip_matmul_add_in_kernel": (C.c_int, [_T, _T, _T, C.POINTER(MatmulAttr), _T]),
     "mlel_hip_conv2d_add_clamp_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Conv2dAttr), _T]),
     "mlel_hip_transpose_conv2d_rescale_clamp_in_kernel": (C.c_int, [_T, _T, _T, _T, C.POINTER(Tconv2dAttr)]),
     "mlel_hip_concat_conv2d_in_kernel": (C.c_int, [_T, _T, _T, _T, _T, C.POINTER(Conv2dAttr)]),

@@ -198,6 +198,24 @@ int mlel_hip_matmul(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const m
     return matmul_generic_launch((hipStream_t)stream, out, a, b, attr);
 }
 
+int mlel_hip_matmul_add_in_kernel(const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b, const mlel_matmul_attr *attr,
+                                  const mlel_tensor *row) {
+    if (out == nullptr || a == nullptr || b == nullptr || attr == nullptr || row == nullptr) return 0;
+    if (out->rank != 3 || a->rank != 3 || b->rank != 3) return 0;
+    return try_matmul_float(nullptr, nullptr, out, a, b, attr, row, true) == 1 ? 1 : 0;
+}
+
+int mlel_hip_matmul_add(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
+                        const mlel_matmul_attr *attr, const mlel_tensor *row) {
+    MLEL_TRY(require_ctx(ctx, "matmul_add"));
+    MLEL_REQUIRE(attr != nullptr && row != nullptr, MLEL_ERR_INVALID, "matmul_add: null argument");
+    for (const mlel_tensor *t : {out, a, b, row}) MLEL_TRY(check_supported(t, "matmul_add"));
+    MLEL_REQUIRE(out->rank == 3 && a->rank == 3 && b->rank == 3 && row->rank == 3, MLEL_ERR_INVALID, "matmul_add: rank must be 3");
+    const int rc = try_matmul_float(ctx, (hipStream_t)stream, out, a, b, attr, row);
+    if (rc != 0) return rc < 0 ? rc : 0;
+    return set_error(MLEL_ERR_UNSUPPORTED, "matmul_add: not a case of the one-launch kernel");
+}
+
 int mlel_hip_rescale(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *in,
                      const mlel_tensor *multiplier, const mlel_tensor *shift, const mlel_rescale_attr *attr) {
     MLEL_TRY(require_ctx(ctx, "rescale"));

@@ -819,9 +819,10 @@ int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     return launch_conv<float>(ctx, g, direct, s);
 }
 
-// MATMUL over fp16, bf16 or fp32 operands with an fp32 result.  Returns 1 when launched, 0 to decline.
+// MATMUL over fp16, bf16 or fp32 operands with an fp32 result, optionally followed by the ADD of an fp32 row (one or N values).
+// Returns 1 when launched (`probe`: when types, extents and strides are covered; pointers are not looked at), 0 to decline.
 int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
-                     const mlel_matmul_attr *attr) {
+                     const mlel_matmul_attr *attr, const mlel_tensor *bias, bool probe) {
     const int dt = a->dtype;
     if ((dt != MLEL_F16 && dt != MLEL_BF16 && dt != MLEL_F32) || b->dtype != dt || out->dtype != MLEL_F32 || attr->a_zp != 0 ||
         attr->b_zp != 0)
@@ -840,7 +841,12 @@ int try_matmul_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     if (M * a->strides[1] >= kLim || (rows ? N : K) * ldw >= kLim || M * out->strides[1] >= kLim || K >= (1 << 24) ||
         M >= (1 << 30) || N >= (1 << 30))
         return 0;
+    if (bias != nullptr && (bias->dtype != MLEL_F32 || bias->rank != 3 || !is_packed(bias) || bias->dims[0] != 1 || bias->dims[1] != 1 ||
+                            (bias->dims[2] != 1 && bias->dims[2] != N)))
+        return 0;
+    if (probe) return 1;
     FArgs g{};
+    if (bias != nullptr) g.bias = static_cast<const char *>(bias->ptr), g.bias_len = (int)bias->dims[2];
     g.x = static_cast<const char *>(a->ptr), g.w = static_cast<const char *>(b->ptr), g.out = static_cast<char *>(out->ptr);
     g.M = (int)M, g.N = (int)N, g.K = (int)K;
     g.IC = (int)K, g.KW = g.KH = 1, g.H = 1, g.W = (int)M, g.sy = g.sx = g.dy = g.dx = 1;

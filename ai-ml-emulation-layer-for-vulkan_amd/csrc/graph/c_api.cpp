@@ -304,6 +304,7 @@ std::string opLabel(const OpNode &op) {
         for (const auto &st : op.chain) reduces = reduces || st.kind == MLEL_CHAIN_REDUCE;
         return (reduces ? "ELEMENTWISE+REDUCE x" : "ELEMENTWISE x") + std::to_string(op.chain.size());
     }
+    case OpKind::FusedMatmulAdd: return "MATMUL+ADD";
     case OpKind::FusedMatmulBiasCast:
     {
         std::string name = std::string(op.hasBias ? "MATMUL+ADD+CAST" : "MATMUL+CAST") + (op.flag ? "+ADD" : "") +

@@ -996,6 +996,27 @@ void GraphPipeline::fuse() {
         if (add) add->fusedAway = true;
     }
 
+    // Pattern 4f (floating-point fully connected layer): MATMUL -> ADD of an fp32 constant of one or N values, the sum an fp32
+    // tensor, on what the one-launch kernel takes (mlel_hip_matmul_add_in_kernel decides).
+    for (const auto &opPtr : ops) {
+        OpNode &mm = *opPtr;
+        if (mm.fusedAway || mm.kind != OpKind::Matmul) continue;
+        const TensorPtr acc = mm.outputs[0];
+        if (acc->getFormat() != MLEL_F32 || !isPrivateIntermediate(*acc)) continue;
+        const auto users = consumersOf(ops, acc.get());
+        if (users.size() != 1 || users[0]->kind != OpKind::Binary || users[0]->selector != MLEL_BIN_ADD) continue;
+        OpNode *add = users[0];
+        const TensorPtr row = add->inputs[add->inputs[0].get() == acc.get() ? 1 : 0], sum = add->outputs[0];
+        if (row->getKind() != TensorKind::Constant || sum->getFormat() != MLEL_F32 || !sameShape(*acc, *sum) || !sum->isPacked()) continue;
+        const mlel_tensor o = sum->view(), a = mm.inputs[0]->view(), b = mm.inputs[1]->view(), r = row->view();
+        if (!mlel_hip_matmul_add_in_kernel(&o, &a, &b, &mm.matmul, &r)) continue;
+        mm.kind = OpKind::FusedMatmulAdd;
+        mm.inputs.push_back(row);
+        mm.outputs[0] = sum;
+        sum->setProducer(&mm);
+        add->fusedAway = true;
+    }
+
     // Pattern 4e (head split / merge behind an fp16 product): the fp16 result [NB, M, N], private, read only by a
     // RESHAPE that splits each of NB, M, N into at most two extents, itself read only by a TRANSPOSE that keeps the
     // innermost extent innermost or makes the inner row extent the innermost one (K transposed for the scores).
@@ -2241,6 +2262,7 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
     case OpKind::Reverse: rc = mlel_hip_reverse(ctx, stream, &out, &in[0], op.axis); break;
     case OpKind::Tile: rc = mlel_hip_tile(ctx, stream, &out, &in[0]); break;
     case OpKind::Select: rc = mlel_hip_select(ctx, stream, &out, &in[0], &in[1], &in[2]); break;
+    case OpKind::FusedMatmulAdd: rc = mlel_hip_matmul_add(ctx, stream, &out, &in[0], &in[1], &op.matmul, &in[2]); break;
     case OpKind::FusedConv2DFloat:
         rc = mlel_hip_conv2d_add_clamp(ctx, stream, &out, &in[0], &in[1], &in[2], &op.conv, op.flag ? &in[3] : nullptr,
                                        op.hasClamp ? &op.clamp : nullptr);

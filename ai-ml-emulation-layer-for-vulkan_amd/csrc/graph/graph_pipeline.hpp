@@ -99,7 +99,7 @@ enum class OpKind {
     // produced by the fusion pass only
     FusedConv2D, FusedDepthwiseConv2D, FusedMatmul, FusedRescaleAddRescale, FusedMatmulBiasCast, FusedElementwise,
     FusedConv2DResidual, FusedAttention, FusedConv2DDepthwise, FusedConv2DConv2D, FusedConv2DAvgPool,
-    FusedConv2DFloat, FusedTransposeConv2D, FusedConcatConv2D, FusedResize,
+    FusedConv2DFloat, FusedMatmulAdd, FusedTransposeConv2D, FusedConcatConv2D, FusedResize,
 };
 
 struct RescaleSpec {
