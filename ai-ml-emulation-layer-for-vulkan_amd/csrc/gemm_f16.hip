@@ -129,13 +129,15 @@ struct ViewDiv {
 
 // BKH: halfs of K per step (32, or 64 for long contractions: half as many barriers and LDS round trips per K)
 // BROWS: B is given row-wise, [N][K] (a weight matrix laid down transposed once, ahead of time): both operands are
-// then rows of K, and the main loop is the direct-to-LDS pipeline of the int8 kernel (gemm_i8_kernel.hpp): 64 bytes of
+// then rows of K, and the main loop is the direct-to-LDS pipeline of the int8 kernel (gemm_i8_kernel.hpp): 64 or 128 bytes of
 // K per step, `buffer_load ... lds` into a ring of four unpadded stages whose 16-byte pieces are XOR-swizzled (piece p
-// of row r in slot p ^ ((r >> 2) & 3)), 128-bit operand reads without bank conflicts and without the transposing
-// reads of the K-major tile, one barrier per step, reads of the next half step issued before the multiplies of this one.
-// The ring is four stages deep, eight for the 64 x 64 tile: it is taken where a compute unit gets one or two blocks, and the
-// stages in flight are then all that hides the trip to memory.
-constexpr int ring_stages(int bm, int bn) { return bm * bn <= 64 * 64 ? 8 : 4; }
+// of row r in slot p ^ ((r >> 2) & 3), or p ^ ((r >> 1) & 7)), 128-bit operand reads without bank conflicts and without the
+// transposing reads of the K-major tile, one barrier per step, reads of the next 16 halfs issued before the multiplies of these.
+// The ring is four stages deep, eight short ones for the 64 x 64 tile: it is taken where a compute unit gets one or two blocks,
+// and the stages in flight are then all that hides the trip to memory.  A width that is no whole number of requests per thread
+// (192 columns over eight wavefronts) is rounded up in shared memory, the rows beyond the tile fetched as zeros.
+constexpr int ring_stages(int bm, int bn, int bkh) { return bm * bn <= 64 * 64 && bkh == 32 ? 8 : 4; }
+constexpr int ring_w_pieces(int bn, int nt, int bkh) { return (bn * bkh / 8 + nt - 1) / nt; }  // of a thread
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int BKH, bool BROWS = false>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const HGemmArgs g) {
     constexpr int NT = 64 * WAVES_M * WAVES_N;  // four or eight wavefronts
@@ -148,7 +150,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const 
     constexpr int WPITCH = 2 * BN + 32;       // bytes per K row of the B tile: 4 rows x 32 B land on distinct banks
     constexpr int WROW16 = BN / 8;            // 16-byte pieces per K row
     constexpr int WCHUNKS = (BKH * WROW16) / NT;
-    static_assert((WAVES_M * WAVES_N == 4 || WAVES_M * WAVES_N == 8) && BM % XPASS == 0 && WM % 32 == 0 && WN % 32 == 0 && (BKH * WROW16) % NT == 0, "tile shape");
+    static_assert((WAVES_M * WAVES_N == 4 || WAVES_M * WAVES_N == 8) && BM % XPASS == 0 && WM % 32 == 0 && WN % 32 == 0 && (BROWS || (BKH * WROW16) % NT == 0), "tile shape");
     constexpr int XBUF = BM * XPITCH, WBUF = BKH * WPITCH;
     extern __shared__ __align__(16) char smem[];
     char *xs = smem;             // [2][BM][XPITCH]
@@ -224,33 +226,34 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const 
     };
     if constexpr (BROWS) {
         // ---- direct-to-LDS main loop (K % 32 == 0: whole 64-byte steps)
-        constexpr int BK = 64, DL_S = ring_stages(BM, BN), DL_STAGE = (BM + BN) * BK;
-        constexpr int XI = BM * 4 / NT, WI = BN * 4 / NT;  // 16-byte pieces per thread and stage
+        constexpr int BK = BKH * 2, PP = BK / 16, SH = BK == 64 ? 2 : 1, KKN = BK / 32;
+        constexpr int XI = BM * PP / NT, WI = ring_w_pieces(BN, NT, BKH);  // 16-byte pieces per thread and stage
+        constexpr int DL_S = ring_stages(BM, BN, BKH), DL_STAGE = (BM + WI * NT / PP) * BK;
         // (request counts above 15 need the upper bits of the vmcnt field, a path no instance has exercised)
-        static_assert((BM * 4) % NT == 0 && (BN * 4) % NT == 0 && (DL_S - 1) * (XI + WI) < 16, "whole pieces per thread");
+        static_assert((BM * PP) % NT == 0 && (DL_S - 1) * (XI + WI) < 16, "whole pieces per thread");
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
         uint32_t xo[XI], wo[WI];
 #pragma unroll
         for (int i = 0; i < XI; i++) {
-            const int q = i * NT + tid, r = q >> 2, p = (q & 3) ^ ((r >> 2) & 3);
+            const int q = i * NT + tid, r = q / PP, p = (q % PP) ^ ((r >> SH) & (PP - 1));
             const int m = m_base + r;
             xo[i] = m < g.M ? (uint32_t)m * g.lda + (uint32_t)(p * 16) : kOob;
         }
 #pragma unroll
         for (int i = 0; i < WI; i++) {
-            const int q = i * NT + tid, r = q >> 2, p = (q & 3) ^ ((r >> 2) & 3);
+            const int q = i * NT + tid, r = q / PP, p = (q % PP) ^ ((r >> SH) & (PP - 1));
             const int n = n_base + r;
-            wo[i] = n < g.N ? (uint32_t)n * g.ldb + (uint32_t)(p * 16) : kOob;
+            wo[i] = n < g.N && r < BN ? (uint32_t)n * g.ldb + (uint32_t)(p * 16) : kOob;  // (beyond the tile: zeros)
         }
         const v4i xres4 = rsrc_words(g.a + (int64_t)batch * g.a_batch, g.a_bytes);
         const v4i wres4 = rsrc_words(o.b + (int64_t)batch * g.b_batch, g.b_bytes);
         const uint32_t lds0 = (uint32_t) reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem) +
                               (uint32_t)(wave_u * 1024);
         // operand addresses inside a stage: row lane % 32 of a 32-row group, the lane half's eight halfs of K half kk
-        const int h = lane >> 5, swz = (lane >> 2) & 3;
-        const char *x_base[2], *w_base[2];
+        const int h = lane >> 5, swz = (lane >> SH) & (PP - 1);
+        const char *x_base[KKN], *w_base[KKN];
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
+        for (int kk = 0; kk < KKN; kk++) {
             const int slot = ((kk * 2 + h) ^ swz) * 16;
             x_base[kk] = smem + (wave_m * WM + (lane & 31)) * BK + slot;
             w_base[kk] = smem + BM * BK + (wave_n * WN + (lane & 31)) * BK + slot;
@@ -258,14 +261,14 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const 
         // The loop, as in the int8 kernel's direct-to-LDS form: a wavefront issues in order, so a K half is one
         // straight line -- a matrix instruction, then a share of the next half's operand reads and of the requests,
         // which issue while the matrix core works, then the next matrix instruction.  Stage s lives in buffer
-        // s % DL_S; a stage's requests ride in the second K half of a step, behind the step's barrier, which frees the
+        // s % DL_S; a stage's requests ride in the last 16 halfs of a step, behind the step's barrier, which frees the
         // buffer (spread over both halves of a step they arrive a step later, which the long contractions whose
         // operands come from memory rather than from the L2 pay for: 4096 x 3072 x 768 ran 5 % slower).  Beyond the last step they go through an
         // empty resource and fetch nothing, so every step has the same requests in flight and the waits count exactly:
         // at most DL_S - 3 stages outstanding at the barrier of step s means this thread's part of stage s + 1 has
         // landed; the barrier extends that to every thread's part and says that every wavefront has received its
         // reads of stage s - 1, whose buffer the step's requests overwrite.
-        const int nk = g.K / 32;
+        const int nk = g.K / BKH;
         const v4i null4 = v4i{xres4[0], xres4[1], 0, xres4[3]};
         constexpr int NLA = XI + WI;
         auto half = [&](auto lp_t, const v8h(&xc)[TM], const v8h(&wc)[TN], v8h(&xn)[TM], v8h(&wn)[TN], int rbuf, int rkk,
@@ -330,6 +333,11 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_f16_kernel(const 
             for (int d = 0; d < DL_S; d++) {
                 if (step + d < nk) {  // uniform
                     half(std::integral_constant<int, 0>{}, xf0, wf0, xf1, wf1, d, 1, 0, 0);
+#pragma unroll
+                    for (int kk = 1; kk + 1 < KKN; kk += 2) {
+                        half(std::integral_constant<int, 0>{}, xf1, wf1, xf0, wf0, d, kk + 1, 0, 0);
+                        half(std::integral_constant<int, 0>{}, xf0, wf0, xf1, wf1, d, kk + 2, 0, 0);
+                    }
                     wait_vmcnt<(DL_S - 3) * NLA>();
                     asm volatile("" ::: "memory");
                     __builtin_amdgcn_s_barrier();
@@ -575,7 +583,8 @@ void launch_k(const HGemmArgs &args, bool cast_epilogue, dim3 grid, hipStream_t 
     g.div_per_batch = make_div_magic((uint32_t)(g.tiles_m * g.tiles_n));
     g.div_tiles_n = make_div_magic((uint32_t)g.tiles_n);
     g.div_group = make_div_magic((uint32_t)(g.tiles_n_group > 0 ? g.tiles_n_group : 1));
-    constexpr size_t operands = BROWS ? (size_t)ring_stages(BM, BN) * (BM + BN) * 64
+    constexpr int NT = 64 * WAVES_M * WAVES_N;
+    constexpr size_t operands = BROWS ? (size_t)ring_stages(BM, BN, BKH) * (BM + ring_w_pieces(BN, NT, BKH) * NT * 8 / BKH) * BKH * 2
                                       : (size_t)2 * BM * (BKH * 2 + 16) + (size_t)2 * BKH * (2 * BN + 32);
     constexpr size_t result = std::max((size_t)BM * (BN * 2 + 16), (size_t)BN * (BM * 2 + 16));
     constexpr size_t sm = std::max(operands, result);
@@ -764,36 +773,49 @@ int launch_args(mlel_ctx *ctx, hipStream_t s, HGemmArgs &g, bool bias_cast) {
     // tile with or without one.
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256) * NB;
     if (g.b_rows) {
-        // row-wise B: the direct-to-LDS loop; 64 x 64 tiles where there are few, the 256 x 256 tile under the same condition as below, else 128 x 128 of
-        // eight wavefronts, whatever the extents (rows beyond M or N are fetched as zeros)
-        const int64_t tn128 = (N + 127) / 128;
-        const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * g.groups * NB;
-        // Few tiles (one or two of 64 x 64 per compute unit): 64 x 64 over four wavefronts.  197 rows, 1536 -> 384: 8 blocks of
-        // 128 x 128 took 15.7 us, 24 of these 6; an encoder block of 8 x 197 rows, 768 columns: 107.7 -> 100.7 us with the
-        // line at two tiles per unit, 105.7 at four.
-        if (tiles64 <= 2 * (int64_t)cus) {
-            g.tiles_m = (int)((M + 63) / 64);
-            g.tiles_n_group = (int)((N + 63) / 64);
+        // Row-wise B: the direct-to-LDS loop, whatever the extents (rows beyond M or N are fetched as zeros).
+        const auto tiles_of = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * g.groups * NB; };
+        const auto go = [&](auto bm, auto bn, auto wm, auto wn, auto bkh) {
+            constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value;
+            g.tiles_m = (int)((M + BM - 1) / BM);
+            g.tiles_n_group = (int)((N + BN - 1) / BN);
             g.tiles_n = g.tiles_n_group * g.groups;
-            g.total_tiles = (int)tiles64;
-            g.chunk = (int)((tiles64 + 7) / 8);
-            launch_k<64, 64, 2, 2, 32, true>(g, bias_cast, dim3((unsigned)(g.chunk * 8)), s);
-        } else if (g.groups == 1 && g.K >= 256 && tiles256 * 4 >= 3 * (int64_t)cus && tiles256 <= 2 * (int64_t)cus) {
-            g.tiles_m = (int)((M + 255) / 256);
-            g.tiles_n_group = (int)((N + 255) / 256);
-            g.tiles_n = g.tiles_n_group;
-            g.total_tiles = (int)tiles256;
-            g.chunk = (int)((tiles256 + 7) / 8);
-            launch_k<256, 256, 2, 4, 32, true>(g, bias_cast, dim3((unsigned)(g.chunk * 8)), s);
-        } else {
-            g.tiles_m = (int)((M + 127) / 128);
-            g.tiles_n_group = (int)tn128;
-            g.tiles_n = (int)(tn128 * g.groups);
-            const int64_t t = (int64_t)g.tiles_m * g.tiles_n * NB;
-            MLEL_REQUIRE(t < (int64_t(1) << 30), MLEL_ERR_LIMIT, "matmul: %lld tiles", (long long)t);
+            const int64_t t = tiles_of(BM, BN);
             g.total_tiles = (int)t;
             g.chunk = (int)((t + 7) / 8);
-            launch_k<128, 128, 2, 4, 32, true>(g, bias_cast, dim3((unsigned)(g.chunk * 8)), s);
+            launch_k<BM, BN, decltype(wm)::value, decltype(wn)::value, decltype(bkh)::value, true>(g, bias_cast, dim3((unsigned)(g.chunk * 8)), s);
+        };
+        MLEL_REQUIRE(tiles_of(64, 64) < (int64_t(1) << 30), MLEL_ERR_LIMIT, "matmul: %lld tiles", (long long)tiles_of(64, 64));
+        constexpr std::integral_constant<int, 2> two;
+        constexpr std::integral_constant<int, 4> four;
+        constexpr std::integral_constant<int, 32> k32;
+        constexpr std::integral_constant<int, 64> k64, t64;
+        constexpr std::integral_constant<int, 128> t128;
+        constexpr std::integral_constant<int, 192> t192;
+        constexpr std::integral_constant<int, 256> t256;
+        const bool whole64 = K % 64 == 0;
+        const auto fills = [&](int64_t tiles, int64_t most) { return tiles * 4 >= 3 * (int64_t)cus && tiles <= most; };
+        // - Few tiles (one or two of 64 x 64 per compute unit): 64 x 64 over four wavefronts.  197 rows, 1536 -> 384: 8 blocks of
+        //   128 x 128 took 15.7 us, 24 of these 6; an encoder block of 8 x 197 rows, 768 columns: 107.7 -> 100.7 us with the
+        //   line at two tiles per unit, 105.7 at four.
+        // - 256 rows where three quarters of the compute units get a tile: a third fewer operand reads from shared memory per
+        //   multiply.  256 x 192 serves the widths between (4096 x 768 x 2304, 192 tiles: 27.2 -> 23.4 us against 576 of
+        //   128 x 128; 256 x 256 would leave 112 units idle).
+        // - 128 x 128 over eight wavefronts otherwise.
+        // Steps of 64 halfs halve the barriers, at twice the shared memory: for the tiles that have a compute unit to themselves
+        // anyway (4096 x 3072 x 768: 30.2 -> 25.1 us, 878 x 896 x 3584: 14.0 -> 12.1, even at K = 768 and below), and for the
+        // 64 x 64 tile, of which two still fit (1576 x 3072 x 768: 25.0 -> 19.9).
+        if (tiles_of(64, 64) <= 2 * (int64_t)cus) {
+            if (whole64) go(t64, t64, two, two, k64);
+            else go(t64, t64, two, two, k32);
+        } else if (g.groups == 1 && K >= 256 && fills(tiles_of(256, 256), 2 * (int64_t)cus)) {
+            go(t256, t256, two, four, k32);
+        } else if (K >= 256 && fills(tiles_of(256, 192), cus)) {
+            go(t256, t192, four, two, k32);
+        } else if (whole64 && K > 768 && tiles_of(128, 128) <= cus) {
+            go(t128, t128, two, four, k64);
+        } else {
+            go(t128, t128, two, four, k32);
         }
         MLEL_TRY(check_launch("matmul fp16, row-wise B"));
         return 1;
