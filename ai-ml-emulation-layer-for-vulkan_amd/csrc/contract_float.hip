@@ -221,8 +221,9 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
 
     const int h = lane / MT, lrow = lane % MT;
 
-    // ---- what the epilogue needs, asked for in front of the operands (behind the loop its trip to memory stands alone): the
-    // bias of this lane's columns and the pieces of the residual.  NQ: register quads this wavefront finishes, of NB columns' worth
+    // ---- what the epilogue needs: the bias of this lane's columns and the pieces of the residual.  Asked for in front of the
+    // operands (behind the loop its trip to memory stands alone) where the loop's loads are counted; a loop whose loads stand
+    // behind conditions would wait for it first (the 3-channel convolution of four images of 224 x 224: 7.7 -> 10.4 us).  NQ: register quads this wavefront finishes, of NB columns' worth
     constexpr int NQ = WK == 1 ? AR / 4 * TM * TN : (AR / 4 > WK ? AR / 4 / WK : 1), NB = WK == 1 ? AR / 4 * TN : NQ;
     static_assert(WK == 1 || TM * TN == 1, "one sub-tile where K is shared");
     auto quad_col = [&](int u) {  // first column of quad u, within the tile
@@ -235,17 +236,21 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
     const __amdgpu_buffer_rsrc_t rres = rsrc(g.res, g.res != nullptr ? g.o_bytes : 0u);
     uint32_t bias_bits[NB][4], off[NP];
     uint4 res[NP];
+    auto ask_epilogue = [&] {
 #pragma unroll
-    for (int u = 0; u < NB; u++)
+        for (int u = 0; u < NB; u++)
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            bias_bits[u][e] = load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)((n_base + quad_col(u) + e) * SO));
+            for (int e = 0; e < 4; e++)
+                bias_bits[u][e] = load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)((n_base + quad_col(u) + e) * SO));
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const int p = i * NT + tid, m = m_base + p / OPPR, n = n_base + (p % OPPR) * EO;
-        off[i] = p < BM * OPPR && m < g.M && n < g.N ? (uint32_t)m * g.ldo + (uint32_t)(n * SO) : kOob;
-        res[i] = load16(rres, g.wide_out ? off[i] : kOob);
-    }
+        for (int i = 0; i < NP; i++) {
+            const int p = i * NT + tid, m = m_base + p / OPPR, n = n_base + (p % OPPR) * EO;
+            off[i] = p < BM * OPPR && m < g.M && n < g.N ? (uint32_t)m * g.ldo + (uint32_t)(n * SO) : kOob;
+            res[i] = load16(rres, g.wide_out ? off[i] : kOob);
+        }
+    };
+    constexpr bool AHEAD = DIRECT || XF == F_ROWS;
+    if constexpr (AHEAD) ask_epilogue();
     // this wavefront's operands of a stage; `between` runs while they are on their way, then they are multiplied
     auto compute = [&](const char *st, auto between) {
         uint4 xf[KKW][TM], wf[KKW][TN];
@@ -578,6 +583,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
         }
     }
 
+    if constexpr (!AHEAD) ask_epilogue();
     // ---- the K shares of a block's wavefronts, added in ascending order of K: they leave their quads in shared memory, and each
     // of the first few takes an equal part of them, in every wavefront what it then rounds and stores
     v4f own[NQ];
