@@ -77,6 +77,7 @@ struct FArgs {
     uint32_t ic_magic, kw_magic;  // k / IC = mulhi(k, ic_magic), tap / KW = tap kw_magic >> 16 (DIRECT)
     int32_t bias_len;
     int32_t wide_out;  // rows of the result in whole aligned 16-byte pieces
+    int32_t border;    // some tap of some position lies outside the image
     int32_t has_clamp, clamp_nan_ignore;
     float clamp_lo, clamp_hi;
 };
@@ -146,6 +147,29 @@ enum { F_PIECES = 0,   // aligned 16-byte pieces
        F_KMAJOR = 4 }; // W of a product only: pieces of the rows of [K][N], from any address, transposed on their way out of
                        // shared memory
 
+// What position m gives for column n before its rounding, over the taps inside the image one after the other, until the sum is
+// NaN for good; false for a position whose taps all lie inside.
+template <typename T, typename TO>
+__device__ __forceinline__ bool sum_inside(const FArgs &g, int m, int n, float &s) {
+    constexpr int SZ = Elem<T>::size, SO = Elem<TO>::size;
+    const int img = div_magic(m, g.div_ohw), pos = m - img * g.OHW, oy = div_magic(pos, g.div_ow), ox = pos - oy * g.OW;
+    const int iy0 = oy * g.sy - g.pt, ix0 = ox * g.sx - g.pl;
+    if (iy0 >= 0 && ix0 >= 0 && iy0 + (g.KH - 1) * g.dy < g.H && ix0 + (g.KW - 1) * g.dx < g.W) return false;
+    const __amdgpu_buffer_rsrc_t xres = rsrc(g.x, g.x_bytes), wres = rsrc(g.w, g.w_bytes), bres = rsrc(g.bias, (uint32_t)(g.bias_len * SO));
+    s = 0.f;
+    for (int tap = 0; tap < g.KH * g.KW && s == s; tap++) {
+        const int ky = tap / g.KW, kx = tap - ky * g.KW, iy = iy0 + ky * g.dy, ix = ix0 + kx * g.dx;
+        if ((uint32_t)iy >= (uint32_t)g.H || (uint32_t)ix >= (uint32_t)g.W) continue;
+        const uint32_t xo = (uint32_t)img * g.x_img + (uint32_t)iy * g.x_row + (uint32_t)ix * g.x_pix;
+        const uint32_t wo = (uint32_t)n * g.ldw + (uint32_t)(tap * g.IC * SZ);
+#pragma unroll 4
+        for (int c = 0; c < g.IC; c++)
+            s += Elem<T>::get(load_elem<SZ>(xres, xo + (uint32_t)(c * SZ))) * Elem<T>::get(load_elem<SZ>(wres, wo + (uint32_t)(c * SZ)));
+    }
+    s += Elem<TO>::get(load_elem<SO>(bres, g.bias_len == 1 ? 0u : (uint32_t)(n * SO)));
+    return true;
+}
+
 constexpr int stage_bytes(int bm, int bn, int bkb, int size, bool km) {
     return km ? bm * bkb + (bkb / size) * (bn * size + 32) : (bm + bn) * bkb;
 }
@@ -160,7 +184,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
     constexpr int TM = BM / WM / MT, TN = BN / WN / MT;
     typedef typename std::conditional<MT == 32, v16f, v4f>::type acc_t;
     constexpr int XI = BM * PPR / NT, WI = BN * PPR / NT;
-    constexpr bool KM = WF == F_KMAJOR;
+    constexpr bool KM = WF == F_KMAJOR, CONV = std::is_same<T, TO>::value && XF != F_ROWS;  // (or an fp32 product of aligned pieces)
     // a K-major W keeps its rows: the pad puts the four rows a transposing read meets (16 bits), or the two the halves of a
     // wavefront read (fp32), on distinct banks
     constexpr int WPITCH = BN * SZ + 32, KROWS = BKB / SZ, WCH = BN * SZ / 16;
@@ -627,6 +651,33 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             if constexpr (SO == 2) *reinterpret_cast<uint2 *>(row) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
             else *reinterpret_cast<uint4 *>(row) = make_uint4(v[0], v[1], v[2], v[3]);
         }
+        // A tap outside the image contributes nothing (conv2d.comp:75-87), but here it is a zero times its weight: no change to
+        // a finite sum, NaN where the weight is infinite or NaN.  So a position with such taps whose sum came out as NaN is
+        // summed again over the taps inside the image, by the lane that holds it.  One comparison per two results where
+        // none is.
+        if constexpr (CONV) {
+            bool nan = false;
+#pragma unroll
+            for (int u = 0; u < NQ; u++) nan |= __builtin_isunordered(own[u][0], own[u][1]) || __builtin_isunordered(own[u][2], own[u][3]);
+            if (g.border && nan) {
+                // (the arguments again, from where the launch left them: held from the start they took 30 scalar registers)
+                typedef const FArgs __attribute__((address_space(4))) *args_t;
+                args_t again = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(again));
+                const FArgs &late = *(const FArgs *)again;
+#pragma clang loop unroll(disable)
+                for (int q = 0; q < 4 * NQ; q++) {
+                    const int u = q / 4, r = (wave_m * TM + u / (AR / 4 * TN)) * MT + lrow, c = quad_col(u) + q % 4;
+                    char *at = smem + r * OP + c * SO;
+                    uint32_t v = 0;
+                    __builtin_memcpy(&v, at, SO);
+                    float sum = Elem<TO>::get(v);
+                    if (sum == sum || m_base + r >= late.M || n_base + c >= late.N || !sum_inside<T, TO>(late, m_base + r, n_base + c, sum)) continue;
+                    v = Elem<TO>::put(sum, false);
+                    __builtin_memcpy(at, &v, SO);
+                }
+            }
+        }
     }
     __syncthreads();
     // ADD of the residual (one rounding, to nearest) and CLAMP, as the stand-alone operators compute them
@@ -809,6 +860,7 @@ int try_conv2d_float(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const
     g.x_bytes = (uint32_t)(N * H * W * IC * sz), g.w_bytes = (uint32_t)(OC * K * sz), g.ldw = (uint32_t)(K * sz);
     g.ldo = (uint32_t)(OC * sz), g.o_bytes = (uint32_t)(M * OC * sz);
     g.bias_len = bias->dims[0] == 1 ? 1 : (int)OC;
+    g.border = a->pad[0] > 0 || a->pad[2] > 0 || (OH - 1) * g.sy - a->pad[0] + (KH - 1) * g.dy >= H || (OW - 1) * g.sx - a->pad[2] + (KW - 1) * g.dx >= W;
     const bool pieces = aligned16(in->ptr, {IC * sz}) && aligned16(w->ptr, {IC * sz});
     // the DIRECT form's taps are bits of a word and its divisions single multiplications
     const bool direct = pieces && KH <= 32 && KW <= 32 && (K + 1024) * IC < (int64_t(1) << 32) &&
