@@ -153,8 +153,10 @@ __global__ void __launch_bounds__(kBlock) resize_argmax_cells_kernel(const Resiz
     __shared__ int32_t reach[256];  // reach[r + 128]: the smallest sum whose RESCALE is at least r
     const int cell = min((int)(blockIdx.x * kBlock + threadIdx.x), g.cells_x - 1);
     const int img = blockIdx.z, qy = (int)blockIdx.y + g.cell_y0, qx = cell + g.cell_x0;
-    // the cell's corners (beyond the border: the border) and its first output position
-    const int y0 = max(qy, 0), y1 = min(qy + 1, g.H - 1), x0 = max(qx, 0), x1 = min(qx + 1, g.W - 1);
+    // the cell's corners (beyond the border: the border; the minimum is unsigned, as in axis_of: a cell two or more in front of
+    // the image pairs its first pixel with its last) and its first output position
+    const int y0 = max(qy, 0), y1 = (int)min((uint32_t)(qy + 1), (uint32_t)g.H - 1u);
+    const int x0 = max(qx, 0), x1 = (int)min((uint32_t)(qx + 1), (uint32_t)g.W - 1u);
     const int8_t *base = g.in + (int64_t)img * g.H * g.W * g.C;
     const int8_t *p[4] = {base + ((int64_t)y0 * g.W + x0) * g.C, base + ((int64_t)y0 * g.W + x1) * g.C,
                           base + ((int64_t)y1 * g.W + x0) * g.C, base + ((int64_t)y1 * g.W + x1) * g.C};

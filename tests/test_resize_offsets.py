@@ -1,0 +1,46 @@
+"""RESIZE with offsets that place positions in front of the image: the one-launch kernels, the operators one by one and the
+oracle."""
+import numpy as np
+import pytest
+
+import test_fused_image_graphs as fused
+from hip_util import abi, gpu_available, hb
+
+graphs = fused.graphs
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = hb.Device(0)
+    yield d
+    d.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("offset", [(-4, -4), (-5, 0), (0, -5), (-13, 1), (-9, -22), (-801, -402)], ids=lambda o: "%d_%d" % o)
+def test_offsets_in_front_of_the_image(dev, oracle, offset):
+    """Scale 4 / 2, offsets from one pixel to hundreds in front of the image: the second corner of a cell two or more in front
+    is the last row or column (the shader's minimum is unsigned), as the operators give it one by one."""
+    rng = np.random.default_rng(-offset[0])
+    n, h, w, c = 2, 200, 331, 7
+    big = (n, 2 * h, 2 * w, c)
+    iattr = [4, 2, 4, 2, *offset, 0, 0, 2]
+    spec = graphs.Spec()
+    spec.inputs.append(("input", abi.I8, (n, h, w, c)))
+    wide, score = spec.tensor("wide", abi.I32, big), spec.tensor("score", abi.I8, big)
+    spec.op("RESIZE", ["input"], [wide], iattr)
+    mult, shift = np.array([1500000011], np.int32), np.array([34], np.int8)
+    spec.op("RESCALE", [wide, spec.const("m", mult), spec.const("s", shift)], [score], [0, 3, 1, 1, 0, 0, 0])
+    spec.op("ARGMAX", [score], ["output"], [3, abi.NAN_PROPAGATE])
+    spec.outputs.append(("output", abi.I32, big[:3]))
+    values = rng.integers(-128, 127, (n, h, w, c), endpoint=True).astype(np.int8)
+    assert fused.both_ways(dev, spec, {"input": values}) == ["RESIZE+RESCALE+ARGMAX"]
+    want = oracle.resize(values, big, abi.I32, abi.resize_attr(iattr[:4], offset, (0, 0), 2))
+    want = oracle.argmax(oracle.rescale(want, mult, shift, abi.I8, abi.rescale_attr(0, 3, True, True, False)), 3)
+    g = graphs.build(dev, spec)
+    g.set_input("input", values)
+    g.dispatch()
+    dev.sync()
+    np.testing.assert_array_equal(g.get_output("output"), want)
+    g.close()
