@@ -340,6 +340,7 @@ bool describe(ResizeArgs &g, const mlel_tensor *out_image, const mlel_tensor *in
     for (int i = 0; i < 2; i++)
         if (a->offset[i] < -(1 << 20) || a->offset[i] > (1 << 20)) return false;
     // the shader's coordinates are int16: they stay so for every position
+    if (a->offset[0] < -32000 * s[0] || a->offset[1] < -32000 * s[2]) return false;
     if (((OH - 1) * s[1] + a->offset[0]) / s[0] > 32000 || ((OW - 1) * s[3] + a->offset[1]) / s[2] > 32000) return false;
     if (OH * s[1] >= (1 << 28) || OW * s[3] >= (1 << 28)) return false;
     // no position lies beyond the last pixel by a pixel or more (the border of a RESIZE is smaller than that)

@@ -1,10 +1,12 @@
 """RESIZE with offsets that place positions in front of the image: the one-launch kernels, the operators one by one and the
 oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import test_fused_image_graphs as fused
-from hip_util import abi, gpu_available, hb
+from hip_util import Runner, abi, gpu_available, hb
 
 graphs = fused.graphs
 
@@ -44,3 +46,25 @@ def test_offsets_in_front_of_the_image(dev, oracle, offset):
     dev.sync()
     np.testing.assert_array_equal(g.get_output("output"), want)
     g.close()
+
+
+# coordinates of the shader are int16: offsets beyond them wrap, which only the general kernel computes
+FAR = [(-32001, 0), (0, -40000), (-70000, -65540)]
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("offset", FAR, ids=lambda o: "%d_%d" % o)
+def test_offsets_beyond_int16_coordinates(dev, oracle, offset):
+    values = np.random.default_rng(1).integers(-128, 127, (1, 9, 11, 5), endpoint=True).astype(np.int8)
+    for mode, dt in ((1, abi.I8), (2, abi.I32)):
+        attr = abi.resize_attr((1, 1, 1, 1), offset, (0, 0), mode)
+        np.testing.assert_array_equal(Runner(dev).resize(values, (1, 9, 11, 5), dt, attr), oracle.resize(values, (1, 9, 11, 5), dt, attr))
+
+
+@pytest.mark.parametrize("offset, taken", [((-32000, -32000), 1)] + [(o, 0) for o in FAR], ids=str)
+def test_offsets_the_one_launch_form_takes(offset, taken):
+    view = lambda dt, shape: abi.make_tensor(0, dt, shape)
+    image, labels = view(abi.I8, (1, 9, 11, 5)), view(abi.I32, (1, 9, 11))
+    attr = abi.resize_attr((1, 1, 1, 1), offset, (0, 0), 2)
+    assert hb.load_library().mlel_hip_resize_rescale_in_kernel(C.byref(labels), C.byref(image), C.byref(attr), 1) == taken
