@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
+#include <optional>
 #include <unordered_map>
 
 #include "session_planner.hpp"
@@ -1626,8 +1627,8 @@ void GraphPipeline::plan() {
     idx++;
     for (const auto &op : ops) {
         if (op->fusedAway) continue;
-        for (const auto &t : op->inputs) touch(t, idx);
-        for (const auto &t : op->outputs) touch(t, idx);
+        for (const auto *list : {&op->inputs, &op->outputs, &op->standIns})
+            for (const auto &t : *list) touch(t, idx);
         for (const auto *spec : {&op->epilogue, &op->scaleA, &op->scaleB, &op->scaleOut}) {
             touch(spec->multiplier, idx);
             touch(spec->shift, idx);
@@ -1884,11 +1885,46 @@ void GraphPipeline::prepackConstants() {
     }
 }
 
+namespace {
+
+// The address alignment the one-launch kernel of a fused operator asks of operand `i` (inputs.size(): the result) and has no
+// other route for; 1 where it asks for none, or its entry point runs the operators one after another instead.
+size_t wantedAlignment(const OpNode &op, const size_t i) {
+    const bool result = i == op.inputs.size();
+    switch (op.kind) {
+    case OpKind::FusedAttention: return result || i < 3 ? 16 : 2;  // q, k, v; the scale
+    case OpKind::FusedConv2DDepthwise: return !result && i < 2 ? 16 : (i == 3 ? 1 : 4);  // x, weights; biases and result
+    case OpKind::FusedResize: return result && op.flag ? 4 : 1;  // the labels
+    default: return 1;
+    }
+}
+
+bool atAlignment(const void *p, const size_t alignment) { return reinterpret_cast<uintptr_t>(p) % alignment == 0; }
+
+}  // namespace
+
+// Fusion is decided before anything is bound, and an external tensor may be bound at any address.  For the operands of a
+// fused kernel that does not take every address, session memory is set aside (alive for that one launch): where the bound
+// address is not one the kernel takes, run() copies the operand there, or the result from there.
+void GraphPipeline::reserveStandIns() {
+    for (const auto &opPtr : ops) {
+        OpNode &op = *opPtr;
+        if (op.fusedAway) continue;
+        for (size_t i = 0; i <= op.inputs.size(); i++) {
+            const TensorPtr &t = i < op.inputs.size() ? op.inputs[i] : op.outputs[0];
+            if (wantedAlignment(op, i) == 1 || t->getKind() != TensorKind::External) continue;
+            op.standIns.resize(op.inputs.size() + 1);
+            op.standIns[i] = makeTensor(t->getFormat(), t->getDimensions());
+        }
+    }
+}
+
 void GraphPipeline::finalize(const bool enableFusion) {
     if (finalized) return;
     const size_t recorded = ops.size();
     if (enableFusion) fuse();
     if (enableFusion) prepackConstants();
+    if (enableFusion) reserveStandIns();
     if (splitRequested) analyzeBatchSplit();
     plan();
     if (splitPrefix > 0) validateSplitPlan();
@@ -2212,7 +2248,23 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
         for (const size_t i : act) halved(in[i], op.inputs[i].get());
         halved(out, op.outputs[0].get());
     }
+    // operands at addresses the kernel does not take: through the session memory set aside for them
+    const auto standIn = [&](const size_t i, const mlel_tensor &bound) -> std::optional<mlel_tensor> {
+        if (i >= op.standIns.size() || !op.standIns[i] || atAlignment(bound.ptr, wantedAlignment(op, i))) return std::nullopt;
+        mlel_tensor t = op.standIns[i]->view();
+        if (half >= 0) halved(t, op.standIns[i].get());  // (in a split run only activations are external)
+        return t;
+    };
     int rc = 0;
+    for (size_t i = 0; i < op.inputs.size() && i < in.size() && rc == 0; i++) {
+        if (const auto t = standIn(i, in[i])) {
+            rc = mlel_hip_reshape(ctx, stream, &*t, &in[i]);
+            in[i] = *t;
+        }
+    }
+    const mlel_tensor result = out;
+    if (const auto t = standIn(op.inputs.size(), out)) out = *t;
+    if (rc != 0) fail(op.tosaName + " (" + op.debugName + "): " + mlel_hip_last_error());
     switch (op.kind) {
     case OpKind::Conv2D: rc = mlel_hip_conv2d(ctx, stream, &out, &in[0], &in[1], &in[2], &op.conv); break;
     case OpKind::DepthwiseConv2D:
@@ -2442,6 +2494,7 @@ void GraphPipeline::run(const OpNode &op, void *stream, const int half) {
         break;
     }
     }
+    if (rc == 0 && out.ptr != result.ptr) rc = mlel_hip_reshape(ctx, stream, &result, &out);
     if (rc != 0) fail(op.tosaName + " (" + op.debugName + "): " + mlel_hip_last_error());
 }
 

@@ -167,6 +167,9 @@ class OpNode {
     mlel_conv2d_attr convFirst{};
     mlel_clamp_attr clampFirst{};
     bool hasClampFirst = false;
+    // Fused kinds whose kernel wants aligned addresses and has no other route: session tensors (one per input, the result's
+    // last; null where none is needed) that stand in for external operands bound elsewhere
+    std::vector<TensorPtr> standIns;
 };
 
 class GraphPipeline {
@@ -387,6 +390,7 @@ class GraphPipeline {
     void *uploadConstant(const TensorDescriptor &t, const void *data);
     void fuse();
     void prepackConstants();
+    void reserveStandIns();
     void plan();
     std::vector<details::BestFitTensor> bestFitTensors(const std::vector<details::LiveInterval> &planned,
                                                        const std::vector<details::UnseenAllocation> &unseen);
