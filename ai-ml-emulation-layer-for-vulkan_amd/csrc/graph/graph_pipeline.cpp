@@ -1984,6 +1984,37 @@ bool batchOperands(const OpNode &op, std::vector<size_t> &ins) {
     }
 }
 
+// Whether the one-launch kernel of a fused operator without another route takes half of the batch as it takes the whole (an
+// image of a few bytes may be the least it reads).
+bool takesHalfBatch(const OpNode &op, const int64_t half) {
+    const auto view = [&](const TensorPtr &t, const bool batch) {
+        mlel_tensor v = t->view();
+        if (batch) v.dims[0] = half;
+        return v;
+    };
+    const auto in = [&](const size_t i, const bool batch) { return view(op.inputs[i], batch); };
+    const mlel_tensor out = view(op.outputs[0], true);
+    switch (op.kind) {
+    case OpKind::FusedTransposeConv2D: {
+        const mlel_tensor x = in(0, true), w = in(1, false), b = in(2, false);
+        return mlel_hip_transpose_conv2d_rescale_clamp_in_kernel(&out, &x, &w, &b, &op.tconv) == 1;
+    }
+    case OpKind::FusedConcatConv2D: {
+        const mlel_tensor x1 = in(0, true), x2 = in(3, true), w = in(1, false), b = in(2, false);
+        return mlel_hip_concat_conv2d_in_kernel(&out, &x1, &x2, &w, &b, &op.conv) == 1;
+    }
+    case OpKind::FusedConv2DFloat: {
+        const mlel_tensor x = in(0, true), w = in(1, false), b = in(2, false), r = in(op.flag ? 3 : 0, true);
+        return mlel_hip_conv2d_add_clamp_in_kernel(&out, &x, &w, &b, &op.conv, op.flag ? &r : nullptr) == 1;
+    }
+    case OpKind::FusedConv2DDepthwise: {
+        const mlel_tensor x = in(0, true), w1 = in(1, false), b1 = in(2, false), w2 = in(3, false), b2 = in(4, false);
+        return mlel_hip_conv2d_dwconv_in_kernel(&out, &x, &w1, &b1, &op.convFirst, &w2, &b2, &op.conv) == 1;
+    }
+    default: return true;
+    }
+}
+
 }  // namespace
 
 void GraphPipeline::analyzeBatchSplit() {
@@ -2016,7 +2047,7 @@ void GraphPipeline::analyzeBatchSplit() {
         }
         for (const auto *spec : {&op->epilogue, &op->scaleA, &op->scaleB, &op->scaleOut})
             for (const auto &t : {spec->multiplier, spec->shift}) ok = ok && (!t || t->getKind() == TensorKind::Constant);
-        if (!ok) break;
+        if (!ok || !takesHalfBatch(*op, n / 2)) break;
         count++;
     }
     if (count < 2) return;
