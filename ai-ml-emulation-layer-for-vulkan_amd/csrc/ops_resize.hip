@@ -115,9 +115,10 @@ __global__ void __launch_bounds__(kBlock) resize_argmax_kernel(const ResizeArgs 
     const int8_t *p10 = base + ((int64_t)y.i1 * g.W + x.i0) * g.C, *p11 = base + ((int64_t)y.i1 * g.W + x.i1) * g.C;
     const int32_t w00 = (g.yn - y.r) * (g.xn - x.r), w01 = (g.yn - y.r) * x.r, w10 = y.r * (g.xn - x.r), w11 = y.r * x.r;
     const ChanScale cs = scale_of(g);
-    // (no sum of this RESIZE may leave int32 when it is scaled, or the order would not survive)
+    // (no sum of this RESIZE may leave int32 when it is scaled, or the order would not survive; the bound holds for the negative
+    // sums too where nothing is subtracted from them first)
     const int64_t bound = (int64_t)128 * g.yn * g.xn;
-    const bool monotone = cs.mult >= 0 && ((bound * cs.mult + cs.round_pos) >> cs.shift) < (int64_t(1) << 30);
+    const bool monotone = g.rp.in_zp == 0 && cs.mult >= 0 && ((bound * cs.mult + cs.round_pos) >> cs.shift) < (int64_t(1) << 30);
     int32_t best = 0, best_r = -128, best_a = INT32_MIN;
     auto channel = [&](int c, int32_t a) {
         if (monotone && a <= best_a && c > 0) return;

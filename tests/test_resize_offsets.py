@@ -1,5 +1,5 @@
-"""RESIZE with offsets that place positions in front of the image: the one-launch kernels, the operators one by one and the
-oracle."""
+"""RESIZE with offsets that place positions in front of the image, and with a RESCALE whose input zero point makes its results
+wrap: the one-launch kernels, the operators one by one and the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -68,3 +68,21 @@ def test_offsets_the_one_launch_form_takes(offset, taken):
     image, labels = view(abi.I8, (1, 9, 11, 5)), view(abi.I32, (1, 9, 11))
     attr = abi.resize_attr((1, 1, 1, 1), offset, (0, 0), 2)
     assert hb.load_library().mlel_hip_resize_rescale_in_kernel(C.byref(labels), C.byref(image), C.byref(attr), 1) == taken
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("zero_point", [0, 2 ** 21, -2 ** 21, 2 ** 31 - 1])
+@pytest.mark.parametrize("h", [6, 400], ids=["few_labels", "many_labels"])
+def test_labels_of_a_rescale_with_an_input_zero_point(dev, h, zero_point):
+    """(a - 2^21) 2^10 leaves int32 on one side of zero: negative sums then scale to the largest value."""
+    spec, big = graphs.Spec(), (1, 2 * h, 2 * 200, 7)
+    spec.inputs.append(("input", abi.I8, (1, h, 200, 7)))
+    wide, score = spec.tensor("wide", abi.I32, big), spec.tensor("score", abi.I8, big)
+    spec.op("RESIZE", ["input"], [wide], [4, 2, 4, 2, -1, -1, 1, 1, 2])
+    scale = [spec.const("m", np.array([2 ** 30], np.int32)), spec.const("s", np.array([20], np.int8))]
+    spec.op("RESCALE", [wide] + scale, [score], [zero_point, 0, 1, 0, 0, 0, 0])
+    spec.op("ARGMAX", [score], ["output"], [3, abi.NAN_PROPAGATE])
+    spec.outputs.append(("output", abi.I32, big[:3]))
+    values = np.random.default_rng(3).integers(-128, 127, (1, h, 200, 7), endpoint=True).astype(np.int8)
+    assert fused.both_ways(dev, spec, {"input": values}) == ["RESIZE+RESCALE+ARGMAX"]
