@@ -1313,7 +1313,7 @@ SPLIT_CONV_CASES = [
     # that K is split over blocks
     ("tap_ic256_3x3", (1, 9, 9, 256), 64, (3, 3), (1, 1, 1, 1), (1, 1), -5, 0),         # one tap per K step
     ("tap_ic320_3x3_s2_zw", (2, 11, 9, 320), 40, (3, 3), (1, 0, 1, 0), (2, 2), 7, -3),
-    ("generic_ic232_3x3", (1, 8, 8, 232), 24, (3, 3), (1, 1, 1, 1), (1, 1), 9, 1),       # byte gathers
+    ("generic_ic232_3x3", (1, 8, 8, 232), 24, (3, 3), (1, 1, 1, 1), (1, 1), 9, 1),       # no whole pieces: rows of any alignment, unsplit
     ("plain_2560_160", (2, 7, 7, 2560), 160, (1, 1), (0, 0, 0, 0), (1, 1), -1, 0),       # 16-byte rows
     ("plain4_ic2200", (1, 6, 6, 2200), 36, (1, 1), (0, 0, 0, 0), (1, 1), 3, 2),          # dword rows, K tail
     ("plain_k_tail_2096", (1, 5, 5, 2096), 130, (1, 1), (0, 0, 0, 0), (1, 1), 0, 0),     # last split shorter
