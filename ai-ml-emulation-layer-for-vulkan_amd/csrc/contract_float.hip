@@ -777,13 +777,15 @@ int launch_shape(mlel_ctx *ctx, FArgs &g, int64_t batches, hipStream_t s) {
         return launch_tile<T, TO, 32, 32, 1, 1, 4, 256, 3, DIRECT, XF, WF>(g, batches, s);
     }
     if constexpr (!DIRECT) {
-        // 128 x 128 tiles from one per compute unit on, unless most of one would be padding; products take eight wavefronts on
+        // K-major W: 128 x 128 tiles from one per compute unit on, unless most of one would be padding; products take eight wavefronts on
         // the smaller tiles where K is long: a wavefront that has a SIMD to itself issues an instruction every 7 clocks, two
         // share the work of a stage (7 x 4000 x 900 fp32: 32.6 -> 25.3 us, 4 x 2274 x 3609 x 32 fp16: 25.2 -> 19.6 us)
-        if (WF == F_KMAJOR && g.M > 64 && g.N > 64 && tiles(128, 128) >= cus) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 2, DIRECT, XF, WF>(g, batches, s);
+        if constexpr (WF == F_KMAJOR)
+            if (g.M > 64 && g.N > 64 && tiles(128, 128) >= cus) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 2, DIRECT, XF, WF>(g, batches, s);
         constexpr int W2 = XF == F_ROWS ? 2 : 1;
         if (tiles(64, 64) * 2 >= cus) {
-            if (W2 == 2 && g.K * (int64_t)Elem<T>::size >= 1024) return launch_tile<T, TO, 64, 64, 2, 2, W2, 128, 2, DIRECT, XF, WF>(g, batches, s);
+            if constexpr (W2 == 2)
+                if (g.K * (int64_t)Elem<T>::size >= 1024) return launch_tile<T, TO, 64, 64, 2, 2, W2, 128, 2, DIRECT, XF, WF>(g, batches, s);
             return launch_tile<T, TO, 64, 64, 2, 2, 1, 128, 2, DIRECT, XF, WF>(g, batches, s);
         }
         return launch_tile<T, TO, 32, 32, 1, 1, 4 * W2, 256, 2, DIRECT, XF, WF>(g, batches, s);

@@ -99,6 +99,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
     constexpr int XI = BM * PPR / NT, STAGE = (BM + BN) * BKB;
     constexpr int WI = (BN * PPR + NT - 1) / NT;  // pieces of W per thread
     static_assert((BM * PPR) % NT == 0 && KK % WK == 0 && TM >= 1 && TN >= 1 && (NT / PPR) % 16 == 0, "tile shape");
+    static_assert(BM + BN <= NT, "a thread per sum");
     extern __shared__ __align__(16) char smem[];
     int32_t *sums = reinterpret_cast<int32_t *>(smem + 2 * STAGE);  // [BM] of X, [BN] of W
     struct Scale {
@@ -145,7 +146,6 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_i8_kernel(const IA
         xb[i] = (img * g.H + y * g.sy + by) * g.W + ix0[i];
     }
     if (tid < BM + BN) sums[tid] = 0;
-    if (BM + BN > NT && tid + NT < BM + BN) sums[tid + NT] = 0;
     for (int c = tid; c < BN; c += NT) {
         const int n = n_base + c;
         Scale s{};
