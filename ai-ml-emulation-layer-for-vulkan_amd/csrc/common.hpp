@@ -465,6 +465,25 @@ __device__ __forceinline__ int32_t requant_acc(int32_t acc, const ChanScale &c, 
     return clamped;
 }
 
+// 16, 8 or 4 bytes from any address
+template <int B>
+__device__ __forceinline__ uint4 load_any(const void *p) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    __builtin_memcpy(&v, p, B);
+    return v;
+}
+// the first `n` (any value) bytes of a dword
+__device__ __forceinline__ uint32_t keep_bytes(uint32_t v, int n) {
+    return n >= 4 ? v : (n <= 0 ? 0u : v & ((1u << (8 * n)) - 1u));
+}
+// acc plus the sixteen signed bytes of a piece
+__device__ __forceinline__ int32_t sum_bytes(uint4 v, int32_t acc) {
+    acc = __builtin_amdgcn_sdot4((int)v.x, 0x01010101, acc, false);
+    acc = __builtin_amdgcn_sdot4((int)v.y, 0x01010101, acc, false);
+    acc = __builtin_amdgcn_sdot4((int)v.z, 0x01010101, acc, false);
+    return __builtin_amdgcn_sdot4((int)v.w, 0x01010101, acc, false);
+}
+
 // 4 rows x 4 channels (bytes) -> 4 channels x 4 vertical taps: output row 0 multiplies the column by the weights
 // (w0, w1, w2, 0), output row 1 by (0, w0, w1, w2), so one transpose serves both rows of a work item
 __device__ __forceinline__ void transpose_4x4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3, uint32_t (&col)[4]) {

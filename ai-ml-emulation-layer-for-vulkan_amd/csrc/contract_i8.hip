@@ -47,17 +47,6 @@ struct IArgs {
     RescaleParams rp;
 };
 
-// 16 or 4 bytes from any address
-template <int B>
-__device__ __forceinline__ uint4 load_any(const int8_t *p) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    __builtin_memcpy(&v, p, B);
-    return v;
-}
-// the first `n` (any value) bytes of a dword
-__device__ __forceinline__ uint32_t keep_bytes(uint32_t v, int n) {
-    return n >= 4 ? v : (n <= 0 ? 0u : v & ((1u << (8 * n)) - 1u));
-}
 // B bytes at offset `off` of an operand of `bytes` bytes (at least B): a chunk that would reach beyond the end is loaded
 // from further in front and shifted down
 template <int B>
@@ -79,12 +68,6 @@ __device__ __forceinline__ uint4 load_chunk(const int8_t *base, uint32_t off, ui
         r[i] = (uint32_t)((((uint64_t)hi << 32) | lo) >> s);
     }
     return make_uint4(r[0], r[1], r[2], r[3]);
-}
-__device__ __forceinline__ int32_t sum_bytes(uint4 v, int32_t acc) {
-    acc = __builtin_amdgcn_sdot4((int)v.x, 0x01010101, acc, false);
-    acc = __builtin_amdgcn_sdot4((int)v.y, 0x01010101, acc, false);
-    acc = __builtin_amdgcn_sdot4((int)v.z, 0x01010101, acc, false);
-    return __builtin_amdgcn_sdot4((int)v.w, 0x01010101, acc, false);
 }
 
 // SO: bytes of a result (1: requantised int8 / uint8, 4: the int32 accumulator, or the requantised int32);

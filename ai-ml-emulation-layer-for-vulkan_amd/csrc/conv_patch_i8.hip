@@ -68,15 +68,6 @@ struct PatchArgs {
 
 // n / d for n < 2^11 and n d < 2^20, `m` = 2^20 / d + 1: two full-rate instructions
 __device__ __forceinline__ int quotient(int n, uint32_t m) { return (int)(__umul24((uint32_t)n, m) >> 20); }
-template <int B>
-__device__ __forceinline__ uint4 load_any(const int8_t *p) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    __builtin_memcpy(&v, p, B);
-    return v;
-}
-__device__ __forceinline__ uint32_t keep_bytes(uint32_t v, int n) {
-    return n >= 4 ? v : (n <= 0 ? 0u : v & ((1u << (8 * n)) - 1u));
-}
 // four bytes at offset `off` of an operand of `bytes` (at least 4): near the end from further in front, shifted down; what
 // lies beyond the end is any value
 __device__ __forceinline__ uint32_t load_dword(const int8_t *base, uint32_t off, uint32_t bytes) {

@@ -45,21 +45,6 @@ struct PArgs {
     RescaleParams rp;
 };
 
-__device__ __forceinline__ uint4 load16(const char *p) {
-    uint4 v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-__device__ __forceinline__ int32_t sum_bytes(uint4 v, int32_t acc) {
-    acc = __builtin_amdgcn_sdot4((int)v.x, 0x01010101, acc, false);
-    acc = __builtin_amdgcn_sdot4((int)v.y, 0x01010101, acc, false);
-    acc = __builtin_amdgcn_sdot4((int)v.z, 0x01010101, acc, false);
-    return __builtin_amdgcn_sdot4((int)v.w, 0x01010101, acc, false);
-}
-// the first `n` (any value) bytes of a dword
-__device__ __forceinline__ uint32_t keep_bytes(uint32_t v, int n) {
-    return n >= 4 ? v : (n <= 0 ? 0u : v & ((1u << (8 * n)) - 1u));
-}
 // a piece moved `by` (at most 15) bytes to the front, zeros behind, and its first `rem` bytes kept
 __device__ __forceinline__ uint4 forward_keep(uint4 v, uint32_t by, int rem) {
     uint32_t w[5] = {v.x, v.y, v.z, v.w, 0};
@@ -124,9 +109,9 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) product_i8_kernel(const PAr
         stage = min(stage, g.whole - 1);
         const char *xa = xp + (int64_t)stage * BKB, *wa = wp + (int64_t)stage * (KM ? (int64_t)BKB * g.ldw : BKB);
 #pragma unroll
-        for (int i = 0; i < XI; i++) v.x[i] = load16(xa + xo[i]);
+        for (int i = 0; i < XI; i++) v.x[i] = load_any<16>(xa + xo[i]);
 #pragma unroll
-        for (int i = 0; i < WI; i++) v.w[i] = load16(wa + wo[i]);
+        for (int i = 0; i < WI; i++) v.w[i] = load_any<16>(wa + wo[i]);
     };
     // the stage at `k0` that may reach beyond K: loads inside the operand ...
     auto tail_x = [&](int i, int k0) { return xo[i] + (uint32_t)k0; };
@@ -136,9 +121,9 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) product_i8_kernel(const PAr
     };
     auto ask_tail = [&](Set &v, int k0) {
 #pragma unroll
-        for (int i = 0; i < XI; i++) v.x[i] = load16(xp + min(tail_x(i, k0), g.x_bytes - 16));
+        for (int i = 0; i < XI; i++) v.x[i] = load_any<16>(xp + min(tail_x(i, k0), g.x_bytes - 16));
 #pragma unroll
-        for (int i = 0; i < WI; i++) v.w[i] = load16(wp + min(tail_w(i, k0), g.w_bytes - 16));
+        for (int i = 0; i < WI; i++) v.w[i] = load_any<16>(wp + min(tail_w(i, k0), g.w_bytes - 16));
     };
     // ... and what of them counts
     auto trim = [&](Set &v, int k0) {
