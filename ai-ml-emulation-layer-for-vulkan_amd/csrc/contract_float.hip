@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             bool nan = false;
 #pragma unroll
             for (int u = 0; u < NQ; u++) nan |= __builtin_isunordered(own[u][0], own[u][1]) || __builtin_isunordered(own[u][2], own[u][3]);
-            if (g.border && nan) {
+            if (__builtin_expect(g.border && nan, 0)) {
                 // (the arguments again, from where the launch left them: held from the start they took 30 scalar registers)
                 typedef const FArgs __attribute__((address_space(4))) *args_t;
                 args_t again = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
