@@ -211,6 +211,12 @@ int mlel_hip_matmul_add(mlel_ctx *ctx, void *stream, const mlel_tensor *out, con
     MLEL_REQUIRE(attr != nullptr && row != nullptr, MLEL_ERR_INVALID, "matmul_add: null argument");
     for (const mlel_tensor *t : {out, a, b, row}) MLEL_TRY(check_supported(t, "matmul_add"));
     MLEL_REQUIRE(out->rank == 3 && a->rank == 3 && b->rank == 3 && row->rank == 3, MLEL_ERR_INVALID, "matmul_add: rank must be 3");
+    // a large fp16 product and the ADD in place behind it, on what the one launch takes too
+    if (try_matmul_float(nullptr, nullptr, out, a, b, attr, row, true) == 1 && matmul_f16_then_add(ctx, out, a, b, attr)) {
+        const int rc = try_matmul_f16_mfma(ctx, (hipStream_t)stream, out, a, b, attr);
+        if (rc < 0) return rc;
+        if (rc == 1) return mlel_hip_elementwise_binary(ctx, stream, MLEL_BIN_ADD, out, out, row, MLEL_NAN_PROPAGATE);
+    }
     const int rc = try_matmul_float(ctx, (hipStream_t)stream, out, a, b, attr, row);
     if (rc != 0) return rc < 0 ? rc : 0;
     return set_error(MLEL_ERR_UNSUPPORTED, "matmul_add: not a case of the one-launch kernel");

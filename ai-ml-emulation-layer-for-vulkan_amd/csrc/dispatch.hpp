@@ -140,6 +140,9 @@ int try_matmul_f16_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, co
 // single fp16 elements, nine steps (ops_float.hip).
 bool chain_is_gelu_tanh(const mlel_chain *chain);
 
+// whether MATMUL with an fp32 row added behind it is faster as the product here and an ADD pass over its result
+bool matmul_f16_then_add(mlel_ctx *ctx, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b, const mlel_matmul_attr *attr);
+
 // two or three fused products (fp16 out = CAST(MATMUL + bias)) of one A in a single launch
 int try_matmul_f16_group(mlel_ctx *ctx, hipStream_t s, int n, const mlel_tensor *const *outs, const mlel_tensor *a,
                          const mlel_tensor *const *bs, const mlel_tensor *const *biases, const mlel_matmul_attr *attr);

@@ -858,6 +858,20 @@ int try_matmul_f16_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, co
     return launch_args(ctx, s, g, bias_cast);
 }
 
+// Whether a product with a row added behind it is better off here, the ADD a pass of its own over the result, than in the kernel
+// that adds in its epilogue (contract_float.hip): where this file's 256 x 256 tile applies and K is long enough for its faster
+// loop to pay for the pass.  us, apart / there -- K-major B: 4096 x 2048 x 4096 110 / 105, 4096 x 3072 x 4096 141 / 146, 4096^3
+// 167 / 189, 3072 x 4096 x 4096 (192 tiles) 143 / 141, 4096 x 2048 x 8192 214 / 210, 4096 x 4096 x 8192 337 / 379; row-wise B:
+// 4096 x 1024 x 4096 74 / 61, 4096 x 2048 x 4096 101 / 102, 4096 x 3072 x 4096 128 / 146, 3072 x 4096 x 4096 124 / 141.
+bool matmul_f16_then_add(mlel_ctx *ctx, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b, const mlel_matmul_attr *attr) {
+    HGemmArgs g{};
+    if (a->dtype != MLEL_F16 || fill_args(out, a, b, attr, false, nullptr, nullptr, &g) != 1) return false;
+    const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+    const int64_t tiles = ((int64_t)(g.M + 255) / 256) * ((g.N + 255) / 256) * g.batches;
+    const bool wide = g.b_rows || (g.N + 127) / 128 * 128 <= (g.N + 63) / 64 * 64;  // (launch_args' condition for that tile)
+    return wide && tiles * 4 >= 3 * cus && tiles <= 2 * cus && g.K * std::min(tiles, cus) >= (g.b_rows ? 2048 : 3072) * cus;
+}
+
 // Up to three fused products of one A in a single launch; 0 unless every product is a case for the kernel and they
 // agree in everything but their B, bias and output.
 int try_matmul_f16_group(mlel_ctx *ctx, hipStream_t s, int n, const mlel_tensor *const *outs, const mlel_tensor *a,

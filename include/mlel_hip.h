@@ -602,9 +602,10 @@ int mlel_hip_conv2d_add_clamp(mlel_ctx *ctx, void *stream, const mlel_tensor *ou
                               const mlel_tensor *residual, const mlel_clamp_attr *clamp);
 int mlel_hip_conv2d_add_clamp_in_kernel(const mlel_tensor *out, const mlel_tensor *in, const mlel_tensor *weights,
                                         const mlel_tensor *bias, const mlel_conv2d_attr *attr, const mlel_tensor *residual);
-/* out(fp32) = ADD(MATMUL(a, b), row) over fp16, bf16 or fp32 operands of zero zero points, one launch: the product's fp32
- * results plus an fp32 row [1, 1, N] or single value [1, 1, 1] (matmul.comp:30-73, elementwise_binary.comp:146-173).
- * Anything else is MLEL_ERR_UNSUPPORTED; the _in_kernel query judges by types, extents and strides. */
+/* out(fp32) = ADD(MATMUL(a, b), row) over fp16, bf16 or fp32 operands of zero zero points, one launch (large fp16 products two,
+ * the row added in place; no memory is allocated): the product's fp32 results plus an fp32 row [1, 1, N] or single value
+ * [1, 1, 1] (matmul.comp:30-73, elementwise_binary.comp:146-173).  Anything else is MLEL_ERR_UNSUPPORTED; the _in_kernel query
+ * judges by types, extents and strides. */
 int mlel_hip_matmul_add(mlel_ctx *ctx, void *stream, const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b,
                         const mlel_matmul_attr *attr, const mlel_tensor *row);
 int mlel_hip_matmul_add_in_kernel(const mlel_tensor *out, const mlel_tensor *a, const mlel_tensor *b, const mlel_matmul_attr *attr,
