@@ -802,7 +802,7 @@ int launch_args(mlel_ctx *ctx, hipStream_t s, HGemmArgs &g, bool bias_cast) {
         //   multiply.  256 x 192 serves the widths between (4096 x 768 x 2304, 192 tiles: 27.2 -> 23.4 us against 576 of
         //   128 x 128; 256 x 256 would leave 112 units idle).
         // - 128 x 128 over eight wavefronts otherwise.
-        // Steps of 64 halfs halve the barriers, at twice the shared memory: for the tiles that have a compute unit to themselves
+        // Steps of 64 halfs, half as many of them at twice the shared memory: for the tiles that have a compute unit to themselves
         // anyway (4096 x 3072 x 768: 30.2 -> 25.1 us, 878 x 896 x 3584: 14.0 -> 12.1, even at K = 768 and below), and for the
         // 64 x 64 tile, of which two still fit (1576 x 3072 x 768: 25.0 -> 19.9).
         if (tiles_of(64, 64) <= 2 * (int64_t)cus) {
