@@ -334,7 +334,7 @@ bool describe(ResizeArgs &g, const mlel_tensor *out_image, const mlel_tensor *in
     const int64_t N = in->dims[0], H = in->dims[1], W = in->dims[2], C = in->dims[3];
     const int64_t OH = out_image->dims[1], OW = out_image->dims[2];
     if (out_image->dims[0] != N || N <= 0 || H <= 0 || W <= 0 || C <= 0 || OH <= 0 || OW <= 0 || N > 65535 || OH > 65535) return false;
-    if (H > 32767 || W > 32767 || OW * C >= (1 << 28) || N * H * W * C >= (int64_t(1) << 40)) return false;
+    if (H > 32767 || W > 32767 || W * C >= (int64_t(1) << 31) || OW * C >= (1 << 28) || N * H * W * C >= (int64_t(1) << 40)) return false;
     const int32_t *s = a->scale;
     for (int i = 0; i < 4; i++)
         if (s[i] <= 0 || s[i] > 2048) return false;

@@ -86,3 +86,11 @@ def test_labels_of_a_rescale_with_an_input_zero_point(dev, h, zero_point):
     spec.outputs.append(("output", abi.I32, big[:3]))
     values = np.random.default_rng(3).integers(-128, 127, (1, h, 200, 7), endpoint=True).astype(np.int8)
     assert fused.both_ways(dev, spec, {"input": values}) == ["RESIZE+RESCALE+ARGMAX"]
+
+
+@pytest.mark.parametrize("w, c, taken", [(32767, 65536, 1), (32767, 65540, 0), (32000, 200000, 0)])
+def test_rows_of_more_than_31_bits_are_left_to_the_general_kernel(w, c, taken):
+    """A place within a row is an int32 in the one-launch kernels (judged without memory)."""
+    image, out = (abi.make_tensor(0, abi.I8, shape) for shape in ((1, 2, w, c), (1, 2, 40, c)))
+    attr = abi.resize_attr((1, 1, 1, 800), (0, 0), (0, 0), 2)
+    assert hb.load_library().mlel_hip_resize_rescale_in_kernel(C.byref(out), C.byref(image), C.byref(attr), 0) == taken
