@@ -651,7 +651,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             if constexpr (SO == 2) *reinterpret_cast<uint2 *>(row) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
             else *reinterpret_cast<uint4 *>(row) = make_uint4(v[0], v[1], v[2], v[3]);
         }
-        // A tap outside the image contributes nothing (conv2d.comp:75-87), but here it is a zero times its weight: no change to
+        // A tap outside the image contributes nothing (conv2d.comp:40-116), but here it is a zero times its weight: no change to
         // a finite sum, NaN where the weight is infinite or NaN.  So a position with such taps whose sum came out as NaN is
         // summed again over the taps inside the image, by the lane that holds it.  One comparison per two results where
         // none is.

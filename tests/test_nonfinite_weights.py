@@ -1,5 +1,5 @@
 """CONV2D over floating-point tensors whose weights hold infinities and NaN: a tap outside the image contributes nothing
-(conv2d.comp:75-87), so what such a weight does to the inside of an image must not reach the positions at its border."""
+(conv2d.comp:40-116), so what such a weight does to the inside of an image must not reach the positions at its border."""
 import zlib
 
 import numpy as np
