@@ -488,6 +488,7 @@ int try_conv_few_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const 
                     const mlel_tensor *w, const mlel_tensor *bias, const FusedEpilogue *epi, int32_t zx, int32_t zw,
                     const int32_t *pad, const int32_t *stride, const int32_t *dilation, bool transposed) {
     if (epi == nullptr || epi->p.in_zp != 0 || zw != 0 || dt_size(out->dtype) != 1) return 0;
+    if (zx < -128 || zx > 127) return 0;  // (-zx is a byte of an operand here; the kernels of more tiles multiply in 32 bits)
     const int64_t B = in->dims[0], H = in->dims[1], W = in->dims[2], IC1 = in->dims[3], IC2 = in2 ? in2->dims[3] : 0, IC = IC1 + IC2;
     const int64_t OC = w->dims[0], KH = w->dims[1], KW = w->dims[2];
     FewArgs g{};

@@ -59,6 +59,18 @@ def test_conv2d_of_few_tiles_vs_oracle(dev, oracle, case):
     np.testing.assert_array_equal(run.conv2d(x, wt, b, shape, abi.I8, attr, epilogue=(mult, shift, rattr, (-100, 90))), exp)
 
 
+@pytest.mark.parametrize("zx", [200, -129])
+@pytest.mark.parametrize("ic", [64, 20], ids=["pieces", "ragged"])
+def test_zero_points_that_are_no_byte(dev, oracle, ic, zx):
+    """The zero point is subtracted in 32 bits, whatever its value: here as a factor of the weights' sums, without borders."""
+    run, rng = Runner(dev), np.random.default_rng(ic)
+    x, wt, b = i8(rng, (1, 9, 8, ic)), i8(rng, (24, 3, 3, ic)), rng.integers(-2 ** 12, 2 ** 12, (24,)).astype(np.int32)
+    attr, rattr = abi.conv2d_attr((0, 0, 0, 0), (1, 1), (1, 1), zx, 0), abi.rescale_attr(0, 3, True, True, True)
+    mult, shift = scale(rng, 24, 9 * ic)
+    exp = np.clip(oracle.rescale(oracle.conv2d(x, wt, b, (1, 7, 6, 24), abi.I32, attr), mult, shift, abi.I8, rattr), -100, 90)
+    np.testing.assert_array_equal(run.conv2d(x, wt, b, (1, 7, 6, 24), abi.I8, attr, epilogue=(mult, shift, rattr, (-100, 90))), exp)
+
+
 @pytest.mark.parametrize("n, h, w, ic, c1, c2, oc, s", [
     (2, 3, 5, 16, 16, 16, 7, (1, 2)), (1, 6, 5, 16, 32, 16, 8, (3, 1)), (1, 8, 7, 64, 32, 48, 40, (2, 2)), (1, 4, 5, 32, 80, 16, 24, (3, 2)),
     (1, 40, 40, 48, 16, 16, 48, (2, 2)),      # tiles of 32
