@@ -43,16 +43,14 @@ __global__ void __launch_bounds__(kColsBlock) conv_cols_mfma_i8_kernel(const Gem
                                                                          const DivMagic div_groups_n, int chunk) {
     // every argument that the tile assignment, the first operand requests and the epilogue depend on, asked for in one
     // batch: left alone the compiler loads most of them behind the early exit, a second trip to memory in a row
+    // (not the residual's: nothing in front of the loop waits for them, and twenty more to wait for cost 0.1 us, or 3 %, at up to 256
+    // channels: 32 -> 24 over 294 positions 4.12 us with them, 3.97 without; over 300 such sizes 1.5 % slower than with neither
+    // this nor the later barrier, 1.5 % faster with the barrier alone)
     asm volatile("" ::"s"(total_waves), "s"(groups_n), "s"(div_groups_n.m), "s"(div_groups_n.s), "s"(chunk), "s"(g.x), "s"(g.w),
                  "s"(g.x_bytes), "s"(g.w_bytes), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.batches), "s"(g.x_sx), "s"(g.ldw), "s"(g.ldo),
                  "s"(g.o_bytes), "s"(g.out), "s"(g.bias), "s"(g.bias_len), "s"(g.zx), "s"(g.mult), "s"(g.shift),
                  "s"(g.mult16), "s"(g.rp.out_zp), "s"(g.rp.out_lo), "s"(g.rp.out_hi), "s"(g.rp.double_round),
                  "s"(g.rp.per_channel));
-    if constexpr (RES)
-        asm volatile("" ::"s"(g.res), "s"(g.rs_res.mult), "s"(g.rs_res.shift), "s"(g.rs_res.mult16), "s"(g.rs_res.p.in_zp), "s"(g.rs_res.p.out_zp),
-                     "s"(g.rs_res.p.double_round), "s"(g.rs_conv.mult), "s"(g.rs_conv.shift), "s"(g.rs_conv.mult16), "s"(g.rs_conv.p.in_zp),
-                     "s"(g.rs_conv.p.out_zp), "s"(g.rs_conv.p.double_round), "s"(g.rs_out.mult), "s"(g.rs_out.shift), "s"(g.rs_out.mult16),
-                     "s"(g.rs_out.p.out_zp), "s"(g.rs_out.p.out_lo), "s"(g.rs_out.p.out_hi), "s"(g.rs_out.p.double_round));
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks are dealt round-robin to the XCDs: XCD k gets the k-th contiguous run of blocks, so the tiles of a
