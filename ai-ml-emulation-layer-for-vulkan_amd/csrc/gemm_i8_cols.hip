@@ -43,9 +43,8 @@ __global__ void __launch_bounds__(kColsBlock) conv_cols_mfma_i8_kernel(const Gem
                                                                          const DivMagic div_groups_n, int chunk) {
     // every argument that the tile assignment, the first operand requests and the epilogue depend on, asked for in one
     // batch: left alone the compiler loads most of them behind the early exit, a second trip to memory in a row
-    // (not the residual's: nothing in front of the loop waits for them, and twenty more to wait for cost 0.1 us, or 3 %, at up to 256
-    // channels: 32 -> 24 over 294 positions 4.12 us with them, 3.97 without; over 300 such sizes 1.5 % slower than with neither
-    // this nor the later barrier, 1.5 % faster with the barrier alone)
+    // (not the residual's, which nothing in front of the loop waits for: with them in the batch 144 -> 120 channels over 12 636
+    // positions took 6.24 us, without 5.96; 196 sizes of up to 256 channels 3.4 % longer on average, 104 of more 0.9 %)
     asm volatile("" ::"s"(total_waves), "s"(groups_n), "s"(div_groups_n.m), "s"(div_groups_n.s), "s"(chunk), "s"(g.x), "s"(g.w),
                  "s"(g.x_bytes), "s"(g.w_bytes), "s"(g.M), "s"(g.N), "s"(g.K), "s"(g.batches), "s"(g.x_sx), "s"(g.ldw), "s"(g.ldo),
                  "s"(g.o_bytes), "s"(g.out), "s"(g.bias), "s"(g.bias_len), "s"(g.zx), "s"(g.mult), "s"(g.shift),
