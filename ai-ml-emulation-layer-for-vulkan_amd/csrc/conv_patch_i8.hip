@@ -749,6 +749,13 @@ int try_conv_patch_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, cons
     bool direct = false;
     int nw = 4, nj = 1, tm = 1;
     size_t sm = 0;
+    // how often a wavefront of the kernel without a loop asks for two columns of four rows of the patch and waits for them: a patch
+    // that is wide and low takes as many trips to memory in a row (1 x 1, 108 -> 16 channels at 101 x 188, batch 11, in tiles of 64 x 2:
+    // 14 of them, 27 us; as before, 13)
+    const auto fetches = [&](int64_t ph, int64_t pw, int which) {
+        const int64_t row = std::max<int64_t>(1, pw * g.cpp[which]), turn = nw * std::max<int64_t>(1, 64 / row);
+        return ((row + 63) / 64 + 1) / 2 * (((ph + turn - 1) / turn + 3) / 4);
+    };
     // the tile: the shape of its positions with the least padding, then the smallest patch; false: none whose shared memory
     // leaves room for two blocks on a compute unit
     const auto choose = [&]() {
@@ -760,6 +767,7 @@ int try_conv_patch_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, cons
             const int64_t patch = ph * pw;
             if (ph > 511 || pw > 255 || patch * g.pitch > 65536) continue;  // what a thread's chunk descriptors hold
             if (per_thread(patch, 0) + per_thread(patch, 1) > kChunks * nw / (direct && unit == 4 ? 2 : 4)) continue;
+            if (direct && std::max(fetches(ph, pw, 0), fetches(ph, pw, 1)) > 3) continue;
             if (best >= 0 && (area > best || (area == best && patch >= best_patch))) continue;
             best = area, best_patch = patch;
             g.log_tw = lt, g.TH = (int)th, g.PH = (int)ph, g.PW = (int)pw;
@@ -808,8 +816,17 @@ int try_conv_patch_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, cons
             nw = 8;
             if (!choose()) nw = 4, choose();
         }
+        // Where the other kernel has 64 channels to a block and this one's shared memory leaves 32, twice as many blocks fetch the
+        // patch: TRANSPOSE_CONV2D 192 -> 97, 3 x 3, eight images of 95 x 18 20.9 us looped, 27.0 here; 9 of 17 such sizes longer, by up to 38 %
+        if (looped && nj0 == 2 && nj == 1) fits = false;
+        // What the other kernel does not take: not where most of a tile lies outside a small image, nor kernels of one or two
+        // taps, for which contract_i8.hip's stages are short (68 -> 398, 2 x 2, over 105 x 1, batch 15: 9.1 us there, 15.6 here; 1 x 1,
+        // 124 -> 128 at 69 x 177, batch 2: 8.3, 19.6; 2 x 1, 84 -> 186 at 139 x 39, batch 4: 11.9, 15.0; 3 x 3 and larger: 23 % faster here on
+        // average over 67 sizes)
+        if (!looped && fits && (positions * 3 < B * g.tiles_x * g.tiles_y * 32 * nw * tm || (!transposed && in2 == nullptr && kh * kw < 3)))
+            fits = false;
         if (!fits) {
-            direct = false, nj = nj0, tm = tm0;
+            direct = false, nw = 4, nj = nj0, tm = tm0;
             if (looped) choose();
         }
     }
