@@ -292,12 +292,28 @@ int try_conv2d_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
         const int rc = try_conv_few_i8(ctx, s, out, in, nullptr, w, bias, epi, a->input_zp, a->weight_zp, a->pad, a->stride, a->dilation, false);
         if (rc != 0) return rc;
     }
-    // 64 channels fill the staged kernel's steps, but its 32 KiB of operands per step for every tap again cost more than a
-    // patch: 64 -> 64, 3 x 3, at 112 x 112, batch 16: 28.8 -> 21.2 us; -> 96, batch 4: 15.2 -> 11.8; -> 160: 20.1 -> 17.2; -> 300, batch 2: 17.1 ->
-    // 18.0; 128 -> 128 at 160 x 160: 13.3 -> 17.6
-    if (packed8 && IC == 64 && KH * KW > 1 && OC <= 192 && static_scratch == nullptr) {
-        const int rc = try_conv_patch_i8(ctx, s, out, in, nullptr, w, bias, epi, a->input_zp, a->weight_zp, a->pad, a->stride, a->dilation, false);
-        if (rc != 0) return rc;
+    // 64 channels fill the staged kernel's steps, but its 32 KiB of operands per step for every tap again can cost more than a patch
+    // (conv_patch_i8.hip): 3 x 3 and larger
+    // - where its tile is the one of 32 channels (OC % 64 in 1 .. 32), which fetches X twice as often (24 % on average over 177
+    //   sizes, one slower);
+    // - where it stores byte by byte (OC % 4 != 0), up to three of its tiles of 64 x 64 per compute unit (20 % over 62 sizes; with four
+    //   and five 64 -> 61 over 67 840 positions 14.9 -> 17.3 us);
+    // - 3 x 3, where it has two tall tiles per unit and the sums of the weights to make (14 % over 174; 112 x 112, batch 16: 28.8 -> 21.2 us;
+    //   no zero point, 64 -> 164 over 106 704 positions: 30.5 there, 33.7 here);
+    // 2 x 2 where both of the first hold (20 % over 30).  Elsewhere it is up to 1.9 times as fast (2 x 2, stride 2, 64 -> 168 over
+    // 14 880 positions 6.6, 12.3).
+    if (packed8 && IC == 64 && OC <= 192 && static_scratch == nullptr) {
+        const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256, taps = KH * KW;
+        const auto up = [](int64_t n, int64_t to) { return (n + to - 1) / to * to; };
+        const bool narrow = up(OC, 32) < up(OC, 64), bytes = OC % 4 != 0;
+        const int64_t width = up(OC, 128) == up(OC, 64) ? 128 : 64, height = width == 128 ? 128 : 256;
+        const bool tall = (M + height - 1) / height * (up(OC, width) / width) >= 2 * cus;
+        if (taps >= 9 ? narrow || (bytes && M * up(OC, 64) <= 3 * 64 * 64 * cus) || (taps < 16 && tall && g.zx != 0)
+                      : taps >= 4 && narrow && bytes && a->stride[0] == 1 && a->stride[1] == 1) {
+            const int rc =
+                try_conv_patch_i8(ctx, s, out, in, nullptr, w, bias, epi, a->input_zp, a->weight_zp, a->pad, a->stride, a->dilation, false);
+            if (rc != 0) return rc;
+        }
     }
     SplitScratch sc;
     if (static_scratch != nullptr) {  // the caller's region instead of the context's workspace

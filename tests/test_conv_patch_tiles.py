@@ -36,6 +36,11 @@ CASES = [
     (1, 90, 100, 20, 20, (7, 7), (1, 1), (1, 1), (3, 3, 3, 3), -5),
     (1, 282, 281, 4, 300, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 5),         # many channels: blocks that walk tiles
     (1, 900, 890, 24, 7, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), -7),         # many tiles of many steps: the same
+    # 64 channels instead of the staged kernel: a result of 1 .. 32 channels modulo 64, of no whole dwords, many tiles
+    (1, 130, 132, 64, 20, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 0),
+    (1, 101, 99, 64, 39, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), -128),
+    (1, 364, 362, 64, 36, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 5),
+    (1, 190, 93, 64, 27, (2, 2), (1, 1), (1, 1), (0, 1, 0, 1), -5),
     (1, 262, 258, 56, 64, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), -3),        # 64 channels to a block where blocks walk tiles, 32 here: the same
     (1, 64, 190, 84, 20, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 6),          # a wide low tile would be fetched in too many turns
     (4, 105, 3, 68, 398, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 127),        # most of a tile outside the image: staged
