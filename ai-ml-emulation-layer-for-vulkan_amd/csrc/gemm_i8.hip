@@ -294,11 +294,11 @@ int try_conv2d_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
     }
     // 64 channels fill the staged kernel's steps, but its 32 KiB of operands per step for every tap again can cost more than a patch
     // (conv_patch_i8.hip): 3 x 3 and larger
-    // - where its tile is the one of 32 channels (OC % 64 in 1 .. 32), which fetches X twice as often (24 % on average over 177
+    // - where its tile is the one of 32 channels (OC % 64 in 1 .. 32), which fetches X twice as often (25 % on average over 169
     //   sizes, one slower);
     // - where it stores byte by byte (OC % 4 != 0), up to three of its tiles of 64 x 64 per compute unit (20 % over 62 sizes; with four
     //   and five 64 -> 61 over 67 840 positions 14.9 -> 17.3 us);
-    // - 3 x 3, where it has two tall tiles per unit and the sums of the weights to make (14 % over 174; 112 x 112, batch 16: 28.8 -> 21.2 us;
+    // - 3 x 3, where it has two tall tiles per unit and the sums of the weights to make (16 % over 174; 112 x 112, batch 16: 28.8 -> 21.2 us;
     //   no zero point, 64 -> 164 over 106 704 positions: 30.5 there, 33.7 here);
     // 2 x 2 where both of the first hold (20 % over 30).  Elsewhere it is up to 1.9 times as fast (2 x 2, stride 2, 64 -> 168 over
     // 14 880 positions 6.6, 12.3).
@@ -392,10 +392,14 @@ int try_matmul_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
     }
     // K-major W, at most one tile of 64 x 64 per compute unit: product_i8.hip, whose wavefronts share K there.  us, here / there:
     // 16 x 1024 x 1024 6.3 / 4.1, 64 x 4096 x 4096 14.3 / 9.2, 512 x 1024 x 1024 (128 tiles) 7.7 / 6.0, 1024^3 (256) 7.9 / 6.2,
-    // 1100 x 1024 x 1024 (288) 8.0 / 8.8, 1920 x 512 x 1024 (480) 6.0 / 6.7.
+    // 1100 x 1024 x 1024 (288) 8.0 / 8.8, 1920 x 512 x 1024 (480) 6.0 / 6.7.  Not a short K with a RESCALE on a quarter to a half of a tile
+    // per unit, which are several of its 32 x 32 with eight wavefronts each: 2 x 45 x 32 x 3888 (122) 3.5 / 4.4, 230 x 688 x 320 five
+    // times (100) 5.1 / 6.2, 1517 x 32 x 176 (72) 3.9 / 4.5; 86 such sizes up to K = 511 took 3 % less there on average but 27 more,
+    // by up to 27 %; 46 longer ones 21 % less, 294 with an int32 result 35 %.
     if (!b_rows) {
         const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
-        if ((M + 63) / 64 * ((N + 63) / 64) * NB <= cus) {
+        const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64) * NB;
+        if (tiles <= cus && !(epi != nullptr && K < 512 && tiles * 4 > cus && tiles * 2 < cus)) {
             const int rc = try_matmul_i8_ragged(ctx, s, out, A, B, attr, epi);
             if (rc != 0) return rc;
         }
