@@ -158,8 +158,9 @@ enum { F_PIECES = 0,   // aligned 16-byte pieces
        F_RUNS = 2,     // convolutions: the taps of a kernel row are one run of KW IC elements, padded to whole pieces of K, that
                        // lie anywhere; elements outside the image or beyond the run are zeros
        F_ELEMS = 3,    // element by element along K (convolutions dilated along the row)
-       F_KMAJOR = 4 }; // W of a product only: pieces of the rows of [K][N], from any address, transposed on their way out of
+       F_KMAJOR = 4,   // W of a product only: pieces of the rows of [K][N], from any address, transposed on their way out of
                        // shared memory
+       F_TAPS = 5 };   // X, DIRECT: F_PIECES with the taps inside the image as a bit each
 
 // What position m gives for column n before its rounding, over the taps inside the image one after the other, until the sum is
 // NaN for good; false for a position whose taps all lie inside.
@@ -413,9 +414,17 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             (uint32_t) reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem) + (uint32_t)(wave * 1024);
         // A wavefront that has its SIMD to itself issues an instruction every 7 clocks or so, and the loop is a few dozen of
         // them beside eight matrix instructions: what a request costs is what the loop takes.  So the place of a piece among the
-        // taps comes from two multiplications, and W's rows advance by the scalar offset alone.  (The taps that a row meets
-        // inside the image were a bit each, made in front of the loop: 1400 clocks there, for one instruction less per request.)
-        uint32_t wo[WI];
+        // taps comes from two multiplications, and W's rows advance by the scalar offset alone.  F_TAPS makes the taps that a
+        // row meets inside the image a bit each in front of the loop: 1400 clocks there, for fewer instructions per request.
+        uint32_t wo[WI], my[XI], mx[XI];
+        if constexpr (XF == F_TAPS) {
+#pragma unroll
+            for (int i = 0; i < XI; i++) {
+                my[i] = mx[i] = 0;
+                for (int y = 0; y < g.KH; y++) my[i] |= (uint32_t)(iy0[i] + y * g.dy) < (uint32_t)g.H ? 1u << y : 0u;  // uniform trip count
+                for (int x = 0; x < g.KW; x++) mx[i] |= (uint32_t)(ix0[i] + x * g.dx) < (uint32_t)g.W ? 1u << x : 0u;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < WI; i++) {
             const int n = n0 + i * (NT / PPR);
@@ -429,17 +438,25 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) contract_float_kernel(const
             const int y = (int)(__umul24((uint32_t)tap, g.kw_magic) >> 16), x = tap - (int)__umul24((uint32_t)y, (uint32_t)g.KW);
             const uint32_t t = __umul24((uint32_t)y, y_step) + __umul24((uint32_t)x, x_step) + (uint32_t)(c * SZ);
             const bool partial = (asked + 1) * PPR * E > g.K;  // uniform: the last stage ends beyond K
-            int yd = y * g.dy;
-            const int xd = x * g.dx;
-            if (partial) {
-                yd = kpos < g.K ? yd : 0x20000000;  // no tap: outside the image
-                asm volatile("" : "+v"(yd));  // (a branch, not a select in every stage)
-            }
+            if constexpr (XF == F_TAPS) {  // (beyond the last tap: bits that are not set; 32 rows of taps are whole stages)
 #pragma unroll
-            for (int i = 0; i < XI; i++) {
-                const bool in = (uint32_t)(iy0[i] + yd) < (uint32_t)g.H && (uint32_t)(ix0[i] + xd) < (uint32_t)g.W;
-                const uint32_t off = in ? (uint32_t)xb[i] + t : kOob;
-                load16_to_lds(xres, d + i * NT * 16, off, 0);
+                for (int i = 0; i < XI; i++) {
+                    const uint32_t in = (uint32_t)(__builtin_amdgcn_sbfe((int)my[i], y, 1) & __builtin_amdgcn_sbfe((int)mx[i], x, 1));
+                    load16_to_lds(xres, d + i * NT * 16, (in & ((uint32_t)xb[i] + t)) | (~in & kOob), 0);
+                }
+            } else {
+                int yd = y * g.dy;
+                const int xd = x * g.dx;
+                if (partial) {
+                    yd = kpos < g.K ? yd : 0x20000000;  // no tap: outside the image
+                    asm volatile("" : "+v"(yd));  // (a branch, not a select in every stage)
+                }
+#pragma unroll
+                for (int i = 0; i < XI; i++) {
+                    const bool in = (uint32_t)(iy0[i] + yd) < (uint32_t)g.H && (uint32_t)(ix0[i] + xd) < (uint32_t)g.W;
+                    const uint32_t off = in ? (uint32_t)xb[i] + t : kOob;
+                    load16_to_lds(xres, d + i * NT * 16, off, 0);
+                }
             }
 #pragma unroll
             for (int i = 0; i < WI; i++) {
@@ -990,6 +1007,12 @@ int launch_shape(mlel_ctx *ctx, FArgs &g, int64_t batches, hipStream_t s) {
     const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
     auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * batches; };
     if constexpr (DIRECT) {
+        // the taps as bits where the loop is long: against the comparisons, over some 600 convolutions and products, fp32 took
+        // 1.02-1.06 of the time up to K = 128, 1.00 at 512, 0.94-0.98 to 1024, 0.92 to 2048, 0.85 beyond 4096 (K = 11760, 16 channels over
+        // four of 2 x 189: 36.7 -> 30.5 us); the halves 1.03-1.14 up to 4096, 0.96-0.98 beyond (K = 21168, 47 channels over five of
+        // 37 x 16: 41.9 -> 35.8)
+        if constexpr (XF == F_PIECES)
+            if (g.K > (Elem<T>::size == 4 ? 512 : 4096)) return launch_shape<T, TO, DIRECT, F_TAPS, WF>(ctx, g, batches, s);
         if (tiles(128, 128) >= 2 * cus && g.N > 64) return launch_tile<T, TO, 128, 128, 2, 4, 1, 64, 4, DIRECT, XF, WF>(g, batches, s);
         if (tiles(64, 64) * 2 >= cus) return launch_tile<T, TO, 64, 64, 2, 2, 2, 128, 3, DIRECT, XF, WF>(g, batches, s);
         if (tiles(32, 32) * 2 <= cus) return launch_tile<T, TO, 16, 16, 1, 1, 4, 256, 3, DIRECT, XF, WF>(g, batches, s);

@@ -151,6 +151,23 @@ def test_convolution_edges(run, case, dt):
     np.testing.assert_allclose(got, want, rtol=1.01 * STEP[dt], atol=1e-5 * max(1.0, np.abs(want).max()))
 
 
+# both sides of the K from which the taps inside the image are bits of a word (fp32 512, fp16 and bf16 4096), every tile
+LONG = [
+    (1, 5, 6, 32, 20, (4, 4), (1, 1), (1, 1), (2, 1, 1, 2)), (1, 5, 6, 40, 20, (4, 4), (1, 1), (1, 1), (2, 1, 1, 2)),
+    (2, 80, 41, 16, 40, (6, 6), (2, 1), (2, 1), (5, 5, 3, 2)), (1, 100, 92, 16, 64, (6, 6), (1, 1), (1, 1), (0, 5, 2, 3)),
+    (1, 256, 257, 64, 72, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (1, 33, 20, 16, 8, (32, 3), (1, 1), (1, 2), (16, 15, 2, 2)),
+    (1, 20, 9, 8, 8, (3, 32), (1, 1), (1, 1), (1, 1, 16, 15)), (1, 6, 5, 256, 24, (4, 4), (1, 1), (1, 1), (1, 2, 2, 1)),
+    (1, 6, 5, 168, 24, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)), (1, 50, 60, 168, 40, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)),
+    (1, 60, 140, 168, 64, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)),
+]
+
+
+@pytest.mark.parametrize("dt", [abi.F16, abi.BF16, abi.F32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", LONG, ids=["_".join(map(str, c[1:5] + c[5] + c[7])) for c in LONG])
+def test_long_sums(run, case, dt):
+    test_convolution_edges(run, case, dt)
+
+
 @pytest.mark.parametrize("dt", [abi.F16, abi.F32], ids=["f16", "f32"])
 @pytest.mark.parametrize("oc", [1, 7, 20, 33, 96])
 def test_residual_of_ragged_rows(run, oc, dt):
