@@ -1051,10 +1051,23 @@ int launch_conv(mlel_ctx *ctx, FArgs &g, bool direct, hipStream_t s) {
     constexpr int E = 16 / Elem<T>::size;
     const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
     const int64_t ppr = (g.KW * (int64_t)g.IC + E - 1) / E, pieces = g.KH * ppr, tiles = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-    if (g.dx == 1 && pieces <= 16 && g.wide_out && g.res == nullptr && g.x_bytes >= 16 && g.w_bytes >= 16 && 4 * tiles >= 11 * cus &&
+    // More than six pieces, against the stages over 2500 calls.  Halves: the seven or eight that fill a stage, and rows that are no
+    // whole words or three pieces and more, lost up to 1.9 of the time (3 x 3 x 7 -> 232 over 43344 fp16: 19.2 us staged, 30.3 without;
+    // 4 x 4 x 6 -> 16 over 22876 bf16: 5.2, 6.1); nine or ten of an even number of channels take 0.55-0.97, most that leave more than
+    // 2048 sub-tiles to 32 channels 0.48-0.98.  Without a border the masks are one and more is won: 32 channels 0.48-1.05, rows of
+    // two pieces 0.57-1.05.  fp32 lost beyond ten pieces of more than 32 channels with a border (0.85-1.26; the others 0.37-1.13).
+    const int64_t steps = (pieces + 1) / 2;
+    const bool narrow = g.N <= 32, words = g.IC % 2 == 0;
+    bool taken;
+    if (Elem<T>::size == 4) taken = steps <= 5 || narrow || !g.border;
+    else if (steps <= 3 || (narrow && tiles > 8 * cus && (words || steps <= 5))) taken = true;
+    else if (g.border) taken = steps == 5 && (words || (ppr <= 2 && narrow));
+    else if (narrow) taken = words || ppr <= 2 || tiles <= 4 * cus;
+    else taken = words ? steps == 5 || steps >= 7 : ppr <= 2;
+    if (g.dx == 1 && pieces <= 16 && taken && g.wide_out && g.res == nullptr && g.x_bytes >= 16 && g.w_bytes >= 16 && 4 * tiles >= 11 * cus &&
         (g.N <= 32 || tiles <= 4 * cus || tiles >= 16 * cus)) {
         g.div_ppr = make_div_magic((uint32_t)ppr);
-        return g.N > 32 && tiles > 4 * cus ? launch_runs<T, 2>(g, (int)(pieces + 1) / 2, s) : launch_runs<T, 1>(g, (int)(pieces + 1) / 2, s);
+        return g.N > 32 && tiles > 4 * cus ? launch_runs<T, 2>(g, (int)steps, s) : launch_runs<T, 1>(g, (int)steps, s);
     }
     return g.dx == 1 ? launch_shape<T, T, false, F_RUNS, F_RUNS>(ctx, g, 1, s) : launch_shape<T, T, false, F_ELEMS, F_ELEMS>(ctx, g, 1, s);
 }

@@ -26,6 +26,14 @@ CASES = [
     (1, 153, 152, 5, 8, (3, 3), (1, 1), (2, 1), (2, 2, 1, 1)),    # dilated along the column; fp32: six steps
     (3, 101, 80, 2, 32, (4, 2), (1, 1), (1, 1), (0, 0, 0, 0)),    # no border
     (1, 40, 700, 3, 8, (3, 3), (1, 1), (1, 1), (4, 4, 5, 5)),     # positions that meet no pixel
+    # more pieces: what stays without stages
+    (1, 262, 260, 4, 16, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)),   # eight steps, more than 2048 sub-tiles of 32 channels at most
+    (1, 258, 257, 7, 24, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),   # five, rows that are no whole words (fp32: a piece too many)
+    (1, 90, 84, 6, 88, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),     # five of an even number of channels (fp32: eight, with stages)
+    (1, 90, 84, 7, 88, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),     # and of an odd one: with stages
+    (1, 90, 84, 4, 88, (4, 4), (1, 1), (1, 1), (2, 1, 1, 2)),     # four: with stages
+    (1, 92, 88, 2, 88, (7, 7), (1, 1), (1, 1), (0, 0, 0, 0)),     # no border: seven of an even number of channels, without
+    (1, 130, 129, 7, 264, (5, 2), (1, 1), (1, 1), (0, 0, 0, 0)),  # five of an odd one, two pieces a row, two groups of channels
 ]
 
 
