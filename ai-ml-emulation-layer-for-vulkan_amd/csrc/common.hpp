@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "../../include/mlel_hip.h"
+#include "fresh_blocks.hpp"
 
 namespace mlel {
 
@@ -622,7 +623,7 @@ constexpr size_t kMaxStageBytes = size_t(2) << 30;
 
 // Small allocations are made and cleared ahead and waited for several at a time (arena_alloc in runtime.hip): of a class both
 // lists together hold at most eight, so all of them less than 1 MiB.
-constexpr int kFreshClasses = 5, kFreshBlocks = 8;
+constexpr int kFreshClasses = 5;
 
 struct mlel_ctx {
     int device;
@@ -638,9 +639,7 @@ struct mlel_ctx {
     char *static_scratch = nullptr;
     hipStream_t clear_stream = nullptr;  // where fresh memory is cleared
     std::mutex fresh_lock;
-    // allocations of 4 KiB << class that are cleared and not handed out yet, and those whose clearing nobody has waited for
-    void *fresh[kFreshClasses][kFreshBlocks], *clearing[kFreshClasses][kFreshBlocks];
-    int n_fresh[kFreshClasses] = {}, n_clearing[kFreshClasses] = {};
+    mlel::FreshBlocks fresh[kFreshClasses];  // of 4 KiB << class each
     int static_last_use = 0;  // what the last call of that entry point kept there: 0 nothing, 1 split-K tiles, 2 accumulator
 };
 

@@ -483,10 +483,7 @@ void mlel_hip_destroy(mlel_ctx *ctx) {
     if (hipSetDevice(ctx->device) == hipSuccess) {
         (void)hipDeviceSynchronize();  // no launch may still be using a workspace that is about to be freed
         free_split_workspaces(ctx);
-        for (int c = 0; c < kFreshClasses; c++) {
-            while (ctx->n_fresh[c] > 0) (void)hipFree(ctx->fresh[c][--ctx->n_fresh[c]]);
-            while (ctx->n_clearing[c] > 0) (void)hipFree(ctx->clearing[c][--ctx->n_clearing[c]]);
-        }
+        for (mlel::FreshBlocks &blocks : ctx->fresh) blocks.clear([](void *p) { (void)hipFree(p); });
         (void)hipStreamDestroy(ctx->clear_stream);
     }
     delete ctx;
@@ -512,9 +509,9 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
     MLEL_HIP_CHECK(hipSetDevice(ctx->device));
     // Tensors start zero-filled, as the reference's test tensors do; the clearing has ended before the memory is handed out, since no
     // stream that may write there next waits for it.  On a stream of its own: on the null stream a clear of 1 MiB and the wait took
-    // 118 us, here 33 (16 MiB 293, 42).  Of an allocation of 4 KiB the wait is 8 of 13 us, so up to 64 KiB they are made ahead and
-    // eight are waited for at a time; each is an allocation of its own, and a call makes at least one, so that what refuses an
-    // allocation (a capture on this thread) refuses every call.
+    // 118 us, here 33 (16 MiB 293, 42).  Of an allocation of 4 KiB the wait is 8 of 13 us, so up to 64 KiB they are made ahead, in
+    // sizes of a power of two from 4 KiB, each an allocation of its own, and eight are waited for at a time.  A call makes at least
+    // one, so that what refuses an allocation (a capture on this thread) refuses every call.
     int cls = 0;
     while (cls < kFreshClasses && bytes > (size_t(4096) << cls)) cls++;
     if (cls == kFreshClasses) {
@@ -528,32 +525,26 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
         }
         return 0;
     }
-    std::lock_guard<std::mutex> lock(ctx->fresh_lock);
-    void **fresh = ctx->fresh[cls], **clearing = ctx->clearing[cls];
-    int &n = ctx->n_fresh[cls], &m = ctx->n_clearing[cls];
     const size_t size = size_t(4096) << cls;
-    auto make = [&] {
-        hipError_t e = hipMalloc(&clearing[m], size);
-        if (e != hipSuccess) return e;
-        e = hipMemsetAsync(clearing[m], 0, size, ctx->clear_stream);
-        if (e != hipSuccess) (void)hipFree(clearing[m]);
-        else m++;
+    const char *call = "";  // the one that failed
+    auto make = [&](void **block) {
+        call = "hipMalloc";
+        hipError_t e = hipMalloc(block, size);
+        if (e == hipSuccess) {
+            call = "hipMemsetAsync";
+            e = hipMemsetAsync(*block, 0, size, ctx->clear_stream);
+            if (e != hipSuccess) (void)hipFree(*block);
+        }
+        if (e != hipSuccess) (void)hipGetLastError();  // (it may be one that is not needed, and the next launch looks there)
         return e;
     };
-    hipError_t e = make();
-    if (e == hipErrorOutOfMemory && n > 0) e = hipSuccess, (void)hipGetLastError();  // (there is one all the same)
-    if (e != hipSuccess) return set_error(MLEL_ERR_DEVICE, "hipMalloc(dptr, bytes) failed: %s", hipGetErrorString(e));
-    if (n == 0) {  // (m is at most the number that were handed out since, and one)
-        while (m < kFreshBlocks && make() == hipSuccess) {}
-        (void)hipGetLastError();
-        e = hipStreamSynchronize(ctx->clear_stream);
-        if (e != hipSuccess) {
-            while (m > 0) (void)hipFree(clearing[--m]);
-            return set_error(MLEL_ERR_DEVICE, "arena_alloc: %s", hipGetErrorString(e));
-        }
-        while (m > 0) fresh[n++] = clearing[--m];
-    }
-    *dptr = fresh[--n];
+    auto wait = [&] {
+        call = "hipStreamSynchronize";
+        return hipStreamSynchronize(ctx->clear_stream);
+    };
+    std::lock_guard<std::mutex> lock(ctx->fresh_lock);
+    const hipError_t e = ctx->fresh[cls].take(dptr, hipErrorOutOfMemory, make, wait, [](void *p) { (void)hipFree(p); });
+    if (e != hipSuccess) return set_error(MLEL_ERR_DEVICE, "arena_alloc: %s of %zu bytes failed: %s", call, size, hipGetErrorString(e));
     return 0;
 }
 
