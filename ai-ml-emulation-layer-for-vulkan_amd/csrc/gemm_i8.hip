@@ -395,11 +395,12 @@ int try_matmul_i8_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, con
     // 1100 x 1024 x 1024 (288) 8.0 / 8.8, 1920 x 512 x 1024 (480) 6.0 / 6.7.  Not a short K with a RESCALE on a quarter to a half of a tile
     // per unit, which are several of its 32 x 32 with eight wavefronts each: 2 x 45 x 32 x 3888 (122) 3.5 / 4.4, 230 x 688 x 320 five
     // times (100) 5.1 / 6.2, 1517 x 32 x 176 (72) 3.9 / 4.5; 86 such sizes up to K = 511 took 3 % less there on average but 27 more,
-    // by up to 27 %; 46 longer ones 21 % less, 294 with an int32 result 35 %.
+    // by up to 27 %; 46 longer ones 21 % less, 294 with an int32 result 35 %.  With at most 48 columns also from a half on: 1954 x 48 x 32
+    // seven times (217) 4.0 / 4.7, and 7 % more over eleven such sizes.
     if (!b_rows) {
         const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
         const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64) * NB;
-        if (tiles <= cus && !(epi != nullptr && K < 512 && tiles * 4 > cus && tiles * 2 < cus)) {
+        if (tiles <= cus && !(epi != nullptr && K < 512 && tiles * 4 > cus && (tiles * 2 < cus || N <= 48))) {
             const int rc = try_matmul_i8_ragged(ctx, s, out, A, B, attr, epi);
             if (rc != 0) return rc;
         }

@@ -227,6 +227,7 @@ MM_CASES = [
     ("zp_b_only", 2, 33, 64, 64, 0, -9),
     ("k_small", 4, 300, 8, 16, 1, 1),
     ("short_k_half_of_the_units", 2, 45, 96, 3888, 2, -1),  # 122 tiles of 64 x 64: with a RESCALE the staged kernel
+    ("short_k_few_columns", 3, 3207, 64, 32, 0, 4),  # 153, of half a tile each
 ]
 
 
