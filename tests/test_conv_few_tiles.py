@@ -59,6 +59,39 @@ def test_conv2d_of_few_tiles_vs_oracle(dev, oracle, case):
     np.testing.assert_array_equal(run.conv2d(x, wt, b, shape, abi.I8, attr, epilogue=(mult, shift, rattr, (-100, 90))), exp)
 
 
+def rescales(rng, oc, taps):
+    """RESCALE as its multiplier, shift, attribute and CLAMP: 16-bit multipliers, one rounding, results without a sign."""
+    for per_channel in (True, False):
+        n = oc if per_channel else 1
+        mult, shift = scale(rng, n, taps)
+        mult16 = rng.integers(2 ** 14, 2 ** 15 - 1, (n,), endpoint=True).astype(np.int16)
+        yield mult16, (shift - 16).astype(np.int8), abi.rescale_attr(0, -3, False, False, per_channel), (-100, 90)
+        yield mult, shift, abi.rescale_attr(0, 3, True, False, per_channel), (-100, 90)
+        yield mult, shift, abi.rescale_attr(0, 120, True, per_channel, per_channel, output_unsigned=True), None
+        yield mult16, (shift - 16).astype(np.int8), abi.rescale_attr(0, 17, False, False, per_channel, output_unsigned=True), None
+
+
+def every_rescale(dev, oracle, case):
+    n, h, w, ic, oc, (kh, kw), (sy, sx), (dy, dx), pad, zx = case
+    run, rng = Runner(dev), np.random.default_rng(zlib.crc32(repr(case).encode()))
+    x, wt, b = i8(rng, (n, h, w, ic)), i8(rng, (oc, kh, kw, ic)), rng.integers(-2 ** 12, 2 ** 12, (oc,)).astype(np.int32)
+    shape = (n, (h + pad[0] + pad[1] - (kh - 1) * dy - 1) // sy + 1, (w + pad[2] + pad[3] - (kw - 1) * dx - 1) // sx + 1, oc)
+    attr = abi.conv2d_attr(pad, (sy, sx), (dy, dx), zx, 0)
+    sums = oracle.conv2d(x, wt, b, shape, abi.I32, attr)
+    for mult, shift, rattr, clamp in rescales(rng, oc, kh * kw * ic):
+        exp = oracle.rescale(sums, mult, shift, abi.I8, rattr)
+        if clamp is not None:
+            exp = np.clip(exp, *clamp)
+        got = run.conv2d(x, wt, b, shape, abi.I8, attr, epilogue=(mult, shift, rattr, clamp))
+        np.testing.assert_array_equal(got.view(np.uint8), exp.astype(got.dtype, copy=False).view(np.uint8))
+        assert len(np.unique(exp)) > 20
+
+
+@pytest.mark.parametrize("case", [CASES[k][:-1] for k in (2, 5, 7, 15, 18)], ids=["rows_of_17", "three_stages", "tiles_of_32", "ragged", "ragged_tiles_of_32"])
+def test_every_rescale_of_few_tiles(dev, oracle, case):
+    every_rescale(dev, oracle, case)
+
+
 @pytest.mark.parametrize("zx", [200, -129])
 @pytest.mark.parametrize("ic", [64, 20], ids=["pieces", "ragged"])
 def test_zero_points_that_are_no_byte(dev, oracle, ic, zx):

@@ -63,6 +63,12 @@ def test_conv2d_of_a_tile_per_block_vs_oracle(dev, oracle, case):
     np.testing.assert_array_equal(run.conv2d(x, wt, b, shape, abi.I8, attr, epilogue=(mult, shift, rattr, (-100, 90))), exp)
 
 
+@pytest.mark.parametrize("case", [CASES[k] for k in (0, 2, 5, 7, 14, 12)],
+                         ids=["4_channels", "stride", "64_to_a_block", "eight_wavefronts", "whole_pieces", "blocks_that_walk"])
+def test_every_rescale_of_a_tile_per_block(dev, oracle, case):
+    few.every_rescale(dev, oracle, case)
+
+
 @pytest.mark.parametrize("n, h, w, ic, c1, c2, oc, s", [(1, 75, 81, 20, 12, 20, 36, (2, 2)), (2, 70, 75, 48, 32, 16, 24, (2, 2)),
                                                         (1, 40, 130, 64, 40, 56, 48, (3, 2)), (1, 180, 160, 24, 24, 24, 24, (2, 2))])
 def test_two_images_and_transposed_convolution_of_a_tile_per_block(dev, n, h, w, ic, c1, c2, oc, s):

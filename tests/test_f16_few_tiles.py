@@ -21,6 +21,7 @@ CASES = [
     (1, 600, 288, 1000),                       # K-major: three tiles per unit; row-wise: 64 x 64, steps of 32
     (1, 1000, 320, 712),                       # row-wise: 64 x 64, steps of 64; K-major: 64 x 64 with the bias
     (1, 1030, 1088, 1048),                     # K-major MATMUL of long rows without shared K
+    (1, 2050, 320, 2056),                      # K-major: 128 x 128
 ]
 
 

@@ -9,7 +9,8 @@ pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="n
 
 CASES = [
     # m, k, n
-    (65, 64, 72), (1, 128, 8), (130, 320, 200), (63, 96, 136),        # 64 x 64: steps of 64 halfs, of 32
+    (65, 64, 72), (1, 128, 8), (130, 320, 200), (63, 96, 136),        # at most two tiles of 32 x 32 per unit: the kernel of few tiles
+    (1005, 320, 712), (999, 288, 600),                                 # 64 x 64: steps of 64 halfs, of 32
     (3900, 256, 2296), (4096, 288, 2304),                              # 256 x 192
     (4000, 256, 3080),                                                 # 256 x 256
     (1700, 832, 1496), (1665, 1024, 1544),                             # 128 x 128, steps of 64

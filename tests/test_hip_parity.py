@@ -1199,9 +1199,11 @@ def test_external_memory_import_by_file_descriptor(run):
     data = np.random.default_rng(3).integers(-128, 127, n, endpoint=True).astype(np.int8)
     dev._check(dev.lib.mlel_hip_memcpy_h2d(dev.ctx, C.c_void_p(src), data.ctypes.data_as(C.c_void_p), n, None))
     fd = C.c_int(-1)
-    if hip.hipMemGetHandleForAddressRange(C.byref(fd), C.c_void_p(src), n, 1, 0) != 0:  # hipMemRangeHandleTypeDmaBufFd
+    status = hip.hipMemGetHandleForAddressRange(C.byref(fd), C.c_void_p(src), n, 1, 0)  # hipMemRangeHandleTypeDmaBufFd
+    if status != 0:
         dev.free(src)
-        pytest.skip("this driver does not export device memory as a dma-buf fd")
+        hip.hipGetErrorName.restype = C.c_char_p
+        pytest.skip(f"hipMemGetHandleForAddressRange of a whole 1 MiB allocation: {hip.hipGetErrorName(status).decode()}")
     mapped, handle = C.c_void_p(), C.c_void_p()
     dev._check(dev.lib.mlel_hip_arena_import_fd(dev.ctx, fd.value, n, C.byref(mapped), C.byref(handle)))
     back = np.zeros(n, np.int8)
