@@ -1192,7 +1192,7 @@ def test_external_memory_import_by_file_descriptor(run):
     the Vulkan export; the imported mapping shows the same bytes, operators run on it, and the import is released."""
     import ctypes as C
     dev = run.dev
-    hip = C.CDLL("libamdhip64.so")
+    hip = C.CDLL(dev.lib._name)  # HIP's functions as the library sees them: another copy of the runtime may be loaded beside its own
     hip.hipMemGetHandleForAddressRange.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_ulonglong]
     n = 1 << 20
     src = dev.alloc(n)
@@ -1203,7 +1203,9 @@ def test_external_memory_import_by_file_descriptor(run):
     if status != 0:
         dev.free(src)
         hip.hipGetErrorName.restype = C.c_char_p
-        pytest.skip(f"hipMemGetHandleForAddressRange of a whole 1 MiB allocation: {hip.hipGetErrorName(status).decode()}")
+        name = hip.hipGetErrorName(status).decode()
+        assert name == "hipErrorNotSupported", f"export of a whole 1 MiB allocation: {name}"
+        pytest.skip("this driver does not export device memory as a dma-buf fd")
     mapped, handle = C.c_void_p(), C.c_void_p()
     dev._check(dev.lib.mlel_hip_arena_import_fd(dev.ctx, fd.value, n, C.byref(mapped), C.byref(handle)))
     back = np.zeros(n, np.int8)
