@@ -622,7 +622,7 @@ struct StageWorkspace {
 constexpr size_t kMaxStageBytes = size_t(2) << 30;
 
 // Small allocations are made and cleared ahead and waited for several at a time (arena_alloc in runtime.hip): of a class both
-// lists together hold at most eight, so all of them less than 1 MiB.
+// lists together hold at most kFreshBlocks, so all of them less than 512 KiB.
 constexpr int kFreshClasses = 5;
 
 struct mlel_ctx {

@@ -510,7 +510,7 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
     // Tensors start zero-filled, as the reference's test tensors do; the clearing has ended before the memory is handed out, since no
     // stream that may write there next waits for it.  On a stream of its own: on the null stream a clear of 1 MiB and the wait took
     // 118 us, here 33 (16 MiB 293, 42).  Of an allocation of 4 KiB the wait is 8 of 13 us, so up to 64 KiB they are made ahead, in
-    // sizes of a power of two from 4 KiB, each an allocation of its own, and eight are waited for at a time.  A call makes at least
+    // sizes of a power of two from 4 KiB, each an allocation of its own, and several are waited for at a time.  A call makes at least
     // one, so that what refuses an allocation (a capture on this thread) refuses every call.
     int cls = 0;
     while (cls < kFreshClasses && bytes > (size_t(4096) << cls)) cls++;

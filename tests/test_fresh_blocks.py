@@ -44,10 +44,10 @@ struct Pool {
     }
 };
 int main() {
-    {   // apart, cleared, and eight to a wait
+    {   // apart, cleared, and as many to a wait as are made ahead
         Pool pool;
         for (int i = 0; i < 100; i++) pool.good();
-        CHECK(pool.waits == 13);
+        CHECK(pool.waits == (100 + mlel::kFreshBlocks - 1) / mlel::kFreshBlocks);
     }
     for (int before = 0; before <= 17; before++) {  // refused whatever lies ready, and taken again
         Pool pool;
