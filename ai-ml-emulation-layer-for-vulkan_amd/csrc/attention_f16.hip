@@ -424,7 +424,7 @@ __global__ void __launch_bounds__(kBlock) attention_f16_kernel(const AttnArgs g)
 // What bounds it: the chain of one block (the chip is not full), of which the kernel above spends two thirds on steps of
 // 64 keys with two barriers and a trip to shared memory each.  Here eight wavefronts fetch all of K and V before anything
 // is computed (K goes to shared memory, V waits in registers until the scores are out of K's way), one wavefront multiplies
-// each 32 keys, sixteen threads share a row, and the block meets six barriers whatever the number of keys.  The two
+// each 32 keys, sixteen threads share a row, and the block meets five barriers whatever the number of keys.  The two
 // wavefronts that multiply P and V read all of V's operands while another folds.  Six heads of 197 queries and keys:
 // 8.4 -> 5.7 us (1.7 of them the launch, 0.9 the fold: 8 clocks per addition is the latency of one); operands of P V
 // fetched a chunk ahead instead of during the fold: 6.0.

@@ -622,7 +622,7 @@ struct StageWorkspace {
 constexpr size_t kMaxStageBytes = size_t(2) << 30;
 
 // Small allocations are made and cleared ahead and waited for several at a time (arena_alloc in runtime.hip): of a class both
-// lists together hold at most kFreshBlocks, so all of them less than 512 KiB.
+// lists together hold at most kFreshBlocks, so all of them less than 768 KiB.
 constexpr int kFreshClasses = 5;
 
 struct mlel_ctx {
@@ -637,7 +637,6 @@ struct mlel_ctx {
     // the statically allocated scratch of the entry point that must not allocate: this device's address of the
     // array (hipGetSymbolAddress at context creation), nullptr if that failed
     char *static_scratch = nullptr;
-    hipStream_t clear_stream = nullptr;  // where fresh memory is cleared
     std::mutex fresh_lock;
     mlel::FreshBlocks fresh[kFreshClasses];  // of 4 KiB << class each
     int static_last_use = 0;  // what the last call of that entry point kept there: 0 nothing, 1 split-K tiles, 2 accumulator

@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(64 * NW, NJ * TM == 1 || U < 16 ? 4 : 3) conv_
         const int c2 = g.IC - g.IC1;
         const uint32_t zx4 = (uint32_t)(uint8_t)g.zx * 0x01010101u;
         const int iy = oy0 * g.sy - g.pt, ix = ox0 * g.sx - g.pl, pix0 = (img * g.H + iy) * g.W + ix;
-        // a patch that lies in the image (and whose last dword does): nothing to decide per chunk
+        // a patch that lies in the image: nothing to decide per chunk
         const bool inside = iy >= 0 && ix >= 0 && iy + g.PH <= g.H && ix + g.PW <= g.W;
         struct Chunks {
             uint4 v[2][4];

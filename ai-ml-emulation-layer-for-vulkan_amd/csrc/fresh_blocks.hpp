@@ -2,9 +2,10 @@
 #pragma once
 
 namespace mlel {
-// As many as share one wait (8 us).  A 4 KiB allocation: 6.2 us with four, 5.5 with six, 7.3 with eight; with eight, instantiating a
-// recorded graph of 38 launches afterwards took 52 us instead of 43.  Preparing such a graph: 12.5, 12.6 and 12.7 ms.
-constexpr int kFreshBlocks = 4;
+// As many as share one wait (8 us).  A 4 KiB allocation: 13 us alone, 5.8 with four, 5.4 with six, 8.8 with eight.  Where the blocks lie moves
+// what the runtime allocates for itself: instantiating a recorded graph of 38 launches afterwards took 44 us with six, 58 with four, 62
+// with three, 50 with two.
+constexpr int kFreshBlocks = 6;
 
 struct FreshBlocks {
     void *fresh[kFreshBlocks], *clearing[kFreshBlocks];  // cleared and not handed out yet; those whose clearing nobody has waited for

@@ -467,10 +467,6 @@ int mlel_hip_init(int device, mlel_ctx **out_ctx) {
         delete ctx;
         return set_error(MLEL_ERR_DEVICE, "init: hipGetDeviceProperties: %s", hipGetErrorString(pe));
     }
-    if (const hipError_t ce = hipStreamCreateWithFlags(&ctx->clear_stream, hipStreamNonBlocking); ce != hipSuccess) {
-        delete ctx;
-        return set_error(MLEL_ERR_DEVICE, "init: hipStreamCreateWithFlags: %s", hipGetErrorString(ce));
-    }
     if (const char *env = std::getenv("MLEL_SPLIT_K")) ctx->split_k = std::atoi(env);  // 0: off, n: at most n splits
     // this device's address of the static scratch array; a failure only disables the entry point that needs it
     (void)static_scratch_init(ctx);
@@ -484,7 +480,6 @@ void mlel_hip_destroy(mlel_ctx *ctx) {
         (void)hipDeviceSynchronize();  // no launch may still be using a workspace that is about to be freed
         free_split_workspaces(ctx);
         for (mlel::FreshBlocks &blocks : ctx->fresh) blocks.clear([](void *p) { (void)hipFree(p); });
-        (void)hipStreamDestroy(ctx->clear_stream);
     }
     delete ctx;
 }
@@ -508,16 +503,19 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
     if (bytes == 0) bytes = 16;
     MLEL_HIP_CHECK(hipSetDevice(ctx->device));
     // Tensors start zero-filled, as the reference's test tensors do; the clearing has ended before the memory is handed out, since no
-    // stream that may write there next waits for it.  On a stream of its own: on the null stream a clear of 1 MiB and the wait took
-    // 118 us, here 33 (16 MiB 293, 42).  Of an allocation of 4 KiB the wait is 8 of 13 us, so up to 64 KiB they are made ahead, in
-    // sizes of a power of two from 4 KiB, each an allocation of its own, and several are waited for at a time.  A call makes at least
-    // one, so that what refuses an allocation (a capture on this thread) refuses every call.
+    // stream that may write there next waits for it.  Asynchronous, and then a wait: of 1 MiB hipMemset took 118 us on its own, this 27.
+    // On the null stream, which every process has: one of the context's own takes part when the runtime deals its few hardware
+    // queues to streams, and the two that a program made next shared one (two launches of 8 x 512 x 1024 x 1024 in flight 10.2 us each, here
+    // 7.3; two MobileNetV2 sessions 0.28 ms, here 0.20).
+    // Of an allocation of 4 KiB the wait is 8 of 13 us, so up to 64 KiB they are made ahead, in sizes of a power of two from 4 KiB,
+    // each an allocation of its own, and several are waited for at a time.  A call makes at least one, so that what refuses an
+    // allocation (a capture on this thread) refuses every call.
     int cls = 0;
     while (cls < kFreshClasses && bytes > (size_t(4096) << cls)) cls++;
     if (cls == kFreshClasses) {
         MLEL_HIP_CHECK(hipMalloc(dptr, bytes));
-        hipError_t e = hipMemsetAsync(*dptr, 0, bytes, ctx->clear_stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->clear_stream);
+        hipError_t e = hipMemsetAsync(*dptr, 0, bytes, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) {
             (void)hipFree(*dptr);
             *dptr = nullptr;
@@ -532,7 +530,7 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
         hipError_t e = hipMalloc(block, size);
         if (e == hipSuccess) {
             call = "hipMemsetAsync";
-            e = hipMemsetAsync(*block, 0, size, ctx->clear_stream);
+            e = hipMemsetAsync(*block, 0, size, nullptr);
             if (e != hipSuccess) (void)hipFree(*block);
         }
         if (e != hipSuccess) (void)hipGetLastError();  // (it may be one that is not needed, and the next launch looks there)
@@ -540,7 +538,7 @@ int mlel_hip_arena_alloc(mlel_ctx *ctx, size_t bytes, void **dptr) {
     };
     auto wait = [&] {
         call = "hipStreamSynchronize";
-        return hipStreamSynchronize(ctx->clear_stream);
+        return hipStreamSynchronize(nullptr);
     };
     std::lock_guard<std::mutex> lock(ctx->fresh_lock);
     const hipError_t e = ctx->fresh[cls].take(dptr, hipErrorOutOfMemory, make, wait, [](void *p) { (void)hipFree(p); });
