@@ -1084,11 +1084,12 @@ int launch_args(mlel_ctx *ctx, hipStream_t s, HGemmArgs &g, bool bias_cast) {
         MLEL_TRY(check_launch("matmul fp16, row-wise B"));
         return 1;
     }
-    // K-major B, few tiles: up to two of 32 x 32 per compute unit, three for longer contractions.  us, before / there: 256 x 1024 x
-    // 1024 11.7 / 4.6, 64 x 2048 x 4096 19.5 / 6.8, 128^3 4.8 / 2.9, 800 x 768 x 768 (600 tiles) 9.9 / 7.8, 512 x 64 x 2048 (1024)
-    // 4.5 / 6.4, 1024^3 (1024) 11.9 / 11.5
+    // K-major B, few tiles: up to two of 32 x 32 per compute unit, three for longer contractions over whole tiles of 128 columns.  us,
+    // before / there: 256 x 1024 x 1024 11.7 / 4.6, 64 x 2048 x 4096 19.5 / 6.8, 128^3 4.8 / 2.9, 800 x 768 x 768 (600 tiles) 9.9 / 7.8,
+    // 512 x 64 x 2048 (1024) 4.5 / 6.4, 1024^3 (1024) 11.9 / 11.5; other columns, whose tiles of 64 x 64 are not half empty, 705 x 264 x 1032
+    // (759) 5.5 / 7.1 (162 such products 10 % slower there, 195 over whole tiles 17 % faster)
     const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32) * g.groups * NB;
-    if (tiles32 <= (K >= 256 ? 3 : 2) * (int64_t)cus) launch_few<true>(g, cus, bias_cast, s);
+    if (tiles32 <= (K >= 256 && BN == 128 ? 3 : 2) * (int64_t)cus) launch_few<true>(g, cus, bias_cast, s);
     else if (BN == 128 && g.groups == 1 && g.act[0] == nullptr && g.K >= 256 && tiles256 * 4 >= 3 * (int64_t)cus && tiles256 <= 2 * (int64_t)cus) {
         g.tiles_n_group = (int)((N + 255) / 256);
         g.total_tiles = (int)tiles256;
@@ -1126,11 +1127,26 @@ int try_matmul_f16_mfma(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, co
     // stores.  us, here / there: 500 x 2048 x 2048 20.1 / 12.6, 1024^3 12.1 / 8.0, 2048^3 30.0 / 25.5, 4096 x 768 x 3072 39.9 / 34.4,
     // 4096 x 1024 x 4096 57.5 / 56.2, 4096 x 2048 x 4096 88 / 100, 4096 x 3072 x 3072 104 / 103, 4096^3 139 / 171, 2048 x 8192 x
     // 2048 (64 tiles of 256) 93 / 84; 8192 x 32 x 64 3.2 / 3.5, 8192 x 128 x 64 3.8 / 3.9, 4096 x 64 x 64 3.3 / 3.2.
+    // Of 4000 such products the kernels here are faster for (mean time there, of here)
+    // - at most 32 rows, K below 512, up to two tiles of 64 x 64 per unit, eight for K up to 128, or 32 columns, 24 for K up to 72, up to
+    //   five tiles: 1.2 (9 x 2 x 72 x 2416 3.5 us here, 4.9 there, 23 x 2576 x 88 x 8 4.5, 8.3)
+    // - N whose last 64 columns a tile of 128 would leave empty and a K of no whole steps, up to a tile of 64 x 64 per unit, or one and a
+    //   half beyond K = 72: 1.06 (705 x 264 x 1032 5.2, 6.9)
+    // - other N, less than a round of tiles of 128 x 128 on five eighths of the units or more from K = 768 on, four fifths from 400: 1.15
+    //   (3356 x 1928 x 1112 30.1, 43.4)
+    // - up to an eighth more tiles of 128 x 128 than units, beyond a short K: 1.04 (22 x 183 x 56 x 672 6.9, 9.0)
+    // and the others, on average, slower: 0.88
     if (!bias_cast && !g.b_rows) {
         const int64_t cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
         const auto tiles = [&](int64_t t) { return ((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.batches; };
         const bool large = tiles(256) * 2 >= cus && g.K * std::min(tiles(256), cus) >= 2048 * cus;
-        if (tiles(32) > 2 * cus && !large && !(g.N <= 64 && g.K <= 128 && g.M >= 8192)) {
+        const bool wide = (g.N + 127) / 128 * 128 <= (g.N + 63) / 64 * 64;  // (launch_args' condition for 128 columns)
+        const bool thin = g.M <= 32 ? g.K < 512 && tiles(64) <= (g.K <= 128 ? 8 : 2) * cus : g.N <= (g.K > 72 ? 32 : 24) && tiles(64) <= 5 * cus;
+        const bool narrow = !wide && g.K % 64 != 0 && tiles(64) * 2 <= (g.K > 72 ? 3 : 2) * cus;
+        const bool round = wide && g.M > 64 && tiles(128) * 8 >= 5 * cus && tiles(128) < cus && g.K >= (tiles(128) * 5 >= 4 * cus ? 400 : 768);
+        const bool second = g.K > (wide ? 128 : 32) && g.M > 64 && g.N > 64 && tiles(128) > cus && tiles(128) * 8 <= 9 * cus;
+        const bool here = large || thin || narrow || round || second || (g.N <= 64 && g.K <= 128 && g.M >= 8192);
+        if (tiles(32) > 2 * cus && !here) {
             const int there = try_matmul_float(ctx, s, out, a, b, attr, nullptr, false, true);
             if (there != 0) return there;
         }

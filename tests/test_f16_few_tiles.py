@@ -19,7 +19,9 @@ CASES = [
     (1, 100, 1536, 264),                       # whole stages, one tile per unit
     (1, 200, 416, 1192), (5, 197, 64, 200),    # two tiles per unit
     (1, 600, 288, 1000),                       # K-major: three tiles per unit; row-wise: 64 x 64, steps of 32
-    (1, 1000, 320, 712),                       # row-wise: 64 x 64, steps of 64; K-major: 64 x 64 with the bias
+    (1, 1000, 320, 712),                       # row-wise: 64 x 64, steps of 64; K-major: three tiles per unit
+    # K-major products that keep to gemm_f16.hip's tiles: few rows, few columns, half of 128 columns, a round of 128 x 128, a little more
+    (9, 3, 32, 2048), (13, 1300, 96, 16), (1, 705, 288, 1032), (1, 1300, 768, 1920), (1, 2500, 160, 1664),
     (1, 1030, 1088, 1048),                     # K-major MATMUL of long rows without shared K
     (1, 2050, 320, 2056),                      # K-major: 128 x 128
 ]
