@@ -525,6 +525,9 @@ int try_conv_few_i8(mlel_ctx *ctx, hipStream_t s, const mlel_tensor *out, const 
     // 4.9, 60 x 60 x 50 -> 100 (452) 8.3 / 7.8, 50 x 50 x 100 -> 170 (474) 10.0 / 7.6; 100 x 100 x 10 -> 20 (313) 5.5 / 5.8, 70 x 70 x 18 ->
     // 64, 5 x 5 (308) 9.2 / 9.5: beyond one tile per unit not where the pieces are more than half as much again as the channels
     if (g.ragged && !small && tiles(32) > cus && (tiles(32) > 2 * cus || 3 * IC < 2 * 16 * ppt)) return 0;
+    // nor where large kernels of a few channels are mostly padding, from a tile of 16 per unit on: 7 x 35 x 3 -> 144 four times, 7 x 7
+    // (558) 5.4 / 7.5, 8 x 248 of 1 channel eleven times (464) 5.5 / 7.6; 18 of 1200 random sizes, on average 14 % longer here
+    if (g.ragged && 2 * IC < 16 * ppt && K - taps * IC > 350 && tiles(16) > cus) return 0;
     g.x = static_cast<const int8_t *>(in->ptr), g.w = static_cast<const int8_t *>(w->ptr);
     g.x2 = in2 != nullptr ? static_cast<const int8_t *>(in2->ptr) : g.x;
     g.out = static_cast<int8_t *>(out->ptr), g.bias = static_cast<const int32_t *>(bias->ptr), g.bias_len = (int)bias->dims[0];

@@ -42,6 +42,8 @@ CASES = [
     (1, 12, 11, 44, 64, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), -128, True),
     (1, 50, 60, 37, 70, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), -7, True),       # tiles of 32
     (1, 61, 63, 25, 100, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 4, False),      # tiles of 32, two per unit
+    (4, 7, 35, 3, 144, (7, 7), (1, 1), (1, 1), (3, 3, 3, 3), -5, True),        # mostly padding: the kernel of image pieces
+    (1, 9, 11, 3, 144, (7, 7), (1, 1), (1, 1), (3, 3, 3, 3), -5, True),        # the same, a tile of 16 per unit at most
 ]
 
 
