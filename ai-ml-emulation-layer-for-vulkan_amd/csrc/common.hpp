@@ -55,6 +55,37 @@ __device__ __forceinline__ int div_magic(int n, const DivMagic &d) {
     return (int)(((uint64_t)(uint32_t)n * d.m) >> (31 + d.s));
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// buffer resources, and loads straight into shared memory
+// ---------------------------------------------------------------------------------------------------------------
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ v4i rsrc_words(const void *p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
+}
+// One wavefront-wide 16-byte-per-lane load from a buffer resource straight into LDS at `lds_addr` + 16 * lane; a lane whose
+// offset lies beyond the resource's extent leaves zeros.  Written as inline assembly on purpose: the compiler orders every LDS
+// read after ALL outstanding loads of this kind (it cannot tell which bytes they write), which would drain the whole stage ring
+// at every step; the loops do their own counting with s_waitcnt vmcnt(N).  M0 holds the LDS address for this one instruction
+// only; nothing else in these kernels keeps a value in M0.
+__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res),
+                 "s"(scalar_offset)
+                 : "memory");
+}
+// the same from an address
+__device__ __forceinline__ void load16_to_lds(const void *from, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(from) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {  // s_waitcnt vmcnt(N) only (expcnt / lgkmcnt untouched)
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
 // The order in which the tiles of a product are dealt out.  Block b runs on XCD b % 8 and takes tile (b % 8) * chunk + b / 8, so
 // an XCD, whose L2 the others cannot use, works on `chunk` consecutive tiles.  They run in bands of `rows` tile rows, column
 // by column inside a band: one row per band is row by row, all of them column by column.  The height is the one whose

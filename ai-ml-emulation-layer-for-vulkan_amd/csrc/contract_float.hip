@@ -31,7 +31,6 @@ typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) v4s lds_v4s;
@@ -85,13 +84,6 @@ struct FArgs {
     float clamp_lo, clamp_hi;
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ v4i rsrc_words(const void *p, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
-}
 __device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const v4i v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
     return make_uint4((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w);
@@ -111,17 +103,6 @@ template <int SIZE>
 __device__ __forceinline__ uint32_t load_elem(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     if constexpr (SIZE == 2) return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0);
     else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
-}
-// one wavefront-wide 16-byte-per-lane load straight into shared memory at lds_addr + 16 * lane; a lane whose offset lies
-// beyond the resource's extent leaves zeros.  The loop counts these loads itself (s_waitcnt vmcnt(N)).
-__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res),
-                 "s"(scalar_offset)
-                 : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
 // 16 x 16: the same over four pieces

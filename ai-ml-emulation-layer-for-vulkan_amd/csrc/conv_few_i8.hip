@@ -27,7 +27,6 @@
 namespace mlel {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kOob = 0x80000000u;
@@ -67,27 +66,6 @@ struct FewArgs {
     int32_t ragged;  // (for the launch) pieces at any address
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ v4i rsrc_words(const void *p, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
-}
-// one wavefront-wide load of 16 bytes per lane straight into shared memory at lds_addr + 16 * lane: from an offset of a
-// resource (zeros beyond its extent), or from an address.  The loop counts these loads itself (s_waitcnt vmcnt(N)).
-__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset), "s"(res),
-                 "s"(scalar_offset)
-                 : "memory");
-}
-__device__ __forceinline__ void load16_to_lds(const void *from, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(from) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
 __device__ __forceinline__ v16i multiply(v4i w, v4i x, v16i acc) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(w, x, acc, 0, 0, 0); }
 __device__ __forceinline__ v4i multiply(v4i w, v4i x, v4i acc) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, x, acc, 0, 0, 0); }
 

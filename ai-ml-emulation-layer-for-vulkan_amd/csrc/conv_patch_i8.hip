@@ -34,7 +34,6 @@
 namespace mlel {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kBlock = 256;

@@ -27,7 +27,6 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4s lds_v4s;
 
 constexpr uint32_t kOob = 0x80000000u;
@@ -89,31 +88,11 @@ struct HProduct {
     uint32_t vs_m1, vs_m2, vs_n1, vs_n2;
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
-}
 __device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const v4i v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
     return make_uint4((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w);
 }
 
-// One wavefront-wide 16-byte-per-lane load from a buffer resource straight into LDS at `lds_addr` + 16 * lane.
-// Inline assembly on purpose: the compiler orders every LDS read after ALL outstanding loads of this kind (it cannot
-// tell which bytes they write), which would drain the stage ring at every step; the loop does its own counting with
-// s_waitcnt vmcnt(N).  M0 holds the LDS address for this one instruction only.
-__device__ __forceinline__ void load16_to_lds(v4i res, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset),
-                 "s"(res), "s"(scalar_offset)
-                 : "memory");
-}
-__device__ __forceinline__ v4i rsrc_words(const void *p, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {  // s_waitcnt vmcnt(N) only (expcnt / lgkmcnt untouched)
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
 
 // Division of the row and column indices of a view by its inner extents, once per 16-byte piece: the extents are the
 // same for every piece, so the quotient is one multiplication by floor((2^32 - 1) / d) + 1 (exact while x * d < 2^32,

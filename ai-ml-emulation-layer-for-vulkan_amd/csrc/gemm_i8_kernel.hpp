@@ -29,7 +29,6 @@
 namespace mlel {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i lds_v2i;
@@ -265,25 +264,6 @@ template <int BM, int BN>
 constexpr int dl_stages() {
     return 4;
 }
-// One wavefront-wide 16-byte-per-lane load from a buffer resource straight into LDS at `lds_addr` + 16 * lane.
-// Written as inline assembly on purpose: the compiler orders every LDS read after ALL outstanding loads of this kind
-// (it cannot tell which bytes they write), which would drain the whole stage ring at every step; the loop below does
-// its own counting with s_waitcnt vmcnt(N).  M0 holds the LDS address for this one instruction only; nothing else
-// in these kernels keeps a value in M0.
-__device__ __forceinline__ void load16_to_lds(v4i rsrc, uint32_t lds_addr, uint32_t offset, uint32_t scalar_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(offset),
-                 "s"(rsrc), "s"(scalar_offset)
-                 : "memory");
-}
-__device__ __forceinline__ v4i make_rsrc_words(const void *p, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, 0x00020000};
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {  // s_waitcnt vmcnt(N) only (expcnt / lgkmcnt untouched)
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 template <int BM, int BN, int WAVES_M, int WAVES_N, int XMODE, int WMODE, bool SUMS, bool Q8, bool RES = false>
 __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) gemm_i8_kernel(const GemmArgs g) {
     static_assert(!RES || Q8, "the residual stage follows the 8-bit epilogue");
@@ -639,7 +619,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) gemm_i8_kernel(const Ge
                 wo[i] = n < g.N ? (uint32_t)kr * (uint32_t)g.ldw + (uint32_t)n : kOobOffset;
             }
         }
-        const v4i xres4 = make_rsrc_words(xb, g.x_bytes), wres4 = make_rsrc_words(wb, g.w_bytes);
+        const v4i xres4 = rsrc_words(xb, g.x_bytes), wres4 = rsrc_words(wb, g.w_bytes);
         const uint32_t lds0 = (uint32_t) reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem) +
                               (uint32_t)(wave_u * 1024);
         const uint32_t w_kstep = WMODE == W_ROWS_DL ? (uint32_t)BK : (uint32_t)BK * (uint32_t)g.ldw;
